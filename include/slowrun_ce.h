@@ -184,7 +184,7 @@ int sce_forward(const sce_args* args);
  * allocate: code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  The call allocates
  * nothing and frees nothing; args->workspace and args->workspace_bytes are ignored, every other field means what it
  * means to sce_forward, and the results are the same bits.  Limit: ceil(N / 256) * 256 * S <= 524288, S the number of
- * vocabulary splits (8 to 16; 8 at N = 65536, V = 50304), else SCE_EINVAL with a message.  All calls on one device
+ * vocabulary splits (8 to 16, 8 at N = 65536, V = 50304; more where N <= 3840, which always fits), else SCE_EINVAL with a message.  All calls on one device
  * share the one array: calls that overlap in time on the same device (two streams, two threads) race. */
 int sce_forward_noalloc(const sce_args* args);
 

@@ -488,7 +488,7 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
   }
 }
 
-// What a block of 256 rows contributes to the mean loss: left by fwd_combine_kernel in the first 16 bytes of the
+// What a block of COMBINE_ROWS rows contributes to the mean loss: left by fwd_combine_kernel in the first 16 bytes of the
 // block's own rows of the partial records (which it has consumed by then), summed by fwd_reduce_kernel.
 struct BlockLoss {
   double sum;      // sum of lse_i - z[i, y_i] over the valid rows
@@ -497,62 +497,93 @@ struct BlockLoss {
 };
 static_assert(sizeof(BlockLoss) == 16, "one float4 slot");
 
-// one thread per row: fold the V-splits, write lse / loss / argmax and the saved row statistics
-__global__ __launch_bounds__(256) void fwd_combine_kernel(float4* __restrict__ partials, int S, int N, int Np, int V,
+// Folds the V-splits of a row and writes lse / loss / argmax and the saved row statistics: COMBINE_ROWS rows to a
+// workgroup, one wave to every G-th split (its 64 rows' records are 1 KB in a row), four records in flight per lane.
+// What bounds it is the chain of loads, not their volume: with one thread per row the records of a call of 61 rows and
+// 197 splits were 197 loads of one workgroup.  G = 4 for up to 16 splits, 16 beyond (rows too few to fill the chip
+// without cutting the vocabulary finer); the order of the sums depends on G alone.
+constexpr int COMBINE_ROWS = 64;
+template <int G>
+__global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* __restrict__ partials, int S, int N, int Np, int V,
                                                          const int64_t* __restrict__ targets, int64_t ignore_index, float cap,
                                                          const float* __restrict__ mtp_weights, int n_predict,
-                                                         float* __restrict__ s_lse, float* __restrict__ s_umax,
-                                                         float* __restrict__ s_zy, float* __restrict__ losses,
+                                                         float* __restrict__ s_lse, float* __restrict__ s_zy, float* __restrict__ losses,
                                                          float* __restrict__ lse_out, int32_t* __restrict__ argmax_out) {
-  __shared__ double ssum[256];
-  __shared__ int scnt[256], sbad[256];
-  const int t = threadIdx.x, i = blockIdx.x * 256 + t;      // the grid covers Np = 256 * gridDim.x rows exactly
-  double term = 0.0;
-  int cnt = 0, bad = 0;
-  if (i >= N) {
-    s_lse[i] = 0.f; s_umax[i] = 0.f;
-    for (int k = 0; k < n_predict; ++k) s_zy[(int64_t)k * Np + i] = 0.f;
-  } else {
+  static_assert(G >= 4, "one wave per prediction offset");
+  __shared__ float rsum[G][COMBINE_ROWS], rmax[G][COMBINE_ROWS], rl[4][COMBINE_ROWS];
+  __shared__ int rarg[G][COMBINE_ROWS];
+  const int r = threadIdx.x & 63, g = threadIdx.x >> 6, i = blockIdx.x * COMBINE_ROWS + r;      // the grid covers Np rows exactly
+  {
     float sum = 0.f, umax = -INFINITY;
     int uarg = 0x7fffffff;
-    for (int s = 0; s < S; ++s) {
-      const float4 o = partials[(int64_t)s * Np + i];
-      const int ua = __float_as_int(o.z);
-      sum += o.x;
-      if (o.y > umax || (o.y == umax && ua < uarg)) { umax = o.y; uarg = ua; }
-    }
-    const float lse = cap + logf(sum);
-    s_lse[i] = lse; s_umax[i] = umax;
-    // the forward kernel left the raw logit at each target that takes part: z_y = cap tanh(u_y / cap) replaces it (0 for the others);
-    // loss_i = sum_k w_k (lse_i - z[i, y_{i+k}]) over the offsets that take part (tiny/cuda_kernels.py:226-240)
-    float l = 0.f;
-    for (int k = 0; k < n_predict; ++k) {
-      float zy = 0.f;
-      if (target_valid(targets, ignore_index, i + k, N, V)) {
-        zy = cap * tanhf(s_zy[(int64_t)k * Np + i] / cap);
-        l += (mtp_weights ? mtp_weights[k] : 1.0f) * (lse - zy);
+    for (int s0 = g; s0 < S; s0 += 4 * G) {
+      float4 o[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int s = s0 + q * G;
+        o[q] = s < S ? partials[(int64_t)s * Np + i] : make_float4(0.f, -INFINITY, __int_as_float(0x7fffffff), 0.f);
       }
-      s_zy[(int64_t)k * Np + i] = zy;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int ua = __float_as_int(o[q].z);
+        sum += o[q].x;
+        if (o[q].y > umax || (o[q].y == umax && ua < uarg)) { umax = o[q].y; uarg = ua; }
+      }
     }
-    if (losses) losses[i] = l;
-    if (lse_out) lse_out[i] = lse;
-    if (argmax_out) argmax_out[i] = (uarg == 0x7fffffff) ? 0 : uarg;
-    const int64_t y = targets[i];
-    if (y != ignore_index) {
-      if (y < 0 || y >= V) bad = 1;
-      else { term = (double)(lse - s_zy[i]); cnt = 1; }
+    rsum[g][r] = sum; rmax[g][r] = umax; rarg[g][r] = uarg;
+  }
+  __syncthreads();               // also: every wave of this block has read its partial records
+  float lse = 0.f;
+  if (g < n_predict && i < N) {
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < G; ++q) sum += rsum[q][r];
+    lse = cap + logf(sum);
+  }
+  // one wave per offset: the raw logit at each target that takes part is there; z_y = cap tanh(u_y / cap) replaces it (0 for the
+  // others); loss_i = sum_k w_k (lse_i - z[i, y_{i+k}]) over the offsets that take part (tiny/cuda_kernels.py:226-240)
+  if (g < n_predict) {
+    float zy = 0.f, l = 0.f;
+    if (i < N && target_valid(targets, ignore_index, i + g, N, V)) {
+      zy = cap * tanhf(s_zy[(int64_t)g * Np + i] / cap);
+      l = (mtp_weights ? mtp_weights[g] : 1.0f) * (lse - zy);
+    }
+    s_zy[(int64_t)g * Np + i] = zy;
+    rl[g][r] = l;
+    if (g == 0) {
+      double term = 0.0;
+      int cnt = 0, bad = 0;
+      s_lse[i] = lse;
+      if (i < N) {
+        if (lse_out) lse_out[i] = lse;
+        if (argmax_out) {
+          float umax = -INFINITY;
+          int uarg = 0x7fffffff;
+          for (int q = 0; q < G; ++q)
+            if (rmax[q][r] > umax || (rmax[q][r] == umax && rarg[q][r] < uarg)) { umax = rmax[q][r]; uarg = rarg[q][r]; }
+          argmax_out[i] = (uarg == 0x7fffffff) ? 0 : uarg;
+        }
+        const int64_t y = targets[i];
+        if (y != ignore_index) {
+          if (y < 0 || y >= V) bad = 1;
+          else { term = (double)(lse - zy); cnt = 1; }
+        }
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) { term += __shfl_xor(term, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
+      if (r == 0) {
+        BlockLoss bl;
+        bl.sum = term; bl.cnt = cnt; bl.bad = bad;
+        *reinterpret_cast<BlockLoss*>(partials + (int64_t)blockIdx.x * COMBINE_ROWS) = bl;
+      }
     }
   }
-  ssum[t] = term; scnt[t] = cnt; sbad[t] = bad;
-  __syncthreads();               // also: every row of this block has read its partial records
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) { ssum[t] += ssum[t + w]; scnt[t] += scnt[t + w]; sbad[t] += sbad[t + w]; }
-    __syncthreads();
-  }
-  if (t == 0) {
-    BlockLoss bl;
-    bl.sum = ssum[0]; bl.cnt = scnt[0]; bl.bad = sbad[0];
-    *reinterpret_cast<BlockLoss*>(partials + (int64_t)blockIdx.x * 256) = bl;
+  if (!losses) return;
+  __syncthreads();
+  if (g == 0 && i < N) {
+    float l = rl[0][r];
+    for (int k = 1; k < n_predict; ++k) l += rl[k][r];
+    losses[i] = l;
   }
 }
 
@@ -580,7 +611,7 @@ __global__ __launch_bounds__(1024) void fwd_reduce_kernel(const float4* __restri
   double acc = 0.0;
   int cnt = 0, bad = 0;
   for (int b = t; b < nblk; b += 1024) {
-    const BlockLoss bl = *reinterpret_cast<const BlockLoss*>(partials + (int64_t)b * 256);
+    const BlockLoss bl = *reinterpret_cast<const BlockLoss*>(partials + (int64_t)b * COMBINE_ROWS);
     acc += bl.sum; cnt += bl.cnt; bad += bl.bad;
   }
   ssum[t] = acc; scnt[t] = cnt; sbad[t] = bad;

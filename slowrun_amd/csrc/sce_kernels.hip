@@ -84,7 +84,8 @@ static std::mutex g_mu;
 static std::atomic<int64_t> g_gather_limit{(int64_t)1 << 32};   // see sce_test_set_gather_limit
 static int g_arch_ok[64];   // 0 unknown, 1 gfx950, -1 other
 static void* g_scratch[64]; // device address of `scratch` on each device, filled with g_arch_ok
-static int g_cus[64];       // compute units, filled with g_arch_ok
+constexpr int MAX_CUS = 256;       // of a gfx950 device
+static int g_cus[64];       // compute units (at most MAX_CUS counted), filled with g_arch_ok
 static inline int device_cus_or_default(int dev) { return (dev >= 0 && dev < 64 && g_cus[dev] > 0) ? g_cus[dev] : 256; }
 
 // Optional per-kernel timing with HIP events on the caller's stream (off by default).
@@ -158,7 +159,7 @@ static int check_device(int dev) {
       void* sp = nullptr;
       HIP_TRY(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));       // this device's copy of the array
       g_scratch[dev] = sp;
-      g_cus[dev] = prop.multiProcessorCount;
+      g_cus[dev] = std::min(prop.multiProcessorCount, MAX_CUS);
       g_arch_ok[dev] = 1;
     }
   }
@@ -309,15 +310,22 @@ extern "C" const char* sce_last_error(void) { return g_err; }
 
 // Forward splits V among S workgroups per row tile (each walks CT / S column tiles).  8 keeps the partial records
 // small and gives every workgroup a long walk; more (up to 16) only where 8 would leave the last round of
-// workgroups, one per CU, mostly empty.
+// workgroups, one per CU, mostly empty.  With fewer than 16 row tiles even 16 splits leave CUs without a workgroup: then as
+// many as there are CUs, down to one column tile to a workgroup.  Measured: N = 2048 (8 row tiles), d = 768, V = 50304
+// forward 221 us with 16 splits (128 workgroups), 135 us with 32; N = 61, d = 2560, bf16 operands 800 us with 16, 85 us with 197.
 constexpr int FWD_MAX_SPLITS = 16;
 static int fwd_splits(int RT, int CT, int ncu) {
+  if (RT * FWD_MAX_SPLITS < ncu) return std::min(CT, ncu / RT);
   if (CT <= 8) return CT;
   auto fill = [&](int S) { const int64_t wg = (int64_t)RT * S; return (double)wg / (double)((wg + ncu - 1) / ncu * ncu); };
   int best = 8;
   for (int S = 9; S <= FWD_MAX_SPLITS && S <= CT; ++S)
     if (fill(S) > fill(best) + 0.03) best = S;
   return best;
+}
+// partial records of a forward pass: enough for any device (fwd_splits makes no more than MAX_CUS workgroups beyond 16 splits)
+static size_t fwd_workspace(int64_t Np) {
+  return (size_t)std::max<int64_t>(FWD_MAX_SPLITS * Np, (int64_t)MAX_CUS * 256) * 16 + 256;
 }
 
 extern "C" int sce_sizes_for(const sce_shape* shape, sce_sizes* out) {
@@ -327,7 +335,7 @@ extern "C" int sce_sizes_for(const sce_shape* shape, sce_sizes* out) {
   out->saved_bytes = S.total;
   out->saved_x_bytes = S.x_total;
   out->wcache_bytes = S.w_total;
-  out->fwd_workspace_bytes = (size_t)FWD_MAX_SPLITS * S.Np * 16 + 256;
+  out->fwd_workspace_bytes = fwd_workspace(S.Np);
   out->bwd_workspace_min_bytes = bwd_layout(S, 256, 256, 1, shape->n_predict).total;
   out->bwd_panel_rows = default_panel(S);
   {
@@ -514,7 +522,7 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   p.sc = bf16ops ? 1.0f : (float)a->x_s * (float)a->w_s; p.k1 = p.sc * 2.0f * LOG2E / a->cap; p.c2 = -2.0f * a->cap * LOG2E; p.ic2 = 1.0f / p.c2; p.em2cap = expf(-2.0f * a->cap);
   p.dc = bf16ops ? nullptr : dcp;
   p.want_argmax = a->argmax != nullptr;
-  const int grid = 8 * nsplit * ((RT + 7) / 8);
+  const int grid = map_tile_grid(RT, nsplit);
   // An fp8 forward pass has its target logits computed ahead of the forward kernel (from a tile of gathered rows of W_q^T,
   // together with the rows' boosts when it emits the dlogits) as long as that tile's 32-bit offsets reach every row of
   // W_q^T; beyond, the forward kernel takes them out of its own accumulators, as the bf16 forward pass does.
@@ -542,12 +550,15 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   }
   KernelTimer tm_red(SCE_K_FWD_REDUCE, st);
   float* s_lse = (float*)(sv + S.off_lse);
-  float* s_umax = (float*)(sv + S.off_umax);
   float* s_zy = (float*)(sv + S.off_zy);
-  fwd_combine_kernel<<<(int)(S.Np / 256), 256, 0, st>>>(p.partials, nsplit, (int)N, (int)S.Np, (int)Vl, a->targets, a->ignore_index,
-                                                       a->cap, a->mtp_weights, a->shape.n_predict, s_lse, s_umax, s_zy, a->losses, a->lse,
-                                                       a->argmax);
-  fwd_reduce_kernel<<<1, 1024, 0, st>>>(p.partials, (int)(S.Np / 256), (int32_t*)(sv + S.off_hdr),
+  const int nblk = (int)(S.Np / COMBINE_ROWS);
+  auto combine = [&](auto kernel, int g) {
+    kernel<<<nblk, COMBINE_ROWS * g, 0, st>>>(p.partials, nsplit, (int)N, (int)S.Np, (int)Vl, a->targets, a->ignore_index, a->cap, a->mtp_weights,
+                                             a->shape.n_predict, s_lse, s_zy, a->losses, a->lse, a->argmax);
+  };
+  if (nsplit <= 16) combine(fwd_combine_kernel<4>, 4);
+  else combine(fwd_combine_kernel<16>, 16);
+  fwd_reduce_kernel<<<1, 1024, 0, st>>>(p.partials, nblk, (int32_t*)(sv + S.off_hdr),
                                         a->reduction == SCE_REDUCE_MEAN ? a->loss : nullptr, a->n_valid,
                                         call_mode(emit, (int)Vl, a->shape.n_predict, a->cap));
   HIP_TRY(hipGetLastError());
@@ -933,7 +944,7 @@ extern "C" int sce_bench_floor(const sce_args* a, int32_t which, int32_t reps, v
   const uint32_t* gexp = (const uint32_t*)(sv + S.total + S.rel_gexp);
   const int RT = (int)(S.Np / 256), CTv = (int)(S.Vp / 256), CTd = (int)(S.dq / 256);
   const int nsplit = fwd_splits(RT, CTv, device_cus_or_default(a->device));
-  const int fgrid = 8 * nsplit * ((RT + 7) / 8);
+  const int fgrid = map_tile_grid(RT, nsplit);
   int maxgrid = std::max(fgrid, std::max(map_tile_grid((int)(P / 256), CTd), map_tile_rr_grid(CTd, CTv)));
   const size_t need = (size_t)maxgrid * 256 * 4 + 2 * 1024 * sizeof(long long);
   if (scratch_bytes < need) return fail(SCE_EINVAL, "scratch too small: %zu < %zu", scratch_bytes, need);
