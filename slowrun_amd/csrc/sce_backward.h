@@ -23,9 +23,12 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
                                                       const float* __restrict__ mtp_weights, int n_predict,
                                                       float cap, int N, int Np, int V, const float* __restrict__ lam,
                                                       float* __restrict__ rho, float* __restrict__ hcoef,
-                                                      float* __restrict__ blockmax, int32_t* __restrict__ rowinfo, CallMode mode) {
+                                                      float* __restrict__ blockmax, int32_t* __restrict__ rowinfo, CallMode mode,
+                                                      int32_t key_none, int32_t* __restrict__ keys, int32_t* __restrict__ vals,
+                                                      int32_t* __restrict__ longlist) {
   __shared__ float smax[256];
   const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i == 0) longlist[0] = 0;        // counter of the long-column list, filled by bwd_segments_kernel
   float r = 0.f;
   float h[4] = {0.f, 0.f, 0.f, 0.f};
   // the forward call that wrote `saved` was asked for something else (kept dlogits, vocabulary limit, offsets, cap):
@@ -56,6 +59,12 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
       if (!ok[k]) continue;
       yk[k] = targets[i + k];
       sw += mtp_weights ? mtp_weights[k] : 1.0f;
+    }
+    // sort keys of the rows grouped by target: one entry per (offset k, row i): key = target y_{i+k} (key_none if the pair
+    // takes no part), value = entry id k * Np + i
+    for (int k = 0; k < n_predict; ++k) {
+      keys[(int64_t)k * N + i] = ok[k] ? (int32_t)yk[k] : key_none;
+      vals[(int64_t)k * N + i] = k * Np + i;
     }
     if (ok[0] || ok[1] || ok[2] || ok[3]) {
       const float lse = s_lse[i];
@@ -91,34 +100,33 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
   if (threadIdx.x == 0) blockmax[blockIdx.x] = smax[0];
 }
 
-__global__ __launch_bounds__(1024) void bwd_xi_kernel(const float* __restrict__ blockmax, int n, float* __restrict__ xi) {
-  __shared__ float smax[1024];
-  float m = 0.f;
-  for (int i = threadIdx.x; i < n; i += 1024) m = fmaxf(m, blockmax[i]);
-  smax[threadIdx.x] = m;
-  __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
-    if (threadIdx.x < w) smax[threadIdx.x] = fmaxf(smax[threadIdx.x], smax[threadIdx.x + w]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) xi[0] = (smax[0] > 0.f && isfinite(smax[0])) ? smax[0] : 1.0f;
-}
-
 // Xt (blocked, dq rows, K = Np) = e4m3( X_q[i][j] * rho_i / xi ), transposed through LDS in 128 x 128 tiles: a row of
 // the tile is one whole 128-byte line of the blocked layout on the way out, and 128 bytes of an X_q row on the way in.
+// xi, the largest |rho|, is folded from bwd_prep_kernel's block maxima by every workgroup for itself (one load a thread at
+// N = 65536, from L2, beside the loads of the tile): a launch of one workgroup for it was 4.7 us of every backward call.
 constexpr int XT_TILE = 128;
 __global__ __launch_bounds__(256) void bwd_xt_kernel(const uint8_t* __restrict__ xq, int64_t dp, int64_t ldx, int64_t kbn,
-                                                    const float* __restrict__ rho, const float* __restrict__ xi,
-                                                    uint8_t* __restrict__ xt) {
+                                                    const float* __restrict__ rho, const float* __restrict__ blockmax, int nblk,
+                                                    float* __restrict__ xi_out, uint8_t* __restrict__ xt) {
   __shared__ uint8_t tile[XT_TILE][XT_TILE + 4];
+  __shared__ float wmax[4];
   const int t = threadIdx.x;
+  float xi = 0.f;
+  for (int n = t; n < nblk; n += 256) xi = fmaxf(xi, blockmax[n]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) xi = fmaxf(xi, __shfl_xor(xi, o));
+  if ((t & 63) == 0) wmax[t >> 6] = xi;
+  __syncthreads();
+  xi = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+  xi = (xi > 0.f && isfinite(xi)) ? xi : 1.0f;
+  if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) xi_out[0] = xi;
   const int64_t i0 = (int64_t)blockIdx.x * XT_TILE, j0 = (int64_t)blockIdx.y * XT_TILE;
   if (j0 < dp) {
 #pragma unroll
     for (int pass = 0; pass < 4; ++pass) {
       const int r = (t >> 3) + 32 * pass, c = (t & 7) * 16;
       const v4i raw = *reinterpret_cast<const v4i*>(xq + (i0 + r) * ldx + j0 + c);
-      const float f = rho[i0 + r] / xi[0];
+      const float f = rho[i0 + r] / xi;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const uint32_t w = (uint32_t)raw[m];
@@ -635,31 +643,6 @@ __global__ __launch_bounds__(256) void bwd_dw_tail_kernel(DwParams p, DwTail tl)
       for (int r = 0; r < 16; ++r) dst0[(a * 32 + 8 * (r >> 2) + (r & 3)) * 256 + b * 32] = acc[a][b][r];
 }
 
-// sort keys: one entry per (offset k, row i): key = target y_{i+k} (V if the pair takes no part; targets at or
-// beyond the vocabulary limit Vl take no part),
-// value = entry id k * Np + i
-__global__ __launch_bounds__(256) void bwd_keys_kernel(const int64_t* __restrict__ targets, int64_t ignore_index, int N, int Np, int Vl,
-                                                      int V, int n_predict, int32_t* __restrict__ keys, int32_t* __restrict__ vals,
-                                                      int32_t* __restrict__ longlist) {
-  const int e = blockIdx.x * 256 + threadIdx.x;
-  if (e == 0) longlist[0] = 0;        // counter of the long-column list, filled later on the same stream
-  if (e >= N * n_predict) return;
-  const int k = e / N, i = e - k * N;
-  keys[e] = target_valid(targets, ignore_index, i + k, N, Vl) ? (int32_t)targets[i + k] : V;
-  vals[e] = k * Np + i;
-}
-
-// segoff[v] = first sorted position whose key >= v, v = 0..V+1
-__global__ __launch_bounds__(256) void bwd_segoff_kernel(const int32_t* __restrict__ skeys, int N, int V,
-                                                        int32_t* __restrict__ segoff) {
-  const int pos = blockIdx.x * 256 + threadIdx.x;
-  if (pos > N) return;
-  const int k = (pos < N) ? skeys[pos] : V + 1;
-  const int kprev = (pos > 0) ? skeys[pos - 1] : -1;
-  for (int v = kprev + 1; v <= k; ++v) segoff[v] = pos;
-}
-
-
 // A column that is the target of at least LONG_SEG rows has its segment of the sorted list cut into
 // nch = ceil(L / LONG_CHUNK) equal chunks (the last one may be shorter); chunk c starts at sorted
 // position s0 + c * ceil(L / nch).
@@ -668,14 +651,40 @@ __device__ __forceinline__ void long_chunks(int L, int& nch, int& len) {
   len = (L + nch - 1) / nch;
 }
 
-// List of (column, chunk) pairs of the long columns (order irrelevant: each pair is handled on its
-// own).  longlist[0] is the count, then two ints per pair; the position of a pair in the list is the slot of its
-// chunk sum, and longbase[v] is the position of column v's first pair.
-__global__ __launch_bounds__(256) void bwd_longlist_kernel(const int32_t* __restrict__ segoff, int V, int32_t* __restrict__ longlist,
-                                                          int32_t* __restrict__ longbase) {
-  const int v = blockIdx.x * 256 + threadIdx.x;
-  if (v >= V) return;
-  const int L = segoff[v + 1] - segoff[v];
+// From the sorted keys: segoff[v] = first position whose key is at least v, v = 0 .. V, and the list of (column, chunk)
+// pairs of the long columns (order irrelevant: each pair is handled on its own).  longlist[0] is the count, then two
+// ints per pair; the position of a pair in the list is the slot of its chunk sum, and longbase[v] is the position of
+// column v's first pair.  One column per thread, by bisection: first among every stride-th key (in LDS), then within one
+// stride.  (A thread per key that fills the gap up to the next key runs as long as the widest gap: with Zipf targets the
+// rare end of the vocabulary holds gaps of thousands of columns, and 2048 rows took 63 us; this takes 4.7.)
+__global__ __launch_bounds__(256) void bwd_segments_kernel(const int32_t* __restrict__ skeys, int n, int V, int32_t* __restrict__ segoff,
+                                                          int32_t* __restrict__ longlist, int32_t* __restrict__ longbase) {
+  __shared__ int32_t top[256], seg[257];
+  const int t = threadIdx.x, v0 = blockIdx.x * 256, stride = (n + 255) / 256;
+  top[t] = t * stride < n ? skeys[t * stride] : 0x7fffffff;
+  __syncthreads();
+  auto lower_bound = [&](int v) {
+    int lo = 0, hi = 256;              // top[lo - 1] < v <= top[hi]
+    while (lo < hi) {
+      const int m = (lo + hi) >> 1;
+      if (top[m] < v) lo = m + 1; else hi = m;
+    }
+    if (lo == 0) return 0;
+    int a = (lo - 1) * stride + 1, b = min(lo * stride, n);      // skeys[a - 1] < v; skeys[b] >= v or b = n
+    while (a < b) {
+      const int m = (a + b) >> 1;
+      if (skeys[m] < v) a = m + 1; else b = m;
+    }
+    return a;
+  };
+  seg[t] = lower_bound(v0 + t);
+  if (t == 255) seg[256] = lower_bound(v0 + 256);
+  __syncthreads();
+  const int v = v0 + t;
+  if (v > V) return;
+  segoff[v] = seg[t];
+  if (v == V) return;
+  const int L = seg[t + 1] - seg[t];
   if (L < LONG_SEG) return;
   int nch, len;
   long_chunks(L, nch, len);

@@ -684,22 +684,19 @@ extern "C" int sce_backward(const sce_args* a) {
   bwd_prep_kernel<<<nblk, 256, 0, st>>>(s_lse, s_zy, a->targets, a->ignore_index, hdr, a->grad_output,
                                         a->reduction == SCE_REDUCE_NONE ? 1 : 0, a->grad_scale, a->mtp_weights, K, a->cap, (int)N,
                                         (int)S.Np, (int)Vl, (const float*)(sv + S.off_lam), rho, hcoef, blockmax, kept ? nullptr : rowinfo,
-                                        call_mode(kept, (int)Vl, K, a->cap));
-  bwd_xi_kernel<<<1, 1024, 0, st>>>(blockmax, nblk, xi);
+                                        call_mode(kept, (int)Vl, K, a->cap), (int32_t)V, keys_in, vals_in, longlist);
   {
     dim3 g((unsigned)(S.Np / XT_TILE), (unsigned)(S.dq / XT_TILE));
-    bwd_xt_kernel<<<g, 256, 0, st>>>(xq, S.dp, S.ldx, S.Np / BK, rho, xi, xt);
+    bwd_xt_kernel<<<g, 256, 0, st>>>(xq, S.dp, S.ldx, S.Np / BK, rho, blockmax, nblk, xi, xt);
   }
   // rows grouped by target, for the one-hot part of dW
   {
-    bwd_keys_kernel<<<(int)((NE + 255) / 256), 256, 0, st>>>(a->targets, a->ignore_index, (int)N, (int)S.Np, (int)Vl, (int)V, K, keys_in, vals_in, longlist);
     int bits = 1;
     while ((1ll << bits) <= V) ++bits;
     size_t tmp = B.sorttmp_bytes;
     if (sce::sort_pairs(ws + B.off_sorttmp, &tmp, keys_in, skeys, vals_in, perm, (size_t)NE, bits, st) != 0)
     { delete tm_prep; return fail(SCE_EHIP, "radix sort of the targets failed"); }
-    bwd_segoff_kernel<<<(int)((NE + 256) / 256), 256, 0, st>>>(skeys, (int)NE, (int)V, segoff);
-    bwd_longlist_kernel<<<(int)((V + 255) / 256), 256, 0, st>>>(segoff, (int)V, longlist, longbase);
+    bwd_segments_kernel<<<(int)(V / 256 + 1), 256, 0, st>>>(skeys, (int)NE, (int)V, segoff, longlist, longbase);
   }
   delete tm_prep;
   const float sc = (float)a->x_s * (float)a->w_s, k1 = sc * 2.0f * LOG2E / a->cap, c2 = -2.0f * a->cap * LOG2E;
