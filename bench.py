@@ -18,7 +18,7 @@ sys.path.insert(0, ROOT)
 PEAK_FP8_TFLOPS = 5000.0        # MI355X dense fp8 MFMA, published
 
 PROFILE_KERNEL = {"fwd": "fwd_kernel", "recompute": "bwd_recompute_kernel", "dx": "bwd_dx_kernel<bf16_t, false>",
-                  "dw": "bwd_dw_kernel<false>"}
+                  "dw": "bwd_dw_out_kernel<bf16_t>"}
 
 
 def measured_traffic(workload, mode, kind):

@@ -657,10 +657,18 @@ __device__ __forceinline__ void long_chunks(int L, int& nch, int& len) {
 // column v's first pair.  One column per thread, by bisection: first among every stride-th key (in LDS), then within one
 // stride.  (A thread per key that fills the gap up to the next key runs as long as the widest gap: with Zipf targets the
 // rare end of the vocabulary holds gaps of thousands of columns, and 2048 rows took 63 us; this takes 4.7.)
-__global__ __launch_bounds__(256) void bwd_segments_kernel(const int32_t* __restrict__ skeys, int n, int V, int32_t* __restrict__ segoff,
-                                                          int32_t* __restrict__ longlist, int32_t* __restrict__ longbase) {
+// Also: row and coefficient of every sorted entry (srow, sh), so that the kernels that walk a segment load them side by
+// side instead of one behind the other.
+__global__ __launch_bounds__(256) void bwd_segments_kernel(const int32_t* __restrict__ skeys, const int32_t* __restrict__ perm,
+                                                          const float* __restrict__ hcoef, int n, int Np, int V, int32_t* __restrict__ segoff,
+                                                          int32_t* __restrict__ longlist, int32_t* __restrict__ longbase,
+                                                          int32_t* __restrict__ srow, float* __restrict__ sh) {
   __shared__ int32_t top[256], seg[257];
   const int t = threadIdx.x, v0 = blockIdx.x * 256, stride = (n + 255) / 256;
+  for (int q = v0 + t; q < n; q += gridDim.x * 256) {
+    const int e = perm[q];             // entry id k * Np + i
+    srow[q] = e % Np; sh[q] = hcoef[e];
+  }
   top[t] = t * stride < n ? skeys[t * stride] : 0x7fffffff;
   __syncthreads();
   auto lower_bound = [&](int v) {
@@ -694,26 +702,29 @@ __global__ __launch_bounds__(256) void bwd_segments_kernel(const int32_t* __rest
 }
 
 // One-hot part of dW for the long columns: longsum[slot][:] = sum over the chunk's rows of h_i X_q[i, :].
-// One workgroup per (chunk, block of 256 rows of dW); the rows of the chunk are split over 16
+// One workgroup per (chunk, block of 256 rows of dW) at a time -- the grid is a fixed one that walks the list, whose
+// length the host does not know; the rows of the chunk are split over 16
 // row-lanes (8 independent loads in flight each) and folded in a fixed order, so the result does
 // not depend on scheduling.
+constexpr int LONG_GRID = 1024;
 __global__ __launch_bounds__(256) void bwd_dw_long_kernel(const int32_t* __restrict__ longlist, const int32_t* __restrict__ segoff,
-                                                         const int32_t* __restrict__ perm, const float* __restrict__ hcoef,
-                                                         const uint8_t* __restrict__ xq, int64_t dp, int64_t ldx, int64_t dq, int Np,
+                                                         const int32_t* __restrict__ srow, const float* __restrict__ sh,
+                                                         const uint8_t* __restrict__ xq, int64_t ldx, int64_t dq,
                                                          float* __restrict__ longsum) {
   __shared__ float red[16][256];
-  if ((int)blockIdx.x >= longlist[0]) return;
-  const int v = longlist[1 + 2 * blockIdx.x], ch = longlist[2 + 2 * blockIdx.x];
-  int nch, len;
-  long_chunks(segoff[v + 1] - segoff[v], nch, len);
-  const int s0 = segoff[v] + ch * len;
-  const int L = (segoff[v + 1] - s0) < len ? (segoff[v + 1] - s0) : len;
-  const int t = threadIdx.x, c = t & 15, rl = t >> 4;
-  const int64_t jb = (int64_t)blockIdx.y * 256;
-  float a[16];
+  const int count = longlist[0];
+  for (int slot = blockIdx.x; slot < count; slot += gridDim.x) {
+    const int v = longlist[1 + 2 * slot], ch = longlist[2 + 2 * slot];
+    int nch, len;
+    const int seg0 = segoff[v], seg1 = segoff[v + 1];
+    long_chunks(seg1 - seg0, nch, len);
+    const int s0 = seg0 + ch * len;
+    const int L = (seg1 - s0) < len ? (seg1 - s0) : len;
+    const int t = threadIdx.x, c = t & 15, rl = t >> 4;
+    const int64_t jb = (int64_t)blockIdx.y * 256;
+    float a[16];
 #pragma unroll
-  for (int m = 0; m < 16; ++m) a[m] = 0.f;
-  if (jb + c * 16 < dp) {
+    for (int m = 0; m < 16; ++m) a[m] = 0.f;
     const uint8_t* xcol = xq + jb + c * 16;
     for (int n0 = rl; n0 < L; n0 += 16 * 8) {
       v4i raw[8];
@@ -721,9 +732,8 @@ __global__ __launch_bounds__(256) void bwd_dw_long_kernel(const int32_t* __restr
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
         const int n = n0 + 16 * u;
-        const int e = n < L ? perm[s0 + n] : -1;          // entry id k * Np + i
-        h[u] = e >= 0 ? hcoef[e] : 0.f;
-        raw[u] = *reinterpret_cast<const v4i*>(xcol + (int64_t)(e >= 0 ? e % Np : 0) * ldx);
+        h[u] = n < L ? sh[s0 + n] : 0.f;
+        raw[u] = *reinterpret_cast<const v4i*>(xcol + (int64_t)srow[n < L ? s0 + n : s0] * ldx);
       }
 #pragma unroll
       for (int u = 0; u < 8; ++u) {        // rows in ascending order within a row-lane
@@ -737,85 +747,292 @@ __global__ __launch_bounds__(256) void bwd_dw_long_kernel(const int32_t* __restr
         }
       }
     }
+#pragma unroll
+    for (int m = 0; m < 16; ++m) red[rl][c * 16 + m] = a[m];
+    __syncthreads();
+    float sfold = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sfold += red[k][t];
+    longsum[(int64_t)slot * dq + jb + t] = sfold;
+    __syncthreads();                       // `red` is written again for the next chunk
   }
-#pragma unroll
-  for (int m = 0; m < 16; ++m) red[rl][c * 16 + m] = a[m];
-  __syncthreads();
-  float sfold = 0.f;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) sfold += red[k][t];
-  longsum[(int64_t)blockIdx.x * dq + jb + t] = sfold;
 }
 
-// dW = x_s * ( xi * (sum of the dW partials) - sum over the target segment of h_i X_q[i, :] ), cast to the output
-// type; the segment sum is formed here for short segments and read from the chunk sums for long ones.  A thread
-// owns one column v and 16 consecutive rows j.
+// Where the one-hot part of dW comes from and where dW goes (bwd_dw_out_kernel, bwd_dw_final_kernel).
+struct DwOut {
+  void* dw;                    // [d][dw_ld], columns [0, V)
+  int64_t dw_ld;
+  const int32_t* segoff;       // entries [segoff[v], segoff[v + 1]) of the sorted list belong to column v
+  const int32_t* srow;         // row i of a sorted entry
+  const float* sh;             // its coefficient h
+  const uint8_t* xq;           // [Np], row stride ldx
+  const float* longsum;        // [slot][dq]: chunk sums of the long columns
+  const int32_t* longbase;     // first slot of a long column
+  const float* xi;
+  const DevConsts* dc;         // non-NULL: x_s comes from here
+  int64_t ldx, dq;
+  float x_s;
+  int d, V;
+};
+
+// dW straight from the main loop: dW = x_s (xi (X~^T G) - sum over the column's target entries of h_i X_q[i, :]), cast and
+// stored by the workgroup that has the tile in its accumulators.  Used whenever one launch covers all rows (N <= 131072, a
+// workspace of the default size).  What the separate pass over an fp32 partial cost was its traffic: 8 bytes an element
+// written and read again (1 GB at d = 2560, V = 50304) around 2 bytes of result, 65 us of a 560 us step at N = 2048,
+// d = 768 and 172 us at N = 30011, d = 2560, whatever the number of rows.
+//
+// The epilogue must not wait on memory: one wave per SIMD has nothing to hide a load behind (gathering the one-hot rows
+// with dependent loads was measured at +0.5 ms of a 20 ms step).  So the rows X_q[i] of the tile's target entries -- the
+// short columns' only; columns with LONG_SEG or more entries have their chunk sums ready -- go to LDS with direct loads:
+// before the main loop, into what the K slots and the block exponents leave free (about 100 entries of 256 bytes), if they
+// fit there -- most tiles of most batches do -- and otherwise into the K slots after it, as many row blocks at a time as
+// fit (a row block's 64 columns have at most 64 (LONG_SEG - 1) = 448 entries).  Each lane then walks the entries of its own
+// column.  A 16-byte chunk c of an entry's 256 bytes lies at position c ^ (entry & 15): the lanes of a wave read the same
+// columns j of neighbouring entries, which would all lie in the same banks.
+// On the way out a bf16 quadrant is turned in LDS, 32 columns x 64 rows at a time, by the transposing read, so that a lane
+// stores 16 bytes of one row of dW and a wave 64 consecutive bytes of 16 rows.
+constexpr int DWO_AUX = 2 * 260 * 4;                         // entry offsets and segment starts of the tile's 256 columns
+constexpr int DWO_STAGE_PITCH = 64 * 2 + 16, DWO_STAGE = 32 * DWO_STAGE_PITCH;      // per wave
+constexpr int DWO_GROUP = 480;                               // entries that the K slots hold (256 bytes of X_q, row and coefficient each)
+static_assert(DWO_GROUP * (256 + 8) <= SMEM_BYTES && DWO_GROUP >= 64 * (LONG_SEG - 1) && DWO_GROUP % 4 == 0, "a row block's entries must fit the K slots");
+constexpr int DWO_MAX_KT = 131072 / BK;
+static_assert(SMEM_MAX - SMEM_BYTES - 8 * DWO_MAX_KT - DWO_AUX >= 4 * DWO_STAGE, "no room for the staging tiles beside the K slots");
+
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restrict__ dwacc, int nparts, int64_t part_stride, int64_t Vp, const int32_t* __restrict__ segoff,
-                                                          const int32_t* __restrict__ perm, const float* __restrict__ hcoef,
-                                                          const uint8_t* __restrict__ xq, int64_t ldx, int Np, const float* __restrict__ xi,
-                                                          const float* __restrict__ longsum, const int32_t* __restrict__ longbase, int64_t dq,
-                                                          float x_s_host, const DevConsts* __restrict__ dc, int d, int V, T* __restrict__ dw, int64_t dw_ld,
-                                                          DwTail tl, int RT, int CT) {
-  const float x_s = dc ? dc->x_s : x_s_host;
-  const int t = threadIdx.x;
-  const int v = blockIdx.x * 64 + (t & 63);
-  const int j0 = blockIdx.y * 64 + (t >> 6) * 16;
-  if (v >= V || j0 >= d) return;
-  const float scale = x_s * xi[0];
-  float o[16];
-  // the block's 64 x 64 elements lie in one 256 x 256 tile: one of the K-split last round (see bwd_dw_tail_kernel)?
-  int tt = -1;
-  if (tl.tile0 >= 0) {
-    const int rt = blockIdx.y >> 2, ct = blockIdx.x >> 2, g8 = ct >> 3, gw = (CT - 8 * g8) < 8 ? (CT - 8 * g8) : 8;
-    tt = g8 * 8 * RT + rt * gw + (ct - 8 * g8) - tl.tile0;       // (tile_from_index the other way round)
+__global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  int rt, ct;
+  if (!map_tile_rr(blockIdx.x, p.RT, p.CT, rt, ct)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wa = wave >> 1, wb = wave & 1;
+  const int KT = p.KT;
+  uint32_t* lsc = reinterpret_cast<uint32_t*>(smem + SMEM_BYTES);            // block exponents of the K loop: [v half][K block]
+  int* ioff = reinterpret_cast<int*>(smem + SMEM_BYTES + 8 * KT);            // [257]: first short entry of column c, counted over the tile
+  int* spos = ioff + 260;                                                    // [257]: segoff of the tile's columns
+  uint8_t* area = reinterpret_cast<uint8_t*>(spos + 260);                    // the rest of LDS
+  const int room = ((SMEM_MAX - SMEM_BYTES - DWO_AUX - 8 * KT) / (256 + 8)) & ~3;
+  // entry q's row and coefficient; its 256 bytes of X_q (columns rt * 256 on) at x + q * 256
+  struct Item { int row; float h; };
+  auto load_rows = [&](const Item* items, int n, uint8_t* x) {
+    const int lane = lane_id();
+    const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)x);
+    for (int q0 = 4 * wave; q0 < n; q0 += 16) {              // one load: four entries; beyond the last one it is loaded again
+      const int q = q0 + (lane >> 4), c = (lane & 15) ^ (q & 15);
+      lds_direct_16_far(__builtin_amdgcn_readfirstlane(lds0 + q0 * 256), o.xq + (int64_t)items[q < n ? q : n - 1].row * o.ldx + rt * 256 + c * 16);
+    }
+  };
+  bool pre;
+  {
+    const int t = threadIdx.x, v = ct * 256 + t;
+    const int s0 = o.segoff[v < o.V ? v : o.V], s1 = o.segoff[v + 1 < o.V ? v + 1 : o.V];
+    for (int e = t; e < 2 * KT; e += NTHREADS) {
+      const int w = e >= KT, kb = e - w * KT;
+      lsc[e] = p.gexp[(int64_t)(2 * ct + w) * p.kbw + kb];
+    }
+    const int cnt = s1 - s0 < LONG_SEG ? s1 - s0 : 0;
+    int incl = cnt;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const int up = __shfl_up(incl, s);
+      if ((t & 63) >= s) incl += up;
+    }
+    int* wtot = reinterpret_cast<int*>(area);
+    if ((t & 63) == 63) wtot[wave] = incl;
+    __syncthreads();
+    for (int w = 0; w < wave; ++w) incl += wtot[w];
+    ioff[t] = incl - cnt; spos[t] = s0;
+    if (t == 255) { ioff[256] = incl; spos[256] = s1; }
+    __syncthreads();
+    const int E = __builtin_amdgcn_readfirstlane(ioff[256]);
+    pre = E <= room;
+    if (pre && E > 0) {
+      Item* items = reinterpret_cast<Item*>(area + room * 256);
+      for (int k = 0; k < cnt; ++k) items[incl - cnt + k].row = s0 + k;
+      __syncthreads();
+      for (int q = t; q < E; q += NTHREADS) {
+        const int at = items[q].row;
+        items[q].row = o.srow[at]; items[q].h = o.sh[at];
+      }
+      __syncthreads();
+      load_rows(items, E, area);
+    }
   }
-  if (tt >= 0) {
-    const int g0 = (tt * tl.kp) / tl.share, g1 = ((tt + 1) * tl.kp - 1) / tl.share;
-    const float* src = tl.buf + (size_t)tt * 65536 + (j0 & 255) * 256 + (v & 255);
+  v16f acc[4][4];
+  mfma_mainloop<false, NoHook, BLOCKED_KSTEP, true, 2>(p.xt + ((int64_t)rt * p.kbn + p.kb0) * BLOCKED_KSTEP, BK, p.ghat_t + (int64_t)(2 * ct) * BLOCKED_KSTEP, BLOCKED_KSTEP, p.KT,
+                                                       smem, acc, ct & 7, 2 * (rt & 3), wave, NoHook(), 128 * BK, p.kbv * BLOCKED_KSTEP, lsc + wb * p.KT);
+  const float x_s = o.dc ? o.dc->x_s : o.x_s, scale = x_s * o.xi[0];
+  T* dw = reinterpret_cast<T*>(o.dw);
+  const bool vec = sizeof(T) == 2 && ((reinterpret_cast<uintptr_t>(o.dw) | (uintptr_t)(o.dw_ld * (int64_t)sizeof(T))) & 15) == 0 && (o.V % 8 == 0 || ct * 256 + 256 <= o.V);
+  uint8_t* stage = (pre ? smem : area) + wave * DWO_STAGE;
+  const uint8_t* xrows = pre ? area : smem;
+  const Item* items = reinterpret_cast<const Item*>(pre ? area + room * 256 : smem + DWO_GROUP * 256);
+  int bend = pre ? 4 : 0, qsub = 0;            // row blocks whose entries are in LDS; what to take off an entry's number for its place there
 #pragma unroll
-    for (int m = 0; m < 16; ++m) o[m] = 0.f;
-    for (int g = g0; g <= g1; ++g) {                      // fixed order; the 16 loads of a piece are in flight together
-#pragma unroll
-      for (int m = 0; m < 16; ++m) o[m] += src[(size_t)g * 65536 + m * 256];
+  for (int b = 0; b < 4; ++b) {
+    if (b >= bend) {
+      // the entries of as many row blocks from b on as fit, of both halves of the columns: first those of the lower half
+      auto upto = [&](int e) { return ioff[32 * e] - ioff[32 * b] + ioff[128 + 32 * e] - ioff[128 + 32 * b]; };
+      bend = b + 1;
+      while (bend < 4 && upto(bend + 1) <= DWO_GROUP) ++bend;
+      bend = __builtin_amdgcn_readfirstlane(bend);
+      const int total = __builtin_amdgcn_readfirstlane(upto(bend)), base0 = ioff[32 * b], sub1 = ioff[128 + 32 * b] - (ioff[32 * bend] - base0);
+      Item* list = reinterpret_cast<Item*>(smem + DWO_GROUP * 256);
+      __syncthreads();                         // every wave is done with the entries that were there
+      const int t = wave * 64 + lane_id(), tb = (t & 127) >> 5;
+      if (tb >= b && tb < bend) {
+        const int first = ioff[t] - (t < 128 ? base0 : sub1), cnt = ioff[t + 1] - ioff[t];
+        for (int k = 0; k < cnt; ++k) list[first + k].row = spos[t] + k;
+      }
+      __syncthreads();
+      for (int q = t; q < total; q += NTHREADS) {
+        const int at = list[q].row;
+        list[q].row = o.srow[at]; list[q].h = o.sh[at];
+      }
+      __syncthreads();
+      load_rows(list, total, smem);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      qsub = __builtin_amdgcn_readfirstlane(wb ? sub1 : base0);
     }
 #pragma unroll
-    for (int m = 0; m < 16; ++m) o[m] *= scale;
+    for (int ah = 0; ah < 2; ++ah) {           // rows 64 ah .. + 63 of the quadrant
+      const int lane = lane_id(), h = lane >> 5, c = wb * 128 + b * 32 + (lane & 31), v = ct * 256 + c;
+      float val[32];
+#pragma unroll
+      for (int m = 0; m < 32; ++m) val[m] = acc[2 * ah + (m >> 4)][b][m & 15] * scale;
+      const int q0 = ioff[c] - qsub, n = ioff[c + 1] - ioff[c];
+      for (int k = 0; __builtin_amdgcn_ballot_w64(k < n) != 0; ++k) {
+        if (k < n) {
+          const int q = q0 + k;
+          const float hx = items[q].h * x_s;
+          const uint8_t* xr = xrows + q * 256 + 4 * h;
+          const int sw = (8 * wa + 4 * ah) ^ (q & 15);
+#pragma unroll
+          for (int g = 0; g < 8; ++g) {        // four rows each: 32 (g / 4) + 8 (g % 4) + 4 h on
+            const uint32_t w = *reinterpret_cast<const uint32_t*>(xr + ((sw ^ (g >> 1)) << 4) + 8 * (g & 1));
+            val[4 * g + 0] -= hx * e4m3_to_float<0>(w);
+            val[4 * g + 1] -= hx * e4m3_to_float<1>(w);
+            val[4 * g + 2] -= hx * e4m3_to_float<2>(w);
+            val[4 * g + 3] -= hx * e4m3_to_float<3>(w);
+          }
+        }
+      }
+      const int L = spos[c + 1] - spos[c];
+      if (__builtin_amdgcn_ballot_w64(L >= LONG_SEG) != 0) {
+        if (L >= LONG_SEG) {
+          int nch, len;
+          long_chunks(L, nch, len);
+          const float* ls = o.longsum + (int64_t)o.longbase[v] * o.dq + rt * 256 + wa * 128 + ah * 64 + 4 * h;
+          for (int k = 0; k < nch; ++k, ls += o.dq) {           // fixed order
+#pragma unroll
+            for (int g = 0; g < 8; ++g) {
+              const v4f s = *reinterpret_cast<const v4f*>(ls + 32 * (g >> 2) + 8 * (g & 3));
+#pragma unroll
+              for (int m = 0; m < 4; ++m) val[4 * g + m] -= s[m] * x_s;
+            }
+          }
+        }
+      }
+      const int j0 = rt * 256 + wa * 128 + ah * 64;
+      if (vec) {
+#pragma unroll
+        for (int g = 0; g < 8; ++g) {
+          typedef __bf16 v4bf __attribute__((ext_vector_type(4)));
+          const v4bf e = {(__bf16)val[4 * g], (__bf16)val[4 * g + 1], (__bf16)val[4 * g + 2], (__bf16)val[4 * g + 3]};
+          *reinterpret_cast<v2i*>(stage + (lane & 31) * DWO_STAGE_PITCH + 2 * (32 * (g >> 2) + 8 * (g & 3) + 4 * h)) = __builtin_bit_cast(v2i, e);
+        }
+        asm volatile("" ::: "memory");         // (a wave's own LDS operations complete in order)
+        // ds_read_b64_tr_b16: of the 4 x 16 matrix that 16 lanes point at, 8 bytes each, lane i gets column i
+        typedef short v4s __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) v4s lds_v4s;
+        const int i = lane & 15, v8 = 8 * (lane >> 4);
+        const uint8_t* src = stage + (v8 + (i >> 2)) * DWO_STAGE_PITCH + 8 * (i & 3);
+        T* dst = dw + (int64_t)(j0 + i) * o.dw_ld + ct * 256 + wb * 128 + b * 32 + v8;
+        const bool in = ct * 256 + wb * 128 + b * 32 + v8 < o.V;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src + 32 * s)));
+          const v2i hi = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src + 32 * s + 4 * DWO_STAGE_PITCH)));
+          if (in && j0 + 16 * s + i < o.d) *reinterpret_cast<v4i*>(dst + (int64_t)(16 * s) * o.dw_ld) = (v4i){lo[0], lo[1], hi[0], hi[1]};
+        }
+        asm volatile("" ::: "memory");
+      } else if (v < o.V) {
+#pragma unroll
+        for (int m = 0; m < 32; ++m) {
+          const int j = j0 + 32 * (m >> 4) + 8 * ((m & 15) >> 2) + 4 * h + (m & 3);
+          if (j < o.d) Elem<T>::store(dw + (int64_t)j * o.dw_ld + v, val[m]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);       // one half at a time: the accumulators of all of them, moved up front, do not fit the registers
+    }
+  }
+}
+
+// The same from fp32 partials: what is left are the tiles of a K-split last round (tl.tile0 >= 0: grid.y = tl.ntail tiles of
+// 16 blocks of 64 x 64 elements), and every tile where dW took more than one launch (grid = blocks of 64 columns x 64
+// rows of dW).  A thread owns one column v and 16 consecutive rows j; the segment sum is formed here for short segments
+// and read from the chunk sums for long ones.
+template <typename T>
+__global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restrict__ dwacc, int nparts, int64_t part_stride, int64_t Vp, DwOut o, DwTail tl, int RT,
+                                                          int CT) {
+  const float x_s = o.dc ? o.dc->x_s : o.x_s;
+  const int t = threadIdx.x;
+  int bx = blockIdx.x, by = blockIdx.y;
+  if (tl.tile0 >= 0) {
+    int rt, ct;
+    tile_from_index(tl.tile0 + by, RT, CT, rt, ct);
+    by = 4 * rt + (bx >> 2); bx = 4 * ct + (bx & 3);
+  }
+  const int v = bx * 64 + (t & 63);
+  const int j0 = by * 64 + (t >> 6) * 16;
+  if (v >= o.V || j0 >= o.d) return;
+  const float scale = x_s * o.xi[0];
+  float val[16];
+  if (tl.tile0 >= 0) {
+    const int tt = blockIdx.y, g0 = (tt * tl.kp) / tl.share, g1 = ((tt + 1) * tl.kp - 1) / tl.share;
+    const float* src = tl.buf + (size_t)tt * 65536 + (j0 & 255) * 256 + (v & 255);
+#pragma unroll
+    for (int m = 0; m < 16; ++m) val[m] = 0.f;
+    for (int g = g0; g <= g1; ++g) {                      // fixed order; the 16 loads of a piece are in flight together
+#pragma unroll
+      for (int m = 0; m < 16; ++m) val[m] += src[(size_t)g * 65536 + m * 256];
+    }
+#pragma unroll
+    for (int m = 0; m < 16; ++m) val[m] *= scale;
   } else {
 #pragma unroll
     for (int m = 0; m < 16; ++m) {
       float sum = dwacc[(int64_t)(j0 + m) * Vp + v];
       for (int q = 1; q < nparts; ++q) sum += dwacc[q * part_stride + (int64_t)(j0 + m) * Vp + v];   // fixed order
-      o[m] = sum * scale;
+      val[m] = sum * scale;
     }
   }
-  const int s0 = segoff[v], L = segoff[v + 1] - s0;
+  const int s0 = o.segoff[v], L = o.segoff[v + 1] - s0;
   if (L >= LONG_SEG) {
     int nch, len;
     long_chunks(L, nch, len);
     for (int c = 0; c < nch; ++c) {                       // fixed order
-      const float* ls = longsum + (int64_t)(longbase[v] + c) * dq + j0;
+      const float* ls = o.longsum + (int64_t)(o.longbase[v] + c) * o.dq + j0;
 #pragma unroll
-      for (int m = 0; m < 16; ++m) o[m] -= ls[m] * x_s;
+      for (int m = 0; m < 16; ++m) val[m] -= ls[m] * x_s;
     }
   } else if (L > 0) {
     for (int n = 0; n < L; ++n) {
-      const int e = perm[s0 + n];                         // entry id k * Np + i
-      const float h = hcoef[e] * x_s;
-      const v4i raw = *reinterpret_cast<const v4i*>(xq + (int64_t)(e % Np) * ldx + j0);
+      const float h = o.sh[s0 + n] * x_s;
+      const v4i raw = *reinterpret_cast<const v4i*>(o.xq + (int64_t)o.srow[s0 + n] * o.ldx + j0);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         const uint32_t w = (uint32_t)raw[m];
-        o[4 * m + 0] -= h * e4m3_to_float<0>(w);
-        o[4 * m + 1] -= h * e4m3_to_float<1>(w);
-        o[4 * m + 2] -= h * e4m3_to_float<2>(w);
-        o[4 * m + 3] -= h * e4m3_to_float<3>(w);
+        val[4 * m + 0] -= h * e4m3_to_float<0>(w);
+        val[4 * m + 1] -= h * e4m3_to_float<1>(w);
+        val[4 * m + 2] -= h * e4m3_to_float<2>(w);
+        val[4 * m + 3] -= h * e4m3_to_float<3>(w);
       }
     }
   }
+  T* dw = reinterpret_cast<T*>(o.dw);
 #pragma unroll
   for (int m = 0; m < 16; ++m)
-    if (j0 + m < d) Elem<T>::store(dw + (int64_t)(j0 + m) * dw_ld + v, o[m]);
+    if (j0 + m < o.d) Elem<T>::store(dw + (int64_t)(j0 + m) * o.dw_ld + v, val[m]);
 }
 
 }  // namespace sce

@@ -156,6 +156,8 @@ static int check_device(int dev) {
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_tail_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
+      HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_out_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
+      HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_out_kernel<bf16_t>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       void* sp = nullptr;
       HIP_TRY(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));       // this device's copy of the array
       g_scratch[dev] = sp;
@@ -672,6 +674,8 @@ extern "C" int sce_backward(const sce_args* a) {
   int32_t* vals_in = perm + NE;
   int32_t* skeys = (int32_t*)(ws + B.off_keys);
   int32_t* keys_in = skeys + NE;
+  int32_t* srow = vals_in;             // (once sorted, the unsorted lists' places are free)
+  float* sh = (float*)keys_in;
   int32_t* segoff = (int32_t*)(ws + B.off_segoff);
   int32_t* longlist = (int32_t*)(ws + B.off_longlist);
   float* longsum = (float*)(ws + B.off_longsum);
@@ -696,14 +700,24 @@ extern "C" int sce_backward(const sce_args* a) {
     size_t tmp = B.sorttmp_bytes;
     if (sce::sort_pairs(ws + B.off_sorttmp, &tmp, keys_in, skeys, vals_in, perm, (size_t)NE, bits, st) != 0)
     { delete tm_prep; return fail(SCE_EHIP, "radix sort of the targets failed"); }
-    bwd_segments_kernel<<<(int)(V / 256 + 1), 256, 0, st>>>(skeys, (int)NE, (int)V, segoff, longlist, longbase);
+    bwd_segments_kernel<<<(int)(V / 256 + 1), 256, 0, st>>>(skeys, perm, hcoef, (int)NE, (int)S.Np, (int)V, segoff, longlist, longbase, srow, sh);
   }
   delete tm_prep;
+  {
+    KernelTimer tm(SCE_K_DW_FINAL, st);
+    bwd_dw_long_kernel<<<dim3((unsigned)std::min<int64_t>(NE / LONG_SEG + 1, LONG_GRID), (unsigned)(S.dq / 256)), 256, 0, st>>>(longlist, segoff, srow, sh, xq, S.ldx,
+                                                                                                                              S.dq, longsum);
+  }
   const float sc = (float)a->x_s * (float)a->w_s, k1 = sc * 2.0f * LOG2E / a->cap, c2 = -2.0f * a->cap * LOG2E;
   const int CTv = (int)(S.Vp / 256), CTd = (int)(S.dq / 256);
   int launch = 0;
   DwTail tail;
   tail.buf = nullptr; tail.tile0 = -1; tail.ntail = 0; tail.kp = 1; tail.share = 1;
+  DwOut wo;
+  wo.dw = a->dw; wo.dw_ld = a->dw_ld; wo.segoff = segoff; wo.srow = srow; wo.sh = sh; wo.xq = xq; wo.longsum = longsum; wo.longbase = longbase;
+  wo.xi = xi; wo.dc = dcp; wo.ldx = S.ldx; wo.dq = S.dq; wo.x_s = (float)a->x_s; wo.d = (int)d; wo.V = (int)V;
+  const bool dw_f32 = a->dw_dtype == SCE_F32;
+  bool dw_done = false;                // every tile is stored, or will be from `tail`
   const bool dx_f32 = a->dx_dtype == SCE_F32;
   const int smem_dx = smem_scaled((int)(S.Vp / BK), SMEM_DX);
   // dX of the rows [p0, p0 + prow) (a multiple of 256), the dlogits buffer standing for rows from gorg on
@@ -754,11 +768,18 @@ extern "C" int sce_backward(const sce_args* a) {
       // shared out along K instead (bwd_dw_tail_kernel): the full rounds run as they are.
       const DwTailPlan tp = dw_tail_plan(S.dq, S.Vp, gathered);
       const bool only = w0 == 0 && last && launch == 0;
-      if (only && tp.use && B.tail_bytes >= tp.bytes && a->workspace_bytes >= B.off_dwtail + tp.bytes) {
-        const int full = tp.full;
-        tail.buf = (float*)(ws + B.off_dwtail); tail.tile0 = tp.full; tail.ntail = tp.ntail; tail.kp = tp.kp; tail.share = tp.share;
-        if (full > 0) bwd_dw_kernel<false><<<full, NTHREADS, smem_scaled(wp.KT, 0), st>>>(wp);
-        bwd_dw_tail_kernel<<<dim3(DW_TAIL_WGS, 2), NTHREADS, smem_scaled(2 * tp.share, 0), st>>>(wp, tail);
+      if (only) {
+        const bool share = tp.use && B.tail_bytes >= tp.bytes && a->workspace_bytes >= B.off_dwtail + tp.bytes;
+        const int grid = share ? tp.full : map_tile_rr_grid(CTd, CTv);
+        if (grid > 0) {
+          if (dw_f32) bwd_dw_out_kernel<float><<<grid, NTHREADS, SMEM_MAX, st>>>(wp, wo);
+          else bwd_dw_out_kernel<bf16_t><<<grid, NTHREADS, SMEM_MAX, st>>>(wp, wo);
+        }
+        if (share) {
+          tail.buf = (float*)(ws + B.off_dwtail); tail.tile0 = tp.full; tail.ntail = tp.ntail; tail.kp = tp.kp; tail.share = tp.share;
+          bwd_dw_tail_kernel<<<dim3(DW_TAIL_WGS, 2), NTHREADS, smem_scaled(2 * tp.share, 0), st>>>(wp, tail);
+        }
+        dw_done = true;
       } else if (launch >= nparts) bwd_dw_kernel<true><<<map_tile_rr_grid(CTd, CTv), NTHREADS, smem_scaled(wp.KT, 0), st>>>(wp);
       else bwd_dw_kernel<false><<<map_tile_rr_grid(CTd, CTv), NTHREADS, smem_scaled(wp.KT, 0), st>>>(wp);
     }
@@ -805,16 +826,12 @@ extern "C" int sce_backward(const sce_args* a) {
     else if (hf) rmsnorm_backward_kernel<bf16_t, float><<<ngrid, 256, 0, st>>>((bf16_t*)a->dx, a->dx_ld, (const float*)a->x, a->x_ld, rstd, N, d);
     else rmsnorm_backward_kernel<bf16_t, bf16_t><<<ngrid, 256, 0, st>>>((bf16_t*)a->dx, a->dx_ld, (const bf16_t*)a->x, a->x_ld, rstd, N, d);
   }
-  KernelTimer tm_fin(SCE_K_DW_FINAL, st);
-  bwd_dw_long_kernel<<<dim3((unsigned)(NE / LONG_SEG + 1), (unsigned)(S.dq / 256)), 256, 0, st>>>(longlist, segoff, perm, hcoef, xq, S.dp, S.ldx, S.dq, (int)S.Np, longsum);
-  {
-    dim3 g((unsigned)((V + 63) / 64), (unsigned)((d + 63) / 64));
-    if (a->dw_dtype == SCE_F32)
-      bwd_dw_final_kernel<float><<<g, 256, 0, st>>>(dwacc, launch < nparts ? launch : nparts, (int64_t)(B.part_stride / 4), S.Vp, segoff, perm, hcoef, xq, S.ldx, (int)S.Np, xi, longsum, longbase, S.dq, (float)a->x_s, dcp, (int)d, (int)V,
-                                                   (float*)a->dw, a->dw_ld, tail, CTd, CTv);
-    else
-      bwd_dw_final_kernel<bf16_t><<<g, 256, 0, st>>>(dwacc, launch < nparts ? launch : nparts, (int64_t)(B.part_stride / 4), S.Vp, segoff, perm, hcoef, xq, S.ldx, (int)S.Np, xi, longsum, longbase, S.dq, (float)a->x_s, dcp, (int)d, (int)V,
-                                                    (bf16_t*)a->dw, a->dw_ld, tail, CTd, CTv);
+  if (!dw_done || tail.tile0 >= 0) {
+    KernelTimer tm_fin(SCE_K_DW_FINAL, st);
+    const dim3 g = dw_done ? dim3(16, (unsigned)tail.ntail) : dim3((unsigned)((V + 63) / 64), (unsigned)((d + 63) / 64));
+    const int np = launch < nparts ? launch : nparts;
+    if (dw_f32) bwd_dw_final_kernel<float><<<g, 256, 0, st>>>(dwacc, np, (int64_t)(B.part_stride / 4), S.Vp, wo, tail, CTd, CTv);
+    else bwd_dw_final_kernel<bf16_t><<<g, 256, 0, st>>>(dwacc, np, (int64_t)(B.part_stride / 4), S.Vp, wo, tail, CTd, CTv);
   }
   HIP_TRY(hipGetLastError());
   return SCE_OK;

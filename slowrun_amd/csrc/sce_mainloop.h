@@ -82,6 +82,11 @@ __device__ __forceinline__ void lds_direct_16(uint32_t lds_addr, uint32_t voff, 
                ::"s"(lds_addr), "n"(LDS_CONST), "v"(voff), "s"(sbase) : "memory", "scc");
 }
 
+// The same with a 64-bit address per lane, for gathers that may span more than 4 GiB.
+__device__ __forceinline__ void lds_direct_16_far(uint32_t lds_addr, const uint8_t* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(src) : "memory");
+}
+
 // Global -> LDS loads of one tile: per wave, 16 instructions per K block (8 for A, 8 for B).
 //
 // TRB = false: both operands are K-contiguous in memory (rows lda / ldb bytes apart) and in LDS.
