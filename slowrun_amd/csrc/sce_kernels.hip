@@ -368,7 +368,7 @@ static int quantize_impl(const void* src, int32_t src_dtype, void* dst, float in
   DeviceGuard guard(device);
   if (!guard.ok) return fail(SCE_EHIP, "cannot select device %d", device);
   hipStream_t st = (hipStream_t)stream;
-  const int grid = grid_for((n + 3) / 4, 256);
+  const int grid = grid_for((n + 15) / 16, 256);
   if (src_dtype == SCE_F32) quantize_flat_kernel<float><<<grid, 256, 0, st>>>((const float*)src, (uint8_t*)dst, n, inv_scale, scale_dev);
   else if (src_dtype == SCE_BF16) quantize_flat_kernel<bf16_t><<<grid, 256, 0, st>>>((const bf16_t*)src, (uint8_t*)dst, n, inv_scale, scale_dev);
   else return fail(SCE_EINVAL, "unsupported dtype %d", src_dtype);
@@ -397,12 +397,12 @@ extern "C" int sce_amax_scale(const void* src, int32_t src_dtype, size_t n, floa
   if (!guard.ok) return fail(SCE_EHIP, "cannot select device %d", device);
   hipStream_t st = (hipStream_t)stream;
   uint32_t* bits = reinterpret_cast<uint32_t*>(scale_out);
-  int grid = grid_for(n, 256 * 16);
-  if (grid > 4096) grid = 4096;
+  const int esz = src_dtype == SCE_F32 ? 4 : 2;
+  int grid = grid_for((n * esz + 15) / 16, 256 * AMAX_LOADS);
+  if (grid > 8 * MAX_CUS) grid = 8 * MAX_CUS;          // as many workgroups as run at one time
   amax_begin_kernel<<<1, 1, 0, st>>>(bits);
   if (src_dtype == SCE_F32) amax_kernel<float><<<grid, 256, 0, st>>>((const float*)src, n, bits);
   else amax_kernel<bf16_t><<<grid, 256, 0, st>>>((const bf16_t*)src, n, bits);
-  amax_end_kernel<<<1, 1, 0, st>>>(bits);
   HIP_TRY(hipGetLastError());
   return SCE_OK;
 }
@@ -414,8 +414,9 @@ extern "C" int sce_transpose_bytes(const void* src, void* dst, int64_t rows, int
   if (int rc = check_device(device)) return rc;
   DeviceGuard guard(device);
   if (!guard.ok) return fail(SCE_EHIP, "cannot select device %d", device);
-  dim3 grid((unsigned)((cols + 63) / 64), (unsigned)((rows + 63) / 64));
-  transpose_bytes_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint8_t*)src, (uint8_t*)dst, rows, cols);
+  dim3 grid((unsigned)((cols + TB_TILE - 1) / TB_TILE), (unsigned)((rows + TB_TILE - 1) / TB_TILE));
+  const int in16 = cols % 16 == 0 && ((uintptr_t)src & 15) == 0, out16 = rows % 16 == 0 && ((uintptr_t)dst & 15) == 0;
+  transpose_bytes_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint8_t*)src, (uint8_t*)dst, rows, cols, in16, out16);
   HIP_TRY(hipGetLastError());
   return SCE_OK;
 }

@@ -205,20 +205,38 @@ __global__ __launch_bounds__(256) void quantize_w_kernel(const T* __restrict__ w
   __shared__ uint8_t tile[QW_TILE][QW_TILE + 4];
   const int t = threadIdx.x;
   const int64_t j0 = (int64_t)blockIdx.y * QW_TILE, v0 = (int64_t)blockIdx.x * QW_TILE;
+  if (sizeof(T) == 4 && v0 + QW_TILE <= V && ((reinterpret_cast<uintptr_t>(w) | (uintptr_t)(ld * 4)) & 15) == 0) {
+    // fp32: four elements a load, so that a wave reads 512 bytes of a row in a row (with 16 a thread its loads lay 64 bytes
+    // apart: 3.2 TB/s at d = 768)
+    v4f x[16];
 #pragma unroll
-  for (int pass = 0; pass < 4; ++pass) {
-    const int r = (t >> 3) + 32 * pass, c = (t & 7) * 16;
-    const int64_t j = j0 + r, v = v0 + c;
-    uint32_t out[4] = {0, 0, 0, 0};
-    if (j < d && v < V) {
-      float x[16];
-      load16_scaled<T>(w + j * ld + v, V - v, scale, x);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) out[m] = cvt4_e4m3(x[4 * m], x[4 * m + 1], x[4 * m + 2], x[4 * m + 3]);
+    for (int pass = 0; pass < 16; ++pass) {
+      const int64_t j = j0 + (t >> 5) + 8 * pass;
+      x[pass] = j < d ? *reinterpret_cast<const v4f*>(reinterpret_cast<const float*>(w) + j * ld + v0 + (t & 31) * 4) : (v4f){0.f, 0.f, 0.f, 0.f};
     }
-    *reinterpret_cast<v4i*>(wq + blocked_offset(j, v, kbv)) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
 #pragma unroll
-    for (int m = 0; m < 4; ++m) *reinterpret_cast<uint32_t*>(&tile[r][c + 4 * m]) = out[m];
+    for (int pass = 0; pass < 16; ++pass) {
+      const int r = (t >> 5) + 8 * pass, c = (t & 31) * 4;
+      const uint32_t out = cvt4_e4m3(scale.apply<T>(x[pass][0]), scale.apply<T>(x[pass][1]), scale.apply<T>(x[pass][2]), scale.apply<T>(x[pass][3]));
+      *reinterpret_cast<uint32_t*>(wq + blocked_offset(j0 + r, v0 + c, kbv)) = out;
+      *reinterpret_cast<uint32_t*>(&tile[r][c]) = out;
+    }
+  } else {
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {
+      const int r = (t >> 3) + 32 * pass, c = (t & 7) * 16;
+      const int64_t j = j0 + r, v = v0 + c;
+      uint32_t out[4] = {0, 0, 0, 0};
+      if (j < d && v < V) {
+        float x[16];
+        load16_scaled<T>(w + j * ld + v, V - v, scale, x);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) out[m] = cvt4_e4m3(x[4 * m], x[4 * m + 1], x[4 * m + 2], x[4 * m + 3]);
+      }
+      *reinterpret_cast<v4i*>(wq + blocked_offset(j, v, kbv)) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
+#pragma unroll
+      for (int m = 0; m < 4; ++m) *reinterpret_cast<uint32_t*>(&tile[r][c + 4 * m]) = out[m];
+    }
   }
   __syncthreads();
   if (j0 < dp) {
@@ -275,59 +293,120 @@ __global__ __launch_bounds__(256) void prep_w_bf16_kernel(const T* __restrict__ 
   }
 }
 
-// flat cast, for the standalone sce_quantize_e4m3 entry point
+// flat cast, for the standalone sce_quantize_e4m3 entry point: 16 elements a thread, their 32 or 64 bytes in 16-byte loads
+// and the result in one 16-byte store where both are aligned (a thread's run starts at a multiple of 16 elements, so
+// that is a matter of the base pointers), element by element otherwise and at the end.  HBM-bound: 3 bytes an element
+// in bf16; with four elements a thread in 2-byte loads 162 us for 2560 x 50304 (2.4 TB/s), now 70.
 template <typename T>
 __global__ __launch_bounds__(256) void quantize_flat_kernel(const T* __restrict__ src, uint8_t* __restrict__ dst,
                                                            size_t n, float inv_scale, const float* __restrict__ scale_dev) {
   const Scaler scale = make_scaler<T>(inv_scale, scale_dev);
-  for (size_t q = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 4; q < n; q += (size_t)gridDim.x * blockDim.x * 4) {
-    float v[4];
+  for (size_t q = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 16; q < n; q += (size_t)gridDim.x * blockDim.x * 16) {
+    const int64_t left = (int64_t)(n - q);
+    float v[16];
+    load16_scaled<T>(src + q, left, scale, v);
+    uint32_t w[4];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) v[m] = (q + m < n) ? scale.apply<T>(Elem<T>::load(src + q + m)) : 0.f;
-    const uint32_t w = cvt4_e4m3(v[0], v[1], v[2], v[3]);
-    if (q + 4 <= n && (((uintptr_t)(dst + q)) & 3) == 0) {
-      *reinterpret_cast<uint32_t*>(dst + q) = w;
+    for (int m = 0; m < 4; ++m) w[m] = cvt4_e4m3(v[4 * m], v[4 * m + 1], v[4 * m + 2], v[4 * m + 3]);
+    if (left >= 16 && ((uintptr_t)dst & 15) == 0) {
+      *reinterpret_cast<v4i*>(dst + q) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     } else {
-      for (int m = 0; m < 4 && q + m < n; ++m) dst[q + m] = (uint8_t)(w >> (8 * m));
+#pragma unroll
+      for (int m = 0; m < 16; ++m)
+        if (m < left) dst[q + m] = (uint8_t)(w[m >> 2] >> (8 * (m & 3)));
     }
   }
 }
 
-// max |src| over n elements, as the bits of a non-negative float (they order like unsigned integers, NaN above
-// everything); *bits starts at 0 (amax_begin_kernel) and ends as max / 448 (amax_end_kernel).
+// max |src| / 448 over n elements into *bits, as the bits of a non-negative float (they order like unsigned integers,
+// NaN above everything); *bits starts at 0 (amax_begin_kernel).  The division comes before the maximum over the
+// workgroups: it is monotonic, so the result is the same and needs no kernel of its own.  HBM-bound: a workgroup walks
+// pieces of AMAX_LOADS x 4 KB with all its 16-byte loads in flight (a 2-byte load at a time: 1.8 TB/s).
 __global__ void amax_begin_kernel(uint32_t* bits) { *bits = 0u; }
+constexpr int AMAX_LOADS = 8;
 template <typename T>
 __global__ __launch_bounds__(256) void amax_kernel(const T* __restrict__ src, size_t n, uint32_t* __restrict__ bits) {
-  __shared__ uint32_t smax[256];
+  __shared__ uint32_t smax[4];
+  constexpr int PER = 16 / sizeof(T);
   uint32_t m = 0u;
-  for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
-    const uint32_t b = __float_as_uint(Elem<T>::load(src + q)) & 0x7fffffffu;
-    m = b > m ? b : m;
+  auto take = [&](uint32_t b) { b &= 0x7fffffffu; m = b > m ? b : m; };
+  // the elements before the first 16-byte boundary, and those after the last whole load, one by one
+  size_t head = ((16 - ((uintptr_t)src & 15)) & 15) / sizeof(T);
+  if (head > n) head = n;
+  const size_t loads = (n - head) / PER, tail = head + loads * PER;
+  const v4i* vec = reinterpret_cast<const v4i*>(src + head);
+  for (size_t q0 = (size_t)blockIdx.x * (256 * AMAX_LOADS) + threadIdx.x; q0 < loads; q0 += (size_t)gridDim.x * (256 * AMAX_LOADS)) {
+    v4i r[AMAX_LOADS];
+#pragma unroll
+    for (int k = 0; k < AMAX_LOADS; ++k) r[k] = vec[q0 + k * 256 < loads ? q0 + k * 256 : q0];
+#pragma unroll
+    for (int k = 0; k < AMAX_LOADS; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (sizeof(T) == 2) { take((uint32_t)r[k][e] << 16); take((uint32_t)r[k][e] & 0xffff0000u); }
+        else take((uint32_t)r[k][e]);
+      }
   }
-  smax[threadIdx.x] = m;
+  if (blockIdx.x == 0) {
+    for (size_t q = threadIdx.x; q < head; q += 256) take(__float_as_uint(Elem<T>::load(src + q)));
+    for (size_t q = tail + threadIdx.x; q < n; q += 256) take(__float_as_uint(Elem<T>::load(src + q)));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { const uint32_t x = (uint32_t)__shfl_xor((int)m, o); m = x > m ? x : m; }
+  if ((threadIdx.x & 63) == 0) smax[threadIdx.x >> 6] = m;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) smax[threadIdx.x] = smax[threadIdx.x] > smax[threadIdx.x + w] ? smax[threadIdx.x] : smax[threadIdx.x + w];
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; ++w) m = smax[w] > m ? smax[w] : m;
+    atomicMax(bits, __float_as_uint(__uint_as_float(m) / 448.0f));
   }
-  if (threadIdx.x == 0) atomicMax(bits, smax[0]);
 }
-__global__ void amax_end_kernel(uint32_t* bits) { *reinterpret_cast<float*>(bits) = __uint_as_float(*bits) / 448.0f; }
 
-// dst (cols, rows) = src (rows, cols)^T, bytes.
+// dst (cols, rows) = src (rows, cols)^T, bytes, in 128 x 128 tiles: whole 128-byte lines both ways.  On the way out of
+// LDS the transposing read gives a lane eight rows of its column at once (16 lanes point at 8 rows of 16 bytes, 8 bytes
+// each, and lane j receives column j).  `in16` / `out16`: every run of 16 bytes along a row of src / dst is aligned; other shapes and the
+// ragged edges go byte by byte.  HBM-bound, 2 bytes an element: 164 us for 2560 x 50304 when every byte was an access
+// of its own (1.6 TB/s), now 50.
+constexpr int TB_TILE = 128, TB_PITCH = TB_TILE + 16;
 __global__ __launch_bounds__(256) void transpose_bytes_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
-                                                             int64_t rows, int64_t cols) {
-  __shared__ uint8_t tile[64][68];
+                                                             int64_t rows, int64_t cols, int in16, int out16) {
+  __shared__ __attribute__((aligned(16))) uint8_t tile[TB_TILE * TB_PITCH];
   const int t = threadIdx.x;
-  const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
-  for (int e = t; e < 64 * 64; e += 256) {
-    const int r = e >> 6, c = e & 63;
-    tile[r][c] = (r0 + r < rows && c0 + c < cols) ? src[(r0 + r) * cols + c0 + c] : 0;
+  const int64_t r0 = (int64_t)blockIdx.y * TB_TILE, c0 = (int64_t)blockIdx.x * TB_TILE;
+  {
+    v4i raw[4];
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) {
+      const int64_t r = r0 + (t >> 3) + 32 * pass, c = c0 + (t & 7) * 16;
+      raw[pass] = (v4i){0, 0, 0, 0};
+      if (r < rows && c < cols) {
+        if (in16) raw[pass] = *reinterpret_cast<const v4i*>(src + r * cols + c);
+        else
+          for (int m = 0; m < 16 && c + m < cols; ++m) raw[pass][m >> 2] |= (int)((uint32_t)src[r * cols + c + m] << (8 * (m & 3)));
+      }
+    }
+#pragma unroll
+    for (int pass = 0; pass < 4; ++pass) *reinterpret_cast<v4i*>(&tile[((t >> 3) + 32 * pass) * TB_PITCH + (t & 7) * 16]) = raw[pass];
   }
   __syncthreads();
-  for (int e = t; e < 64 * 64; e += 256) {
-    const int c = e >> 6, r = e & 63;
-    if (r0 + r < rows && c0 + c < cols) dst[(c0 + c) * rows + r0 + r] = tile[r][c];
+  // a wave takes 16 columns at a time: group g of 16 lanes the rows [16 g, +16) and [64 + 16 g, +16) of the tile
+  const int lane = t & 63, wave = t >> 6, g = lane >> 4, i = lane & 15;
+  typedef __attribute__((address_space(3))) v2i lds_v2i;
+#pragma unroll
+  for (int pass = 0; pass < 4; ++pass) {
+    const int cc = (wave * 2 + (pass & 1)) * 16, rr = 16 * g + 64 * (pass >> 1);
+    const uint8_t* s = &tile[(rr + (i >> 1)) * TB_PITCH + cc + 8 * (i & 1)];
+    const v2i lo = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)s), hi = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_v2i*)(s + 8 * TB_PITCH));
+    const int64_t c = c0 + cc + i, r = r0 + rr;
+    if (c < cols && r < rows) {
+      uint8_t* d = dst + c * rows + r;
+      if (out16) *reinterpret_cast<v4i*>(d) = (v4i){lo[0], lo[1], hi[0], hi[1]};
+      else {
+        const int w[4] = {lo[0], lo[1], hi[0], hi[1]};
+#pragma unroll
+        for (int m = 0; m < 16; ++m)
+          if (r + m < rows) d[m] = (uint8_t)((uint32_t)w[m >> 2] >> (8 * (m & 3)));
+      }
+    }
   }
 }
 

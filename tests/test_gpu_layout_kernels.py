@@ -1,0 +1,34 @@
+"""The casts, maxima and transposes at the edges of their vector paths: lengths around a load, misaligned bases, ragged
+tiles.  All exact: bytes of a defined cast, a maximum, a permutation."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (16, 16), (128, 128), (129, 127), (144, 272), (127, 4096), (1008, 130), (300, 1024)])
+@pytest.mark.parametrize("off", [0, 5])
+def test_transpose_copy_edges(rows, cols, off):
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    src = torch.randint(0, 256, (rows * cols + off,), dtype=torch.uint8, device="cuda", generator=gen)[off:].view(rows, cols)
+    buf = torch.full((rows * cols + 32,), 77, dtype=torch.uint8, device="cuda")
+    dst = buf[off: off + rows * cols].view(cols, rows)
+    ck.transpose_copy(src, dst)
+    assert torch.equal(dst, src.t().contiguous())
+    assert bool((buf[:off] == 77).all()) and bool((buf[off + rows * cols:] == 77).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [1, 7, 16, 17, 2047, 4096 * 8 + 3, 1 << 20])
+@pytest.mark.parametrize("off", [0, 1])
+def test_amax_and_cast_edges(dtype, n, off):
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    t = torch.randn(n + off, device="cuda", generator=gen).to(dtype)[off:]
+    for at in {0, n - 1, n // 2}:             # the largest value in the first, the last and a middle place
+        u = t.clone() if off == 0 else torch.cat([t[:1], t])[1:]
+        u[at] = -9.0
+        assert float(ck.amax_scale(u)) == float(u.float().abs().max().cpu() / 448)      # (a true division; torch multiplies by 1 / 448 on the GPU)
+    for scale in (0.0123, ck.amax_scale(u)):
+        assert torch.equal(ck.quantize_e4m3(u, scale).view(torch.uint8), u.div(scale).to(torch.float8_e4m3fn).view(torch.uint8))
