@@ -482,7 +482,7 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
       if (a->x_dtype == SCE_F32) prep_x_bf16_kernel<float><<<grid, 256, 0, st>>>((const float*)a->x, a->x_ld, N, d, (uint16_t*)xq, S.Np, S.dp / 2, S.ldx / 2);
       else if (a->x_dtype == SCE_BF16) prep_x_bf16_kernel<bf16_t><<<grid, 256, 0, st>>>((const bf16_t*)a->x, a->x_ld, N, d, (uint16_t*)xq, S.Np, S.dp / 2, S.ldx / 2);
       else return fail(SCE_EINVAL, "unsupported x dtype %d", a->x_dtype);
-      dim3 gw((unsigned)(S.Vp / 64), (unsigned)(S.dp / 2 / 64));
+      dim3 gw((unsigned)(S.Vp / 128), (unsigned)(S.dp / 2 / PREP_W_ROWS));
       if (a->w_dtype == SCE_F32) prep_w_bf16_kernel<float><<<gw, 256, 0, st>>>((const float*)a->w, a->w_ld, d, V, (uint16_t*)wqt, S.ldx / 2);
       else if (a->w_dtype == SCE_BF16) prep_w_bf16_kernel<bf16_t><<<gw, 256, 0, st>>>((const bf16_t*)a->w, a->w_ld, d, V, (uint16_t*)wqt, S.ldx / 2);
       else return fail(SCE_EINVAL, "unsupported w dtype %d", a->w_dtype);

@@ -255,6 +255,28 @@ __global__ __launch_bounds__(256) void quantize_w_kernel(const T* __restrict__ w
 }
 
 // bf16 operands (the eval head, tiny/train.py:741 under bf16 autocast): no quantisation, only the layout.
+// 8 consecutive elements as bf16 bits; `vec`: all 8 are there and the run is 16-byte aligned.  Elements at or beyond `valid` are 0.
+template <typename T>
+__device__ __forceinline__ v4i load8_bf16(const T* __restrict__ p, int64_t valid, bool vec) {
+  if constexpr (sizeof(T) == 2) {
+    if (vec) return *reinterpret_cast<const v4i*>(p);
+  }
+  uint32_t out[4] = {0, 0, 0, 0};
+  if (vec) {
+    const v4f a = *reinterpret_cast<const v4f*>(p), b = *reinterpret_cast<const v4f*>(p + 4);
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      out[m] = (uint32_t)float_to_bf16_bits(a[2 * m]) | ((uint32_t)float_to_bf16_bits(a[2 * m + 1]) << 16);
+      out[2 + m] = (uint32_t)float_to_bf16_bits(b[2 * m]) | ((uint32_t)float_to_bf16_bits(b[2 * m + 1]) << 16);
+    }
+  } else {
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+      if (m < valid) out[m >> 1] |= (uint32_t)float_to_bf16_bits(Elem<T>::load(p + m)) << (16 * (m & 1));
+  }
+  return (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
+}
+
 // dst [rows_p][cols_p] bf16 = src [rows][cols] rounded to bf16 (RNE, as autocast's cast), zero outside; 8 outputs per thread.
 template <typename T>
 __global__ __launch_bounds__(256) void prep_x_bf16_kernel(const T* __restrict__ src, int64_t ld, int64_t rows, int64_t cols,
@@ -263,33 +285,62 @@ __global__ __launch_bounds__(256) void prep_x_bf16_kernel(const T* __restrict__ 
   const int64_t total = rows_p * chunks_per_row;
   for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
     const int64_t r = q / chunks_per_row, c0 = (q - r * chunks_per_row) * 8;
-    uint32_t out[4] = {0, 0, 0, 0};
-    if (r < rows) {
-#pragma unroll
-      for (int m = 0; m < 8; ++m) {
-        const uint32_t h = (c0 + m < cols) ? float_to_bf16_bits(Elem<T>::load(src + r * ld + c0 + m)) : 0u;
-        out[m >> 1] |= h << (16 * (m & 1));
-      }
+    v4i out = (v4i){0, 0, 0, 0};
+    if (r < rows && c0 < cols) {
+      const T* p = src + r * ld + c0;
+      out = load8_bf16<T>(p, cols - c0, cols - c0 >= 8 && ((uintptr_t)p & 15) == 0);
     }
-    *reinterpret_cast<v4i*>(dst + r * dst_ld + c0) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
+    *reinterpret_cast<v4i*>(dst + r * dst_ld + c0) = out;
   }
 }
 
-// W (d, V) -> W^T [Vp][dp2 / 2] in bf16 (row stride ldw elements); 64 x 64 tiles through LDS.
+// W (d, V) -> W^T [Vp][dp2 / 2] in bf16 (row stride ldw elements), in tiles of 64 rows x 128 columns through LDS: loads and stores of 16
+// bytes, whole 256-byte pieces of the rows of W and whole 128-byte lines of W^T.  The transposing read (ds_read_b64_tr_b16: of the 4 x 16
+// matrix that 16 lanes point at, 8 bytes each, lane i gets column i) hands a lane eight rows of its column in two reads.
+// HBM-bound, 4 bytes an element from bf16: 2560 x 50304 in 197 us with an element to an access (2.6 TB/s), 163 with 16-byte
+// accesses and tiles of 128 rows (36 KB of LDS leave a CU four workgroups), 88 with these (5.8 TB/s, eight workgroups).
+constexpr int PREP_W_ROWS = 64;
 template <typename T>
 __global__ __launch_bounds__(256) void prep_w_bf16_kernel(const T* __restrict__ w, int64_t ld, int64_t d, int64_t V,
                                                          uint16_t* __restrict__ wt, int64_t ldw) {
-  __shared__ uint16_t tile[64][66];
+  constexpr int TILE = 128, TJ = PREP_W_ROWS, PITCH = 2 * TILE + 32;
+  __shared__ __attribute__((aligned(16))) uint8_t tile[TJ * PITCH];
   const int t = threadIdx.x;
-  const int64_t j0 = (int64_t)blockIdx.y * 64, v0 = (int64_t)blockIdx.x * 64;
-  for (int e = t; e < 64 * 64; e += 256) {
-    const int r = e >> 6, c = e & 63;
-    tile[r][c] = (j0 + r < d && v0 + c < V) ? float_to_bf16_bits(Elem<T>::load(w + (j0 + r) * ld + v0 + c)) : (uint16_t)0;
+  const int64_t j0 = (int64_t)blockIdx.y * TJ, v0 = (int64_t)blockIdx.x * TILE;
+  const bool aligned = ((reinterpret_cast<uintptr_t>(w) | (uintptr_t)(ld * (int64_t)sizeof(T))) & 15) == 0;
+  {
+    v4i x[TJ / 16];
+    const int64_t v = v0 + (t & 15) * 8;
+#pragma unroll
+    for (int pass = 0; pass < TJ / 16; ++pass) {
+      const int64_t j = j0 + (t >> 4) + 16 * pass;
+      x[pass] = (v4i){0, 0, 0, 0};
+      if (j < d && v < V) x[pass] = load8_bf16<T>(w + j * ld + v, V - v, aligned && v + 8 <= V);
+    }
+#pragma unroll
+    for (int pass = 0; pass < TJ / 16; ++pass) *reinterpret_cast<v4i*>(tile + ((t >> 4) + 16 * pass) * PITCH + (t & 15) * 16) = x[pass];
   }
   __syncthreads();
-  for (int e = t; e < 64 * 64; e += 256) {
-    const int vr = e >> 6, jc = e & 63;
-    wt[(v0 + vr) * ldw + j0 + jc] = tile[jc][vr];
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4s lds_v4s;
+  const int lane = t & 63, wave = t >> 6, g = lane >> 4, i = lane & 15;
+#pragma unroll
+  for (int vb = 0; vb < 2; ++vb) {
+    const int vc = wave * 32 + vb * 16;                        // 16 columns of the tile, one for each lane of a group
+#pragma unroll
+    for (int s = 0; s < TJ / 32; s += 2) {                     // rows 32 s + 8 g on, and 32 (s + 1) + 8 g on
+      v4i q[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const uint8_t* src = tile + (32 * (s + u) + 8 * g + (i >> 2)) * PITCH + 2 * vc + 8 * (i & 3);
+        const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)src));
+        const v2i hi = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src + 4 * PITCH)));
+        q[u] = (v4i){lo[0], lo[1], hi[0], hi[1]};
+      }
+      uint16_t* dst = wt + (v0 + vc + i) * ldw + j0 + 32 * s + 8 * g;
+      *reinterpret_cast<v4i*>(dst) = q[0];
+      *reinterpret_cast<v4i*>(dst + 32) = q[1];
+    }
   }
 }
 
