@@ -301,6 +301,114 @@ __global__ __launch_bounds__(256) void fwd_sample_kernel(FwdParams p_in, int ct,
   }
 }
 
+// The same numbers, bit for bit, for a forward pass of few rows, where one workgroup to a row tile leaves most of the chip idle and
+// walks two K loops one behind the other at the latency of memory.  Here a workgroup has 32 rows, and each
+// of its eight waves two blocks of 32 columns (waves 0 - 3 of the sampled tile, 4 - 7 of the targets'): fragments straight
+// from memory to registers, four steps ahead.  A fragment holds the same bytes in the same registers and an accumulator
+// block adds up in the same order as in mfma_mainloop.  The price is that every 32 rows read all 512 rows of W_q^T again, from L2,
+// in pieces of 16 bytes, so it is used up to SAMPLE_FEW_TILES row tiles (one workgroup to a CU).  Measured, V = 50304, against
+// fwd_sample_kernel: d = 1024 25.6 us for 39.4 (2048 rows), 28.5 for 46.7 (8192), but 55.4 for 51.5 (16384); d = 2560 55.8 for 61.5,
+// 61.2 for 82.9, and 121 for 92; d = 256, V = 4096, 1000 rows 11 for 28.5; without the boosts, 8192 rows of d = 2560, 18 for 41.
+// BOOST = false: only the band of the target logits is computed: wave 0 the blocks on the diagonal and right of it, wave 1
+// (a second wave only if there are several offsets) the last block of the first tile for the last rows of a row tile.
+constexpr int SAMPLE_FEW_ROWS = 32, SAMPLE_FEW_TILES = 32;
+template <bool BOOST>
+__global__ __launch_bounds__(512) void fwd_sample_few_kernel(FwdParams p_in, int ct, float* __restrict__ lam_out) {
+  __shared__ float gmins[4][SAMPLE_FEW_ROWS], tops[8][SAMPLE_FEW_ROWS];
+  FwdParams p = p_in;
+  if (p.dc) { p.sc = p.dc->sc; p.k1 = p.dc->k1; }
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), h = lane >> 5;
+  const int rt = blockIdx.x >> 3, rb = blockIdx.x & 7;          // row tile, block of 32 rows in it
+  const int ntail = p.n_predict - 1;
+  const bool second = BOOST ? wave >= 4 : wave == 0;            // this wave's columns are the targets
+  const int ab[2] = {BOOST ? 2 * (wave & 3) : second ? rb : 6, BOOST ? 2 * (wave & 3) + 1 : second ? min(rb + 1, 7) : 7};
+  if (!BOOST && !second && rb != 7) return;
+  auto target_of = [&](int row) { return row < p.N ? p.targets[row] : p.ignore_index; };
+  auto column_of = [&](int64_t y) { return (y != p.ignore_index && y >= 0 && y < p.V) ? (int)y : 0; };
+  auto row_of_w = [&](int j) {                                   // the row of W^T that column j of the wave's tile is
+    const int q = j - (256 - ntail);
+    if (second) return column_of(target_of(rt * 256 + j));
+    return q < 0 ? ct * 256 + j : column_of(target_of(rt * 256 + 256 + q));
+  };
+  const int i = rb * 32 + (lane & 31);                           // the lane's row in the row tile
+  const uint8_t* xr = p.xq + (int64_t)(rt * 256 + i) * p.ldx + 32 * h;
+  const uint8_t* wr0 = p.wqt + (int64_t)row_of_w(ab[0] * 32 + (lane & 31)) * p.ldx + 32 * h;
+  const uint8_t* wr1 = p.wqt + (int64_t)row_of_w(ab[1] * 32 + (lane & 31)) * p.ldx + 32 * h;
+  bool dead = true;
+  if (BOOST && wave == 0)
+    for (int k = 0; k < p.n_predict; ++k) dead = dead && !(rt * 256 + i < p.N && target_valid(p.targets, p.ignore_index, rt * 256 + i + k, p.N, p.V));
+  typedef int v8i_16 __attribute__((ext_vector_type(8), aligned(16)));
+  constexpr int AHEAD = 4;                                       // steps of 64 bytes; the K extent is a multiple of 256
+  v8i fx[AHEAD], fw[AHEAD][2];
+  auto load = [&](int u, int64_t k) {
+    fx[u] = *reinterpret_cast<const v8i_16*>(xr + k);
+    fw[u][0] = *reinterpret_cast<const v8i_16*>(wr0 + k);
+    fw[u][1] = *reinterpret_cast<const v8i_16*>(wr1 + k);
+  };
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) load(u, 64 * u);
+  v16f acc[2];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) { acc[0][r] = 0.f; acc[1][r] = 0.f; }
+  for (int64_t k = 0; k < p.dp; k += 64 * AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int a = 0; a < 2; ++a) acc[a] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fw[u][a], fx[u], acc[a], 0, 0, 0, 0, 0, 0);
+      if (k + 64 * AHEAD < p.dp) load(u, k + 64 * (AHEAD + u));
+    }
+  }
+  // element (row i, column j) of the wave's tile is in register r of block a: j = 32 ab[a] + 8 (r / 4) + 4 h + r % 4
+  if (second) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+      if (ab[a] == rb || ab[a] == rb + 1)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int k = 32 * ab[a] + 8 * (r >> 2) + 4 * h + (r & 3) - i;
+          if (k >= 0 && k < p.n_predict) p.s_uy[(int64_t)k * p.Np + rt * 256 + i] = acc[a][r] * p.sc;
+        }
+  } else if (rb == 7 && ab[1] == 7) {                            // the next row tile's targets: columns 256 - ntail on of the first tile
+#pragma unroll
+    for (int r = 12; r < 16; ++r) {
+      const int j = 252 + (r & 3), k = 256 + (j - (256 - ntail)) - i;
+      if (h == 1 && j >= 256 - ntail && k >= 1 && k < p.n_predict) p.s_uy[(int64_t)k * p.Np + rt * 256 + i] = acc[1][r] * p.sc;
+    }
+  }
+  if (!BOOST) return;
+  const int vlim = second ? 256 : min(p.V - ct * 256, 256 - ntail);
+  float gmin = INFINITY, top = -INFINITY;
+#pragma unroll
+  for (int a = 0; a < 2; ++a) {
+    float sum = 0.f, cnt = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float pt = fast_exp2(fast_rcp(fmaf(fast_exp2(acc[a][r] * p.k1), p.ic2, p.ic2)));
+      const bool live = 32 * ab[a] + 8 * (r >> 2) + 4 * h + (r & 3) < vlim;
+      sum += live ? pt : 0.f;
+      cnt += live ? 1.f : 0.f;
+      top = live ? fmaxf(top, acc[a][r]) : top;
+    }
+    if (cnt > 0.f) gmin = fminf(gmin, sum / cnt);
+  }
+  gmin = fminf(gmin, __shfl_xor(gmin, 32));
+  top = fmaxf(top, __shfl_xor(top, 32));
+  if (h == 0) {
+    if (!second) gmins[wave][lane] = gmin;
+    tops[wave][lane] = top;
+  }
+  __syncthreads();
+  if (wave == 0 && h == 0) {
+    for (int w = 1; w < 4; ++w) gmin = fminf(gmin, gmins[w][lane]);
+    for (int w = 1; w < 8; ++w) top = fmaxf(top, tops[w][lane]);
+    const float peak = fast_exp2(fast_rcp(fmaf(fast_exp2(top * p.k1), p.ic2, p.ic2)));
+    float l = floorf(-log2f(fmaxf((float)p.V * gmin, peak)));
+    l = l > -64.f ? (l < 120.f ? l : 120.f) : -64.f;
+    lam_out[rt * 256 + i] = dead ? -64.f : (l == l ? l : 0.f);
+  }
+}
+
 // The target entries of the dlogits that a forward pass has emitted are set to zero: they take no part in D (their
 // share goes into the one-hot coefficient in fp32, see bwd_prep_kernel).  One thread per row.
 __global__ __launch_bounds__(256) void fwd_knock_kernel(uint8_t* __restrict__ ghat, int64_t kbv, const int64_t* __restrict__ targets,

@@ -536,7 +536,10 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
     KernelTimer tm(SCE_K_QUANT, st);
     float* lam = (float*)(sv + S.off_lam);
     p.lam = lam;
-    if (!bf16ops && emit) {
+    const bool few = pre && RT <= SAMPLE_FEW_TILES;
+    if (few && emit) fwd_sample_few_kernel<true><<<8 * RT, 512, 0, st>>>(p, CT / 2, lam);
+    else if (few) fwd_sample_few_kernel<false><<<8 * RT, a->shape.n_predict > 1 ? 128 : 64, 0, st>>>(p, CT / 2, lam);
+    else if (!bf16ops && emit) {
       if (pre) fwd_sample_kernel<true><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2, lam);
       else fwd_sample_kernel<false><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2, lam);
     } else if (pre) fwd_sample_kernel<true, false><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2, lam);
