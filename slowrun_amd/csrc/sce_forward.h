@@ -596,6 +596,180 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
   }
 }
 
+// The bf16 forward pass of few rows (scoring one short text): W (d, V) read as it lies, once, without the transposed copy.
+// What bounds it is that read (2 bytes an element); the copy costs as many bytes again in each direction and a second
+// read.  One workgroup to 256 columns (the split of fwd_splits), each of its eight waves to 32 of them and all 32 NB rows.
+// The whole LDS is a ring of FEW_K-deep slices of W and x, filled by direct loads up to STAGES - 1 slices ahead, with one barrier a slice.  K runs along the rows of W, so the A fragments come through the transposing read: ds_read_b64_tr_b16 gives lane i
+// of 16 column i of the 4 x 16 matrix that the 16 lanes point at, four K values, and two reads the eight of an instruction.
+// d is a multiple of 16, the K of one instruction: the last slice may be half a one, and nothing is padded.
+// In a slice the pair of 16-byte chunks c / 2 of W's row k lies at position (c / 2) ^ (k & 3), chunk c of a row of x at
+// c ^ (row / 2 & 3): the rows that one read touches would otherwise lie in the same banks.
+// 61 rows, d = 2560, V = 50304: copy 88 us and general kernel 86, now 44.7 (5.8 TB/s).  The whole pass, copy and general kernel
+// against this: 200 us against 51 (64 rows), 66 (128) and 101 (256); d = 4096, V = 4096, where 16 workgroups do it all:
+// 95 against 64 and 81, but 97 against 125 for 256 rows (a CU's LDS reads are the bound then): beyond 128 rows only with
+// FEW_TILES column tiles, half as many as there are CUs; d = 512, V = 8192: 36 against 18 and 23.
+constexpr int FEW_K = 32;
+constexpr int FEW_MAX_ROWS = 256, FEW_TILES = 128, FEW_THREADS = 512;
+template <int NB>
+struct FewRows {
+  static constexpr int W_BYTES = FEW_K * 512, STAGE = W_BYTES + NB * 2048, STAGES = NB == 2 ? 7 : NB == 4 ? 6 : 4;
+  static constexpr int XL = NB == 8 ? 2 : 1, LOADS = 2 + XL;      // direct loads of a wave per slice (NB = 2: the second four waves load x again)
+  static constexpr int TGT_OFF = STAGES * STAGE, SMEM = TGT_OFF + 4 * 32 * NB * 4;
+  static_assert(SMEM <= SMEM_MAX && (STAGES - 2) * LOADS < 64, "LDS, and what s_waitcnt can count");
+};
+struct FewParams {
+  const uint8_t* x;        // bf16, row stride x_ldb bytes
+  const uint8_t* w;        // bf16 (d, Vw), row stride w_ldb bytes; 16-byte aligned rows, Vw a multiple of 8
+  int64_t x_ldb, w_ldb;
+  int d, Vw;
+};
+
+template <int NB>
+__global__ __launch_bounds__(FEW_THREADS) void fwd_few_rows_kernel(FwdParams p, FewParams f) {
+  using F = FewRows<NB>;
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), h = lane >> 5;
+  const int ct0 = (int)((int64_t)p.CT * blockIdx.x / p.S), ct1 = (int)((int64_t)p.CT * (blockIdx.x + 1) / p.S);
+  int* tgt = reinterpret_cast<int*>(smem + F::TGT_OFF);           // [4 offsets][32 NB]
+  for (int e = threadIdx.x; e < p.n_predict * 32 * NB; e += FEW_THREADS) {
+    const int row = e % (32 * NB), i = row + e / (32 * NB);
+    tgt[e] = (row < p.N && target_valid(p.targets, p.ignore_index, i, p.N, p.V)) ? (int)p.targets[i] : -1;
+  }
+  __syncthreads();
+  const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem);
+  // W: load n of a wave is rows 4 wave + 2 n and + 1 of the slice, 32 chunks each; x: load q is 16 rows of 4 chunks
+  auto xload = [&](int n) { return NB == 2 ? wave & 3 : wave * F::XL + n; };
+  uint32_t xo[F::XL];
+  const int xc = (lane & 3) ^ ((lane >> 3) & 3);
+#pragma unroll
+  for (int n = 0; n < F::XL; ++n) xo[n] = (uint32_t)(min(xload(n) * 16 + (lane >> 2), p.N - 1) * f.x_ldb + xc * 16);
+  const uint32_t xhalf = (xc & 2) ? 32u : 0u;                     // the last slice's second half does not exist: its first half again
+  uint32_t wo[2];
+  auto columns = [&](int ct) {                                    // (the last tile may reach beyond W: its last chunk again)
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int pc = lane & 31, c = (((pc >> 1) ^ ((2 * n + h) & 3)) << 1) | (pc & 1);
+      wo[n] = (uint32_t)((wave * 4 + 2 * n + h) * f.w_ldb + 2 * min(ct * 256 + c * 8, f.Vw - 8));
+    }
+  };
+  const int nk = (f.d + FEW_K - 1) / FEW_K, total = (ct1 - ct0) * nk;
+  const bool half_slice = f.d % FEW_K != 0;
+  int ict = ct0, ik = 0, islot = 0;                               // the slice that is loaded next
+  auto issue = [&]() {
+    if (ik == 0) columns(ict);
+    const bool tail = half_slice && ik == nk - 1;
+    const uint8_t* wb = f.w + (int64_t)(ik * FEW_K - (tail && wave >= 4 ? 16 : 0)) * f.w_ldb;
+    const uint8_t* xb = f.x + (int64_t)ik * (2 * FEW_K);
+    const uint32_t l = lds0 + islot * F::STAGE;
+    lds_direct_16<0>(l + wave * 2048, wo[0], wb);
+    lds_direct_16<1024>(l + wave * 2048, wo[1], wb);
+#pragma unroll
+    for (int n = 0; n < F::XL; ++n) lds_direct_16<F::W_BYTES>(l + xload(n) * 1024, xo[n] - (tail ? xhalf : 0u), xb);
+    if (++ik == nk) { ik = 0; ++ict; }
+    if (++islot == F::STAGES) islot = 0;
+  };
+#pragma unroll 1
+  for (int g = 0; g < F::STAGES - 1 && g < total; ++g) issue();
+  float sum[NB], amax[NB];
+  int uarg[NB];
+#pragma unroll
+  for (int b = 0; b < NB; ++b) { sum[b] = 0.f; amax[b] = -INFINITY; uarg[b] = 0x7fffffff; }
+  v16f acc[NB];
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4s lds_v4s;
+  const int i16 = lane & 15, g4 = lane >> 4;                      // group g4 of 16 lanes: columns 16 (g4 & 1) on, K values 8 (g4 / 2) on
+  int slot = 0, done = 0;
+#pragma unroll 1
+  for (int ct = ct0; ct < ct1; ++ct) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[b][r] = 0.f;
+#pragma unroll 1
+    for (int k = 0; k < nk; ++k, ++done) {
+      // this wave's loads of the slice have landed and its reads of the one before are complete; after the barrier that holds
+      // for every wave, and the slot of the slice before is free
+      if (done + F::STAGES - 1 <= total) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((F::STAGES - 2) * F::LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (done + F::STAGES - 1 < total) issue();
+      const uint8_t* ws = smem + slot * F::STAGE;
+      const uint8_t* xs = ws + F::W_BYTES;
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {                               // 16 K values
+        v8bf fa, fb[NB];
+        if (s == 1 && half_slice && k == nk - 1) {                // not there: products of zeros (a branch around the MFMAs would have the accumulators moved in every slice)
+          fa = __builtin_bit_cast(v8bf, (v4i){0, 0, 0, 0});
+#pragma unroll
+          for (int b = 0; b < NB; ++b) fb[b] = fa;
+        } else {
+          const int kr = 16 * s + 8 * (g4 >> 1) + (i16 >> 2), pair = wave * 2 + (g4 & 1);      // (32 bytes of columns)
+          const uint8_t* src = ws + kr * 512 + ((pair ^ (kr & 3)) << 5) + 8 * (i16 & 3);
+          const v2i lo = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)src));
+          const v2i hi = __builtin_bit_cast(v2i, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s*)(src + 4 * 512)));
+          fa = __builtin_bit_cast(v8bf, (v4i){lo[0], lo[1], hi[0], hi[1]});
+#pragma unroll
+          for (int b = 0; b < NB; ++b) {
+            const int r = b * 32 + (lane & 31);
+            fb[b] = __builtin_bit_cast(v8bf, *reinterpret_cast<const v4i*>(xs + r * 64 + (((2 * s + h) ^ ((r >> 1) & 3)) << 4)));
+          }
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa, fb[b], acc[b], 0, 0, 0);
+      }
+      if (++slot == F::STAGES) slot = 0;
+    }
+    // the lane's 16 columns of a row: v0 + 8 (r / 4) + r % 4; logits rounded to bf16 as the eager head's GEMM returns them
+    const int v0 = ct * 256 + wave * 32 + 4 * h;
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      __builtin_amdgcn_sched_barrier(0);                          // one row block at a time
+      const int row = b * 32 + (lane & 31);
+      float s = 0.f;
+      int arg = -1;
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int v = 8 * (r >> 2) + (r & 3);
+        float x = round_to_bf16_hw(acc[b][r]), pt = fast_exp2(fast_rcp(fmaf(fast_exp2(x * p.k1), p.ic2, p.ic2)));
+        if (v >= p.V - v0) { pt = 0.f; x = -INFINITY; }
+        s += pt;
+        if (x > amax[b]) { amax[b] = x; arg = v; }                // ascending columns: the lowest wins
+      }
+      if (arg >= 0) uarg[b] = v0 + arg;
+      sum[b] += s;
+      for (int k = 0; k < p.n_predict; ++k) {
+        const int rel = tgt[k * 32 * NB + row] - v0;
+        if ((unsigned)rel < 32u && (rel & 4) == 0) {
+          float x = 0.f;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) x = rel == 8 * (r >> 2) + (r & 3) ? acc[b][r] : x;
+          p.s_uy[(int64_t)k * p.Np + row] = round_to_bf16_hw(x) * p.sc;
+        }
+      }
+    }
+  }
+  // fold the two half-waves and the eight waves: all hold different columns of the same rows
+  __syncthreads();
+  float4* red = reinterpret_cast<float4*>(smem);                  // [8 waves][32 NB]
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    const float s2 = __shfl_xor(sum[b], 32), um2 = __shfl_xor(amax[b], 32);
+    const int ua2 = __shfl_xor(uarg[b], 32);
+    sum[b] += s2;
+    if (um2 > amax[b] || (um2 == amax[b] && ua2 < uarg[b])) { amax[b] = um2; uarg[b] = ua2; }
+    if (h == 0) red[wave * 32 * NB + b * 32 + lane] = make_float4(sum[b], amax[b], __int_as_float(uarg[b]), 0.f);
+  }
+  __syncthreads();
+  if (threadIdx.x < 32 * NB) {
+    float4 o = red[threadIdx.x];
+    for (int w = 1; w < 8; ++w) {
+      const float4 q = red[w * 32 * NB + threadIdx.x];
+      o.x += q.x;
+      if (q.y > o.y || (q.y == o.y && __float_as_int(q.z) < __float_as_int(o.z))) { o.y = q.y; o.z = q.z; }
+    }
+    p.partials[(int64_t)blockIdx.x * p.Np + threadIdx.x] = make_float4(o.x, o.y * p.sc, o.z, 0.f);
+  }
+}
+
 // What a block of COMBINE_ROWS rows contributes to the mean loss: left by fwd_combine_kernel in the first 16 bytes of the
 // block's own rows of the partial records (which it has consumed by then), summed by fwd_reduce_kernel.
 struct BlockLoss {

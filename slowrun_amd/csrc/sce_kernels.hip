@@ -148,6 +148,9 @@ static int check_device(int dev) {
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_sample_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_SAMPLE));
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_sample_kernel<true, false>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_SAMPLE));
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_kernel<false, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_FWD));
+      HIP_TRY(hipFuncSetAttribute((const void*)fwd_few_rows_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, FewRows<2>::SMEM));
+      HIP_TRY(hipFuncSetAttribute((const void*)fwd_few_rows_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, FewRows<4>::SMEM));
+      HIP_TRY(hipFuncSetAttribute((const void*)fwd_few_rows_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, FewRows<8>::SMEM));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_recompute_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_RECOMPUTE));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dx_kernel<float, false>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dx_kernel<bf16_t, false>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
@@ -475,13 +478,22 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   const bool devsc = a->x_s_dev || a->w_s_dev;
   DevConsts* dcp = devsc ? (DevConsts*)(sv + S.off_hdr + 32) : nullptr;
   const float inv_xs = a->x_s_dev ? 0.f : (float)(1.0 / a->x_s), inv_ws = a->w_s_dev ? 0.f : (float)(1.0 / a->w_s);
+  // a bf16 pass of few rows reads W as it lies (and x too) if the kernel's 16-byte loads and 32-bit offsets can: whole
+  // pieces of aligned rows
+  auto direct = [&](const void* q, int32_t dtype, int64_t ld, int64_t rows) {
+    return dtype == SCE_BF16 && ((uintptr_t)q & 15) == 0 && ld % 8 == 0 && ld < ((int64_t)1 << 31) / rows;
+  };
+  const bool few = bf16ops && (N <= 128 || (N <= FEW_MAX_ROWS && CT >= FEW_TILES)) && V % 8 == 0 && direct(a->w, a->w_dtype, a->w_ld, FEW_K);
+  const bool few_x = few && direct(a->x, a->x_dtype, a->x_ld, FEW_MAX_ROWS);
   {
     KernelTimer tm(SCE_K_QUANT, st);
-    if (bf16ops) {
+    if (bf16ops && !few_x) {
       const int grid = grid_for((size_t)S.Np * (S.dp / 16), 256);
       if (a->x_dtype == SCE_F32) prep_x_bf16_kernel<float><<<grid, 256, 0, st>>>((const float*)a->x, a->x_ld, N, d, (uint16_t*)xq, S.Np, S.dp / 2, S.ldx / 2);
       else if (a->x_dtype == SCE_BF16) prep_x_bf16_kernel<bf16_t><<<grid, 256, 0, st>>>((const bf16_t*)a->x, a->x_ld, N, d, (uint16_t*)xq, S.Np, S.dp / 2, S.ldx / 2);
       else return fail(SCE_EINVAL, "unsupported x dtype %d", a->x_dtype);
+    }
+    if (bf16ops && !few) {
       dim3 gw((unsigned)(S.Vp / 128), (unsigned)(S.dp / 2 / PREP_W_ROWS));
       if (a->w_dtype == SCE_F32) prep_w_bf16_kernel<float><<<gw, 256, 0, st>>>((const float*)a->w, a->w_ld, d, V, (uint16_t*)wqt, S.ldx / 2);
       else if (a->w_dtype == SCE_BF16) prep_w_bf16_kernel<bf16_t><<<gw, 256, 0, st>>>((const bf16_t*)a->w, a->w_ld, d, V, (uint16_t*)wqt, S.ldx / 2);
@@ -550,6 +562,14 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
       fwd_kernel<true, false, true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
       fwd_knock_kernel<<<(int)(S.Np / 256), 256, 0, st>>>(p.ghat_t, p.kbv, a->targets, a->ignore_index, (int)N, (int)Vl, a->shape.n_predict);
     } else if (emit) fwd_kernel<true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
+    else if (few) {
+      FewParams f;
+      f.w = (const uint8_t*)a->w; f.w_ldb = a->w_ld * 2; f.d = (int)d; f.Vw = (int)V;
+      f.x = few_x ? (const uint8_t*)a->x : xq; f.x_ldb = few_x ? a->x_ld * 2 : S.ldx;
+      if (N <= 64) fwd_few_rows_kernel<2><<<nsplit, FEW_THREADS, FewRows<2>::SMEM, st>>>(p, f);
+      else if (N <= 128) fwd_few_rows_kernel<4><<<nsplit, FEW_THREADS, FewRows<4>::SMEM, st>>>(p, f);
+      else fwd_few_rows_kernel<8><<<nsplit, FEW_THREADS, FewRows<8>::SMEM, st>>>(p, f);
+    }
     else if (bf16ops) fwd_kernel<false, true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
     else if (pre) fwd_kernel<false, false, true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
     else fwd_kernel<false><<<grid, NTHREADS, SMEM_FWD, st>>>(p);

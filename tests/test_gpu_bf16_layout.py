@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("N,d,V", [(1, 16, 7), (5, 112, 130), (61, 144, 1000), (257, 128, 256), (300, 256, 515)])
+@pytest.mark.parametrize("N,d,V", [(1, 16, 7), (5, 112, 130), (61, 144, 1002), (257, 128, 256), (300, 256, 515)])
 def test_aligned_and_unaligned_rows_give_the_same_loss(dtype, N, d, V):
     from slowrun_amd import cuda_kernels as ck
     gen = torch.Generator(device="cuda").manual_seed(N)
@@ -29,3 +29,30 @@ def test_aligned_and_unaligned_rows_give_the_same_loss(dtype, N, d, V):
     ref = F.cross_entropy(15.0 * torch.tanh(u / 15.0), y, reduction="none")
     assert float((losses[0] - ref).abs().max()) < 8 * 2 ** -8
     assert float((losses[0] - ref).abs().mean()) < 2e-3
+
+
+@pytest.mark.parametrize("xdtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,d,V,vocab,offsets", [(1, 16, 8, 8, 1), (31, 48, 248, 241, 1), (64, 64, 256, 256, 2), (65, 272, 264, 257, 4), (128, 1040, 3000, 2999, 1),
+                                                 (129, 96, 33000, 32990, 3), (256, 528, 32776, 32776, 1), (61, 32, 131072, 131072, 1), (200, 16, 70000, 69999, 1)])
+def test_few_rows_against_the_general_path(xdtype, N, d, V, vocab, offsets):
+    """Few rows (up to 128, or 256 of a large vocabulary) of aligned bf16 weights are read as they lie; the same weights in rows of odd length take the general path.
+    Small whole numbers make every logit exact, whatever the order of its sum: the maximum's column is the same, and the
+    losses differ by the order of the row sums (fp32 sums of at most V positive terms)."""
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(V + N)
+    x = torch.randint(-2, 3, (N, d), device="cuda", generator=gen).to(xdtype) / 4
+    w = torch.randint(-2, 3, (d, V), device="cuda", generator=gen).bfloat16() / 4
+    y = torch.randint(0, vocab, (N,), device="cuda", generator=gen)
+    y[::5] = -1
+    odd = torch.zeros(d, V + 1, device="cuda", dtype=torch.bfloat16)
+    odd[:, :V] = w
+    mtp = torch.tensor([1.0, 0.5, 0.25, 0.125][:offsets], device="cuda")
+    got = [ck.ce_forward(x, m, y, 1.0, 1.0, 15.0, "none", want_argmax=True, mtp_weights=mtp, vocab_size=vocab, operand_dtype=torch.bfloat16)
+           for m in (w, odd[:, :V])]
+    (l0, _, lse0, am0, nv0), (l1, _, lse1, am1, nv1) = got
+    assert torch.equal(am0, am1) and torch.equal(nv0, nv1)
+    assert torch.allclose(lse0, lse1, rtol=2e-6, atol=2e-5) and torch.allclose(l0, l1, rtol=2e-6, atol=2e-5)
+    if offsets == 1:
+        u = (x.float() @ w.float())[:, :vocab].bfloat16().float()
+        ref = F.cross_entropy(15.0 * torch.tanh(u / 15.0), y, reduction="none", ignore_index=-1)
+        assert torch.allclose(l0, ref, rtol=1e-5, atol=1e-4)
