@@ -248,7 +248,7 @@ struct DxParams {
   const float* hcoef;     // [n_predict][Np], offset to the panel
   const int64_t* targets; // offset to the panel
   void* dx;               // offset to the panel's first row
-  float* part;            // [ksplit][RT * 256][dq] fp32 partial sums (ksplit > 1 only)
+  float* part;            // [ksplit][RT][CT] tiles of fp32 partial sums, as dx_part_offset lays them out (ksplit > 1 only)
   int64_t dx_ld, Vp, ldx, Np, dq;        // Vp: K extent; ldx: row stride of wqt
   int64_t kbw;                           // blocks of 128 rows i that gexp counts per block of 128 columns
   int RT, CT, rows, d, V;  // rows: valid rows in this panel
@@ -300,6 +300,12 @@ struct DxRowTerms {
   }
 };
 
+// The partial sums of a tile are private to the two kernels, so they lie as the accumulators do: for every 32 rows x 128 columns
+// (il / 32, wa) the 16 registers quads (a, q) one behind the other, 64 lanes x 16 bytes each -- a wave's store is 1 KB in a row.
+// In row order it was 32 pieces of 32 bytes, and waiting to issue them took two thirds of the kernel at 1000 rows, d = 256,
+// V = 4096: 16.8 -> 12.6 us there, 89.5 -> 86 at 2048 rows, d = 1024, V = 50304.
+__device__ __forceinline__ int64_t dx_part_offset(int64_t tile, int wb, int b, int wa) { return ((tile * 2 + wb) * 4 + b) * 8192 + wa * 4096; }
+
 // SPLIT = false: one workgroup per 256 x 256 tile of dX, whole K loop, finished values stored.
 // SPLIT = true : a panel with too few tiles to fill the chip; each tile's K loop is shared by ksplit
 //                workgroups that store raw fp32 partial sums, and bwd_dx_finish_kernel adds them up.
@@ -309,11 +315,20 @@ __global__ __launch_bounds__(256) void bwd_dx_kernel(DxParams p_in) {
   DxParams p = p_in;
   if (p.dc) p.w_s = p.dc->w_s;
   int rt, ct, ks = 0;
-  if (!map_tile(blockIdx.x, p.RT, SPLIT ? p.CT * p.ksplit : p.CT, rt, ct)) return;
   int64_t k0 = 0;
   int KD = (int)(p.Vp / BK);
-  if (SPLIT) {
-    ks = ct % p.ksplit; ct /= p.ksplit;
+  if (!SPLIT) {
+    if (!map_tile(blockIdx.x, p.RT, p.CT, rt, ct)) return;
+  } else {
+    // The parts of the K loop are the slowest index of the order that the XCDs take eighths of: what one L2 serves is all (or
+    // many) tiles of the panel over one stretch of K, so both operands come through it once and not once for every row
+    // and column of tiles.  With the parts of a tile side by side instead, G was read by four XCDs and W_q by two each
+    // (515 MB instead of 154 at N = 2048, d = 1024, V = 50304): 95.4 -> 89.5 us there.
+    int lin, none;
+    if (!map_tile(blockIdx.x, 1, p.RT * p.CT * p.ksplit, none, lin)) return;
+    ks = __builtin_amdgcn_readfirstlane(lin / (p.RT * p.CT));
+    tile_from_index(lin - ks * (p.RT * p.CT), p.RT, p.CT, rt, ct);
+    rt = __builtin_amdgcn_readfirstlane(rt); ct = __builtin_amdgcn_readfirstlane(ct);
     const int pairs = KD >> 1;
     const int q0 = (int)((int64_t)pairs * ks / p.ksplit), q1 = (int)((int64_t)pairs * (ks + 1) / p.ksplit);
     k0 = (int64_t)q0 * 2 * BK; KD = 2 * (q1 - q0);
@@ -507,12 +522,12 @@ __global__ __launch_bounds__(256) void bwd_dx_kernel(DxParams p_in) {
   for (int b = 0; b < 4; ++b) {
     const int il = rt * 256 + wb * 128 + b * 32 + (lane & 31);
     if (SPLIT) {
-      float* dst = p.part + ((int64_t)ks * p.RT * 256 + il) * p.dq;
+      float* dst = p.part + dx_part_offset(((int64_t)ks * p.RT + rt) * p.CT + ct, wb, b, wa) + lane * 4;
 #pragma unroll
       for (int a = 0; a < 4; ++a)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
-          *reinterpret_cast<v4f*>(dst + jbase + a * 32 + 8 * q) =
+          *reinterpret_cast<v4f*>(dst + (4 * a + q) * 256) =
               (v4f){acc[a][b][4 * q + 0], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
       continue;
     }
@@ -531,20 +546,56 @@ __global__ __launch_bounds__(256) void bwd_dx_kernel(DxParams p_in) {
   }
 }
 
-// sum of the K-split partials, row scale, one-hot term, cast: a thread per (row, four columns)
+// Sum of the K-split partials, row scale, one-hot term, cast: a workgroup per 32 rows x 128 columns, a wave per 32 of the
+// columns.  A thread's values are four quads of one row; they go out through LDS as whole pieces of rows.
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_dx_finish_kernel(DxParams p_in) {
   DxParams p = p_in;
   if (p.dc) p.w_s = p.dc->w_s;
-  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int per_row = p.d / 4;
-  const int il = (int)(q / per_row), j = (int)(q - (int64_t)il * per_row) * 4;
-  if (il >= p.rows) return;
-  v4f sum = (v4f){0.f, 0.f, 0.f, 0.f};
-  for (int ks = 0; ks < p.ksplit; ++ks)      // fixed order
-    sum += *reinterpret_cast<const v4f*>(p.part + ((int64_t)ks * p.RT * 256 + il) * p.dq + j);
-  const DxRowTerms row(p, il);
-  row.store4<T>(p, reinterpret_cast<T*>(p.dx) + (int64_t)il * p.dx_ld + j, j, sum[0], sum[1], sum[2], sum[3]);
+  constexpr int RB = 128 * (int)sizeof(T), PITCH = RB + 16, CH = RB / 16;
+  __shared__ __attribute__((aligned(16))) uint8_t stage[32 * PITCH];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wa = blockIdx.x & 1, b = (blockIdx.x >> 1) & 3, wb = (blockIdx.x >> 3) & 1;
+  const int tile = blockIdx.x >> 4, rt = tile / p.CT, ct = tile - rt * p.CT, i0 = rt * 256 + wb * 128 + b * 32, j0 = ct * 256 + wa * 128;
+  if (i0 >= p.rows || j0 >= p.d) return;
+  v4f sum[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) sum[q] = (v4f){0.f, 0.f, 0.f, 0.f};
+  const float* src = p.part + dx_part_offset(tile, wb, b, wa) + wave * 1024 + lane * 4;
+  const int64_t step = (int64_t)p.RT * p.CT * 65536;
+  for (int k0 = 0; k0 < p.ksplit; k0 += 4) {              // fixed order, the loads of four parts in flight together
+    v4f x[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) x[u][q] = k0 + u < p.ksplit ? *reinterpret_cast<const v4f*>(src + (k0 + u) * step + q * 256) : (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sum[q] += x[u][q];
+  }
+  const int il = i0 + (lane & 31);
+  if (il < p.rows) {
+    const DxRowTerms row(p, il);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int c = wave * 32 + 8 * q + 4 * (lane >> 5);
+      row.store4<T>(p, reinterpret_cast<T*>(stage + (lane & 31) * PITCH) + c, j0 + c, sum[q][0], sum[q][1], sum[q][2], sum[q][3]);
+    }
+  }
+  __syncthreads();
+  T* dx = reinterpret_cast<T*>(p.dx);
+  const bool vec = ((reinterpret_cast<uintptr_t>(p.dx) | (uintptr_t)(p.dx_ld * (int64_t)sizeof(T))) & 15) == 0;
+#pragma unroll
+  for (int n = 0; n < 32 * CH / 256; ++n) {
+    const int e = t + 256 * n, r = e / CH, k = e % CH, col = j0 + k * (16 / (int)sizeof(T));
+    if (i0 + r >= p.rows || col >= p.d) continue;          // (d is a multiple of 16: a piece is in range as a whole)
+    T* dst = dx + (int64_t)(i0 + r) * p.dx_ld + col;
+    const T* from = reinterpret_cast<const T*>(stage + r * PITCH + k * 16);
+    if (vec) *reinterpret_cast<v4i*>(dst) = *reinterpret_cast<const v4i*>(from);
+    else
+#pragma unroll
+      for (int m = 0; m < 16 / (int)sizeof(T); ++m) dst[m] = from[m];
+  }
 }
 
 struct DwParams {
@@ -634,13 +685,14 @@ __global__ __launch_bounds__(256) void bwd_dw_tail_kernel(DwParams p, DwTail tl)
                                                        uniform_ptr(p.ghat_t + ((int64_t)k0 * p.kbv + 2 * ct) * BLOCKED_KSTEP), BLOCKED_KSTEP,
                                                        KD, smem, acc, ct & 7, 2 * (rt & 3), __builtin_amdgcn_readfirstlane(wave), NoHook(), 128 * BK, p.kbv * BLOCKED_KSTEP,
                                                        lsc + __builtin_amdgcn_readfirstlane(wb) * KD);
-  float* dst0 = tl.buf + (size_t)(g + tt) * 65536 + (wa * 128 + 4 * (lane >> 5)) * 256 + wb * 128 + (lane & 31);
+  float* dst0 = tl.buf + (size_t)(g + tt) * 65536 + (wa * 2 + wb) * 16384 + lane * 4;       // as the accumulators lie: [wa][wb][a][b][quad][lane]
 #pragma unroll
   for (int b = 0; b < 4; ++b)
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) dst0[(a * 32 + 8 * (r >> 2) + (r & 3)) * 256 + b * 32] = acc[a][b][r];
+      for (int q = 0; q < 4; ++q)
+        *reinterpret_cast<v4f*>(dst0 + (4 * a + b) * 1024 + q * 256) = (v4f){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
 }
 
 // A column that is the target of at least LONG_SEG rows has its segment of the sorted list cut into
@@ -969,43 +1021,51 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
 
 // The same from fp32 partials: what is left are the tiles of a K-split last round (tl.tile0 >= 0: grid.y = tl.ntail tiles of
 // 16 blocks of 64 x 64 elements), and every tile where dW took more than one launch (grid = blocks of 64 columns x 64
-// rows of dW).  A thread owns one column v and 16 consecutive rows j; the segment sum is formed here for short segments
+// rows of dW).  A thread owns one column v and four groups of four rows j: 16 consecutive rows, or, of the pieces of a K-split
+// tile, the rows that one lane's accumulators of a 32 x 32 block are.  The segment sum is formed here for short segments
 // and read from the chunk sums for long ones.
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restrict__ dwacc, int nparts, int64_t part_stride, int64_t Vp, DwOut o, DwTail tl, int RT,
                                                           int CT) {
   const float x_s = o.dc ? o.dc->x_s : o.x_s;
-  const int t = threadIdx.x;
-  int bx = blockIdx.x, by = blockIdx.y;
-  if (tl.tile0 >= 0) {
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const bool pieces = tl.tile0 >= 0;
+  int v = blockIdx.x * 64 + lane, j0 = blockIdx.y * 64 + wave * 16;
+  int wa = 0, wb = 0, a = 0, b = 0;
+  if (pieces) {
     int rt, ct;
-    tile_from_index(tl.tile0 + by, RT, CT, rt, ct);
-    by = 4 * rt + (bx >> 2); bx = 4 * ct + (bx & 3);
+    tile_from_index(tl.tile0 + blockIdx.y, RT, CT, rt, ct);
+    const int by = blockIdx.x >> 2, bx = blockIdx.x & 3;            // 64 rows and 64 columns of the tile
+    wa = by >> 1; a = 2 * (by & 1) + (wave >> 1); wb = bx >> 1; b = 2 * (bx & 1) + (wave & 1);
+    v = ct * 256 + wb * 128 + b * 32 + (lane & 31);
+    j0 = rt * 256 + wa * 128 + a * 32 + 4 * (lane >> 5);
   }
-  const int v = bx * 64 + (t & 63);
-  const int j0 = by * 64 + (t >> 6) * 16;
+  const int step = pieces ? 8 : 4;                                  // rows from one group of four to the next
   if (v >= o.V || j0 >= o.d) return;
   const float scale = x_s * o.xi[0];
-  float val[16];
-  if (tl.tile0 >= 0) {
+  v4f val[4];
+  if (pieces) {
     const int tt = blockIdx.y, g0 = (tt * tl.kp) / tl.share, g1 = ((tt + 1) * tl.kp - 1) / tl.share;
-    const float* src = tl.buf + (size_t)tt * 65536 + (j0 & 255) * 256 + (v & 255);
+    const float* src = tl.buf + (size_t)tt * 65536 + (wa * 2 + wb) * 16384 + (4 * a + b) * 1024 + lane * 4;
 #pragma unroll
-    for (int m = 0; m < 16; ++m) val[m] = 0.f;
-    for (int g = g0; g <= g1; ++g) {                      // fixed order; the 16 loads of a piece are in flight together
+    for (int q = 0; q < 4; ++q) val[q] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int g = g0; g <= g1; ++g) {                      // fixed order; the loads of a piece are in flight together
 #pragma unroll
-      for (int m = 0; m < 16; ++m) val[m] += src[(size_t)g * 65536 + m * 256];
+      for (int q = 0; q < 4; ++q) val[q] += *reinterpret_cast<const v4f*>(src + (size_t)g * 65536 + q * 256);
     }
-#pragma unroll
-    for (int m = 0; m < 16; ++m) val[m] *= scale;
   } else {
 #pragma unroll
-    for (int m = 0; m < 16; ++m) {
-      float sum = dwacc[(int64_t)(j0 + m) * Vp + v];
-      for (int q = 1; q < nparts; ++q) sum += dwacc[q * part_stride + (int64_t)(j0 + m) * Vp + v];   // fixed order
-      val[m] = sum * scale;
-    }
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const float* src = dwacc + (int64_t)(j0 + 4 * q + m) * Vp + v;
+        float sum = src[0];
+        for (int n = 1; n < nparts; ++n) sum += src[n * part_stride];                                   // fixed order
+        val[q][m] = sum;
+      }
   }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) val[q] *= scale;
   const int s0 = o.segoff[v], L = o.segoff[v + 1] - s0;
   if (L >= LONG_SEG) {
     int nch, len;
@@ -1013,26 +1073,30 @@ __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restri
     for (int c = 0; c < nch; ++c) {                       // fixed order
       const float* ls = o.longsum + (int64_t)(o.longbase[v] + c) * o.dq + j0;
 #pragma unroll
-      for (int m = 0; m < 16; ++m) val[m] -= ls[m] * x_s;
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int m = 0; m < 4; ++m) val[q][m] -= ls[q * step + m] * x_s;
     }
   } else if (L > 0) {
     for (int n = 0; n < L; ++n) {
       const float h = o.sh[s0 + n] * x_s;
-      const v4i raw = *reinterpret_cast<const v4i*>(o.xq + (int64_t)o.srow[s0 + n] * o.ldx + j0);
+      const uint8_t* row = o.xq + (int64_t)o.srow[s0 + n] * o.ldx + j0;
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const uint32_t w = (uint32_t)raw[m];
-        val[4 * m + 0] -= h * e4m3_to_float<0>(w);
-        val[4 * m + 1] -= h * e4m3_to_float<1>(w);
-        val[4 * m + 2] -= h * e4m3_to_float<2>(w);
-        val[4 * m + 3] -= h * e4m3_to_float<3>(w);
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(row + q * step);
+        val[q][0] -= h * e4m3_to_float<0>(w);
+        val[q][1] -= h * e4m3_to_float<1>(w);
+        val[q][2] -= h * e4m3_to_float<2>(w);
+        val[q][3] -= h * e4m3_to_float<3>(w);
       }
     }
   }
   T* dw = reinterpret_cast<T*>(o.dw);
 #pragma unroll
-  for (int m = 0; m < 16; ++m)
-    if (j0 + m < o.d) Elem<T>::store(dw + (int64_t)(j0 + m) * o.dw_ld + v, val[m]);
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      if (j0 + q * step + m < o.d) Elem<T>::store(dw + (int64_t)(j0 + q * step + m) * o.dw_ld + v, val[q][m]);
 }
 
 }  // namespace sce

@@ -769,7 +769,7 @@ extern "C" int sce_backward(const sce_args* a) {
       if (dx_f32) bwd_dx_kernel<float, false><<<map_tile_grid(dp_.RT, CTd), NTHREADS, smem_dx, st>>>(dp_);
       else bwd_dx_kernel<bf16_t, false><<<map_tile_grid(dp_.RT, CTd), NTHREADS, smem_dx, st>>>(dp_);
     } else if (dp_.rows > 0) {
-      const int fgrid = (int)(((int64_t)dp_.rows * (d / 4) + 255) / 256);
+      const int fgrid = tiles * 16;
       if (dx_f32) {
         bwd_dx_kernel<float, true><<<map_tile_grid(dp_.RT, CTd * ksplit), NTHREADS, smem_dx, st>>>(dp_);
         bwd_dx_finish_kernel<float><<<fgrid, 256, 0, st>>>(dp_);
