@@ -8,6 +8,45 @@ namespace sce {
 // ------------------------------------------------------------------------------------------
 // backward
 // ------------------------------------------------------------------------------------------
+// Up to RANK_MAX (offset, row) entries are put in the order of their targets by counting: entry e goes to the place that is
+// the number of entries before it, n compares spread over 16 lanes, all n keys in LDS.  (target, e) is one 32-bit number, so ties
+// keep their order, as in the radix sort that larger calls use.  That sort is 3 to 4 launches of 4.8 us each whatever
+// the size (20 us at 2048 entries, 16 at 4096); this is blocks of bwd_prep_kernel's own launch, for it needs nothing but the targets, and
+// takes that kernel from 5 us to 7 and 9.8.  n^2 grows past the sort soon after.
+constexpr int RANK_BITS = 12, RANK_MAX = 1 << RANK_BITS, RANK_PER_BLOCK = 16;
+__device__ __forceinline__ void rank_targets(uint32_t* keys, int block, const int64_t* __restrict__ targets, int64_t ignore_index, int N, int Np, int V,
+                                             int32_t key_none, int n_predict, int32_t* __restrict__ skeys, int32_t* __restrict__ perm) {
+  const int n = N * n_predict, n64 = (n + 63) & ~63, t = threadIdx.x;
+  for (int e0 = t; e0 < n64; e0 += 8 * 256) {
+    int64_t y[8];                        // (eight loads in flight: one at a time they were the whole time, 13 us for 4096 entries)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = e0 + 256 * u, k = e / N, i = e - k * N + k;
+      y[u] = e < n && i < N ? targets[i] : ignore_index;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = e0 + 256 * u;
+      const uint32_t key = y[u] != ignore_index && y[u] >= 0 && y[u] < V ? (uint32_t)y[u] : (uint32_t)key_none;
+      if (e < n64) keys[e] = e < n ? (key << RANK_BITS) | (uint32_t)e : ~0u;
+    }
+  }
+  __syncthreads();
+  const int e = block * RANK_PER_BLOCK + (t >> 4);
+  const uint32_t mine = e < n ? keys[e] : 0u;
+  int before = 0;
+  for (int q = 4 * (t & 15); q < n64; q += 64) {
+    const uint4 c = *reinterpret_cast<const uint4*>(keys + q);
+    before += (c.x < mine) + (c.y < mine) + (c.z < mine) + (c.w < mine);
+  }
+#pragma unroll
+  for (int o = 8; o > 0; o >>= 1) before += __shfl_xor(before, o);
+  if ((t & 15) == 0 && e < n) {
+    skeys[before] = (int32_t)(mine >> RANK_BITS);
+    perm[before] = (e / N) * Np + e % N;
+  }
+}
+
 // per row: rho (row factor of the block-scaled dlogits) and h_k (one-hot coefficients).
 //   dz_iv = g_i ( S_i p_iv - sum_k w_k [v = y_{i+k}] ),  S_i = sum of w_k over the offsets that take part,
 //   S_i p_iv (1 - t^2) = rho_i (D_iv 2^{lam_i})  with  rho_i = g_i S_i e^{cap - lse_i} 2^{-lam_i}.
@@ -25,10 +64,13 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
                                                       float* __restrict__ rho, float* __restrict__ hcoef,
                                                       float* __restrict__ blockmax, int32_t* __restrict__ rowinfo, CallMode mode,
                                                       int32_t key_none, int32_t* __restrict__ keys, int32_t* __restrict__ vals,
-                                                      int32_t* __restrict__ longlist) {
+                                                      int32_t* __restrict__ longlist, int32_t* __restrict__ skeys, int32_t* __restrict__ perm) {
   __shared__ float smax[256];
+  __shared__ __attribute__((aligned(16))) uint32_t rank_keys[RANK_MAX];
+  // blocks beyond the rows' (there are some with few entries only): the entries' places
+  if ((int)blockIdx.x >= Np / 256) return rank_targets(rank_keys, blockIdx.x - Np / 256, targets, ignore_index, N, Np, V, key_none, n_predict, skeys, perm);
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i == 0) longlist[0] = 0;        // counter of the long-column list, filled by bwd_segments_kernel
+  if (i == 0) longlist[0] = 0;        // counter of the long-column list, filled by column_segments
   float r = 0.f;
   float h[4] = {0.f, 0.f, 0.f, 0.f};
   // the forward call that wrote `saved` was asked for something else (kept dlogits, vocabulary limit, offsets, cap):
@@ -60,9 +102,9 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
       yk[k] = targets[i + k];
       sw += mtp_weights ? mtp_weights[k] : 1.0f;
     }
-    // sort keys of the rows grouped by target: one entry per (offset k, row i): key = target y_{i+k} (key_none if the pair
+    // sort keys of the rows grouped by target (keys == NULL: ranked by this launch's other blocks): one entry per (offset k, row i): key = target y_{i+k} (key_none if the pair
     // takes no part), value = entry id k * Np + i
-    for (int k = 0; k < n_predict; ++k) {
+    for (int k = 0; k < n_predict && keys; ++k) {
       keys[(int64_t)k * N + i] = ok[k] ? (int32_t)yk[k] : key_none;
       vals[(int64_t)k * N + i] = k * Np + i;
     }
@@ -105,11 +147,12 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
 // xi, the largest |rho|, is folded from bwd_prep_kernel's block maxima by every workgroup for itself (one load a thread at
 // N = 65536, from L2, beside the loads of the tile): a launch of one workgroup for it was 4.7 us of every backward call.
 constexpr int XT_TILE = 128;
-__global__ __launch_bounds__(256) void bwd_xt_kernel(const uint8_t* __restrict__ xq, int64_t dp, int64_t ldx, int64_t kbn,
-                                                    const float* __restrict__ rho, const float* __restrict__ blockmax, int nblk,
-                                                    float* __restrict__ xi_out, uint8_t* __restrict__ xt) {
-  __shared__ uint8_t tile[XT_TILE][XT_TILE + 4];
-  __shared__ float wmax[4];
+struct XtShared { uint8_t tile[XT_TILE][XT_TILE + 4]; float wmax[4]; };
+__device__ __forceinline__ void xt_tile(XtShared& shared, int bx, int by, const uint8_t* __restrict__ xq, int64_t dp, int64_t ldx, int64_t kbn,
+                                        const float* __restrict__ rho, const float* __restrict__ blockmax, int nblk,
+                                        float* __restrict__ xi_out, uint8_t* __restrict__ xt) {
+  auto& tile = shared.tile;
+  auto& wmax = shared.wmax;
   const int t = threadIdx.x;
   float xi = 0.f;
   for (int n = t; n < nblk; n += 256) xi = fmaxf(xi, blockmax[n]);
@@ -119,8 +162,8 @@ __global__ __launch_bounds__(256) void bwd_xt_kernel(const uint8_t* __restrict__
   __syncthreads();
   xi = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
   xi = (xi > 0.f && isfinite(xi)) ? xi : 1.0f;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) xi_out[0] = xi;
-  const int64_t i0 = (int64_t)blockIdx.x * XT_TILE, j0 = (int64_t)blockIdx.y * XT_TILE;
+  if (bx == 0 && by == 0 && t == 0) xi_out[0] = xi;
+  const int64_t i0 = (int64_t)bx * XT_TILE, j0 = (int64_t)by * XT_TILE;
   if (j0 < dp) {
 #pragma unroll
     for (int pass = 0; pass < 4; ++pass) {
@@ -711,13 +754,15 @@ __device__ __forceinline__ void long_chunks(int L, int& nch, int& len) {
 // rare end of the vocabulary holds gaps of thousands of columns, and 2048 rows took 63 us; this takes 4.7.)
 // Also: row and coefficient of every sorted entry (srow, sh), so that the kernels that walk a segment load them side by
 // side instead of one behind the other.
-__global__ __launch_bounds__(256) void bwd_segments_kernel(const int32_t* __restrict__ skeys, const int32_t* __restrict__ perm,
-                                                          const float* __restrict__ hcoef, int n, int Np, int V, int32_t* __restrict__ segoff,
-                                                          int32_t* __restrict__ longlist, int32_t* __restrict__ longbase,
-                                                          int32_t* __restrict__ srow, float* __restrict__ sh) {
-  __shared__ int32_t top[256], seg[257];
-  const int t = threadIdx.x, v0 = blockIdx.x * 256, stride = (n + 255) / 256;
-  for (int q = v0 + t; q < n; q += gridDim.x * 256) {
+struct SegShared { int32_t top[256], seg[257]; };
+__device__ __forceinline__ void column_segments(SegShared& shared, int block, int nblocks, const int32_t* __restrict__ skeys, const int32_t* __restrict__ perm,
+                                                const float* __restrict__ hcoef, int n, int Np, int V, int32_t* __restrict__ segoff,
+                                                int32_t* __restrict__ longlist, int32_t* __restrict__ longbase,
+                                                int32_t* __restrict__ srow, float* __restrict__ sh) {
+  auto& top = shared.top;
+  auto& seg = shared.seg;
+  const int t = threadIdx.x, v0 = block * 256, stride = (n + 255) / 256;
+  for (int q = v0 + t; q < n; q += nblocks * 256) {
     const int e = perm[q];             // entry id k * Np + i
     srow[q] = e % Np; sh[q] = hcoef[e];
   }
@@ -751,6 +796,26 @@ __global__ __launch_bounds__(256) void bwd_segments_kernel(const int32_t* __rest
   const int at = atomicAdd(&longlist[0], nch);
   longbase[v] = at;
   for (int c = 0; c < nch; ++c) { longlist[1 + 2 * (at + c)] = v; longlist[2 + 2 * (at + c)] = c; }
+}
+
+// The two in one launch, blocks [0, nxt) the tiles of X~ and the rest the segments: neither needs the other, and on few rows
+// a launch of its own costs more than the work (2 x 4.8 us at 2048 rows, 5.8 together; 34 us, 27 together, at 32768 of three offsets).
+struct XtSegParams {
+  const uint8_t* xq;
+  int64_t dp, ldx, kbn;
+  const float *rho, *blockmax, *hcoef;
+  float* xi;
+  uint8_t* xt;
+  const int32_t *skeys, *perm;
+  int32_t *segoff, *longlist, *longbase, *srow;
+  float* sh;
+  int nblk, nxt, nx, n, Np, V;
+};
+__global__ __launch_bounds__(256) void bwd_xt_segments_kernel(XtSegParams p) {
+  __shared__ union { XtShared x; SegShared s; } shared;
+  const int bid = blockIdx.x;
+  if (bid < p.nxt) xt_tile(shared.x, bid % p.nx, bid / p.nx, p.xq, p.dp, p.ldx, p.kbn, p.rho, p.blockmax, p.nblk, p.xi, p.xt);
+  else column_segments(shared.s, bid - p.nxt, gridDim.x - p.nxt, p.skeys, p.perm, p.hcoef, p.n, p.Np, p.V, p.segoff, p.longlist, p.longbase, p.srow, p.sh);
 }
 
 // One-hot part of dW for the long columns: longsum[slot][:] = sum over the chunk's rows of h_i X_q[i, :].

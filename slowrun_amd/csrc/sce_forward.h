@@ -409,16 +409,19 @@ __global__ __launch_bounds__(512) void fwd_sample_few_kernel(FwdParams p_in, int
   }
 }
 
-// The target entries of the dlogits that a forward pass has emitted are set to zero: they take no part in D (their
-// share goes into the one-hot coefficient in fp32, see bwd_prep_kernel).  One thread per row.
+// The target entries of the dlogits that a forward pass has emitted are set to zero (fwd_combine_kernel, which looks at every
+// row's targets anyway; in backward, of dlogits formed again, fwd_knock_kernel, one thread per row): they take no part in D
+// (their share goes into the one-hot coefficient in fp32, see bwd_prep_kernel).
+__device__ __forceinline__ void knock_target(uint8_t* __restrict__ ghat, int64_t kbv, int i, int64_t y) {
+  ghat[((int64_t)(i >> 8) * kbv + (y >> 7)) * BLOCKED_KSTEP + (i & 255) * BK + (y & 127)] = 0;
+}
 __global__ __launch_bounds__(256) void fwd_knock_kernel(uint8_t* __restrict__ ghat, int64_t kbv, const int64_t* __restrict__ targets,
                                                        int64_t ignore_index, int N, int V, int n_predict) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= N) return;
   for (int k = 0; k < n_predict; ++k) {
     if (!target_valid(targets, ignore_index, i + k, N, V)) continue;
-    const int64_t y = targets[i + k];
-    ghat[((int64_t)(i >> 8) * kbv + (y >> 7)) * BLOCKED_KSTEP + (i & 255) * BK + (y & 127)] = 0;
+    knock_target(ghat, kbv, i, targets[i + k]);
   }
 }
 
@@ -436,7 +439,7 @@ static_assert(SMEM_BYTES <= FWD_UY_OFF, "K slots and row data overlap");
 // BF16 (without EMIT): bf16 operands, logits rounded to bf16 as the eager head's GEMM returns them (forward only).
 // PRE: the target logits are in s_uy already (fwd_sample_kernel<true, .>) and this kernel does not look for them in
 // its accumulators.  With EMIT the target entries go through the epilogue like any other, except that they are kept out
-// of the block exponents (form_dlogits, EXCL), and fwd_knock_kernel clears their bytes of G afterwards.
+// of the block exponents (form_dlogits, EXCL), and fwd_combine_kernel clears their bytes of G afterwards.
 template <bool EMIT, bool BF16 = false, bool PRE = false>
 __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
   static_assert(!PRE || !BF16, "PRE is for the fp8 kernels");
@@ -790,7 +793,8 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
                                                          const int64_t* __restrict__ targets, int64_t ignore_index, float cap,
                                                          const float* __restrict__ mtp_weights, int n_predict,
                                                          float* __restrict__ s_lse, float* __restrict__ s_zy, float* __restrict__ losses,
-                                                         float* __restrict__ lse_out, int32_t* __restrict__ argmax_out) {
+                                                         float* __restrict__ lse_out, int32_t* __restrict__ argmax_out,
+                                                         uint8_t* __restrict__ ghat, int64_t kbv) {
   static_assert(G >= 4, "one wave per prediction offset");
   __shared__ float rsum[G][COMBINE_ROWS], rmax[G][COMBINE_ROWS], rl[4][COMBINE_ROWS];
   __shared__ int rarg[G][COMBINE_ROWS];
@@ -827,6 +831,7 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
   if (g < n_predict) {
     float zy = 0.f, l = 0.f;
     if (i < N && target_valid(targets, ignore_index, i + g, N, V)) {
+      if (ghat) knock_target(ghat, kbv, i, targets[i + g]);
       zy = cap * tanhf(s_zy[(int64_t)g * Np + i] / cap);
       l = (mtp_weights ? mtp_weights[g] : 1.0f) * (lse - zy);
     }

@@ -558,10 +558,8 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   }
   {
     KernelTimer tm(SCE_K_FWD, st);
-    if (emit && pre) {
-      fwd_kernel<true, false, true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
-      fwd_knock_kernel<<<(int)(S.Np / 256), 256, 0, st>>>(p.ghat_t, p.kbv, a->targets, a->ignore_index, (int)N, (int)Vl, a->shape.n_predict);
-    } else if (emit) fwd_kernel<true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
+    if (emit && pre) fwd_kernel<true, false, true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
+    else if (emit) fwd_kernel<true><<<grid, NTHREADS, SMEM_FWD, st>>>(p);
     else if (few) {
       FewParams f;
       f.w = (const uint8_t*)a->w; f.w_ldb = a->w_ld * 2; f.d = (int)d; f.Vw = (int)V;
@@ -580,7 +578,7 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   const int nblk = (int)(S.Np / COMBINE_ROWS);
   auto combine = [&](auto kernel, int g) {
     kernel<<<nblk, COMBINE_ROWS * g, 0, st>>>(p.partials, nsplit, (int)N, (int)S.Np, (int)Vl, a->targets, a->ignore_index, a->cap, a->mtp_weights,
-                                             a->shape.n_predict, s_lse, s_zy, a->losses, a->lse, a->argmax);
+                                             a->shape.n_predict, s_lse, s_zy, a->losses, a->lse, a->argmax, emit && pre ? p.ghat_t : nullptr, p.kbv);
   };
   if (nsplit <= 16) combine(fwd_combine_kernel<4>, 4);
   else combine(fwd_combine_kernel<16>, 16);
@@ -709,22 +707,26 @@ extern "C" int sce_backward(const sce_args* a) {
 
   const int nblk = (int)(S.Np / 256);
   KernelTimer* tm_prep = new KernelTimer(SCE_K_BWD_PREP, st);
-  bwd_prep_kernel<<<nblk, 256, 0, st>>>(s_lse, s_zy, a->targets, a->ignore_index, hdr, a->grad_output,
-                                        a->reduction == SCE_REDUCE_NONE ? 1 : 0, a->grad_scale, a->mtp_weights, K, a->cap, (int)N,
-                                        (int)S.Np, (int)Vl, (const float*)(sv + S.off_lam), rho, hcoef, blockmax, kept ? nullptr : rowinfo,
-                                        call_mode(kept, (int)Vl, K, a->cap), (int32_t)V, keys_in, vals_in, longlist);
-  {
-    dim3 g((unsigned)(S.Np / XT_TILE), (unsigned)(S.dq / XT_TILE));
-    bwd_xt_kernel<<<g, 256, 0, st>>>(xq, S.dp, S.ldx, S.Np / BK, rho, blockmax, nblk, xi, xt);
-  }
+  static_assert((int64_t)MAX_SCALE_KBLOCKS * BK << RANK_BITS < (int64_t)1 << 32, "a target (at most V, for none) and an entry number in 32 bits");
+  const bool ranked = NE <= RANK_MAX;
+  bwd_prep_kernel<<<nblk + (ranked ? (int)((NE + RANK_PER_BLOCK - 1) / RANK_PER_BLOCK) : 0), 256, 0, st>>>(
+      s_lse, s_zy, a->targets, a->ignore_index, hdr, a->grad_output, a->reduction == SCE_REDUCE_NONE ? 1 : 0, a->grad_scale, a->mtp_weights, K, a->cap, (int)N,
+      (int)S.Np, (int)Vl, (const float*)(sv + S.off_lam), rho, hcoef, blockmax, kept ? nullptr : rowinfo, call_mode(kept, (int)Vl, K, a->cap), (int32_t)V,
+      ranked ? nullptr : keys_in, vals_in, longlist, skeys, perm);
   // rows grouped by target, for the one-hot part of dW
-  {
+  if (!ranked) {
     int bits = 1;
     while ((1ll << bits) <= V) ++bits;
     size_t tmp = B.sorttmp_bytes;
     if (sce::sort_pairs(ws + B.off_sorttmp, &tmp, keys_in, skeys, vals_in, perm, (size_t)NE, bits, st) != 0)
     { delete tm_prep; return fail(SCE_EHIP, "radix sort of the targets failed"); }
-    bwd_segments_kernel<<<(int)(V / 256 + 1), 256, 0, st>>>(skeys, perm, hcoef, (int)NE, (int)S.Np, (int)V, segoff, longlist, longbase, srow, sh);
+  }
+  {
+    XtSegParams q;
+    q.xq = xq; q.dp = S.dp; q.ldx = S.ldx; q.kbn = S.Np / BK; q.rho = rho; q.blockmax = blockmax; q.hcoef = hcoef; q.xi = xi; q.xt = xt;
+    q.skeys = skeys; q.perm = perm; q.segoff = segoff; q.longlist = longlist; q.longbase = longbase; q.srow = srow; q.sh = sh;
+    q.nblk = nblk; q.nx = (int)(S.Np / XT_TILE); q.nxt = q.nx * (int)(S.dq / XT_TILE); q.n = (int)NE; q.Np = (int)S.Np; q.V = (int)V;
+    bwd_xt_segments_kernel<<<q.nxt + (int)(V / 256 + 1), 256, 0, st>>>(q);
   }
   delete tm_prep;
   {

@@ -1,0 +1,55 @@
+"""The rows grouped by target: up to 4096 (offset, row) entries are ranked in one launch, more go through the radix sort.  A
+batch just below that limit and the same batch with ignored rows behind it (no gradient of their own, past the limit) have
+the same gradients: dX row by row, dW up to the order of its fp32 sums over the rows."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("keep", [True, False])
+@pytest.mark.parametrize("N,offsets,d,V", [(4096, 1, 64, 300), (2048, 2, 272, 5000), (1365, 3, 128, 40000), (1024, 4, 16, 3)])
+def test_ranked_and_sorted_targets_give_the_same_gradients(N, offsets, d, V, keep):
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(V)
+    more = 4096 // offsets + 40
+    x = torch.randn(more, d, device="cuda", generator=gen)
+    w = torch.randn(d, V, device="cuda", generator=gen) * d ** -0.5
+    y = (torch.rand(more, device="cuda", generator=gen) ** 3 * V).long()          # some columns hit by many rows, most by few
+    y[torch.rand(more, device="cuda", generator=gen) < 0.1] = -1
+    y[N:] = -1
+    mtp = torch.tensor([1.0, 0.5, 0.25, 0.125][:offsets], device="cuda")
+    got = []
+    for n in (N, more):
+        loss, saved, *_ = ck.ce_forward(x[:n], w, y[:n], 0.02, 0.01, 15.0, "none", mtp_weights=mtp, keep_dlogits=keep)
+        go = torch.rand(more, device="cuda", generator=torch.Generator(device="cuda").manual_seed(1))[:n]
+        dx, dw = ck.ce_backward(saved, y[:n], go, n, d, V, 0.02, 0.01, 15.0, 1.0, "none", torch.float32, torch.float32, mtp_weights=mtp, keep_dlogits=keep)
+        got.append((loss[:N], dx[:N], dw))
+    for a, b in zip(got[0], got[1]):
+        assert float((a - b).norm() / b.norm()) < 2e-5
+
+
+@pytest.mark.parametrize("N,offsets,V", [(1, 1, 5), (15, 4, 3), (65, 2, 1000)])
+def test_one_hot_part_of_dw_of_few_entries(N, offsets, V):
+    """x = 0: every logit is 0, p = 1 / V, and what is left of dW is zero too; with x = e_0 in row i only, row 0 of dW is the
+    row's (p - onehot), summed here in fp64."""
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    d = 16
+    x = torch.zeros(N, d, device="cuda")
+    x[:, 0] = 1.0
+    w = torch.zeros(d, V, device="cuda")
+    y = torch.randint(0, V, (N,), device="cuda", generator=gen)
+    mtp = torch.tensor([1.0, 0.5, 0.25, 0.125][:offsets], device="cuda")
+    loss, saved, *_ = ck.ce_forward(x, w, y, 1.0, 1.0, 15.0, "none", mtp_weights=mtp, keep_dlogits=True)
+    dx, dw = ck.ce_backward(saved, y, torch.ones(N, device="cuda"), N, d, V, 1.0, 1.0, 15.0, 1.0, "none", torch.float32, torch.float32, mtp_weights=mtp, keep_dlogits=True)
+    ref = torch.zeros(V, dtype=torch.float64)
+    for i in range(N):
+        for k in range(offsets):
+            if i + k < N:
+                ref += float(mtp[k]) / V
+                ref[int(y[i + k])] -= float(mtp[k])
+    # the softmax part goes through e4m3 (3 bits of mantissa: half a unit is 2^-4 of it), the one-hot part does not
+    soft = float(mtp.sum()) * N / V
+    assert float((dw[0].double().cpu() - ref).abs().max()) <= soft * 2 ** -4 + 1e-5
+    assert float(dw[1:].abs().max()) == 0.0
