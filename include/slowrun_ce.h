@@ -166,6 +166,12 @@ int sce_quantize_e4m3_dev(const void* src, int32_t src_dtype, void* dst, const f
  * scales are constants, tiny/train.py:188-189; a trainer that rescales per step does this). */
 int sce_amax_scale(const void* src, int32_t src_dtype, size_t n, float* scale_out, int32_t device, void* stream);
 
+/* out[i] = exp(-losses[i]), the probability that row i gives its target (losses: the per-row losses of a forward call with a
+ * single offset), or 0 where targets[i] == ignore_index.  What the reference's ensemble evaluation takes from the full
+ * logits (_forward_pgt, unlimited/train.py:1063-1069). */
+int sce_target_probability(const float* losses, const int64_t* targets, int64_t n, int64_t ignore_index, float* out,
+                           int32_t device, void* stream);
+
 /* dst (cols, rows) = transpose of src (rows, cols), one byte per element.  Replaces
  * transpose_copy (tiny/cuda_kernels.py:56-78) for callers that still want it; the fused
  * path itself never materialises a transposed N x V matrix. */

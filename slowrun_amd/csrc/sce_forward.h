@@ -874,6 +874,14 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
   }
 }
 
+// p(target) = exp(-loss) of every row, 0 for the rows without a target.  Bound by its launch: in place of five elementwise operations of
+// torch's (compare, zeros, negate, exp, where) a call that scores 61 rows at d = 2560, V = 50304 takes 65.6 us for 73.6.
+__global__ __launch_bounds__(256) void target_probability_kernel(const float* __restrict__ losses, const int64_t* __restrict__ targets, int64_t n,
+                                                                int64_t ignore_index, float* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = targets[i] == ignore_index ? 0.f : expf(-losses[i]);
+}
+
 // What a forward call was asked for, as far as the matching backward call must have been asked the same: left in the header
 // of the saved state (HDR_MODE_OFF bytes in) by fwd_reduce_kernel and compared by bwd_prep_kernel.  A backward call whose
 // flags differ would read dlogits that were never written, or mask other columns: it gets NaN gradients instead.

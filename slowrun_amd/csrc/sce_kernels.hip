@@ -410,6 +410,18 @@ extern "C" int sce_amax_scale(const void* src, int32_t src_dtype, size_t n, floa
   return SCE_OK;
 }
 
+extern "C" int sce_target_probability(const float* losses, const int64_t* targets, int64_t n, int64_t ignore_index, float* out, int32_t device,
+                                      void* stream) {
+  if (!losses || !targets || !out) return fail(SCE_EINVAL, "losses/targets/out is NULL");
+  if (n <= 0 || n > ((int64_t)1 << 31)) return fail(SCE_EINVAL, "n = %lld out of range", (long long)n);
+  if (int rc = check_device(device)) return rc;
+  DeviceGuard guard(device);
+  if (!guard.ok) return fail(SCE_EHIP, "cannot select device %d", device);
+  target_probability_kernel<<<(unsigned)((n + 255) / 256), 256, 0, (hipStream_t)stream>>>(losses, targets, n, ignore_index, out);
+  HIP_TRY(hipGetLastError());
+  return SCE_OK;
+}
+
 extern "C" int sce_transpose_bytes(const void* src, void* dst, int64_t rows, int64_t cols, int32_t device, void* stream) {
   if (!src || !dst) return fail(SCE_EINVAL, "src/dst is NULL");
   if (rows <= 0 || cols <= 0) return fail(SCE_EINVAL, "rows and cols must be positive");

@@ -439,7 +439,10 @@ def target_probability(x, lm_head_weight, targets, x_s=None, w_s=None, cap=15.0,
     ``softcapped_cross_entropy(..., reduction='none')``, same arguments; a row whose target is -1 has no target
     probability and gets 0."""
     losses = softcapped_cross_entropy(x, lm_head_weight, targets, x_s, w_s, cap, vocab_size, "none", norm_eps, operand_dtype)
-    return torch.where(targets.reshape(losses.shape) == -1, torch.zeros_like(losses), torch.exp(-losses))
+    y, out = targets.reshape(-1).contiguous(), torch.empty_like(losses)
+    _lib.check(_lib.lib().sce_target_probability(losses.data_ptr(), y.data_ptr(), losses.numel(), IGNORE_INDEX, out.data_ptr(), losses.device.index,
+                                                _stream_ptr(losses.device)), "sce_target_probability")
+    return out
 
 
 def quantize_e4m3(t, scale):

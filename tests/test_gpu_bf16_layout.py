@@ -56,3 +56,16 @@ def test_few_rows_against_the_general_path(xdtype, N, d, V, vocab, offsets):
         u = (x.float() @ w.float())[:, :vocab].bfloat16().float()
         ref = F.cross_entropy(15.0 * torch.tanh(u / 15.0), y, reduction="none", ignore_index=-1)
         assert torch.allclose(l0, ref, rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("n,shape", [(1, (1,)), (255, (255,)), (257, (257,)), (4098, (2, 2049))])
+def test_target_probability_is_the_exponential_of_the_losses(n, shape):
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn(*shape, 32, device="cuda", generator=gen).bfloat16()
+    w = torch.randn(32, 200, device="cuda", generator=gen).bfloat16()
+    y = torch.randint(0, 200, (2 * n,), device="cuda", generator=gen)[::2].reshape(shape)      # (strided where it is one row)
+    y.view(-1)[::7] = -1 if n > 1 else 3
+    p = ck.target_probability(x, w, y, operand_dtype=torch.bfloat16)
+    losses = ck.softcapped_cross_entropy(x, w, y, reduction="none", operand_dtype=torch.bfloat16)
+    assert p.shape == losses.shape and torch.allclose(p, torch.where(y == -1, torch.zeros_like(losses), torch.exp(-losses)), rtol=1e-6, atol=0)
