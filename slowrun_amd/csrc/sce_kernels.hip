@@ -430,8 +430,7 @@ extern "C" int sce_transpose_bytes(const void* src, void* dst, int64_t rows, int
   DeviceGuard guard(device);
   if (!guard.ok) return fail(SCE_EHIP, "cannot select device %d", device);
   dim3 grid((unsigned)((cols + TB_TILE - 1) / TB_TILE), (unsigned)((rows + TB_TILE - 1) / TB_TILE));
-  const int in16 = cols % 16 == 0 && ((uintptr_t)src & 15) == 0, out16 = rows % 16 == 0 && ((uintptr_t)dst & 15) == 0;
-  transpose_bytes_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint8_t*)src, (uint8_t*)dst, rows, cols, in16, out16);
+  transpose_bytes_kernel<<<grid, 256, 0, (hipStream_t)stream>>>((const uint8_t*)src, (uint8_t*)dst, rows, cols);
   HIP_TRY(hipGetLastError());
   return SCE_OK;
 }

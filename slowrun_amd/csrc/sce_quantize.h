@@ -414,12 +414,13 @@ __global__ __launch_bounds__(256) void amax_kernel(const T* __restrict__ src, si
 
 // dst (cols, rows) = src (rows, cols)^T, bytes, in 128 x 128 tiles: whole 128-byte lines both ways.  On the way out of
 // LDS the transposing read gives a lane eight rows of its column at once (16 lanes point at 8 rows of 16 bytes, 8 bytes
-// each, and lane j receives column j).  `in16` / `out16`: every run of 16 bytes along a row of src / dst is aligned; other shapes and the
-// ragged edges go byte by byte.  HBM-bound, 2 bytes an element: 164 us for 2560 x 50304 when every byte was an access
-// of its own (1.6 TB/s), now 50.
+// each, and lane j receives column j).  Both sides move 16 bytes at a time wherever 16 are there, aligned or not; only the
+// last few of a row go byte by byte.  HBM-bound, 2 bytes an element: 50 us for
+// 2560 x 50304 (164 with every byte an access of its own), 89 for 2561 x 50257 where no row is aligned (131 with bytes, 341
+// with a lane's 16 bytes one by one: neighbouring lanes then touch different lines).
 constexpr int TB_TILE = 128, TB_PITCH = TB_TILE + 16;
 __global__ __launch_bounds__(256) void transpose_bytes_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
-                                                             int64_t rows, int64_t cols, int in16, int out16) {
+                                                             int64_t rows, int64_t cols) {
   __shared__ __attribute__((aligned(16))) uint8_t tile[TB_TILE * TB_PITCH];
   const int t = threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.y * TB_TILE, c0 = (int64_t)blockIdx.x * TB_TILE;
@@ -430,7 +431,7 @@ __global__ __launch_bounds__(256) void transpose_bytes_kernel(const uint8_t* __r
       const int64_t r = r0 + (t >> 3) + 32 * pass, c = c0 + (t & 7) * 16;
       raw[pass] = (v4i){0, 0, 0, 0};
       if (r < rows && c < cols) {
-        if (in16) raw[pass] = *reinterpret_cast<const v4i*>(src + r * cols + c);
+        if (c + 16 <= cols) raw[pass] = *reinterpret_cast<const v4i_any*>(src + r * cols + c);
         else
           for (int m = 0; m < 16 && c + m < cols; ++m) raw[pass][m >> 2] |= (int)((uint32_t)src[r * cols + c + m] << (8 * (m & 3)));
       }
@@ -450,7 +451,7 @@ __global__ __launch_bounds__(256) void transpose_bytes_kernel(const uint8_t* __r
     const int64_t c = c0 + cc + i, r = r0 + rr;
     if (c < cols && r < rows) {
       uint8_t* d = dst + c * rows + r;
-      if (out16) *reinterpret_cast<v4i*>(d) = (v4i){lo[0], lo[1], hi[0], hi[1]};
+      if (r + 16 <= rows) *reinterpret_cast<v4i_any*>(d) = (v4i){lo[0], lo[1], hi[0], hi[1]};
       else {
         const int w[4] = {lo[0], lo[1], hi[0], hi[1]};
 #pragma unroll

@@ -19,6 +19,20 @@ def test_transpose_copy_edges(rows, cols, off):
     assert bool((buf[:off] == 77).all()) and bool((buf[off + rows * cols:] == 77).all())
 
 
+@pytest.mark.parametrize("rows,cols", [(15, 17), (143, 129), (300, 257), (65, 2561)])
+@pytest.mark.parametrize("soff,doff", [(1, 2), (3, 0), (0, 7), (9, 15)])
+def test_transpose_copy_of_rows_at_any_address(rows, cols, soff, doff):
+    """Rows and bases that are no multiple of 16 bytes move in 16-byte accesses too: nothing beside the output is written."""
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(rows + soff)
+    src = torch.randint(0, 256, (rows * cols + soff,), dtype=torch.uint8, device="cuda", generator=gen)[soff:].view(rows, cols)
+    buf = torch.full((rows * cols + 32,), 77, dtype=torch.uint8, device="cuda")
+    dst = buf[doff: doff + rows * cols].view(cols, rows)
+    ck.transpose_copy(src, dst)
+    assert torch.equal(dst, src.t().contiguous())
+    assert bool((buf[:doff] == 77).all()) and bool((buf[doff + rows * cols:] == 77).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("n", [1, 7, 16, 17, 2047, 4096 * 8 + 3, 1 << 20])
 @pytest.mark.parametrize("off", [0, 1])
