@@ -13,6 +13,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // 16 bytes of global memory at any address: one access all the same (the target's unaligned access mode), for rows whose
 // length is no multiple of 16 bytes.
 typedef int v4i_any __attribute__((ext_vector_type(4), aligned(1)));
+typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
 
 // One workgroup (4 wavefronts of 64) owns a TM x TN tile of C = A * B^T where both
 // operands are stored K-contiguous ("NT").  A rows land on the accumulator registers,

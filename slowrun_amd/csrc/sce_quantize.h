@@ -9,12 +9,13 @@ namespace sce {
 // quantisation
 // ------------------------------------------------------------------------------------------
 // 16 consecutive elements starting at p as floats after the scaling; elements at or beyond
-// `valid` are 0.  One or two 16/32-byte vector loads when the run is complete and 16-byte aligned.
+// `valid` are 0.  16-byte loads when the run is complete, aligned or not: one element at a time, a wave's lanes touch
+// a different cache line each, 16 times over.
 template <typename T>
 __device__ __forceinline__ void load16_scaled(const T* __restrict__ p, int64_t valid, const Scaler scale, float (&v)[16]) {
-  if (valid >= 16 && (((uintptr_t)p) & 15) == 0) {
+  if (valid >= 16) {
     if constexpr (sizeof(T) == 2) {
-      const v4i r0 = *reinterpret_cast<const v4i*>(p), r1 = *reinterpret_cast<const v4i*>(p + 8);
+      const v4i r0 = *reinterpret_cast<const v4i_any*>(p), r1 = *reinterpret_cast<const v4i_any*>(p + 8);
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         v[2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] << 16));
@@ -25,7 +26,7 @@ __device__ __forceinline__ void load16_scaled(const T* __restrict__ p, int64_t v
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const v4f r = *reinterpret_cast<const v4f*>(p + 4 * q);
+        const v4f r = *reinterpret_cast<const v4f_any*>(p + 4 * q);
 #pragma unroll
         for (int m = 0; m < 4; ++m) v[4 * q + m] = scale.apply<T>(r[m]);
       }
@@ -345,9 +346,9 @@ __global__ __launch_bounds__(256) void prep_w_bf16_kernel(const T* __restrict__ 
 }
 
 // flat cast, for the standalone sce_quantize_e4m3 entry point: 16 elements a thread, their 32 or 64 bytes in 16-byte loads
-// and the result in one 16-byte store where both are aligned (a thread's run starts at a multiple of 16 elements, so
-// that is a matter of the base pointers), element by element otherwise and at the end.  HBM-bound: 3 bytes an element
-// in bf16; with four elements a thread in 2-byte loads 162 us for 2560 x 50304 (2.4 TB/s), now 70.
+// and the result in one 16-byte store, at whatever address they lie; element by element at the end.  HBM-bound: 3 bytes an
+// element in bf16; 75 us for 2560 x 50257 whether the source is aligned or one element off (four elements a thread in
+// 2-byte loads: 145 and 153; 16 a thread one by one: 268).
 template <typename T>
 __global__ __launch_bounds__(256) void quantize_flat_kernel(const T* __restrict__ src, uint8_t* __restrict__ dst,
                                                            size_t n, float inv_scale, const float* __restrict__ scale_dev) {
@@ -359,8 +360,8 @@ __global__ __launch_bounds__(256) void quantize_flat_kernel(const T* __restrict_
     uint32_t w[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) w[m] = cvt4_e4m3(v[4 * m], v[4 * m + 1], v[4 * m + 2], v[4 * m + 3]);
-    if (left >= 16 && ((uintptr_t)dst & 15) == 0) {
-      *reinterpret_cast<v4i*>(dst + q) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+    if (left >= 16) {
+      *reinterpret_cast<v4i_any*>(dst + q) = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
     } else {
 #pragma unroll
       for (int m = 0; m < 16; ++m)

@@ -46,3 +46,19 @@ def test_amax_and_cast_edges(dtype, n, off):
         assert float(ck.amax_scale(u)) == float(u.float().abs().max().cpu() / 448)      # (a true division; torch multiplies by 1 / 448 on the GPU)
     for scale in (0.0123, ck.amax_scale(u)):
         assert torch.equal(ck.quantize_e4m3(u, scale).view(torch.uint8), u.div(scale).to(torch.float8_e4m3fn).view(torch.uint8))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [5, 16, 31, 4096 + 17])
+@pytest.mark.parametrize("soff,doff", [(1, 0), (0, 1), (3, 13), (7, 6)])
+def test_cast_between_any_addresses(dtype, n, soff, doff):
+    """The C entry takes source and destination wherever they lie (elements of the source aligned to themselves): the same bytes, and
+    none beside them."""
+    from slowrun_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(n + soff)
+    t = torch.randn(n + soff, device="cuda", generator=gen).to(dtype)[soff:]
+    buf = torch.full((n + 32,), 77, dtype=torch.uint8, device="cuda")
+    _lib.check(_lib.lib().sce_quantize_e4m3(t.data_ptr(), _lib.SCE_F32 if dtype == torch.float32 else _lib.SCE_BF16, buf.data_ptr() + doff, 0.0123, n, t.device.index,
+                                           torch.cuda.current_stream().cuda_stream), "sce_quantize_e4m3")
+    assert torch.equal(buf[doff: doff + n], t.div(0.0123).to(torch.float8_e4m3fn).view(torch.uint8))
+    assert bool((buf[:doff] == 77).all()) and bool((buf[doff + n:] == 77).all())
