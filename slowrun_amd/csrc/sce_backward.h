@@ -753,7 +753,10 @@ __device__ __forceinline__ void long_chunks(int L, int& nch, int& len) {
 // stride.  (A thread per key that fills the gap up to the next key runs as long as the widest gap: with Zipf targets the
 // rare end of the vocabulary holds gaps of thousands of columns, and 2048 rows took 63 us; this takes 4.7.)
 // Also: row and coefficient of every sorted entry (srow, sh), so that the kernels that walk a segment load them side by
-// side instead of one behind the other.
+// side instead of one behind the other: at most SEG_ENTRIES to a block, with blocks beyond the columns' if need be (three
+// offsets of 65536 rows over a vocabulary of 512 took the columns' 3 blocks 135 us, with 384 it is 17; V = 4096 39 -> 18).
+constexpr int SEG_ENTRIES = 512;
+static inline int segment_blocks(int64_t n, int64_t V) { return (int)std::max<int64_t>(V / 256 + 1, (n + SEG_ENTRIES - 1) / SEG_ENTRIES); }
 struct SegShared { int32_t top[256], seg[257]; };
 __device__ __forceinline__ void column_segments(SegShared& shared, int block, int nblocks, const int32_t* __restrict__ skeys, const int32_t* __restrict__ perm,
                                                 const float* __restrict__ hcoef, int n, int Np, int V, int32_t* __restrict__ segoff,
@@ -766,6 +769,7 @@ __device__ __forceinline__ void column_segments(SegShared& shared, int block, in
     const int e = perm[q];             // entry id k * Np + i
     srow[q] = e % Np; sh[q] = hcoef[e];
   }
+  if (v0 > V) return;                  // a block beyond the columns': entries only
   top[t] = t * stride < n ? skeys[t * stride] : 0x7fffffff;
   __syncthreads();
   auto lower_bound = [&](int v) {

@@ -737,7 +737,7 @@ extern "C" int sce_backward(const sce_args* a) {
     q.xq = xq; q.dp = S.dp; q.ldx = S.ldx; q.kbn = S.Np / BK; q.rho = rho; q.blockmax = blockmax; q.hcoef = hcoef; q.xi = xi; q.xt = xt;
     q.skeys = skeys; q.perm = perm; q.segoff = segoff; q.longlist = longlist; q.longbase = longbase; q.srow = srow; q.sh = sh;
     q.nblk = nblk; q.nx = (int)(S.Np / XT_TILE); q.nxt = q.nx * (int)(S.dq / XT_TILE); q.n = (int)NE; q.Np = (int)S.Np; q.V = (int)V;
-    bwd_xt_segments_kernel<<<q.nxt + (int)(V / 256 + 1), 256, 0, st>>>(q);
+    bwd_xt_segments_kernel<<<q.nxt + segment_blocks(NE, V), 256, 0, st>>>(q);
   }
   delete tm_prep;
   {

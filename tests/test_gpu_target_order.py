@@ -53,3 +53,25 @@ def test_one_hot_part_of_dw_of_few_entries(N, offsets, V):
     soft = float(mtp.sum()) * N / V
     assert float((dw[0].double().cpu() - ref).abs().max()) <= soft * 2 ** -4 + 1e-5
     assert float(dw[1:].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("N,offsets,V", [(513, 1, 256), (5000, 2, 512), (3000, 2, 64), (40000, 1, 1024)])
+def test_one_hot_part_of_dw_of_more_entries_than_columns(N, offsets, V):
+    """A small vocabulary with many entries: workgroups beyond those of the columns bring the entries' rows and coefficients.  With
+    x = e_0, a zero head and powers of two for V and for the row's weight, p = 1 / V is exact in e4m3 (dlogits formed again in
+    backward are stored as the probability), so row 0 of dW is sum_i sum_k (1 / V - onehot) up to the fp32 sums: 2^-20 of the N additions that a column sees."""
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    d = 16
+    x = torch.zeros(N, d, device="cuda")
+    x[:, 0] = 1.0
+    w = torch.zeros(d, V, device="cuda")
+    y = torch.randint(0, V, (N,), device="cuda", generator=gen)
+    y[::9] = V // 2                        # one column in chunks
+    mtp = torch.ones(offsets, device="cuda")
+    loss, saved, *_ = ck.ce_forward(x, w, y, 1.0, 1.0, 15.0, "none", mtp_weights=mtp, keep_dlogits=False)
+    dx, dw = ck.ce_backward(saved, y, torch.ones(N, device="cuda"), N, d, V, 1.0, 1.0, 15.0, 1.0, "none", torch.float32, torch.float32, mtp_weights=mtp, keep_dlogits=False)
+    count = sum(torch.bincount(y[k:], minlength=V).double() for k in range(offsets))
+    ref = float(sum(N - k for k in range(offsets))) / V - count
+    assert float((dw[0].double() - ref).abs().max()) <= 2.0 ** -20 * N * offsets
+    assert float(dw[1:].abs().max()) == 0.0
