@@ -55,7 +55,9 @@ typedef struct sce_sizes {
   size_t saved_bytes;        /* state written by sce_forward and read by sce_backward        */
   size_t saved_x_bytes;      /* the same when the quantised W lives in a weight cache        */
   size_t wcache_bytes;       /* size of that weight cache                                    */
-  size_t fwd_workspace_bytes;
+  size_t fwd_workspace_bytes;       /* room for as many vocabulary splits as fill the chip; with less, down to
+                                       16 (ceil(N / 256) * 256) S bytes (S as in sce_forward_noalloc, 8 to 16), a
+                                       forward of few rows makes fewer splits                */
   size_t bwd_workspace_min_bytes;   /* backward with the smallest row panel (256 rows)       */
   size_t bwd_workspace_bytes;       /* backward with the default row panel (with room for the partial tiles of a
                                        K-split last round of dW where there is to be one; less is accepted)   */
@@ -190,7 +192,8 @@ int sce_forward(const sce_args* args);
  * allocate: code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc.  The call allocates
  * nothing and frees nothing; args->workspace and args->workspace_bytes are ignored, every other field means what it
  * means to sce_forward, and the results are the same bits.  Limit: ceil(N / 256) * 256 * S <= 524288, S the number of
- * vocabulary splits (8 to 16, 8 at N = 65536, V = 50304; more where N <= 3840, which always fits), else SCE_EINVAL with a message.  All calls on one device
+ * vocabulary splits (8 to 16, 8 at N = 65536, V = 50304, the number of column tiles where that is less; few rows take
+ * more of them while the array has the room), else SCE_EINVAL with a message.  All calls on one device
  * share the one array: calls that overlap in time on the same device (two streams, two threads) race. */
 int sce_forward_noalloc(const sce_args* args);
 

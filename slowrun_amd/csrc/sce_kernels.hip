@@ -315,18 +315,22 @@ extern "C" const char* sce_last_error(void) { return g_err; }
 
 // Forward splits V among S workgroups per row tile (each walks CT / S column tiles).  8 keeps the partial records
 // small and gives every workgroup a long walk; more (up to 16) only where 8 would leave the last round of
-// workgroups, one per CU, mostly empty.  With fewer than 16 row tiles even 16 splits leave CUs without a workgroup: then as
-// many as there are CUs, down to one column tile to a workgroup.  Measured: N = 2048 (8 row tiles), d = 768, V = 50304
-// forward 221 us with 16 splits (128 workgroups), 135 us with 32; N = 61, d = 2560, bf16 operands 800 us with 16, 85 us with 197.
+// workgroups, one per CU, mostly empty.
 constexpr int FWD_MAX_SPLITS = 16;
-static int fwd_splits(int RT, int CT, int ncu) {
-  if (RT * FWD_MAX_SPLITS < ncu) return std::min(CT, ncu / RT);
+static int fwd_least_splits(int RT, int CT, int ncu) {
   if (CT <= 8) return CT;
   auto fill = [&](int S) { const int64_t wg = (int64_t)RT * S; return (double)wg / (double)((wg + ncu - 1) / ncu * ncu); };
   int best = 8;
   for (int S = 9; S <= FWD_MAX_SPLITS && S <= CT; ++S)
     if (fill(S) > fill(best) + 0.03) best = S;
   return best;
+}
+// With fewer than 16 row tiles even 16 splits leave CUs without a workgroup: then as many as there are CUs, down to one column
+// tile to a workgroup.  Measured: N = 2048 (8 row tiles), d = 768, V = 50304 forward 221 us with 16 splits (128
+// workgroups), 135 us with 32; N = 61, d = 2560, bf16 operands 800 us with 16, 85 us with 197.  A workspace that has not the room
+// for their records is taken as it is, down to the splits above: fewer of them, not an error.
+static int fwd_splits(int RT, int CT, int ncu) {
+  return RT * FWD_MAX_SPLITS < ncu ? std::min(CT, ncu / RT) : fwd_least_splits(RT, CT, ncu);
 }
 // partial records of a forward pass: enough for any device (fwd_splits makes no more than MAX_CUS workgroups beyond 16 splits)
 static size_t fwd_workspace(int64_t Np) {
@@ -537,9 +541,9 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   }
   const bool emit = a->dlogits_from_forward != 0;
   const int CTw = emit ? (int)(S.Vp / 256) : CT;       // with the dlogits every tile is visited: the masked ones must read as zero later
-  const int nsplit = fwd_splits(RT, CTw, device_cus_or_default(a->device));
-  const size_t need_ws = (size_t)nsplit * S.Np * 16;
+  const size_t split_bytes = (size_t)S.Np * 16, need_ws = (size_t)fwd_least_splits(RT, CTw, device_cus_or_default(a->device)) * split_bytes;
   if (!ws || ws_bytes < need_ws) return fail(SCE_EINVAL, "%s too small: %zu < %zu", ws_name, ws_bytes, need_ws);
+  const int nsplit = (int)std::min<size_t>(fwd_splits(RT, CTw, device_cus_or_default(a->device)), ws_bytes / split_bytes);
   FwdParams p;
   p.xq = xq; p.wqt = wqt; p.partials = (float4*)ws;
   p.targets = a->targets; p.ignore_index = a->ignore_index; p.n_predict = a->shape.n_predict; p.s_uy = (float*)(sv + S.off_zy);
