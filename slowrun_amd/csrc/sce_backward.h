@@ -738,7 +738,7 @@ __global__ __launch_bounds__(256) void bwd_dw_tail_kernel(DwParams p, DwTail tl)
         *reinterpret_cast<v4f*>(dst0 + (4 * a + b) * 1024 + q * 256) = (v4f){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
 }
 
-// A column that is the target of at least LONG_SEG rows has its segment of the sorted list cut into
+// A column that is the target of at least long_seg (LONG_SEG or LONG_SEG_PARTS) rows has its segment of the sorted list cut into
 // nch = ceil(L / LONG_CHUNK) equal chunks (the last one may be shorter); chunk c starts at sorted
 // position s0 + c * ceil(L / nch).
 __device__ __forceinline__ void long_chunks(int L, int& nch, int& len) {
@@ -759,7 +759,7 @@ constexpr int SEG_ENTRIES = 512;
 static inline int segment_blocks(int64_t n, int64_t V) { return (int)std::max<int64_t>(V / 256 + 1, (n + SEG_ENTRIES - 1) / SEG_ENTRIES); }
 struct SegShared { int32_t top[256], seg[257]; };
 __device__ __forceinline__ void column_segments(SegShared& shared, int block, int nblocks, const int32_t* __restrict__ skeys, const int32_t* __restrict__ perm,
-                                                const float* __restrict__ hcoef, int n, int Np, int V, int32_t* __restrict__ segoff,
+                                                const float* __restrict__ hcoef, int n, int Np, int V, int long_seg, int32_t* __restrict__ segoff,
                                                 int32_t* __restrict__ longlist, int32_t* __restrict__ longbase,
                                                 int32_t* __restrict__ srow, float* __restrict__ sh) {
   auto& top = shared.top;
@@ -794,7 +794,7 @@ __device__ __forceinline__ void column_segments(SegShared& shared, int block, in
   segoff[v] = seg[t];
   if (v == V) return;
   const int L = seg[t + 1] - seg[t];
-  if (L < LONG_SEG) return;
+  if (L < long_seg) return;
   int nch, len;
   long_chunks(L, nch, len);
   const int at = atomicAdd(&longlist[0], nch);
@@ -813,13 +813,13 @@ struct XtSegParams {
   const int32_t *skeys, *perm;
   int32_t *segoff, *longlist, *longbase, *srow;
   float* sh;
-  int nblk, nxt, nx, n, Np, V;
+  int nblk, nxt, nx, n, Np, V, long_seg;
 };
 __global__ __launch_bounds__(256) void bwd_xt_segments_kernel(XtSegParams p) {
   __shared__ union { XtShared x; SegShared s; } shared;
   const int bid = blockIdx.x;
   if (bid < p.nxt) xt_tile(shared.x, bid % p.nx, bid / p.nx, p.xq, p.dp, p.ldx, p.kbn, p.rho, p.blockmax, p.nblk, p.xi, p.xt);
-  else column_segments(shared.s, bid - p.nxt, gridDim.x - p.nxt, p.skeys, p.perm, p.hcoef, p.n, p.Np, p.V, p.segoff, p.longlist, p.longbase, p.srow, p.sh);
+  else column_segments(shared.s, bid - p.nxt, gridDim.x - p.nxt, p.skeys, p.perm, p.hcoef, p.n, p.Np, p.V, p.long_seg, p.segoff, p.longlist, p.longbase, p.srow, p.sh);
 }
 
 // One-hot part of dW for the long columns: longsum[slot][:] = sum over the chunk's rows of h_i X_q[i, :].
@@ -893,12 +893,12 @@ struct DwOut {
   const DevConsts* dc;         // non-NULL: x_s comes from here
   int64_t ldx, dq;
   float x_s;
-  int d, V;
+  int d, V, long_seg;          // long_seg: LONG_SEG wherever bwd_dw_out_kernel runs
 };
 
 // dW straight from the main loop: dW = x_s (xi (X~^T G) - sum over the column's target entries of h_i X_q[i, :]), cast and
-// stored by the workgroup that has the tile in its accumulators.  Used whenever one launch covers all rows (N <= 131072, a
-// workspace of the default size).  What the separate pass over an fp32 partial cost was its traffic: 8 bytes an element
+// stored by the workgroup that has the tile in its accumulators.  Used whenever one launch covers all rows: up to 131072 with
+// the dlogits kept; formed again, as many whole dX panels as fit in 131072 rows, and a workspace of the default size.  What the separate pass over an fp32 partial cost was its traffic: 8 bytes an element
 // written and read again (1 GB at d = 2560, V = 50304) around 2 bytes of result, 65 us of a 560 us step at N = 2048,
 // d = 768 and 172 us at N = 30011, d = 2560, whatever the number of rows.
 //
@@ -1088,6 +1088,13 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
   }
 }
 
+// s + a b with the product rounded first
+__device__ __forceinline__ float add_product(float s, float a, float b) {
+#pragma clang fp contract(off)
+  const float p = a * b;
+  return s + p;
+}
+
 // The same from fp32 partials: what is left are the tiles of a K-split last round (tl.tile0 >= 0: grid.y = tl.ntail tiles of
 // 16 blocks of 64 x 64 elements), and every tile where dW took more than one launch (grid = blocks of 64 columns x 64
 // rows of dW).  A thread owns one column v and four groups of four rows j: 16 consecutive rows, or, of the pieces of a K-split
@@ -1136,7 +1143,7 @@ __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restri
 #pragma unroll
   for (int q = 0; q < 4; ++q) val[q] *= scale;
   const int s0 = o.segoff[v], L = o.segoff[v + 1] - s0;
-  if (L >= LONG_SEG) {
+  if (L >= o.long_seg) {
     int nch, len;
     long_chunks(L, nch, len);
     for (int c = 0; c < nch; ++c) {                       // fixed order
@@ -1146,6 +1153,27 @@ __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restri
 #pragma unroll
         for (int m = 0; m < 4; ++m) val[q][m] -= ls[q * step + m] * x_s;
     }
+  } else if (L >= LONG_SEG) {
+    // where dW took several launches: the entries' sum first and then x_s, as it comes from the chunk sums otherwise
+    v4f sum[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum[q] = (v4f){0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < L; ++n) {
+      const float h = o.sh[s0 + n];
+      const uint8_t* row = o.xq + (int64_t)o.srow[s0 + n] * o.ldx + j0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(row + q * step);
+        sum[q][0] = add_product(sum[q][0], h, e4m3_to_float<0>(w));
+        sum[q][1] = add_product(sum[q][1], h, e4m3_to_float<1>(w));
+        sum[q][2] = add_product(sum[q][2], h, e4m3_to_float<2>(w));
+        sum[q][3] = add_product(sum[q][3], h, e4m3_to_float<3>(w));
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+      for (int m = 0; m < 4; ++m) val[q][m] -= sum[q][m] * x_s;
   } else if (L > 0) {
     for (int n = 0; n < L; ++n) {
       const float h = o.sh[s0 + n] * x_s;

@@ -28,7 +28,10 @@ constexpr int NTHREADS = 256;
 constexpr int SMEM_MAX = 160 * 1024;              // LDS a workgroup may hold on gfx950
 
 constexpr float LOG2E = 1.4426950408889634f;
-constexpr int LONG_SEG = 8;      // target columns hit by at least this many rows get their own reduction kernel
+// Target columns hit by at least this many rows get their own reduction kernel: 8 where dW is stored from its accumulators (that
+// kernel has LDS for the entries of shorter columns only), 16 where dW takes several launches, for the sake of the
+// workspace (a chunk sum of dq floats for every LONG_SEG entries).
+constexpr int LONG_SEG = 8, LONG_SEG_PARTS = 16;
 constexpr int LONG_CHUNK = 256;  // ... which handles at most about this many rows per workgroup
 
 // Lane index within the wavefront, computed from the execution mask each time it is asked for.  Kernels
@@ -92,6 +95,8 @@ struct BwdLayout {
   size_t off_gexp, off_rho, off_rowinfo, off_hcoef, off_blockmax, off_xi, off_xt, off_dwacc, off_perm, off_keys,
       off_segoff, off_longlist, off_longbase, off_longsum, off_sorttmp, off_dxpart, off_ghat_t, fixed, total;
   size_t sorttmp_bytes, part_stride;   // part_stride: bytes between consecutive fp32 dW partials
+  bool one;                            // one dW launch covers all rows: dW is stored from its accumulators, without partials
+  int64_t long_seg, long_slots;        // what makes a column long, and the most chunk sums there can be
   size_t off_dwtail, tail_bytes;       // partial tiles of the K-split last round of dW: behind `total`, used when the workspace reaches that far
   int nparts;
 };

@@ -221,7 +221,8 @@ static DwTailPlan dw_tail_plan(int64_t dq, int64_t Vp, int64_t krows) {
 // kept: the dlogits come with `saved` (the forward pass emitted them): no panel scratch here
 static BwdLayout bwd_layout(const SavedLayout& S, int64_t P, int64_t Pw, int nparts, int K, bool kept = false) {
   BwdLayout B;
-  B.P = P; B.Pw = Pw; B.nparts = nparts;
+  B.P = P; B.Pw = Pw; B.nparts = nparts; B.one = S.Np <= Pw;
+  const int64_t NE = S.N * K;
   size_t o = 0;
   auto take = [&](size_t bytes) { size_t r = o; o += (bytes + 255) / 256 * 256; return r; };
   B.off_rho = take((size_t)S.Np * 4);
@@ -230,23 +231,41 @@ static BwdLayout bwd_layout(const SavedLayout& S, int64_t P, int64_t Pw, int npa
   B.off_blockmax = take((size_t)(S.Np / 256) * 4);
   B.off_xi = take(256);
   B.off_xt = take((size_t)S.dq * S.Np);
-  B.off_perm = take((size_t)S.N * K * 4 * 2);  // sorted values + unsorted values, one entry per (offset, row)
-  B.off_keys = take((size_t)S.N * K * 4 * 2);  // sorted keys + unsorted keys
+  B.off_perm = take((size_t)NE * 4 * 2);  // sorted values + unsorted values, one entry per (offset, row)
+  B.off_keys = take((size_t)NE * 4 * 2);  // sorted keys + unsorted keys
   B.off_segoff = take((size_t)(S.V + 2) * 4);
-  B.off_longlist = take((size_t)(2 * (S.N * K / LONG_SEG + 1) + 2) * 4);   // (column, chunk) pairs: at most one per LONG_SEG entries
   B.off_longbase = take((size_t)S.V * 4);                                  // first slot of each long column
-  B.off_longsum = take((size_t)(S.N * K / LONG_SEG + 1) * S.dq * 4);      // chunk sums: a long column has at most one chunk per LONG_SEG of its entries
-  B.sorttmp_bytes = sort_tmp_bytes(S.N * K, S.V);
+  B.sorttmp_bytes = sort_tmp_bytes(NE, S.V);
   B.off_sorttmp = take(B.sorttmp_bytes);
   B.off_dxpart = take(DX_PART_BYTES);
-  B.fixed = o;
+  const size_t before = o;
   B.off_ghat_t = take(kept ? 0 : (size_t)S.Vp * Pw);
   B.off_gexp = take(kept ? 0 : (size_t)(S.Vp / 128) * (Pw / 128) * 4);      // block exponents of the dlogits
   B.part_stride = ((size_t)S.dq * S.Vp * 4 + 255) / 256 * 256;
-  B.off_dwacc = take(B.part_stride * (size_t)nparts);     // fp32 dW partials, one per dW launch
+  // The long columns' (column, chunk) pairs and chunk sums -- a column has at most one chunk per long_seg of its entries, and one
+  // more per LONG_CHUNK -- and behind them the fp32 partials of dW, one per launch.  A single launch has none.  With the
+  // dlogits kept it needs no room for them either; a workspace for dlogits that are formed again has it (with less of them in
+  // hand at a time the same workspace serves several launches), and the sums of the shorter columns lie there.
+  const size_t dlogits_end = o;
+  auto long_columns = [&](int64_t slots) {
+    B.long_slots = slots;
+    B.off_longlist = take((size_t)(2 * slots + 2) * 4);
+    B.off_longsum = take((size_t)slots * S.dq * 4);
+  };
+  long_columns(NE / LONG_SEG_PARTS + 1);
+  B.fixed = before + (o - dlogits_end);
+  B.off_dwacc = take(B.part_stride * (size_t)nparts);
   B.total = o;
-  B.off_dwtail = o;
-  B.tail_bytes = S.Np <= Pw ? dw_tail_plan(S.dq, S.Vp, S.Np).bytes : 0;       // (one dW launch over all rows, or no K-split)
+  B.long_seg = LONG_SEG_PARTS;
+  if (B.one) {
+    o = dlogits_end;
+    B.long_seg = LONG_SEG;
+    long_columns(std::min<int64_t>(NE / LONG_SEG, S.V + NE / LONG_CHUNK) + 1);
+    B.off_dwacc = o;                                       // (not used)
+    B.total = kept ? o : std::max(o, B.total);
+  }
+  B.off_dwtail = B.total;
+  B.tail_bytes = B.one ? dw_tail_plan(S.dq, S.Vp, S.Np).bytes : 0;       // (one dW launch over all rows, or no K-split)
   return B;
 }
 
@@ -268,6 +287,9 @@ static int64_t default_dw_panel(const SavedLayout& S, int64_t P) {
   const int64_t cap = round_up(S.Np, P);
   return Pw < cap ? Pw : cap;
 }
+
+// With the dlogits of all rows in hand (kept), nothing ties a dW launch to the dX panels: as many rows as its K loop takes.
+static int64_t kept_dw_panel(const SavedLayout& S) { return std::min<int64_t>(S.Np, 131072); }
 
 // One fp32 dW partial per dW launch (plain stores, summed once at the end) as long as there are
 // at most 8; beyond that the last buffer is read, added to and rewritten.
@@ -353,7 +375,8 @@ extern "C" int sce_sizes_for(const sce_shape* shape, sce_sizes* out) {
     const BwdLayout Bd = bwd_layout(S, out->bwd_panel_rows, Pw, dw_launches(S, Pw), shape->n_predict);
     out->bwd_workspace_bytes = Bd.total + Bd.tail_bytes;
     out->dlogits_bytes = S.g_total;
-    const BwdLayout Bk = bwd_layout(S, out->bwd_panel_rows, Pw, dw_launches(S, Pw), shape->n_predict, true);
+    const int64_t Pk = kept_dw_panel(S);
+    const BwdLayout Bk = bwd_layout(S, out->bwd_panel_rows, Pk, dw_launches(S, Pk), shape->n_predict, true);
     out->bwd_workspace_kept_bytes = Bk.total + Bk.tail_bytes;
   }
   out->saved_bf16_bytes = saved_layout(shape->N, shape->d, shape->V, shape->n_predict, 2).total;
@@ -646,7 +669,7 @@ extern "C" int sce_backward(const sce_args* a) {
   const bool kept = a->dlogits_from_forward != 0;        // the dlogits came with `saved`
   if (kept && a->saved_bytes < need_saved + S.g_total)
     return fail(SCE_EINVAL, "saved buffer too small for the dlogits: %zu < %zu", a->saved_bytes, need_saved + S.g_total);
-  const BwdLayout Bmin = bwd_layout(S, 256, 256, 1, K, kept);
+  const BwdLayout Bmin = bwd_layout(S, 256, kept ? kept_dw_panel(S) : 256, 1, K, kept);
   if (a->workspace_bytes < Bmin.total) return fail(SCE_EINVAL, "backward workspace too small: %zu < %zu", a->workspace_bytes, Bmin.total);
   if (a->panel_rows % 256) return fail(SCE_EINVAL, "panel_rows must be a multiple of 256");
   // panel sizes from what the caller gave: P rows per recompute/dX panel, Pw = m * P rows per dW launch
@@ -657,7 +680,7 @@ extern "C" int sce_backward(const sce_args* a) {
     P = a->panel_rows > 0 ? a->panel_rows : default_panel(S);
     if (P > S.Np) P = S.Np;
     if (P > 131072) P = 131072;
-    Pw = default_dw_panel(S, P);
+    Pw = kept_dw_panel(S);
     nparts = dw_launches(S, Pw);
     while (nparts > 1 && bwd_layout(S, P, Pw, nparts, K, true).total > a->workspace_bytes) --nparts;
   } else {
@@ -741,12 +764,13 @@ extern "C" int sce_backward(const sce_args* a) {
     q.xq = xq; q.dp = S.dp; q.ldx = S.ldx; q.kbn = S.Np / BK; q.rho = rho; q.blockmax = blockmax; q.hcoef = hcoef; q.xi = xi; q.xt = xt;
     q.skeys = skeys; q.perm = perm; q.segoff = segoff; q.longlist = longlist; q.longbase = longbase; q.srow = srow; q.sh = sh;
     q.nblk = nblk; q.nx = (int)(S.Np / XT_TILE); q.nxt = q.nx * (int)(S.dq / XT_TILE); q.n = (int)NE; q.Np = (int)S.Np; q.V = (int)V;
+    q.long_seg = (int)B.long_seg;
     bwd_xt_segments_kernel<<<q.nxt + segment_blocks(NE, V), 256, 0, st>>>(q);
   }
   delete tm_prep;
   {
     KernelTimer tm(SCE_K_DW_FINAL, st);
-    bwd_dw_long_kernel<<<dim3((unsigned)std::min<int64_t>(NE / LONG_SEG + 1, LONG_GRID), (unsigned)(S.dq / 256)), 256, 0, st>>>(longlist, segoff, srow, sh, xq, S.ldx,
+    bwd_dw_long_kernel<<<dim3((unsigned)std::min<int64_t>(B.long_slots, LONG_GRID), (unsigned)(S.dq / 256)), 256, 0, st>>>(longlist, segoff, srow, sh, xq, S.ldx,
                                                                                                                               S.dq, longsum);
   }
   const float sc = (float)a->x_s * (float)a->w_s, k1 = sc * 2.0f * LOG2E / a->cap, c2 = -2.0f * a->cap * LOG2E;
@@ -756,7 +780,7 @@ extern "C" int sce_backward(const sce_args* a) {
   tail.buf = nullptr; tail.tile0 = -1; tail.ntail = 0; tail.kp = 1; tail.share = 1;
   DwOut wo;
   wo.dw = a->dw; wo.dw_ld = a->dw_ld; wo.segoff = segoff; wo.srow = srow; wo.sh = sh; wo.xq = xq; wo.longsum = longsum; wo.longbase = longbase;
-  wo.xi = xi; wo.dc = dcp; wo.ldx = S.ldx; wo.dq = S.dq; wo.x_s = (float)a->x_s; wo.d = (int)d; wo.V = (int)V;
+  wo.xi = xi; wo.dc = dcp; wo.ldx = S.ldx; wo.dq = S.dq; wo.x_s = (float)a->x_s; wo.d = (int)d; wo.V = (int)V; wo.long_seg = (int)B.long_seg;
   const bool dw_f32 = a->dw_dtype == SCE_F32;
   bool dw_done = false;                // every tile is stored, or will be from `tail`
   const bool dx_f32 = a->dx_dtype == SCE_F32;
@@ -797,7 +821,7 @@ extern "C" int sce_backward(const sce_args* a) {
     }
   };
   // dW over the rows [w0, w0 + gathered)
-  auto dw_launch = [&](int64_t w0, int64_t gathered, int64_t gorg, bool last) {
+  auto dw_launch = [&](int64_t w0, int64_t gathered, int64_t gorg) {
     DwParams wp;
     const int part = launch < nparts ? launch : nparts - 1;
     wp.xt = xt; wp.ghat_t = ghat_t + ((w0 - gorg) / 256) * (S.Vp / BK) * BLOCKED_KSTEP; wp.gexp = gexp + (w0 - gorg) / BK; wp.dwacc = (float*)((uint8_t*)dwacc + (size_t)part * B.part_stride);
@@ -808,8 +832,7 @@ extern "C" int sce_backward(const sce_args* a) {
       // When this launch is the only one and its last round of tiles would leave many CUs idle, that round is
       // shared out along K instead (bwd_dw_tail_kernel): the full rounds run as they are.
       const DwTailPlan tp = dw_tail_plan(S.dq, S.Vp, gathered);
-      const bool only = w0 == 0 && last && launch == 0;
-      if (only) {
+      if (B.one) {                       // (then w0 = 0, and this is the last launch as well as the first)
         const bool share = tp.use && B.tail_bytes >= tp.bytes && a->workspace_bytes >= B.off_dwtail + tp.bytes;
         const int grid = share ? tp.full : map_tile_rr_grid(CTd, CTv);
         if (grid > 0) {
@@ -833,7 +856,7 @@ extern "C" int sce_backward(const sce_args* a) {
     // 0.58 ms where one of 250 takes 0.56.  Under fp8 MFMA load the part runs at the clock its power limit allows, and
     // compute units left idle leave the others a higher one.)
     for (int64_t p0 = 0; p0 < S.Np; p0 += P) dx_panel(p0, (S.Np - p0 < P) ? (S.Np - p0) : P, 0);
-    for (int64_t w0 = 0; w0 < S.Np; w0 += Pw) dw_launch(w0, (S.Np - w0 < Pw) ? (S.Np - w0) : Pw, 0, w0 + Pw >= S.Np);
+    for (int64_t w0 = 0; w0 < S.Np; w0 += Pw) dw_launch(w0, (S.Np - w0 < Pw) ? (S.Np - w0) : Pw, 0);
   } else {
     int64_t w0 = 0;                      // first row of the rows gathered for the next dW launch
     for (int64_t p0 = 0; p0 < S.Np; p0 += P) {
@@ -853,7 +876,7 @@ extern "C" int sce_backward(const sce_args* a) {
       dx_panel(p0, prow, gorg);
       const int64_t gathered = p0 + prow - w0;
       if (gathered + P > Pw || p0 + prow >= S.Np) {      // the transposed scratch is full, or this was the last panel
-        dw_launch(w0, gathered, gorg, p0 + prow >= S.Np);
+        dw_launch(w0, gathered, gorg);
         w0 = p0 + prow;
       }
     }
