@@ -785,7 +785,7 @@ static_assert(sizeof(BlockLoss) == 16, "one float4 slot");
 // Folds the V-splits of a row and writes lse / loss / argmax and the saved row statistics: COMBINE_ROWS rows to a
 // workgroup, one wave to every G-th split (its 64 rows' records are 1 KB in a row), four records in flight per lane.
 // What bounds it is the chain of loads, not their volume: with one thread per row the records of a call of 61 rows and
-// 197 splits were 197 loads of one workgroup.  G = 4 for up to 16 splits, 16 beyond (rows too few to fill the chip
+// 197 splits were 197 loads of one workgroup.  Rows beyond N have no records (fwd_few_rows_kernel writes none).  G = 4 for up to 16 splits, 16 beyond (rows too few to fill the chip
 // without cutting the vocabulary finer); the order of the sums depends on G alone.
 constexpr int COMBINE_ROWS = 64;
 template <int G>
@@ -807,7 +807,7 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int s = s0 + q * G;
-        o[q] = s < S ? partials[(int64_t)s * Np + i] : make_float4(0.f, -INFINITY, __int_as_float(0x7fffffff), 0.f);
+        o[q] = s < S && i < N ? partials[(int64_t)s * Np + i] : make_float4(0.f, -INFINITY, __int_as_float(0x7fffffff), 0.f);
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {

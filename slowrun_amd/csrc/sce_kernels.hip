@@ -634,8 +634,8 @@ extern "C" int sce_forward(const sce_args* a) {
 
 // The same launches as sce_forward with the partial records in the library's static device array instead of a
 // caller's workspace: no allocation, by the caller for this call or by the library ever.  Calls on one device share
-// the array; nothing in it has to start at zero (the forward kernel writes every record that the combine kernel
-// reads), so nothing is cleared, but two calls in flight on one device at a time would overwrite each other's records.
+// the array; nothing in it has to start at zero (the forward kernels write the records of all N rows, and the combine kernel
+// reads no others), so nothing is cleared, but two calls in flight on one device at a time would overwrite each other's records.
 extern "C" int sce_forward_noalloc(const sce_args* a) {
   if (int rc = check_common(a, true)) return rc;
   void* sp = g_scratch[a->device];              // set by check_device (inside check_common) for this very device

@@ -92,3 +92,31 @@ def test_one_launch_of_dw_up_to_131072_rows():
     torch.nn.functional.cross_entropy(15.0 * torch.tanh(xf @ wf / 15.0), y).backward()
     assert float((dw - wf.grad).norm() / wf.grad.norm()) < 1e-2
     assert float((dx - xf.grad).norm() / xf.grad.norm()) < 4e-2      # (a row's 300 dlogits: their e4m3 rounding, 2^-4 / sqrt(3) of each at most)
+
+
+@pytest.mark.parametrize("bf16,keep", [(True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("N,offsets,d,V", [(1, 1, 16, 264), (61, 1, 272, 33000), (129, 2, 96, 33000), (300, 3, 1040, 4096), (1100, 1, 528, 263), (4200, 2, 256, 2056)])
+def test_nothing_depends_on_what_the_buffers_held(monkeypatch, N, offsets, d, V, bf16, keep):
+    """State and workspaces full of ones (NaN as floats, -1 as indices) or of zeros before the calls: the same bits after them."""
+    from slowrun_amd import cuda_kernels as ck
+    inp = configs.make_inputs("tiny_track", N=N, d=d, V=V)
+    x, w, y = inp.x.cuda().bfloat16(), inp.w.cuda().bfloat16(), inp.targets.cuda()
+    y[::5] = -1
+    mw = torch.tensor([1.0, 0.5, 0.25, 0.125][:offsets], device="cuda") if offsets > 1 else None
+    go = torch.rand(N, generator=torch.Generator().manual_seed(N)).cuda() / N
+    real, res = torch.empty, []
+    for fill in (0, 255):
+        def empty(*a, **k):
+            t = real(*a, **k)
+            if t.is_cuda:
+                t.view(torch.uint8).fill_(fill) if t.dtype == torch.uint8 else t.fill_(float("nan") if fill and t.is_floating_point() else 0)
+            return t
+        monkeypatch.setattr(torch, "empty", empty)
+        out, saved, lse, argmax, n_valid = ck.ce_forward(x, w, y, inp.x_s, inp.w_s, 15.0, "none", want_argmax=True, mtp_weights=mw, keep_dlogits=keep,
+                                                         operand_dtype=torch.bfloat16 if bf16 else None)
+        grads = () if bf16 else ck.ce_backward(saved, y, go, N, d, V, inp.x_s, inp.w_s, 15.0, 1.0, "none", torch.bfloat16, torch.float32, mtp_weights=mw,
+                                               keep_dlogits=keep)
+        monkeypatch.undo()
+        res.append((out, lse, argmax, n_valid, *grads))
+    for a, b in zip(*res):
+        assert torch.equal(a, b) and bool(torch.isfinite(a.float()).all())
