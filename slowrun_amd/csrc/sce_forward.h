@@ -611,8 +611,11 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
 // against this: 200 us against 51 (64 rows), 66 (128) and 101 (256); d = 4096, V = 4096, where 16 workgroups do it all:
 // 95 against 64 and 81, but 97 against 125 for 256 rows (a CU's LDS reads are the bound then): beyond 128 rows only with
 // FEW_TILES column tiles, half as many as there are CUs; d = 512, V = 8192: 36 against 18 and 23.
+// With so few column tiles that their workgroups' K loops are all there is, 128 rows go the general way from FEW_DEEP on, where its loop
+// is the shorter one and the copy small beside it (128 rows, cold weight: d = 32768, V = 256 510 us against 570, V = 1024 563 and
+// 575, V = 2048 750 and 572; d = 8192 160 and 158); 64 rows never (507 and 459 there).
 constexpr int FEW_K = 32;
-constexpr int FEW_MAX_ROWS = 256, FEW_TILES = 128, FEW_THREADS = 512;
+constexpr int FEW_MAX_ROWS = 256, FEW_TILES = 128, FEW_THREADS = 512, FEW_DEEP = 8192, FEW_DEEP_TILES = 8;
 template <int NB>
 struct FewRows {
   static constexpr int W_BYTES = FEW_K * 512, STAGE = W_BYTES + NB * 2048, STAGES = NB == 2 ? 7 : NB == 4 ? 6 : 4;

@@ -521,7 +521,7 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   auto direct = [&](const void* q, int32_t dtype, int64_t ld, int64_t rows) {
     return dtype == SCE_BF16 && ((uintptr_t)q & 15) == 0 && ld % 8 == 0 && ld < ((int64_t)1 << 31) / rows;
   };
-  const bool few = bf16ops && (N <= 128 || (N <= FEW_MAX_ROWS && CT >= FEW_TILES)) && V % 8 == 0 && direct(a->w, a->w_dtype, a->w_ld, FEW_K);
+  const bool few = bf16ops && (N <= 64 || (N <= 128 && (d <= FEW_DEEP || CT >= FEW_DEEP_TILES)) || (N <= FEW_MAX_ROWS && CT >= FEW_TILES)) && V % 8 == 0 && direct(a->w, a->w_dtype, a->w_ld, FEW_K);
   const bool few_x = few && direct(a->x, a->x_dtype, a->x_ld, FEW_MAX_ROWS);
   {
     KernelTimer tm(SCE_K_QUANT, st);

@@ -58,6 +58,12 @@ def test_few_rows_against_the_general_path(xdtype, N, d, V, vocab, offsets):
         assert torch.allclose(l0, ref, rtol=1e-5, atol=1e-4)
 
 
+@pytest.mark.parametrize("N,d,V", [(64, 8208, 264), (65, 8192, 264), (128, 8208, 1792), (128, 8208, 1800)])
+def test_deep_contractions_of_few_column_tiles(N, d, V):
+    """The lines in d and in column tiles at which 65 to 128 rows change their way: exact logits, as above."""
+    test_few_rows_against_the_general_path(torch.bfloat16, N, d, V, V, 1)
+
+
 @pytest.mark.parametrize("n,shape", [(1, (1,)), (255, (255,)), (257, (257,)), (4098, (2, 2049))])
 def test_target_probability_is_the_exponential_of_the_losses(n, shape):
     from slowrun_amd import cuda_kernels as ck
