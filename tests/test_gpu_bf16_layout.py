@@ -75,3 +75,29 @@ def test_target_probability_is_the_exponential_of_the_losses(n, shape):
     p = ck.target_probability(x, w, y, operand_dtype=torch.bfloat16)
     losses = ck.softcapped_cross_entropy(x, w, y, reduction="none", operand_dtype=torch.bfloat16)
     assert p.shape == losses.shape and torch.allclose(p, torch.where(y == -1, torch.zeros_like(losses), torch.exp(-losses)), rtol=1e-6, atol=0)
+
+
+@pytest.mark.parametrize("N,d,V", [(3, 48, 264), (64, 64, 2056), (128, 96, 520), (200, 32, 33000)])
+def test_infinities_and_nan_of_few_rows_as_in_the_general_path(N, d, V):
+    """Rows with an infinity, a NaN, a largest finite value, and a column of W with each: the few-rows kernel gives what the general
+    path gives -- the same maxima, the same infinities and NaN, and the same losses elsewhere (row sums in another order)."""
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(V)
+    inf, big = float("inf"), float(torch.finfo(torch.bfloat16).max)
+    for case in ("rows", "columns"):
+        x = torch.randint(-2, 3, (N, d), device="cuda", generator=gen).bfloat16() / 4
+        w = torch.randint(-2, 3, (d, V), device="cuda", generator=gen).bfloat16() / 4
+        if case == "rows":
+            for i, v in enumerate((inf, -inf, float("nan"), big)):
+                x[i * 7 % N, i] = v
+        else:
+            for i, v in enumerate((inf, -inf, float("nan"), big)):
+                w[i, (i * 61 + 5) % V] = v
+        y = torch.randint(0, V, (N,), device="cuda", generator=gen)
+        y[0], y[N // 2] = 5, 66
+        odd = torch.zeros(d, V + 1, device="cuda", dtype=torch.bfloat16)
+        odd[:, :V] = w
+        got = [ck.ce_forward(x, m, y, 1.0, 1.0, 15.0, "none", want_argmax=True, operand_dtype=torch.bfloat16) for m in (w, odd[:, :V])]
+        (l0, _, lse0, am0, nv0), (l1, _, lse1, am1, nv1) = got
+        assert torch.equal(am0, am1) and torch.equal(nv0, nv1)
+        assert torch.allclose(lse0, lse1, rtol=2e-6, atol=2e-5, equal_nan=True) and torch.allclose(l0, l1, rtol=2e-6, atol=2e-5, equal_nan=True)
