@@ -898,16 +898,18 @@ struct DwOut {
 
 // dW straight from the main loop: dW = x_s (xi (X~^T G) - sum over the column's target entries of h_i X_q[i, :]), cast and
 // stored by the workgroup that has the tile in its accumulators.  Used whenever one launch covers all rows: up to 131072 with
-// the dlogits kept; formed again, as many whole dX panels as fit in 131072 rows, and a workspace of the default size.  What the separate pass over an fp32 partial cost was its traffic: 8 bytes an element
-// written and read again (1 GB at d = 2560, V = 50304) around 2 bytes of result, 65 us of a 560 us step at N = 2048,
-// d = 768 and 172 us at N = 30011, d = 2560, whatever the number of rows.
+// the dlogits kept; formed again, as many whole dX panels as fit in 131072 rows, and a workspace of the default size.  What
+// the separate pass over an fp32 partial cost was its traffic: 8 bytes an element written and read again (1 GB at
+// d = 2560, V = 50304) around 2 bytes of result, 65 us of a 560 us step at N = 2048, d = 768 and 172 us at N = 30011,
+// d = 2560, whatever the number of rows.
 //
 // The epilogue must not wait on memory: one wave per SIMD has nothing to hide a load behind (gathering the one-hot rows
 // with dependent loads was measured at +0.5 ms of a 20 ms step).  So the rows X_q[i] of the tile's target entries -- the
 // short columns' only; columns with LONG_SEG or more entries have their chunk sums ready -- go to LDS with direct loads:
-// before the main loop, into what the K slots and the block exponents leave free (about 100 entries of 256 bytes), if they
-// fit there -- most tiles of most batches do -- and otherwise into the K slots after it, as many row blocks at a time as
-// fit (a row block's 64 columns have at most 64 (LONG_SEG - 1) = 448 entries).  Each lane then walks the entries of its own
+// before the main loop, into what the K slots and the block exponents leave free (100 to 112 entries of 256 bytes), if they
+// fit there -- all tiles' do of 16384 rows with uniform targets over 50257 columns, four fifths of the tiles' of 65536
+// rows with Zipf targets, next to none of 26400 uniform ones -- and otherwise into the K slots after it, as many row blocks at a
+// time as fit (a row block's 64 columns have at most 64 (LONG_SEG - 1) = 448 entries).  Each lane then walks the entries of its own
 // column.  A 16-byte chunk c of an entry's 256 bytes lies at position c ^ (entry & 15): the lanes of a wave read the same
 // columns j of neighbouring entries, which would all lie in the same banks.
 // On the way out a bf16 quadrant is turned in LDS, 32 columns x 64 rows at a time, by the transposing read, so that a lane

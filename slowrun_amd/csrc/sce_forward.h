@@ -607,7 +607,10 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
 // d is a multiple of 16, the K of one instruction: the last slice may be half a one, and nothing is padded.
 // In a slice the pair of 16-byte chunks c / 2 of W's row k lies at position (c / 2) ^ (k & 3), chunk c of a row of x at
 // c ^ (row / 2 & 3): the rows that one read touches would otherwise lie in the same banks.
-// 61 rows, d = 2560, V = 50304: copy 88 us and general kernel 86, now 44.7 (5.8 TB/s).  The whole pass, copy and general kernel
+// 61 rows, d = 2560, V = 50304: copy 88 us and general kernel 86, now 44.7 with the weight just
+// read before (5.8 TB/s: part of its 257 MB is still in the 256 MB memory-side cache) and 92 right
+// after a 1 GiB fill (whose lines are then still on their way out; the copy 225 and the general kernel 811 there, with 16
+// splits).  The whole pass, copy and general kernel
 // against this: 200 us against 51 (64 rows), 66 (128) and 101 (256); d = 4096, V = 4096, where 16 workgroups do it all:
 // 95 against 64 and 81, but 97 against 125 for 256 rows (a CU's LDS reads are the bound then): beyond 128 rows only with
 // FEW_TILES column tiles, half as many as there are CUs; d = 512, V = 8192: 36 against 18 and 23.

@@ -641,7 +641,7 @@ extern "C" int sce_forward_noalloc(const sce_args* a) {
   void* sp = g_scratch[a->device];              // set by check_device (inside check_common) for this very device
   if (!sp) return fail(SCE_EHIP, "no static scratch on device %d", a->device);
   return forward_impl(a, sp, NOALLOC_SCRATCH_BYTES,
-                      "the static scratch of sce_forward_noalloc (8 MiB: N rounded up to 256 times the number of V-splits, 8 to 16, "
+                      "the static scratch of sce_forward_noalloc (8 MiB: N rounded up to 256 times the least number of V-splits, up to 16, "
                       "may not exceed 524288; use sce_forward with a workspace)");
 }
 

@@ -101,3 +101,33 @@ def test_infinities_and_nan_of_few_rows_as_in_the_general_path(N, d, V):
         (l0, _, lse0, am0, nv0), (l1, _, lse1, am1, nv1) = got
         assert torch.equal(am0, am1) and torch.equal(nv0, nv1)
         assert torch.allclose(lse0, lse1, rtol=2e-6, atol=2e-5, equal_nan=True) and torch.allclose(l0, l1, rtol=2e-6, atol=2e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("N,d,V", [(61, 272, 33000), (200, 96, 33000)])
+def test_scoring_captured_in_a_hip_graph(N, d, V):
+    """The scoring call captured once and replayed on new rows, weights and targets: each replay the bits of the direct call."""
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(N, d, device="cuda", generator=gen).bfloat16()
+    w = (torch.randn(d, V, device="cuda", generator=gen) * d ** -0.5).bfloat16()
+    y = torch.randint(0, V, (N,), device="cuda", generator=gen)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ck.target_probability(x, w, y, operand_dtype=torch.bfloat16)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = ck.target_probability(x, w, y, operand_dtype=torch.bfloat16)
+    for trial in range(4):
+        x.copy_(torch.randn(N, d, device="cuda", generator=gen).bfloat16())
+        w.mul_(1.25)
+        y.copy_(torch.randint(0, V, (N,), device="cuda", generator=gen))
+        y[trial::5] = -1
+        graph.replay()
+        torch.cuda.synchronize()
+        got = captured.clone()
+        want = ck.target_probability(x, w, y, operand_dtype=torch.bfloat16)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and bool((got[y != -1] > 0).all()) and bool((got[y == -1] == 0).all())
