@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
   // blocks beyond the rows' (there are some with few entries only): the entries' places
   if ((int)blockIdx.x >= Np / 256) return rank_targets(rank_keys, blockIdx.x - Np / 256, targets, ignore_index, N, Np, V, key_none, n_predict, skeys, perm);
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i == 0) longlist[0] = 0;        // counter of the long-column list, filled by column_segments
+  if (i == 0) { longlist[0] = 0; longlist[1] = 0; }        // counters of the long-column lists, filled by column_segments
   float r = 0.f;
   float h[4] = {0.f, 0.f, 0.f, 0.f};
   // the forward call that wrote `saved` was asked for something else (kept dlogits, vocabulary limit, offsets, cap):
@@ -589,10 +589,52 @@ __global__ __launch_bounds__(256) void bwd_dx_kernel(DxParams p_in) {
   }
 }
 
+// A column that is the target of at least long_seg (LONG_SEG or LONG_SEG_PARTS) rows has its segment of the sorted list cut into
+// nch = ceil(L / LONG_CHUNK) equal chunks (the last one may be shorter); chunk c starts at sorted
+// position s0 + c * ceil(L / nch).
+__device__ __forceinline__ void long_chunks(int L, int& nch, int& len) {
+  nch = (L + LONG_CHUNK - 1) / LONG_CHUNK;
+  len = (L + nch - 1) / nch;
+}
+
+// The chunk sums of the columns of several chunks are added up, in order, into the first one's place, where everything after finds a
+// long column's sum.  One block of 256 rows of dW of one column at a time, all its loads but for every eighth in flight together.  A
+// few microseconds of work that only the kernels storing dW wait for: it rides in the grid of bwd_dx_finish_kernel where there is
+// one before them.  (Left to its readers it was a walk at the latency of memory, one wave to a SIMD: with Zipf targets the
+// tiles of the first columns took 100 us longer than the rest, which a dW of one or two rounds of tiles waits for whole.
+// 24064 rows of three offsets, d = 416, V = 27712: bwd_dw_out_kernel 406 us, now
+// 306; 29184 rows of three, d = 2512, V = 9664: 512, now 356 and 8 for the fold.)
+struct FoldParams {
+  const int32_t *longlist, *longbase, *segoff;
+  float* longsum;
+  int64_t dq;
+  int slots, first;            // first: the first workgroup of the grid that folds
+};
+__device__ __forceinline__ void fold_chunks(const FoldParams& f, int block, int nblocks) {
+  const int ny = (int)(f.dq / 256), items = f.longlist[1] * ny;
+  for (int item = block; item < items; item += nblocks) {
+    const int v = f.longlist[2 + f.slots + item / ny];
+    int nch, len;
+    long_chunks(f.segoff[v + 1] - f.segoff[v], nch, len);
+    float* s = f.longsum + (int64_t)f.longbase[v] * f.dq + (item % ny) * 256 + threadIdx.x;
+    float sum = 0.f;
+    for (int c0 = 0; c0 < nch; c0 += 8) {
+      float x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = c0 + u < nch ? s[(int64_t)(c0 + u) * f.dq] : 0.f;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += x[u];
+    }
+    *s = sum;
+  }
+}
+__global__ __launch_bounds__(256) void bwd_dw_fold_kernel(FoldParams f) { fold_chunks(f, blockIdx.x, gridDim.x); }
+
 // Sum of the K-split partials, row scale, one-hot term, cast: a workgroup per 32 rows x 128 columns, a wave per 32 of the
 // columns.  A thread's values are four quads of one row; they go out through LDS as whole pieces of rows.
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_dx_finish_kernel(DxParams p_in) {
+__global__ __launch_bounds__(256) void bwd_dx_finish_kernel(DxParams p_in, FoldParams f) {
+  if ((int)blockIdx.x >= f.first) return fold_chunks(f, blockIdx.x - f.first, gridDim.x - f.first);
   DxParams p = p_in;
   if (p.dc) p.w_s = p.dc->w_s;
   constexpr int RB = 128 * (int)sizeof(T), PITCH = RB + 16, CH = RB / 16;
@@ -738,18 +780,10 @@ __global__ __launch_bounds__(256) void bwd_dw_tail_kernel(DwParams p, DwTail tl)
         *reinterpret_cast<v4f*>(dst0 + (4 * a + b) * 1024 + q * 256) = (v4f){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
 }
 
-// A column that is the target of at least long_seg (LONG_SEG or LONG_SEG_PARTS) rows has its segment of the sorted list cut into
-// nch = ceil(L / LONG_CHUNK) equal chunks (the last one may be shorter); chunk c starts at sorted
-// position s0 + c * ceil(L / nch).
-__device__ __forceinline__ void long_chunks(int L, int& nch, int& len) {
-  nch = (L + LONG_CHUNK - 1) / LONG_CHUNK;
-  len = (L + nch - 1) / nch;
-}
-
-// From the sorted keys: segoff[v] = first position whose key is at least v, v = 0 .. V, and the list of (column, chunk)
-// pairs of the long columns (order irrelevant: each pair is handled on its own).  longlist[0] is the count, then two
-// ints per pair; the position of a pair in the list is the slot of its chunk sum, and longbase[v] is the position of
-// column v's first pair.  One column per thread, by bisection: first among every stride-th key (in LDS), then within one
+// From the sorted keys: segoff[v] = first position whose key is at least v, v = 0 .. V, and the list of the long
+// columns, one entry per chunk (order irrelevant: each is handled on its own): longlist[0] is the count, the column of slot n
+// stands in longlist[2 + n], and longbase[v] is the slot of column v's first chunk sum.  Behind them the columns of several
+// chunks once more, longlist[1] of them.  One column per thread, by bisection: first among every stride-th key (in LDS), then within one
 // stride.  (A thread per key that fills the gap up to the next key runs as long as the widest gap: with Zipf targets the
 // rare end of the vocabulary holds gaps of thousands of columns, and 2048 rows took 63 us; this takes 4.7.)
 // Also: row and coefficient of every sorted entry (srow, sh), so that the kernels that walk a segment load them side by
@@ -759,7 +793,7 @@ constexpr int SEG_ENTRIES = 512;
 static inline int segment_blocks(int64_t n, int64_t V) { return (int)std::max<int64_t>(V / 256 + 1, (n + SEG_ENTRIES - 1) / SEG_ENTRIES); }
 struct SegShared { int32_t top[256], seg[257]; };
 __device__ __forceinline__ void column_segments(SegShared& shared, int block, int nblocks, const int32_t* __restrict__ skeys, const int32_t* __restrict__ perm,
-                                                const float* __restrict__ hcoef, int n, int Np, int V, int long_seg, int32_t* __restrict__ segoff,
+                                                const float* __restrict__ hcoef, int n, int Np, int V, int long_seg, int slots, int32_t* __restrict__ segoff,
                                                 int32_t* __restrict__ longlist, int32_t* __restrict__ longbase,
                                                 int32_t* __restrict__ srow, float* __restrict__ sh) {
   auto& top = shared.top;
@@ -799,7 +833,8 @@ __device__ __forceinline__ void column_segments(SegShared& shared, int block, in
   long_chunks(L, nch, len);
   const int at = atomicAdd(&longlist[0], nch);
   longbase[v] = at;
-  for (int c = 0; c < nch; ++c) { longlist[1 + 2 * (at + c)] = v; longlist[2 + 2 * (at + c)] = c; }
+  for (int c = 0; c < nch; ++c) longlist[2 + at + c] = v;
+  if (nch > 1) longlist[2 + slots + atomicAdd(&longlist[1], 1)] = v;
 }
 
 // The two in one launch, blocks [0, nxt) the tiles of X~ and the rest the segments: neither needs the other, and on few rows
@@ -813,13 +848,13 @@ struct XtSegParams {
   const int32_t *skeys, *perm;
   int32_t *segoff, *longlist, *longbase, *srow;
   float* sh;
-  int nblk, nxt, nx, n, Np, V, long_seg;
+  int nblk, nxt, nx, n, Np, V, long_seg, slots;
 };
 __global__ __launch_bounds__(256) void bwd_xt_segments_kernel(XtSegParams p) {
   __shared__ union { XtShared x; SegShared s; } shared;
   const int bid = blockIdx.x;
   if (bid < p.nxt) xt_tile(shared.x, bid % p.nx, bid / p.nx, p.xq, p.dp, p.ldx, p.kbn, p.rho, p.blockmax, p.nblk, p.xi, p.xt);
-  else column_segments(shared.s, bid - p.nxt, gridDim.x - p.nxt, p.skeys, p.perm, p.hcoef, p.n, p.Np, p.V, p.long_seg, p.segoff, p.longlist, p.longbase, p.srow, p.sh);
+  else column_segments(shared.s, bid - p.nxt, gridDim.x - p.nxt, p.skeys, p.perm, p.hcoef, p.n, p.Np, p.V, p.long_seg, p.slots, p.segoff, p.longlist, p.longbase, p.srow, p.sh);
 }
 
 // One-hot part of dW for the long columns: longsum[slot][:] = sum over the chunk's rows of h_i X_q[i, :].
@@ -827,15 +862,15 @@ __global__ __launch_bounds__(256) void bwd_xt_segments_kernel(XtSegParams p) {
 // length the host does not know; the rows of the chunk are split over 16
 // row-lanes (8 independent loads in flight each) and folded in a fixed order, so the result does
 // not depend on scheduling.
-constexpr int LONG_GRID = 1024;
+constexpr int LONG_GRID = 1024, FOLD_GRID = 512;
 __global__ __launch_bounds__(256) void bwd_dw_long_kernel(const int32_t* __restrict__ longlist, const int32_t* __restrict__ segoff,
                                                          const int32_t* __restrict__ srow, const float* __restrict__ sh,
                                                          const uint8_t* __restrict__ xq, int64_t ldx, int64_t dq,
-                                                         float* __restrict__ longsum) {
+                                                         const int32_t* __restrict__ longbase, float* __restrict__ longsum) {
   __shared__ float red[16][256];
   const int count = longlist[0];
   for (int slot = blockIdx.x; slot < count; slot += gridDim.x) {
-    const int v = longlist[1 + 2 * slot], ch = longlist[2 + 2 * slot];
+    const int v = longlist[2 + slot], ch = slot - longbase[v];
     int nch, len;
     const int seg0 = segoff[v], seg1 = segoff[v + 1];
     long_chunks(seg1 - seg0, nch, len);
@@ -887,8 +922,8 @@ struct DwOut {
   const int32_t* srow;         // row i of a sorted entry
   const float* sh;             // its coefficient h
   const uint8_t* xq;           // [Np], row stride ldx
-  const float* longsum;        // [slot][dq]: chunk sums of the long columns
-  const int32_t* longbase;     // first slot of a long column
+  const float* longsum;        // [slot][dq]: sums of the long columns
+  const int32_t* longbase;     // slot of a long column
   const float* xi;
   const DevConsts* dc;         // non-NULL: x_s comes from here
   int64_t ldx, dq;
@@ -905,7 +940,7 @@ struct DwOut {
 //
 // The epilogue must not wait on memory: one wave per SIMD has nothing to hide a load behind (gathering the one-hot rows
 // with dependent loads was measured at +0.5 ms of a 20 ms step).  So the rows X_q[i] of the tile's target entries -- the
-// short columns' only; columns with LONG_SEG or more entries have their chunk sums ready -- go to LDS with direct loads:
+// short columns' only; columns with LONG_SEG or more entries have their sums ready -- go to LDS with direct loads:
 // before the main loop, into what the K slots and the block exponents leave free (100 to 112 entries of 256 bytes), if they
 // fit there -- all tiles' do of 16384 rows with uniform targets over 50257 columns, four fifths of the tiles' of 65536
 // rows with Zipf targets, next to none of 26400 uniform ones -- and otherwise into the K slots after it, as many row blocks at a
@@ -1042,16 +1077,12 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
       const int L = spos[c + 1] - spos[c];
       if (__builtin_amdgcn_ballot_w64(L >= LONG_SEG) != 0) {
         if (L >= LONG_SEG) {
-          int nch, len;
-          long_chunks(L, nch, len);
           const float* ls = o.longsum + (int64_t)o.longbase[v] * o.dq + rt * 256 + wa * 128 + ah * 64 + 4 * h;
-          for (int k = 0; k < nch; ++k, ls += o.dq) {           // fixed order
 #pragma unroll
-            for (int g = 0; g < 8; ++g) {
-              const v4f s = *reinterpret_cast<const v4f*>(ls + 32 * (g >> 2) + 8 * (g & 3));
+          for (int g = 0; g < 8; ++g) {
+            const v4f s = *reinterpret_cast<const v4f*>(ls + 32 * (g >> 2) + 8 * (g & 3));
 #pragma unroll
-              for (int m = 0; m < 4; ++m) val[4 * g + m] -= s[m] * x_s;
-            }
+            for (int m = 0; m < 4; ++m) val[4 * g + m] -= s[m] * x_s;
           }
         }
       }
@@ -1101,7 +1132,7 @@ __device__ __forceinline__ float add_product(float s, float a, float b) {
 // 16 blocks of 64 x 64 elements), and every tile where dW took more than one launch (grid = blocks of 64 columns x 64
 // rows of dW).  A thread owns one column v and four groups of four rows j: 16 consecutive rows, or, of the pieces of a K-split
 // tile, the rows that one lane's accumulators of a 32 x 32 block are.  The segment sum is formed here for short segments
-// and read from the chunk sums for long ones.
+// and read from the sums of the long columns for the others.
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restrict__ dwacc, int nparts, int64_t part_stride, int64_t Vp, DwOut o, DwTail tl, int RT,
                                                           int CT) {
@@ -1146,17 +1177,13 @@ __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restri
   for (int q = 0; q < 4; ++q) val[q] *= scale;
   const int s0 = o.segoff[v], L = o.segoff[v + 1] - s0;
   if (L >= o.long_seg) {
-    int nch, len;
-    long_chunks(L, nch, len);
-    for (int c = 0; c < nch; ++c) {                       // fixed order
-      const float* ls = o.longsum + (int64_t)(o.longbase[v] + c) * o.dq + j0;
+    const float* ls = o.longsum + (int64_t)o.longbase[v] * o.dq + j0;
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
-        for (int m = 0; m < 4; ++m) val[q][m] -= ls[q * step + m] * x_s;
-    }
+      for (int m = 0; m < 4; ++m) val[q][m] -= ls[q * step + m] * x_s;
   } else if (L >= LONG_SEG) {
-    // where dW took several launches: the entries' sum first and then x_s, as it comes from the chunk sums otherwise
+    // where dW took several launches: the entries' sum first and then x_s, as it comes from the long columns' sums otherwise
     v4f sum[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) sum[q] = (v4f){0.f, 0.f, 0.f, 0.f};

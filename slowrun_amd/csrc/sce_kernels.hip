@@ -242,14 +242,14 @@ static BwdLayout bwd_layout(const SavedLayout& S, int64_t P, int64_t Pw, int npa
   B.off_ghat_t = take(kept ? 0 : (size_t)S.Vp * Pw);
   B.off_gexp = take(kept ? 0 : (size_t)(S.Vp / 128) * (Pw / 128) * 4);      // block exponents of the dlogits
   B.part_stride = ((size_t)S.dq * S.Vp * 4 + 255) / 256 * 256;
-  // The long columns' (column, chunk) pairs and chunk sums -- a column has at most one chunk per long_seg of its entries, and one
+  // The long columns' lists and chunk sums -- a column has at most one chunk per long_seg of its entries, and one
   // more per LONG_CHUNK -- and behind them the fp32 partials of dW, one per launch.  A single launch has none.  With the
   // dlogits kept it needs no room for them either; a workspace for dlogits that are formed again has it (with less of them in
   // hand at a time the same workspace serves several launches), and the sums of the shorter columns lie there.
   const size_t dlogits_end = o;
   auto long_columns = [&](int64_t slots) {
     B.long_slots = slots;
-    B.off_longlist = take((size_t)(2 * slots + 2) * 4);
+    B.off_longlist = take((size_t)(2 * slots + 2) * 4);      // two counters, a column for every slot, the columns of several slots
     B.off_longsum = take((size_t)slots * S.dq * 4);
   };
   long_columns(NE / LONG_SEG_PARTS + 1);
@@ -764,14 +764,14 @@ extern "C" int sce_backward(const sce_args* a) {
     q.xq = xq; q.dp = S.dp; q.ldx = S.ldx; q.kbn = S.Np / BK; q.rho = rho; q.blockmax = blockmax; q.hcoef = hcoef; q.xi = xi; q.xt = xt;
     q.skeys = skeys; q.perm = perm; q.segoff = segoff; q.longlist = longlist; q.longbase = longbase; q.srow = srow; q.sh = sh;
     q.nblk = nblk; q.nx = (int)(S.Np / XT_TILE); q.nxt = q.nx * (int)(S.dq / XT_TILE); q.n = (int)NE; q.Np = (int)S.Np; q.V = (int)V;
-    q.long_seg = (int)B.long_seg;
+    q.long_seg = (int)B.long_seg; q.slots = (int)B.long_slots;
     bwd_xt_segments_kernel<<<q.nxt + segment_blocks(NE, V), 256, 0, st>>>(q);
   }
   delete tm_prep;
   {
     KernelTimer tm(SCE_K_DW_FINAL, st);
     bwd_dw_long_kernel<<<dim3((unsigned)std::min<int64_t>(B.long_slots, LONG_GRID), (unsigned)(S.dq / 256)), 256, 0, st>>>(longlist, segoff, srow, sh, xq, S.ldx,
-                                                                                                                              S.dq, longsum);
+                                                                                                                              S.dq, longbase, longsum);
   }
   const float sc = (float)a->x_s * (float)a->w_s, k1 = sc * 2.0f * LOG2E / a->cap, c2 = -2.0f * a->cap * LOG2E;
   const int CTv = (int)(S.Vp / 256), CTd = (int)(S.dq / 256);
@@ -784,6 +784,14 @@ extern "C" int sce_backward(const sce_args* a) {
   const bool dw_f32 = a->dw_dtype == SCE_F32;
   bool dw_done = false;                // every tile is stored, or will be from `tail`
   const bool dx_f32 = a->dx_dtype == SCE_F32;
+  FoldParams fold;
+  fold.longlist = longlist; fold.longbase = longbase; fold.segoff = segoff; fold.longsum = longsum; fold.dq = S.dq; fold.slots = (int)B.long_slots; fold.first = 0;
+  const int fold_blocks = (int)std::min<int64_t>(NE / (LONG_CHUNK + 1) * (S.dq / 256), FOLD_GRID);      // (0: no column can have two chunks)
+  bool folded = fold_blocks == 0;      // launched, with the finishing kernel of a K-split dX panel or by itself
+  auto ensure_folded = [&]() {
+    if (!folded) bwd_dw_fold_kernel<<<fold_blocks, 256, 0, st>>>(fold);
+    folded = true;
+  };
   const int smem_dx = smem_scaled((int)(S.Vp / BK), SMEM_DX);
   // dX of the rows [p0, p0 + prow) (a multiple of 256), the dlogits buffer standing for rows from gorg on
   auto dx_params = [&](int64_t p0, int64_t prow, int64_t gorg) {
@@ -810,13 +818,16 @@ extern "C" int sce_backward(const sce_args* a) {
       if (dx_f32) bwd_dx_kernel<float, false><<<map_tile_grid(dp_.RT, CTd), NTHREADS, smem_dx, st>>>(dp_);
       else bwd_dx_kernel<bf16_t, false><<<map_tile_grid(dp_.RT, CTd), NTHREADS, smem_dx, st>>>(dp_);
     } else if (dp_.rows > 0) {
-      const int fgrid = tiles * 16;
+      FoldParams f = fold;
+      f.first = tiles * 16;
+      const int fgrid = f.first + (folded ? 0 : fold_blocks);
+      folded = true;
       if (dx_f32) {
         bwd_dx_kernel<float, true><<<map_tile_grid(dp_.RT, CTd * ksplit), NTHREADS, smem_dx, st>>>(dp_);
-        bwd_dx_finish_kernel<float><<<fgrid, 256, 0, st>>>(dp_);
+        bwd_dx_finish_kernel<float><<<fgrid, 256, 0, st>>>(dp_, f);
       } else {
         bwd_dx_kernel<bf16_t, true><<<map_tile_grid(dp_.RT, CTd * ksplit), NTHREADS, smem_dx, st>>>(dp_);
-        bwd_dx_finish_kernel<bf16_t><<<fgrid, 256, 0, st>>>(dp_);
+        bwd_dx_finish_kernel<bf16_t><<<fgrid, 256, 0, st>>>(dp_, f);
       }
     }
   };
@@ -829,6 +840,7 @@ extern "C" int sce_backward(const sce_args* a) {
     wp.RT = CTd; wp.CT = CTv; wp.KT = (int)(gathered / BK);
     {
       KernelTimer tm(SCE_K_DW, st);
+      if (B.one) ensure_folded();
       // When this launch is the only one and its last round of tiles would leave many CUs idle, that round is
       // shared out along K instead (bwd_dw_tail_kernel): the full rounds run as they are.
       const DwTailPlan tp = dw_tail_plan(S.dq, S.Vp, gathered);
@@ -892,6 +904,7 @@ extern "C" int sce_backward(const sce_args* a) {
   }
   if (!dw_done || tail.tile0 >= 0) {
     KernelTimer tm_fin(SCE_K_DW_FINAL, st);
+    ensure_folded();
     const dim3 g = dw_done ? dim3(16, (unsigned)tail.ntail) : dim3((unsigned)((V + 63) / 64), (unsigned)((d + 63) / 64));
     const int np = launch < nparts ? launch : nparts;
     if (dw_f32) bwd_dw_final_kernel<float><<<g, 256, 0, st>>>(dwacc, np, (int64_t)(B.part_stride / 4), S.Vp, wo, tail, CTd, CTv);

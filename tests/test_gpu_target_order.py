@@ -75,3 +75,37 @@ def test_one_hot_part_of_dw_of_more_entries_than_columns(N, offsets, V):
     ref = float(sum(N - k for k in range(offsets))) / V - count
     assert float((dw[0].double() - ref).abs().max()) <= 2.0 ** -20 * N * offsets
     assert float(dw[1:].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("panel_rows", [0, 256])
+@pytest.mark.parametrize("N,offsets,d,V", [(257, 1, 16, 64), (3000, 1, 272, 256), (9000, 2, 64, 512), (2000, 1, 4352, 256), (1100, 2, 8448, 64), (70000, 1, 32, 1024)])
+def test_columns_of_many_rows(N, offsets, d, V, panel_rows):
+    """Columns that are the target of hundreds to tens of thousands of rows: the sums of their chunks are added up before dW is
+    stored, in the grid that finishes a K-split dX or by themselves, for one launch of dW and for several.  Whole numbers in x
+    and a zero head: every product and sum is exact, and dW is sum_i x_i (1 / V - onehot), to the last fp32 rounding of each step."""
+    from slowrun_amd import _lib
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randint(-2, 3, (N, d), device="cuda", generator=gen).float()
+    w = torch.zeros(d, V, device="cuda")
+    y = torch.randint(0, V, (N,), device="cuda", generator=gen)
+    r = torch.rand(N, device="cuda", generator=gen)
+    y[r < 0.6], y[r < 0.2] = V - 1, 5
+    y[::11] = -1
+    mtp = torch.ones(offsets, device="cuda")
+    _out, saved, *_ = ck.ce_forward(x, w, y, 1.0, 1.0, 15.0, "none", mtp_weights=mtp, keep_dlogits=False)
+    args = (saved, y, torch.ones(N, device="cuda"), N, d, V, 1.0, 1.0, 15.0, 1.0, "none", torch.float32, torch.float32)
+    nbytes = _lib.sizes_for(N, d, V, offsets).bwd_workspace_min_bytes if panel_rows else None
+    first = None
+    for _ in range(3):                     # (the same bits every time)
+        dx, dw = ck.ce_backward(*args, mtp_weights=mtp, panel_rows=panel_rows, workspace_bytes=nbytes)
+        assert first is None or torch.equal(dw, first)
+        first = dw
+    ref = torch.zeros(d, V, dtype=torch.float64, device="cuda")
+    xd = x.double()
+    for k in range(offsets):
+        ok = torch.arange(N - k, device="cuda")[y[k:] >= 0]
+        ref += xd[ok].sum(0)[:, None] / V
+        ref.index_add_(1, y[k:][ok], -xd[ok].t().contiguous())
+    # 2 |x| N offsets bounds what any partial sum reaches; a handful of roundings of it at 2^-24
+    assert float((dw.double() - ref).abs().max()) <= 2.0 ** -20 * 2 * N * offsets
