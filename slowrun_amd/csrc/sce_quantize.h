@@ -8,29 +8,36 @@ namespace sce {
 // ------------------------------------------------------------------------------------------
 // quantisation
 // ------------------------------------------------------------------------------------------
-// 16 consecutive elements starting at p as floats after the scaling; elements at or beyond
-// `valid` are 0.  16-byte loads when the run is complete, aligned or not: one element at a time, a wave's lanes touch
-// a different cache line each, 16 times over.
-template <typename T>
-__device__ __forceinline__ void load16_scaled(const T* __restrict__ p, int64_t valid, const Scaler scale, float (&v)[16]) {
-  if (valid >= 16) {
-    if constexpr (sizeof(T) == 2) {
-      const v4i r0 = *reinterpret_cast<const v4i_any*>(p), r1 = *reinterpret_cast<const v4i_any*>(p + 8);
+// 16 consecutive elements starting at p as floats after the scaling; elements at or beyond `valid` are 0.  16-byte loads when the
+// run is complete, in a branch of their own where it is not aligned (one element at a time, the lanes of a wave touch a different
+// cache line each, 16 times over; one branch for both, with the accesses of the unaligned one, was 4 % slower on aligned rows
+// in quantize_w_kernel).  ANY = false, where the branch costs the kernel a wave per SIMD: aligned runs only.
+template <typename T, typename VI, typename VF>
+__device__ __forceinline__ void load16_whole(const T* __restrict__ p, const Scaler scale, float (&v)[16]) {
+  if constexpr (sizeof(T) == 2) {
+    const v4i r0 = *reinterpret_cast<const VI*>(p), r1 = *reinterpret_cast<const VI*>(p + 8);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        v[2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] << 16));
-        v[2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] & 0xffff0000u));
-        v[8 + 2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] << 16));
-        v[8 + 2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] & 0xffff0000u));
-      }
-    } else {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const v4f r = *reinterpret_cast<const v4f_any*>(p + 4 * q);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) v[4 * q + m] = scale.apply<T>(r[m]);
-      }
+    for (int m = 0; m < 4; ++m) {
+      v[2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] << 16));
+      v[2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] & 0xffff0000u));
+      v[8 + 2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] << 16));
+      v[8 + 2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] & 0xffff0000u));
     }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const v4f r = *reinterpret_cast<const VF*>(p + 4 * q);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) v[4 * q + m] = scale.apply<T>(r[m]);
+    }
+  }
+}
+template <typename T, bool ANY = true>
+__device__ __forceinline__ void load16_scaled(const T* __restrict__ p, int64_t valid, const Scaler scale, float (&v)[16]) {
+  if (valid >= 16 && (((uintptr_t)p) & 15) == 0) {
+    load16_whole<T, v4i, v4f>(p, scale, v);
+  } else if (ANY && valid >= 16) {
+    load16_whole<T, v4i_any, v4f_any>(p, scale, v);
   } else {
 #pragma unroll
     for (int m = 0; m < 16; ++m) v[m] = (m < valid) ? scale.apply<T>(Elem<T>::load(p + m)) : 0.f;
@@ -88,7 +95,7 @@ __global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const T* __restri
   float ss = 0.f;
   for (int64_t c = lane; c * 16 < cols; c += 64) {
     float v[16];
-    load16_scaled<T>(row + c * 16, cols - c * 16, one, v);      // scaling by 1 is exact: the values themselves
+    load16_scaled<T, false>(row + c * 16, cols - c * 16, one, v);      // scaling by 1 is exact: the values themselves
 #pragma unroll
     for (int m = 0; m < 16; ++m) ss = fmaf(v[m], v[m], ss);
   }
@@ -99,7 +106,7 @@ __global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const T* __restri
     uint32_t out[4] = {0, 0, 0, 0};
     if (c * 16 < cols) {
       float v[16];
-      load16_scaled<T>(row + c * 16, cols - c * 16, one, v);
+      load16_scaled<T, false>(row + c * 16, cols - c * 16, one, v);
 #pragma unroll
       for (int m = 0; m < 16; ++m) {
         float y = v[m] * rstd;

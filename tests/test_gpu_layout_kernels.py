@@ -62,3 +62,26 @@ def test_cast_between_any_addresses(dtype, n, soff, doff):
                                            torch.cuda.current_stream().cuda_stream), "sce_quantize_e4m3")
     assert torch.equal(buf[doff: doff + n], t.div(0.0123).to(torch.float8_e4m3fn).view(torch.uint8))
     assert bool((buf[:doff] == 77).all()) and bool((buf[doff + n:] == 77).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("norm", [None, 1e-6])
+@pytest.mark.parametrize("N,d,V", [(5, 48, 130), (61, 272, 1003), (300, 144, 515)])
+def test_operands_quantised_from_rows_at_any_address(dtype, norm, N, d, V):
+    """The e4m3 operands of a step from aligned rows, from rows of odd length and from an odd base: the same bytes, so the same bits."""
+    from slowrun_amd import cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(N, d, device="cuda", generator=gen).to(dtype)
+    w = (torch.randn(d, V, device="cuda", generator=gen) * d ** -0.5).to(dtype)
+    y = torch.randint(0, V, (N,), device="cuda", generator=gen)
+    res = []
+    for wpad, xpad, off in ((-V % 8, 0, 0), (-V % 8 + 1, 1, 0), (-V % 8 + 8, 8, 1), (-V % 8 + 8, 16, 3)):
+        wb, xb = torch.full((d * (V + wpad) + 8,), 9.0, device="cuda", dtype=dtype), torch.full((N * (d + xpad) + 8,), 9.0, device="cuda", dtype=dtype)
+        wv, xv = wb.as_strided((d, V), (V + wpad, 1), off), xb.as_strided((N, d), (d + xpad, 1), off)
+        wv.copy_(w); xv.copy_(x)
+        out, saved, lse, am, _n = ck.ce_forward(xv, wv, y, 0.02, 0.01, 15.0, "none", want_argmax=True, norm_eps=norm, keep_dlogits=True)
+        dx, dw = ck.ce_backward(saved, y, torch.ones(N, device="cuda"), N, d, V, 0.02, 0.01, 15.0, 1.0, "none", dtype, dtype, keep_dlogits=True,
+                                hidden=xv if norm else None, norm_eps=norm)
+        res.append((out, lse, am, dx, dw))
+    for r in res[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(r, res[0]))
