@@ -8,41 +8,40 @@ namespace sce {
 // ------------------------------------------------------------------------------------------
 // quantisation
 // ------------------------------------------------------------------------------------------
-// 16 consecutive elements starting at p as floats after the scaling; elements at or beyond `valid` are 0.  16-byte loads when the
-// run is complete, in a branch of their own where it is not aligned (one element at a time, the lanes of a wave touch a different
-// cache line each, 16 times over; one branch for both, with the accesses of the unaligned one, was 4 % slower on aligned rows
-// in quantize_w_kernel).  ANY = false, where the branch costs the kernel a wave per SIMD: aligned runs only.
-template <typename T, typename VI, typename VF>
-__device__ __forceinline__ void load16_whole(const T* __restrict__ p, const Scaler scale, float (&v)[16]) {
-  if constexpr (sizeof(T) == 2) {
-    const v4i r0 = *reinterpret_cast<const VI*>(p), r1 = *reinterpret_cast<const VI*>(p + 8);
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      v[2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] << 16));
-      v[2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] & 0xffff0000u));
-      v[8 + 2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] << 16));
-      v[8 + 2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] & 0xffff0000u));
-    }
-  } else {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const v4f r = *reinterpret_cast<const VF*>(p + 4 * q);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) v[4 * q + m] = scale.apply<T>(r[m]);
-    }
-  }
-}
-template <typename T, bool ANY = true>
+// 16 consecutive elements starting at p as floats after the scaling; elements at or beyond `valid` are 0.  One or two 16/32-byte
+// vector loads when the run is complete and 16-byte aligned -- with ANY, aligned or not: for rows of which all or most runs are not
+// (element by element, the lanes of a wave touch a different cache line each, 16 times over).  The kernels choose once, by base
+// and row length: the choice made for each run was 2 to 4 % slower on aligned rows.
+template <typename T, bool ANY>
 __device__ __forceinline__ void load16_scaled(const T* __restrict__ p, int64_t valid, const Scaler scale, float (&v)[16]) {
-  if (valid >= 16 && (((uintptr_t)p) & 15) == 0) {
-    load16_whole<T, v4i, v4f>(p, scale, v);
-  } else if (ANY && valid >= 16) {
-    load16_whole<T, v4i_any, v4f_any>(p, scale, v);
+  using VI = std::conditional_t<ANY, v4i_any, v4i>;
+  using VF = std::conditional_t<ANY, v4f_any, v4f>;
+  if (valid >= 16 && (ANY || (((uintptr_t)p) & 15) == 0)) {
+    if constexpr (sizeof(T) == 2) {
+      const v4i r0 = *reinterpret_cast<const VI*>(p), r1 = *reinterpret_cast<const VI*>(p + 8);
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        v[2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] << 16));
+        v[2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r0[m] & 0xffff0000u));
+        v[8 + 2 * m] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] << 16));
+        v[8 + 2 * m + 1] = scale.apply<T>(__uint_as_float((uint32_t)r1[m] & 0xffff0000u));
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v4f r = *reinterpret_cast<const VF*>(p + 4 * q);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) v[4 * q + m] = scale.apply<T>(r[m]);
+      }
+    }
   } else {
 #pragma unroll
     for (int m = 0; m < 16; ++m) v[m] = (m < valid) ? scale.apply<T>(Elem<T>::load(p + m)) : 0.f;
   }
 }
+// every run of 16 elements that starts at a multiple of 16 in a row is aligned
+template <typename T>
+__device__ __forceinline__ bool rows_aligned(const T* p, int64_t ld) { return (((uintptr_t)p | (uintptr_t)(ld * (int64_t)sizeof(T))) & 15) == 0; }
 
 // dst [rows_p][cols_p] e4m3 = src [rows][cols] / s, zero outside; 16 outputs per thread.  In all the quantising
 // kernels inv_scale is the reciprocal 1 / s taken once on the host, or, with scale_dev, s is read from the device.
@@ -54,17 +53,20 @@ __global__ __launch_bounds__(256) void quantize_pad_kernel(const T* __restrict__
   const Scaler scale = make_scaler<T>(inv_scale, scale_dev);
   const int64_t chunks_per_row = cols_p / 16;
   const int64_t total = rows_p * chunks_per_row;
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = q / chunks_per_row, c0 = (q - r * chunks_per_row) * 16;
-    uint32_t out[4] = {0, 0, 0, 0};
-    if (r < rows && c0 < cols) {
-      float v[16];
-      load16_scaled<T>(src + r * ld + c0, cols - c0, scale, v);
+  auto walk = [&](auto any) {
+    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
+      const int64_t r = q / chunks_per_row, c0 = (q - r * chunks_per_row) * 16;
+      uint32_t out[4] = {0, 0, 0, 0};
+      if (r < rows && c0 < cols) {
+        float v[16];
+        load16_scaled<T, decltype(any)::value>(src + r * ld + c0, cols - c0, scale, v);
 #pragma unroll
-      for (int m = 0; m < 4; ++m) out[m] = cvt4_e4m3(v[4 * m], v[4 * m + 1], v[4 * m + 2], v[4 * m + 3]);
+        for (int m = 0; m < 4; ++m) out[m] = cvt4_e4m3(v[4 * m], v[4 * m + 1], v[4 * m + 2], v[4 * m + 3]);
+      }
+      *reinterpret_cast<v4i*>(dst + r * dst_ld + c0) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
     }
-    *reinterpret_cast<v4i*>(dst + r * dst_ld + c0) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
-  }
+  };
+  if (rows_aligned(src, ld)) walk(std::false_type()); else walk(std::true_type());
 }
 
 __device__ __forceinline__ float wave_sum(float v) {
@@ -230,21 +232,24 @@ __global__ __launch_bounds__(256) void quantize_w_kernel(const T* __restrict__ w
       *reinterpret_cast<uint32_t*>(&tile[r][c]) = out;
     }
   } else {
+    auto fill = [&](auto any) {
 #pragma unroll
-    for (int pass = 0; pass < 4; ++pass) {
-      const int r = (t >> 3) + 32 * pass, c = (t & 7) * 16;
-      const int64_t j = j0 + r, v = v0 + c;
-      uint32_t out[4] = {0, 0, 0, 0};
-      if (j < d && v < V) {
-        float x[16];
-        load16_scaled<T>(w + j * ld + v, V - v, scale, x);
+      for (int pass = 0; pass < 4; ++pass) {
+        const int r = (t >> 3) + 32 * pass, c = (t & 7) * 16;
+        const int64_t j = j0 + r, v = v0 + c;
+        uint32_t out[4] = {0, 0, 0, 0};
+        if (j < d && v < V) {
+          float x[16];
+          load16_scaled<T, decltype(any)::value>(w + j * ld + v, V - v, scale, x);
 #pragma unroll
-        for (int m = 0; m < 4; ++m) out[m] = cvt4_e4m3(x[4 * m], x[4 * m + 1], x[4 * m + 2], x[4 * m + 3]);
+          for (int m = 0; m < 4; ++m) out[m] = cvt4_e4m3(x[4 * m], x[4 * m + 1], x[4 * m + 2], x[4 * m + 3]);
+        }
+        *reinterpret_cast<v4i*>(wq + blocked_offset(j, v, kbv)) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
+#pragma unroll
+        for (int m = 0; m < 4; ++m) *reinterpret_cast<uint32_t*>(&tile[r][c + 4 * m]) = out[m];
       }
-      *reinterpret_cast<v4i*>(wq + blocked_offset(j, v, kbv)) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
-#pragma unroll
-      for (int m = 0; m < 4; ++m) *reinterpret_cast<uint32_t*>(&tile[r][c + 4 * m]) = out[m];
-    }
+    };
+    if (rows_aligned(w, ld)) fill(std::false_type()); else fill(std::true_type());
   }
   __syncthreads();
   if (j0 < dp) {
@@ -363,7 +368,7 @@ __global__ __launch_bounds__(256) void quantize_flat_kernel(const T* __restrict_
   for (size_t q = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * 16; q < n; q += (size_t)gridDim.x * blockDim.x * 16) {
     const int64_t left = (int64_t)(n - q);
     float v[16];
-    load16_scaled<T>(src + q, left, scale, v);
+    load16_scaled<T, true>(src + q, left, scale, v);
     uint32_t w[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) w[m] = cvt4_e4m3(v[4 * m], v[4 * m + 1], v[4 * m + 2], v[4 * m + 3]);
