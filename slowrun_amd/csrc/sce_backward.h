@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
   // blocks beyond the rows' (there are some with few entries only): the entries' places
   if ((int)blockIdx.x >= Np / 256) return rank_targets(rank_keys, blockIdx.x - Np / 256, targets, ignore_index, N, Np, V, key_none, n_predict, skeys, perm);
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i == 0) { longlist[0] = 0; longlist[1] = 0; }        // counters of the long-column lists, filled by column_segments
+  if (i < 3) longlist[i] = 0;         // counters of the long-column lists, filled by column_segments
   float r = 0.f;
   float h[4] = {0.f, 0.f, 0.f, 0.f};
   // the forward call that wrote `saved` was asked for something else (kept dlogits, vocabulary limit, offsets, cap):
@@ -611,9 +611,9 @@ struct FoldParams {
   int slots, first;            // first: the first workgroup of the grid that folds
 };
 __device__ __forceinline__ void fold_chunks(const FoldParams& f, int block, int nblocks) {
-  const int ny = (int)(f.dq / 256), items = f.longlist[1] * ny;
+  const int ny = (int)(f.dq / 256), items = f.longlist[2] * ny;
   for (int item = block; item < items; item += nblocks) {
-    const int v = f.longlist[2 + f.slots + item / ny];
+    const int v = f.longlist[3 + f.slots + item / ny];
     int nch, len;
     long_chunks(f.segoff[v + 1] - f.segoff[v], nch, len);
     float* s = f.longsum + (int64_t)f.longbase[v] * f.dq + (item % ny) * 256 + threadIdx.x;
@@ -780,10 +780,11 @@ __global__ __launch_bounds__(256) void bwd_dw_tail_kernel(DwParams p, DwTail tl)
         *reinterpret_cast<v4f*>(dst0 + (4 * a + b) * 1024 + q * 256) = (v4f){acc[a][b][4 * q], acc[a][b][4 * q + 1], acc[a][b][4 * q + 2], acc[a][b][4 * q + 3]};
 }
 
-// From the sorted keys: segoff[v] = first position whose key is at least v, v = 0 .. V, and the list of the long
-// columns, one entry per chunk (order irrelevant: each is handled on its own): longlist[0] is the count, the column of slot n
-// stands in longlist[2 + n], and longbase[v] is the slot of column v's first chunk sum.  Behind them the columns of several
-// chunks once more, longlist[1] of them.  One column per thread, by bisection: first among every stride-th key (in LDS), then within one
+// From the sorted keys: segoff[v] = first position whose key is at least v, v = 0 .. V, and the long columns (order
+// irrelevant: each is handled on its own).  A long column has a slot for its sum, or one for each of its chunks if it has more
+// than LONG_WAVE rows; longbase[v] is its first.  longlist[0] counts the slots of the former, which are given out from the
+// first on, [1] those of the latter, from the last one down; behind the counters stands the column of every slot, and behind
+// those, longlist[2] of them, the columns of several chunks once more.  One column per thread, by bisection: first among every stride-th key (in LDS), then within one
 // stride.  (A thread per key that fills the gap up to the next key runs as long as the widest gap: with Zipf targets the
 // rare end of the vocabulary holds gaps of thousands of columns, and 2048 rows took 63 us; this takes 4.7.)
 // Also: row and coefficient of every sorted entry (srow, sh), so that the kernels that walk a segment load them side by
@@ -829,12 +830,12 @@ __device__ __forceinline__ void column_segments(SegShared& shared, int block, in
   if (v == V) return;
   const int L = seg[t + 1] - seg[t];
   if (L < long_seg) return;
-  int nch, len;
-  long_chunks(L, nch, len);
-  const int at = atomicAdd(&longlist[0], nch);
+  int nch = 1, len;
+  if (L > LONG_WAVE) long_chunks(L, nch, len);
+  const int at = L > LONG_WAVE ? slots - nch - atomicAdd(&longlist[1], nch) : atomicAdd(&longlist[0], 1);
   longbase[v] = at;
-  for (int c = 0; c < nch; ++c) longlist[2 + at + c] = v;
-  if (nch > 1) longlist[2 + slots + atomicAdd(&longlist[1], 1)] = v;
+  for (int c = 0; c < nch; ++c) longlist[3 + at + c] = v;
+  if (nch > 1) longlist[3 + slots + atomicAdd(&longlist[2], 1)] = v;
 }
 
 // The two in one launch, blocks [0, nxt) the tiles of X~ and the rest the segments: neither needs the other, and on few rows
@@ -857,37 +858,31 @@ __global__ __launch_bounds__(256) void bwd_xt_segments_kernel(XtSegParams p) {
   else column_segments(shared.s, bid - p.nxt, gridDim.x - p.nxt, p.skeys, p.perm, p.hcoef, p.n, p.Np, p.V, p.long_seg, p.slots, p.segoff, p.longlist, p.longbase, p.srow, p.sh);
 }
 
-// One-hot part of dW for the long columns: longsum[slot][:] = sum over the chunk's rows of h_i X_q[i, :].
-// One workgroup per (chunk, block of 256 rows of dW) at a time -- the grid is a fixed one that walks the list, whose
-// length the host does not know; the rows of the chunk are split over 16
-// row-lanes (8 independent loads in flight each) and folded in a fixed order, so the result does
-// not depend on scheduling.
+// One-hot part of dW for the long columns: longsum[slot][:] = sum over the column's (or the chunk's) rows of h_i X_q[i, :], 256 rows
+// of dW at a time (blockIdx.y).  What bounds it is the latency of the gathered rows, of which 16 lanes read 256 bytes: a
+// wave has four rows' worth of lanes and eight loads in flight in each.  A chunk is a workgroup's, folded in LDS in a fixed order; a
+// column of up to LONG_WAVE rows is one wave's, without a barrier (a workgroup each, with most of its lanes idle, took the many
+// columns of 8 to 15 rows of a mid-sized vocabulary 138 us at 50000 rows of three offsets, d = 1024, V = 16384: now 48).  The grid is a
+// fixed one that walks the lists, whose lengths the host does not know.  The result does not depend on scheduling.
 constexpr int LONG_GRID = 1024, FOLD_GRID = 512;
-__global__ __launch_bounds__(256) void bwd_dw_long_kernel(const int32_t* __restrict__ longlist, const int32_t* __restrict__ segoff,
+__global__ __launch_bounds__(256, 5) void bwd_dw_long_kernel(const int32_t* __restrict__ longlist, int slots, const int32_t* __restrict__ segoff,
                                                          const int32_t* __restrict__ srow, const float* __restrict__ sh,
                                                          const uint8_t* __restrict__ xq, int64_t ldx, int64_t dq,
                                                          const int32_t* __restrict__ longbase, float* __restrict__ longsum) {
   __shared__ float red[16][256];
-  const int count = longlist[0];
-  for (int slot = blockIdx.x; slot < count; slot += gridDim.x) {
-    const int v = longlist[2 + slot], ch = slot - longbase[v];
-    int nch, len;
-    const int seg0 = segoff[v], seg1 = segoff[v + 1];
-    long_chunks(seg1 - seg0, nch, len);
-    const int s0 = seg0 + ch * len;
-    const int L = (seg1 - s0) < len ? (seg1 - s0) : len;
-    const int t = threadIdx.x, c = t & 15, rl = t >> 4;
-    const int64_t jb = (int64_t)blockIdx.y * 256;
-    float a[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = t & 15, rl = t >> 4, q = lane >> 4;
+  const int64_t jb = (int64_t)blockIdx.y * 256;
+  const uint8_t* xcol = xq + jb + c * 16;
+  // a[m] = sum over entries first, first + stride, ... of the L from s0 on, in that order, of the lane's 16 rows of dW
+  auto rows = [&](int s0, int L, int first, int stride, float (&a)[16]) {
 #pragma unroll
     for (int m = 0; m < 16; ++m) a[m] = 0.f;
-    const uint8_t* xcol = xq + jb + c * 16;
-    for (int n0 = rl; n0 < L; n0 += 16 * 8) {
+    for (int n0 = first; n0 < L; n0 += stride * 8) {
       v4i raw[8];
       float h[8];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int n = n0 + 16 * u;
+        const int n = n0 + stride * u;
         h[u] = n < L ? sh[s0 + n] : 0.f;
         raw[u] = *reinterpret_cast<const v4i*>(xcol + (int64_t)srow[n < L ? s0 + n : s0] * ldx);
       }
@@ -903,6 +898,16 @@ __global__ __launch_bounds__(256) void bwd_dw_long_kernel(const int32_t* __restr
         }
       }
     }
+  };
+  float a[16];
+  const int nwave = longlist[0], nchunk = longlist[1];
+  for (int i = blockIdx.x; i < nchunk; i += gridDim.x) {
+    const int slot = slots - 1 - i, v = longlist[3 + slot], ch = slot - longbase[v];
+    int nch, len;
+    const int seg0 = segoff[v], seg1 = segoff[v + 1];
+    long_chunks(seg1 - seg0, nch, len);
+    const int s0 = seg0 + ch * len;
+    rows(s0, min(seg1 - s0, len), rl, 16, a);
 #pragma unroll
     for (int m = 0; m < 16; ++m) red[rl][c * 16 + m] = a[m];
     __syncthreads();
@@ -911,6 +916,19 @@ __global__ __launch_bounds__(256) void bwd_dw_long_kernel(const int32_t* __restr
     for (int k = 0; k < 16; ++k) sfold += red[k][t];
     longsum[(int64_t)slot * dq + jb + t] = sfold;
     __syncthreads();                       // `red` is written again for the next chunk
+  }
+  for (int slot = blockIdx.x * 4 + wave; slot < nwave; slot += gridDim.x * 4) {
+    const int v = longlist[3 + slot], s0 = segoff[v];
+    rows(s0, segoff[v + 1] - s0, q, 4, a);
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {         // over the four row lanes, pairwise; all of them get it
+      a[m] += __shfl_xor(a[m], 16);
+      a[m] += __shfl_xor(a[m], 32);
+    }
+    v4f mine;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) mine[m] = q == 0 ? a[m] : q == 1 ? a[4 + m] : q == 2 ? a[8 + m] : a[12 + m];
+    *reinterpret_cast<v4f*>(longsum + (int64_t)slot * dq + jb + c * 16 + q * 4) = mine;
   }
 }
 
@@ -1121,13 +1139,6 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
   }
 }
 
-// s + a b with the product rounded first
-__device__ __forceinline__ float add_product(float s, float a, float b) {
-#pragma clang fp contract(off)
-  const float p = a * b;
-  return s + p;
-}
-
 // The same from fp32 partials: what is left are the tiles of a K-split last round (tl.tile0 >= 0: grid.y = tl.ntail tiles of
 // 16 blocks of 64 x 64 elements), and every tile where dW took more than one launch (grid = blocks of 64 columns x 64
 // rows of dW).  A thread owns one column v and four groups of four rows j: 16 consecutive rows, or, of the pieces of a K-split
@@ -1183,26 +1194,32 @@ __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restri
 #pragma unroll
       for (int m = 0; m < 4; ++m) val[q][m] -= ls[q * step + m] * x_s;
   } else if (L >= LONG_SEG) {
-    // where dW took several launches: the entries' sum first and then x_s, as it comes from the long columns' sums otherwise
-    v4f sum[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) sum[q] = (v4f){0.f, 0.f, 0.f, 0.f};
-    for (int n = 0; n < L; ++n) {
-      const float h = o.sh[s0 + n];
-      const uint8_t* row = o.xq + (int64_t)o.srow[s0 + n] * o.ldx + j0;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t w = *reinterpret_cast<const uint32_t*>(row + q * step);
-        sum[q][0] = add_product(sum[q][0], h, e4m3_to_float<0>(w));
-        sum[q][1] = add_product(sum[q][1], h, e4m3_to_float<1>(w));
-        sum[q][2] = add_product(sum[q][2], h, e4m3_to_float<2>(w));
-        sum[q][3] = add_product(sum[q][3], h, e4m3_to_float<3>(w));
+    // where dW took several launches: the entries' sum first and then x_s, in the order in which a wave of bwd_dw_long_kernel adds
+    // them (four row lanes, then the lanes pairwise)
+#pragma unroll 1
+    for (int q = 0; q < 4; ++q) {
+      v4f sum = (v4f){0.f, 0.f, 0.f, 0.f}, even = sum;
+#pragma unroll 1
+      for (int u = 0; u < 4; ++u) {
+        v4f a = (v4f){0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int n = u; n < L; n += 4) {
+          const float h = o.sh[s0 + n];
+          const uint32_t w = *reinterpret_cast<const uint32_t*>(o.xq + (int64_t)o.srow[s0 + n] * o.ldx + j0 + q * step);
+          a[0] = fmaf(h, e4m3_to_float<0>(w), a[0]);
+          a[1] = fmaf(h, e4m3_to_float<1>(w), a[1]);
+          a[2] = fmaf(h, e4m3_to_float<2>(w), a[2]);
+          a[3] = fmaf(h, e4m3_to_float<3>(w), a[3]);
+        }
+        if (u & 1) { even += a; sum = u == 1 ? even : sum + even; }
+        else even = a;
       }
+#pragma unroll
+      for (int k = 0; k < 4; ++k)                         // (registers are not indexed)
+        if (k == q)
+#pragma unroll
+          for (int m = 0; m < 4; ++m) val[k][m] -= sum[m] * x_s;
     }
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int m = 0; m < 4; ++m) val[q][m] -= sum[q][m] * x_s;
   } else if (L > 0) {
     for (int n = 0; n < L; ++n) {
       const float h = o.sh[s0 + n] * x_s;

@@ -249,7 +249,7 @@ static BwdLayout bwd_layout(const SavedLayout& S, int64_t P, int64_t Pw, int npa
   const size_t dlogits_end = o;
   auto long_columns = [&](int64_t slots) {
     B.long_slots = slots;
-    B.off_longlist = take((size_t)(2 * slots + 2) * 4);      // two counters, a column for every slot, the columns of several slots
+    B.off_longlist = take((size_t)(2 * slots + 2) * 4);      // three counters, a column for every slot, the columns of several slots
     B.off_longsum = take((size_t)slots * S.dq * 4);
   };
   long_columns(NE / LONG_SEG_PARTS + 1);
@@ -770,8 +770,8 @@ extern "C" int sce_backward(const sce_args* a) {
   delete tm_prep;
   {
     KernelTimer tm(SCE_K_DW_FINAL, st);
-    bwd_dw_long_kernel<<<dim3((unsigned)std::min<int64_t>(B.long_slots, LONG_GRID), (unsigned)(S.dq / 256)), 256, 0, st>>>(longlist, segoff, srow, sh, xq, S.ldx,
-                                                                                                                              S.dq, longbase, longsum);
+    bwd_dw_long_kernel<<<dim3((unsigned)std::min<int64_t>(B.long_slots, LONG_GRID), (unsigned)(S.dq / 256)), 256, 0, st>>>(
+        longlist, (int)B.long_slots, segoff, srow, sh, xq, S.ldx, S.dq, longbase, longsum);
   }
   const float sc = (float)a->x_s * (float)a->w_s, k1 = sc * 2.0f * LOG2E / a->cap, c2 = -2.0f * a->cap * LOG2E;
   const int CTv = (int)(S.Vp / 256), CTd = (int)(S.dq / 256);
