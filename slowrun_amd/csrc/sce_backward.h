@@ -862,7 +862,8 @@ __global__ __launch_bounds__(256) void bwd_xt_segments_kernel(XtSegParams p) {
 // of dW at a time (blockIdx.y).  What bounds it is the latency of the gathered rows, of which 16 lanes read 256 bytes: a
 // wave has four rows' worth of lanes and eight loads in flight in each.  A chunk is a workgroup's, folded in LDS in a fixed order; a
 // column of up to LONG_WAVE rows is one wave's, without a barrier (a workgroup each, with most of its lanes idle, took the many
-// columns of 8 to 15 rows of a mid-sized vocabulary 138 us at 50000 rows of three offsets, d = 1024, V = 16384: now 48).  The grid is a
+// columns of 8 to 15 rows of a mid-sized vocabulary 138 us at 50000 rows of three offsets, d = 1024, V = 16384: now 53; LONG_WAVE = 64
+// is faster there and at 48 rows a column, 16 for 22 us, but a wave's second round of loads is 2 us of a small step).  The grid is a
 // fixed one that walks the lists, whose lengths the host does not know.  The result does not depend on scheduling.
 constexpr int LONG_GRID = 1024, FOLD_GRID = 512;
 __global__ __launch_bounds__(256, 5) void bwd_dw_long_kernel(const int32_t* __restrict__ longlist, int slots, const int32_t* __restrict__ segoff,
@@ -917,7 +918,8 @@ __global__ __launch_bounds__(256, 5) void bwd_dw_long_kernel(const int32_t* __re
     longsum[(int64_t)slot * dq + jb + t] = sfold;
     __syncthreads();                       // `red` is written again for the next chunk
   }
-  for (int slot = blockIdx.x * 4 + wave; slot < nwave; slot += gridDim.x * 4) {
+  // (from the other end of the grid: while there are workgroups without a chunk, none has both to do one behind the other)
+  for (int slot = (gridDim.x - 1 - blockIdx.x) * 4 + wave; slot < nwave; slot += gridDim.x * 4) {
     const int v = longlist[3 + slot], s0 = segoff[v];
     rows(s0, segoff[v + 1] - s0, q, 4, a);
 #pragma unroll

@@ -32,7 +32,7 @@ constexpr float LOG2E = 1.4426950408889634f;
 // kernel has LDS for the entries of shorter columns only), 16 where dW takes several launches, for the sake of the
 // workspace (a chunk sum of dq floats for every LONG_SEG entries).
 constexpr int LONG_SEG = 8, LONG_SEG_PARTS = 16;
-constexpr int LONG_WAVE = 64;    // up to so many rows are one wave's work there; more are ...
+constexpr int LONG_WAVE = 32;    // up to so many rows are one wave's work there; more are ...
 constexpr int LONG_CHUNK = 256;  // ... shared out in chunks of at most about this many, a workgroup each
 
 // Lane index within the wavefront, computed from the execution mask each time it is asked for.  Kernels
