@@ -429,7 +429,7 @@ extern "C" int sce_amax_scale(const void* src, int32_t src_dtype, size_t n, floa
   uint32_t* bits = reinterpret_cast<uint32_t*>(scale_out);
   const int esz = src_dtype == SCE_F32 ? 4 : 2;
   int grid = grid_for((n * esz + 15) / 16, 256 * AMAX_LOADS);
-  if (grid > 8 * MAX_CUS) grid = 8 * MAX_CUS;          // as many workgroups as run at one time
+  if (grid > AMAX_GRID) grid = AMAX_GRID;
   amax_begin_kernel<<<1, 1, 0, st>>>(bits);
   if (src_dtype == SCE_F32) amax_kernel<float><<<grid, 256, 0, st>>>((const float*)src, n, bits);
   else amax_kernel<bf16_t><<<grid, 256, 0, st>>>((const bf16_t*)src, n, bits);
