@@ -34,37 +34,32 @@ namespace sce {
 //     b2 on, or earlier behind an extra barrier `b1_after` that tells that every wave has its last fragments of this
 //     block; ldL = the rest of the next block's loads.  The wait that publishes a block comes at b2 of the block before.
 // The four waves of a workgroup run in step and share the compute unit's one path from L2 (64 bytes a clock: 16 clocks
-// for a wave's 1 KB load), so one load per wave and 64-clock MFMA slot already fills that path while it lasts.  Measured
-// at N = 65536, d = 2560, V = 50304, all three big kernels alike: two loads to a slot -- all 16 early, behind the publishing
-// barrier, or all late -- 5 to 10 % slower than schedule 0; reads spread one to a slot (1), loads spread over 22 slots behind
-// an extra barrier (2), and mixtures of the two: within 0.5 % of schedule 0.  At the clock this part grants under fp8 MFMA
-// load the loop is bound neither by where its LDS reads sit nor by the lead its loads have.
-#ifndef SCE_SCHED
-#define SCE_SCHED 0
-#endif
+// for a wave's 1 KB load), so one load per wave and 64-clock MFMA slot already fills that path while it lasts.  What
+// costs is a slot that has both a load and fragment reads: both end in LDS, and the reads of the four waves (8 KB a slot)
+// then wait for the loads' 4 KB.  So a block's slots are four groups of eight: loads, reads, loads, reads.  The loads of the
+// third group go into this block's own LDS slot, behind an extra barrier that waits for the second group's reads; that
+// barrier comes a slot after the last of them, when they have landed, which leaves one load for the fourth group.
+// Measured against the schedule before it (reads in the second half of each sub-step too, but eight of the loads in the
+// slots with reads, no extra barrier), two builds in turn on one card, whole steps: 2048 rows of d = 768 476 -> 466 us, two
+// micro-batches of 2048 rows of d = 1024 974 -> 952, 4096 rows of d = 1600 1194 -> 1154, 32768 rows of d = 1024 4824 -> 4673,
+// 65536 rows of d = 2560 19370 -> 19170, the bf16 eval pass the same.  Also measured: six or more loads in slots with reads
+// (1 % slower than this), all loads as early as their LDS slot is free (2 %), one barrier and a load and a read in every slot
+// of the second half (2 to 4 %), the extra barrier right behind the last read (0 to 0.5 %), reads three to a slot (0.5 %), two loads
+// of a wave in one slot (5 to 10 %).
 struct KSched {
   signed char ldL[32], ldEM[32], r1[32], c0[32], n0[32];
   int b1_after, b2;
 };
-constexpr KSched KSCHEDS[] = {
-    // 0: fragment reads two to a slot in the second half of each sub-step, loads behind the barrier in the middle of the second
-    {{1, 1, 1, 1, 1, 1, 1, 1}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 1, 1},
-     {0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 2, 2, 2, 2, 2, 2}, {0}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 2, 2, 2, 2, 2, 2}, -1, 24},
-    // 1: one read unit to a slot almost everywhere, barrier at slot 22, loads 22..31 and 0..5
-    {{1, 1, 1, 1, 1, 1}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1},
-     {0, 0, 0, 0, 0, 0, 2, 2, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, {1, 1, 1, 1, 1, 1},
-     {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1}, -1, 22},
-    // 2: the reads of 0; an extra barrier after slot 17 lets six loads go out in slots 18..23, the slots with reads take a load every other time
-    {{1, 1, 0, 1, 1, 0, 1, 1}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 1, 0, 1, 0, 1, 0, 1, 0},
-     {0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 2, 2, 2, 2, 2, 2}, {0}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 2, 2, 2, 2, 2, 2}, 17, 24},
-};
-constexpr KSched KS = KSCHEDS[SCE_SCHED];
+constexpr KSched KS = {{1, 1, 1, 1, 1, 1, 1, 1}, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 1, 1, 1, 1, 1, 1, 1, 0, 0, 0, 1, 0, 0, 0, 0},
+                       {0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 2, 2, 2, 2, 2, 2}, {0},
+                       {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 2, 2, 2, 2, 2, 2, 2, 2}, 16, 24};
 constexpr int ksum(const signed char (&a)[32], int n) { int t = 0; for (int i = 0; i < n; ++i) t += a[i]; return t; }
 constexpr int LOADS_E = ksum(KS.ldEM, KS.b2), LOADS_EM = ksum(KS.ldEM, 32), UNITS_N0 = ksum(KS.n0, 32);
 static_assert(LOADS_EM + ksum(KS.ldL, 32) == 16, "a K block is 16 loads per wave");
 static_assert(ksum(KS.r1, 32) == 16 && UNITS_N0 + ksum(KS.c0, 32) == 16, "a sub-step is 16 read units");
 static_assert(ksum(KS.n0, KS.b2) == 0, "the next block cannot be read before the barrier that publishes it");
 static_assert(LOADS_E == 0 || (KS.b1_after >= 0 && ksum(KS.ldEM, KS.b1_after + 1) == 0), "loads before b2 need the extra barrier");
+static_assert(KS.b1_after < 0 || ksum(KS.r1, KS.b1_after + 1) == 16, "the extra barrier frees the block's LDS slot: all its reads are before it");
 constexpr int AHEAD_LOADS = LOADS_EM;      // loads of K block 1 that a prefetch (or the prologue) puts in flight
 constexpr int UNIT_FRAG[8] = {0, 4, 5, 6, 7, 1, 2, 3};      // fragment (0-3: A, 4-7: B) of the q-th pair of read units
 
