@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
                                                       int64_t ignore_index, const int32_t* __restrict__ hdr,
                                                       const float* __restrict__ grad_output, int per_row, float grad_scale,
                                                       const float* __restrict__ mtp_weights, int n_predict,
-                                                      float cap, int N, int Np, int V, const float* __restrict__ lam,
+                                                      float cap, int N, int Np, int V, const float* __restrict__ lam, const float* __restrict__ lam2,
                                                       float* __restrict__ rho, float* __restrict__ hcoef,
                                                       float* __restrict__ blockmax, int32_t* __restrict__ rowinfo, CallMode mode,
                                                       int32_t key_none, int32_t* __restrict__ keys, int32_t* __restrict__ vals,
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(256) void bwd_prep_kernel(const float* __restrict__
   // the boost is what makes the stored value the probability itself, D 2^lam = p (1 - t^2): rows
   // that share a block are then weighed by what their entries contribute, whatever the shapes of their distributions.
   float lam_i = 0.f;
-  if (i < N) lam_i = rowinfo ? (cap - s_lse[i]) * LOG2E : lam[i];
+  if (i < N) lam_i = rowinfo ? (cap - s_lse[i]) * LOG2E : row_boost(lam, lam2, i);
   if (!(lam_i >= -64.f && lam_i <= 120.f)) lam_i = 0.f;      // (ignored rows have no lse to speak of)
   if (rowinfo && i < Np) {          // what the recompute kernel wants to know of a row: its boost and its target columns
     rowinfo[i] = __float_as_int(lam_i);

@@ -56,7 +56,7 @@ static inline int64_t row_stride(int64_t k) { return k + 128; }
 struct SavedLayout {
   int64_t ldx;                       // row stride in bytes of the [..][dp] e4m3 arrays
   int64_t N, d, V, Np, dp, dq, Vp;   // all padded sizes are multiples of 256 (every K loop runs over an even number of 128-byte blocks); dp: row bytes of X_q / W_q^T (= dq for e4m3)
-  size_t off_hdr, off_xq, off_lse, off_zy, off_rstd, off_lam, x_total;
+  size_t off_hdr, off_xq, off_lse, off_zy, off_rstd, off_lam, off_lam2, x_total;
   size_t rel_wqt, rel_wq, w_total;   // relative to the start of the W region
   size_t total;                      // x_total + w_total
   size_t rel_g, rel_gexp, g_total;   // dlogits emitted by the forward pass (optional; behind whatever else `saved` holds)
@@ -74,10 +74,10 @@ static inline SavedLayout saved_layout(int64_t N, int64_t d, int64_t V, int n_pr
   L.off_hdr = take(256);
   L.off_xq = take((size_t)L.Np * L.ldx);       // X_q   [Np][dp]  e4m3, zero padded, row stride ldx
   L.off_lse = take((size_t)L.Np * 4);
-  (void)take((size_t)L.Np * 4);                // not used: the offsets behind it stay where they have been
+  L.off_lam2 = take((size_t)L.Np * 4);         // the second of a row's two numbers (off_lam)
   L.off_zy = take((size_t)L.Np * 4 * n_predict);
   L.off_rstd = take((size_t)L.Np * 4);         // 1 / rms of each row when the final norm is part of the call
-  L.off_lam = take((size_t)L.Np * 4);          // per-row exponent boost of the dlogits (an integer in a float)
+  L.off_lam = take((size_t)L.Np * 4);          // per-row exponent boost of the dlogits: the smaller of two integers in floats (row_boost)
   L.x_total = o;
   o = 0;
   L.rel_wqt = take((size_t)L.Vp * L.ldx);      // W_q^T [Vp][dp], row stride ldx

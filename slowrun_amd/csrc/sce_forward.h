@@ -16,7 +16,7 @@ struct FwdParams {
   float* s_uy;             // [n_predict][Np]: raw logit u at the target of (offset, row): from fwd_sample_kernel (PRE), else written by the workgroup that meets it
   uint8_t* ghat_t;         // EMIT: G, all Np rows, tile by tile (kbv blocks of 128 columns per tile of 256 rows)
   uint32_t* gexp;          // EMIT: its block exponents [Vp / 128][kbw]
-  const float* lam;        // EMIT: exponent boost of every row
+  float *lam, *lam2;       // EMIT: the two numbers of every row's exponent boost (row_boost), from the sample kernels
   int64_t ignore_index;
   int64_t dp, ldx;         // K extent and row stride of xq / wqt
   int64_t kbw, kbv;        // blocks of 128 rows (the exponents' row stride) and of 128 columns
@@ -146,6 +146,12 @@ __device__ __forceinline__ void take_target_logits(v16f (&acc)[4][4], const int*
   }
 }
 
+// A row's boost from the two numbers that were left for it (see sample_rows; fwd_sample_kernel leaves its one number twice).
+__device__ __forceinline__ float row_boost(const float* __restrict__ lam, const float* __restrict__ lam2, int64_t i) {
+  const float l = fminf(lam[i], lam2[i]);
+  return l > -64.f ? (l < 120.f ? l : 120.f) : -64.f;            // (NaN: -64)
+}
+
 // The exponent boost of every row: lam_i = floor(-log2 Z^_i), Z^_i an estimate of the row's softmax sum Z_i = sum_v e^{z_iv - cap}
 // made before the forward kernel starts, so that the stored value D 2^lam is close to the row's probabilities
 // (times 1 - t^2) whatever the level of its logits.  Two tiles of logits go into it (one workgroup per row tile):
@@ -171,7 +177,7 @@ constexpr int SMEM_SAMPLE = SMEM_BYTES + 2 * 256 * 4 + 8 * 256 * 4;      // the 
 // BOOST = false (with GATHER): the target logits only, for a forward pass that emits nothing (the first tile is then
 // computed only for the sake of its last columns, i.e. with more than one offset).
 template <bool GATHER, bool BOOST = true>
-__global__ __launch_bounds__(256) void fwd_sample_kernel(FwdParams p_in, int ct, float* __restrict__ lam_out) {
+__global__ __launch_bounds__(256) void fwd_sample_kernel(FwdParams p_in, int ct) {
   static_assert(GATHER || BOOST, "nothing to do");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   FwdParams p = p_in;
@@ -296,33 +302,188 @@ __global__ __launch_bounds__(256) void fwd_sample_kernel(FwdParams p_in, int ct,
       const float peak = fast_exp2(fast_rcp(fmaf(fast_exp2(u * p.k1), p.ic2, p.ic2)));       // (u = -inf: e^{-2 cap})
       float l = floorf(-log2f(fmaxf((float)p.V * m, peak)));
       l = l > -64.f ? (l < 120.f ? l : 120.f) : -64.f;
-      lam_out[rt * 256 + wb * 128 + b * 32 + lane] = dead[wb * 128 + b * 32 + lane] ? -64.f : (l == l ? l : 0.f);
+      l = dead[wb * 128 + b * 32 + lane] ? -64.f : (l == l ? l : 0.f);
+      const int i = rt * 256 + wb * 128 + b * 32 + lane;
+      p.lam[i] = l; p.lam2[i] = l;
     }
   }
 }
 
-// The same numbers, bit for bit, for a forward pass of few rows, where one workgroup to a row tile leaves most of the chip idle and
-// walks two K loops one behind the other at the latency of memory.  Here a workgroup has 32 rows, and each
-// of its eight waves two blocks of 32 columns (waves 0 - 3 of the sampled tile, 4 - 7 of the targets'): fragments straight
-// from memory to registers, four steps ahead.  A fragment holds the same bytes in the same registers and an accumulator
-// block adds up in the same order as in mfma_mainloop.  The price is that every 32 rows read all 512 rows of W_q^T again, from L2,
-// in pieces of 16 bytes, so it is used up to SAMPLE_FEW_TILES row tiles (one workgroup to a CU).  Measured, V = 50304, against
-// fwd_sample_kernel: d = 1024 25.6 us for 39.4 (2048 rows), 28.5 for 46.7 (8192), but 55.4 for 51.5 (16384); d = 2560 55.8 for 61.5,
-// 61.2 for 82.9, and 121 for 92; d = 256, V = 4096, 1000 rows 11 for 28.5; without the boosts, 8192 rows of d = 2560, 18 for 41.
-// BOOST = false: only the band of the target logits is computed: wave 0 the blocks on the diagonal and right of it, wave 1
-// (a second wave only if there are several offsets) the last block of the first tile for the last rows of a row tile.
-constexpr int SAMPLE_FEW_ROWS = 32, SAMPLE_FEW_TILES = 32;
+// The same numbers, bit for bit, with 32 RB rows and one of the two tiles to a workgroup instead of 256 rows and both: there
+// are 16 / RB workgroups to a row tile, and the two K loops do not run one behind the other.  The eight waves of a workgroup take 32 of
+// the tile's 256 columns each.  A 128-byte K block of the 256 rows of W_q^T and of the workgroup's own rows comes by direct loads,
+// whole 128-byte pieces of rows, into a ring of STAGES LDS slots, STAGES - 1 blocks ahead; the swizzle, the bytes of a fragment
+// and the order in which an accumulator block adds up are those of mfma_mainloop.  What bounds it is the path from L2 (32 + 4 RB KB a K
+// block, 64 bytes a clock).  Before, each lane fetched its own 32 bytes of a row straight into registers, 64 pieces of 16
+// bytes of 32 rows to an instruction, and the address unit took a clock for each.  Measured, V = 50304 unless said, that kernel or
+// (over 8192 rows) fwd_sample_kernel against this: 1000 rows, d = 256, V = 4096 10.8 -> 5.7 us; 2048 rows, d = 768 21 -> 8.4, d = 1024
+// 26 -> 9.9; 4096, d = 1600 45 -> 15; 8192, d = 1024 28 -> 13.7, d = 2560 61 -> 23; 16384, d = 1024 47 -> 18, d = 4096 and V = 131072 108 -> 45;
+// 30011, d = 2560 85 -> 61; 32768, d = 1024 50 -> 35; 65536, d = 1024 58 for its 73, d = 2560 106 for 121.  So up to SAMPLE_RING_TILES row
+// tiles, two rounds of workgroups with RB = 4 (three take as long as fwd_sample_kernel).  RB: the least with which one round of
+// workgroups, one to a CU, is enough (8192 rows, d = 1024: 20, 13.7 and 18 us with 1, 2 and 4; 2048 rows: 9.9, 11.3, 14.9).
+// What the two tiles say of a row stays apart -- lam[i] from the first, lam2[i] from the second, floor(-log2 of its
+// estimate) each -- and row_boost takes the smaller: the floor of the larger estimate's.
+constexpr int SAMPLE_THREADS = 512, SAMPLE_RING_TILES = 128;
+static inline int sample_row_blocks(int RT) { return RT <= 16 ? 1 : RT <= 32 ? 2 : 4; }
+template <int RB>
+struct SampleRing {
+  static constexpr int X_BYTES = 32 * RB * BK, STAGE = 256 * BK + X_BYTES, STAGES = RB == 4 ? 3 : 4;
+  static constexpr int XL = RB == 4 ? 2 : 1, LOADS = 4 + XL;      // direct loads of a wave per K block (RB = 1: the second four waves load x again)
+  static constexpr int SMEM = STAGES * STAGE;
+  static_assert(SMEM <= SMEM_MAX && 2 * 8 * 32 * RB * 4 <= SMEM, "LDS: the ring, and after it the results of the waves");
+};
+template <int RB>
+__device__ __forceinline__ void sample_rows(const FwdParams& p, int ct, uint8_t* smem) {
+  using R = SampleRing<RB>;
+  constexpr int GROUPS = 8 / RB;                                 // workgroups to the 256 rows of a tile
+  // neighbours in this order run on one XCD: those of a row tile, whose gathered rows of W_q^T are the same
+  const int total = p.RT * 2 * GROUPS, per = (total + 7) >> 3, idx = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || idx >= total) return;
+  const int rt = idx / (2 * GROUPS), rest = idx - rt * (2 * GROUPS);
+  const bool second = rest >= GROUPS;                            // this workgroup's columns are the targets
+  const int r0 = (second ? rest - GROUPS : rest) * 32 * RB;      // its first row in the row tile
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), h = lane >> 5;
+  const int ntail = p.n_predict - 1;
+  auto target_of = [&](int row) { return row < p.N ? p.targets[row] : p.ignore_index; };
+  auto column_of = [&](int64_t y) { return (y != p.ignore_index && y >= 0 && y < p.V) ? (int)y : 0; };
+  auto row_of_w = [&](int j) {                                   // the row of W^T that column j of the tile is
+    const int q = j - (256 - ntail);
+    if (second) return column_of(target_of(rt * 256 + j));
+    return q < 0 ? ct * 256 + j : column_of(target_of(rt * 256 + 256 + q));
+  };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)smem);
+  // one load: 8 rows of 128 bytes; a wave loads the W rows of its own 32 columns
+  const int lr = lane >> 3, pc = lane & 7;
+  auto swizzled = [&](int row) { return (uint32_t)((pc ^ ((row & 7) ^ ((row >> 3) & 1))) * 16); };
+  auto xload = [&](int n) { return RB == 1 ? wave & 3 : wave * R::XL + n; };
+  uint32_t wo[4], xo[R::XL];
+#pragma unroll
+  for (int n = 0; n < 4; ++n) wo[n] = (uint32_t)(row_of_w(wave * 32 + n * 8 + lr) * p.ldx) + swizzled(n * 8 + lr);
+#pragma unroll
+  for (int n = 0; n < R::XL; ++n) { const int row = xload(n) * 8 + lr; xo[n] = (uint32_t)(row * p.ldx) + swizzled(row); }
+  const uint8_t* xbase = uniform_ptr(p.xq + (int64_t)(rt * 256 + r0) * p.ldx);
+  const int nk = (int)(p.dp / BK);
+  int ik = 0, islot = 0;                                         // the K block that is loaded next
+  auto issue = [&]() {
+    const uint32_t l = lds0 + islot * R::STAGE;
+    const uint8_t* wb = p.wqt + (int64_t)ik * BK;
+    const uint8_t* xb = xbase + (int64_t)ik * BK;
+    lds_direct_16<0>(l + wave * 4096, wo[0], wb);
+    lds_direct_16<1024>(l + wave * 4096, wo[1], wb);
+    lds_direct_16<2048>(l + wave * 4096, wo[2], wb);
+    lds_direct_16<3072>(l + wave * 4096, wo[3], wb);
+#pragma unroll
+    for (int n = 0; n < R::XL; ++n) lds_direct_16<256 * BK>(l + xload(n) * 1024, xo[n], xb);
+    ++ik;
+    if (++islot == R::STAGES) islot = 0;
+  };
+#pragma unroll 1
+  for (int g = 0; g < R::STAGES - 1 && g < nk; ++g) issue();
+  v16f acc[RB];
+#pragma unroll
+  for (int q = 0; q < RB; ++q)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
+  const int fr = lane & 31, fsw = (fr & 7) ^ ((fr >> 3) & 1);
+  int slot = 0;
+#pragma unroll 1
+  for (int k = 0; k < nk; ++k) {
+    // this wave's loads of the block have landed and its reads of the one before are complete; after the barrier that holds for
+    // every wave, and the slot of the block before is free
+    if (k + R::STAGES - 1 <= nk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((R::STAGES - 2) * R::LOADS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (k + R::STAGES - 1 < nk) issue();
+    const uint8_t* ws = smem + slot * R::STAGE;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      const int c0 = ((4 * half + 2 * h) ^ fsw) * 16;
+      auto fragment = [&](const uint8_t* rows) {
+        const v4i lo = *reinterpret_cast<const v4i*>(rows + fr * BK + c0), hi = *reinterpret_cast<const v4i*>(rows + fr * BK + (c0 ^ 16));
+        return (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      };
+      const v8i fw = fragment(ws + wave * 4096);
+      v8i fx[RB];
+#pragma unroll
+      for (int q = 0; q < RB; ++q) fx[q] = fragment(ws + 256 * BK + q * 4096);
+#pragma unroll
+      for (int q = 0; q < RB; ++q) acc[q] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fw, fx[q], acc[q], 0, 0, 0, 0, 0, 0);
+    }
+    if (++slot == R::STAGES) slot = 0;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // the ring is free for the waves' results
+  float* gmins = reinterpret_cast<float*>(smem);                 // [8 waves][32 RB]
+  float* tops = gmins + 8 * 32 * RB;
+  // element (row i, column j) of the tile is in register r: j = 32 wave + 8 (r / 4) + 4 h + r % 4
+  const int vlim = second ? 256 : min(p.V - ct * 256, 256 - ntail);
+#pragma unroll
+  for (int q = 0; q < RB; ++q) {
+    const int rb = r0 / 32 + q, i = rb * 32 + (lane & 31);       // block of 32 rows, the lane's row in the row tile
+    if (second) {
+      if (wave == rb || wave == rb + 1)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int k = 32 * wave + 8 * (r >> 2) + 4 * h + (r & 3) - i;
+          if (k >= 0 && k < p.n_predict) p.s_uy[(int64_t)k * p.Np + rt * 256 + i] = acc[q][r] * p.sc;
+        }
+    } else if (rb == 7 && wave == 7) {                           // the next row tile's targets: columns 256 - ntail on of the first tile
+#pragma unroll
+      for (int r = 12; r < 16; ++r) {
+        const int j = 252 + (r & 3), k = 256 + (j - (256 - ntail)) - i;
+        if (h == 1 && j >= 256 - ntail && k >= 1 && k < p.n_predict) p.s_uy[(int64_t)k * p.Np + rt * 256 + i] = acc[q][r] * p.sc;
+      }
+    }
+    float gmin = INFINITY, top = -INFINITY, sum = 0.f, cnt = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const bool live = 32 * wave + 8 * (r >> 2) + 4 * h + (r & 3) < vlim;
+      if (!second) {
+        const float pt = fast_exp2(fast_rcp(fmaf(fast_exp2(acc[q][r] * p.k1), p.ic2, p.ic2)));
+        sum += live ? pt : 0.f;
+        cnt += live ? 1.f : 0.f;
+      }
+      top = live ? fmaxf(top, acc[q][r]) : top;
+    }
+    if (cnt > 0.f) gmin = sum / cnt;
+    gmin = fminf(gmin, __shfl_xor(gmin, 32));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    if (h == 0) { gmins[(wave * RB + q) * 32 + lane] = gmin; tops[(wave * RB + q) * 32 + lane] = top; }
+  }
+  __syncthreads();
+  const int t = threadIdx.x;
+  if (t >= 32 * RB) return;
+  float gmin = INFINITY, top = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) { gmin = fminf(gmin, gmins[w * 32 * RB + t]); top = fmaxf(top, tops[w * 32 * RB + t]); }
+  const float peak = fast_exp2(fast_rcp(fmaf(fast_exp2(top * p.k1), p.ic2, p.ic2)));
+  const int row = rt * 256 + r0 + t;
+  float l = floorf(-log2f(second ? peak : fmaxf((float)p.V * gmin, peak)));
+  bool dead = true;
+  for (int k = 0; k < p.n_predict; ++k) dead = dead && !(row < p.N && target_valid(p.targets, p.ignore_index, row + k, p.N, p.V));
+  (second ? p.lam2 : p.lam)[row] = dead ? -64.f : l;
+}
+
+// BOOST = false: the target logits only, for a forward pass that emits nothing: 32 rows to a workgroup, fragments
+// straight from memory to registers, four steps ahead; wave 0 computes the blocks on the diagonal and right of it, wave 1
+// (a second wave only if there are several offsets) the last block of the first tile for the last rows of a row tile.  8192 rows of d = 2560
+// 18 us for the 41 of fwd_sample_kernel; used up to SAMPLE_FEW_TILES row tiles.
+constexpr int SAMPLE_FEW_TILES = 32;
 template <bool BOOST>
-__global__ __launch_bounds__(512) void fwd_sample_few_kernel(FwdParams p_in, int ct, float* __restrict__ lam_out) {
-  __shared__ float gmins[4][SAMPLE_FEW_ROWS], tops[8][SAMPLE_FEW_ROWS];
+__global__ __launch_bounds__(SAMPLE_THREADS) void fwd_sample_few_kernel(FwdParams p_in, int ct, int row_blocks) {
   FwdParams p = p_in;
   if (p.dc) { p.sc = p.dc->sc; p.k1 = p.dc->k1; }
+  if constexpr (BOOST) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    if (row_blocks == 1) sample_rows<1>(p, ct, smem);
+    else if (row_blocks == 2) sample_rows<2>(p, ct, smem);
+    else sample_rows<4>(p, ct, smem);
+    return;
+  }
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), h = lane >> 5;
   const int rt = blockIdx.x >> 3, rb = blockIdx.x & 7;          // row tile, block of 32 rows in it
   const int ntail = p.n_predict - 1;
-  const bool second = BOOST ? wave >= 4 : wave == 0;            // this wave's columns are the targets
-  const int ab[2] = {BOOST ? 2 * (wave & 3) : second ? rb : 6, BOOST ? 2 * (wave & 3) + 1 : second ? min(rb + 1, 7) : 7};
-  if (!BOOST && !second && rb != 7) return;
+  const bool second = wave == 0;                                // this wave's columns are the targets
+  const int ab[2] = {second ? rb : 6, second ? min(rb + 1, 7) : 7};
+  if (!second && rb != 7) return;
   auto target_of = [&](int row) { return row < p.N ? p.targets[row] : p.ignore_index; };
   auto column_of = [&](int64_t y) { return (y != p.ignore_index && y >= 0 && y < p.V) ? (int)y : 0; };
   auto row_of_w = [&](int j) {                                   // the row of W^T that column j of the wave's tile is
@@ -334,9 +495,6 @@ __global__ __launch_bounds__(512) void fwd_sample_few_kernel(FwdParams p_in, int
   const uint8_t* xr = p.xq + (int64_t)(rt * 256 + i) * p.ldx + 32 * h;
   const uint8_t* wr0 = p.wqt + (int64_t)row_of_w(ab[0] * 32 + (lane & 31)) * p.ldx + 32 * h;
   const uint8_t* wr1 = p.wqt + (int64_t)row_of_w(ab[1] * 32 + (lane & 31)) * p.ldx + 32 * h;
-  bool dead = true;
-  if (BOOST && wave == 0)
-    for (int k = 0; k < p.n_predict; ++k) dead = dead && !(rt * 256 + i < p.N && target_valid(p.targets, p.ignore_index, rt * 256 + i + k, p.N, p.V));
   typedef int v8i_16 __attribute__((ext_vector_type(8), aligned(16)));
   constexpr int AHEAD = 4;                                       // steps of 64 bytes; the K extent is a multiple of 256
   v8i fx[AHEAD], fw[AHEAD][2];
@@ -375,37 +533,6 @@ __global__ __launch_bounds__(512) void fwd_sample_few_kernel(FwdParams p_in, int
       const int j = 252 + (r & 3), k = 256 + (j - (256 - ntail)) - i;
       if (h == 1 && j >= 256 - ntail && k >= 1 && k < p.n_predict) p.s_uy[(int64_t)k * p.Np + rt * 256 + i] = acc[1][r] * p.sc;
     }
-  }
-  if (!BOOST) return;
-  const int vlim = second ? 256 : min(p.V - ct * 256, 256 - ntail);
-  float gmin = INFINITY, top = -INFINITY;
-#pragma unroll
-  for (int a = 0; a < 2; ++a) {
-    float sum = 0.f, cnt = 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const float pt = fast_exp2(fast_rcp(fmaf(fast_exp2(acc[a][r] * p.k1), p.ic2, p.ic2)));
-      const bool live = 32 * ab[a] + 8 * (r >> 2) + 4 * h + (r & 3) < vlim;
-      sum += live ? pt : 0.f;
-      cnt += live ? 1.f : 0.f;
-      top = live ? fmaxf(top, acc[a][r]) : top;
-    }
-    if (cnt > 0.f) gmin = fminf(gmin, sum / cnt);
-  }
-  gmin = fminf(gmin, __shfl_xor(gmin, 32));
-  top = fmaxf(top, __shfl_xor(top, 32));
-  if (h == 0) {
-    if (!second) gmins[wave][lane] = gmin;
-    tops[wave][lane] = top;
-  }
-  __syncthreads();
-  if (wave == 0 && h == 0) {
-    for (int w = 1; w < 4; ++w) gmin = fminf(gmin, gmins[w][lane]);
-    for (int w = 1; w < 8; ++w) top = fmaxf(top, tops[w][lane]);
-    const float peak = fast_exp2(fast_rcp(fmaf(fast_exp2(top * p.k1), p.ic2, p.ic2)));
-    float l = floorf(-log2f(fmaxf((float)p.V * gmin, peak)));
-    l = l > -64.f ? (l < 120.f ? l : 120.f) : -64.f;
-    lam_out[rt * 256 + i] = dead ? -64.f : (l == l ? l : 0.f);
   }
 }
 
@@ -457,7 +584,7 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
       stat[(0 + b) * NTHREADS] = 0.f;
       stat[(4 + b) * NTHREADS] = -INFINITY;
       stat[(8 + b) * NTHREADS] = __int_as_float(0x7fffffff);
-      if (EMIT) stat[(12 + b) * NTHREADS] = p.lam[rt * 256 + wb * 128 + b * 32 + (lane_id() & 31)];
+      if (EMIT) stat[(12 + b) * NTHREADS] = row_boost(p.lam, p.lam2, rt * 256 + wb * 128 + b * 32 + (lane_id() & 31));
     }
     int* tgt = reinterpret_cast<int*>(smem + FWD_TGT_OFF);
     for (int e = threadIdx.x; e < p.n_predict * 256; e += NTHREADS) {

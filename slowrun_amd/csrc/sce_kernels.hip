@@ -147,6 +147,7 @@ static int check_device(int dev) {
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_sample_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_SAMPLE));
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_sample_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_SAMPLE));
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_sample_kernel<true, false>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_SAMPLE));
+      HIP_TRY(hipFuncSetAttribute((const void*)fwd_sample_few_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_kernel<false, false, true>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_FWD));
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_few_rows_kernel<2>, hipFuncAttributeMaxDynamicSharedMemorySize, FewRows<2>::SMEM));
       HIP_TRY(hipFuncSetAttribute((const void*)fwd_few_rows_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, FewRows<4>::SMEM));
@@ -584,15 +585,16 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
     // the exponent boosts of the rows, estimated from two tiles of their logits: only for a forward pass
     // that emits the dlogits (a backward pass that forms them again knows the rows' sums and takes the boosts from those)
     KernelTimer tm(SCE_K_QUANT, st);
-    float* lam = (float*)(sv + S.off_lam);
-    p.lam = lam;
+    p.lam = (float*)(sv + S.off_lam); p.lam2 = (float*)(sv + S.off_lam2);
     const bool few = pre && RT <= SAMPLE_FEW_TILES;
-    if (few && emit) fwd_sample_few_kernel<true><<<8 * RT, 512, 0, st>>>(p, CT / 2, lam);
-    else if (few) fwd_sample_few_kernel<false><<<8 * RT, a->shape.n_predict > 1 ? 128 : 64, 0, st>>>(p, CT / 2, lam);
+    if (pre && emit && RT <= SAMPLE_RING_TILES) {
+      const int rb = sample_row_blocks(RT), smem = rb == 1 ? SampleRing<1>::SMEM : rb == 2 ? SampleRing<2>::SMEM : SampleRing<4>::SMEM;
+      fwd_sample_few_kernel<true><<<(RT * 16 / rb + 7) / 8 * 8, SAMPLE_THREADS, smem, st>>>(p, CT / 2, rb);
+    } else if (few && !emit) fwd_sample_few_kernel<false><<<8 * RT, a->shape.n_predict > 1 ? 128 : 64, 0, st>>>(p, CT / 2, 1);
     else if (!bf16ops && emit) {
-      if (pre) fwd_sample_kernel<true><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2, lam);
-      else fwd_sample_kernel<false><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2, lam);
-    } else if (pre) fwd_sample_kernel<true, false><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2, lam);
+      if (pre) fwd_sample_kernel<true><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2);
+      else fwd_sample_kernel<false><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2);
+    } else if (pre) fwd_sample_kernel<true, false><<<RT, NTHREADS, SMEM_SAMPLE, st>>>(p, CT / 2);
   }
   {
     KernelTimer tm(SCE_K_FWD, st);
@@ -749,7 +751,7 @@ extern "C" int sce_backward(const sce_args* a) {
   const bool ranked = NE <= RANK_MAX;
   bwd_prep_kernel<<<nblk + (ranked ? (int)((NE + RANK_PER_BLOCK - 1) / RANK_PER_BLOCK) : 0), 256, 0, st>>>(
       s_lse, s_zy, a->targets, a->ignore_index, hdr, a->grad_output, a->reduction == SCE_REDUCE_NONE ? 1 : 0, a->grad_scale, a->mtp_weights, K, a->cap, (int)N,
-      (int)S.Np, (int)Vl, (const float*)(sv + S.off_lam), rho, hcoef, blockmax, kept ? nullptr : rowinfo, call_mode(kept, (int)Vl, K, a->cap), (int32_t)V,
+      (int)S.Np, (int)Vl, (const float*)(sv + S.off_lam), (const float*)(sv + S.off_lam2), rho, hcoef, blockmax, kept ? nullptr : rowinfo, call_mode(kept, (int)Vl, K, a->cap), (int32_t)V,
       ranked ? nullptr : keys_in, vals_in, longlist, skeys, perm);
   // rows grouped by target, for the one-hot part of dW
   if (!ranked) {
