@@ -976,26 +976,26 @@ static_assert(DWO_GROUP * (256 + 8) <= SMEM_BYTES && DWO_GROUP >= 64 * (LONG_SEG
 constexpr int DWO_MAX_KT = 131072 / BK;
 static_assert(SMEM_MAX - SMEM_BYTES - 8 * DWO_MAX_KT - DWO_AUX >= 4 * DWO_STAGE, "no room for the staging tiles beside the K slots");
 
-template <typename T>
-__global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  int rt, ct;
-  if (!map_tile_rr(blockIdx.x, p.RT, p.CT, rt, ct)) return;
+// NA = 2: 128 rows of dW (rt counts those), see bwd_dw_half_kernel.
+template <typename T, int NA>
+__device__ __forceinline__ void dw_out_tile(const DwParams& p, const DwOut& o, uint8_t* smem, int rt, int ct) {
+  constexpr int TROWS = 64 * NA, EB = TROWS, CHUNKS = EB / 16;               // rows of dW in the tile = bytes of X_q of an entry
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wa = wave >> 1, wb = wave & 1;
   const int KT = p.KT;
   uint32_t* lsc = reinterpret_cast<uint32_t*>(smem + SMEM_BYTES);            // block exponents of the K loop: [v half][K block]
   int* ioff = reinterpret_cast<int*>(smem + SMEM_BYTES + 8 * KT);            // [257]: first short entry of column c, counted over the tile
   int* spos = ioff + 260;                                                    // [257]: segoff of the tile's columns
   uint8_t* area = reinterpret_cast<uint8_t*>(spos + 260);                    // the rest of LDS
-  const int room = ((SMEM_MAX - SMEM_BYTES - DWO_AUX - 8 * KT) / (256 + 8)) & ~3;
-  // entry q's row and coefficient; its 256 bytes of X_q (columns rt * 256 on) at x + q * 256
+  const int room = ((SMEM_MAX - SMEM_BYTES - DWO_AUX - 8 * KT) / (EB + 8)) & ~(64 / CHUNKS - 1);
+  // entry q's row and coefficient; its EB bytes of X_q (columns rt * TROWS on) at x + q * EB
   struct Item { int row; float h; };
   auto load_rows = [&](const Item* items, int n, uint8_t* x) {
     const int lane = lane_id();
     const uint32_t lds0 = (uint32_t)(uintptr_t)((__attribute__((address_space(3))) void*)x);
-    for (int q0 = 4 * wave; q0 < n; q0 += 16) {              // one load: four entries; beyond the last one it is loaded again
-      const int q = q0 + (lane >> 4), c = (lane & 15) ^ (q & 15);
-      lds_direct_16_far(__builtin_amdgcn_readfirstlane(lds0 + q0 * 256), o.xq + (int64_t)items[q < n ? q : n - 1].row * o.ldx + rt * 256 + c * 16);
+    constexpr int PER = 64 / CHUNKS;                         // entries to one load: four (NA = 4); beyond the last one it is loaded again
+    for (int q0 = PER * wave; q0 < n; q0 += 4 * PER) {
+      const int q = q0 + lane / CHUNKS, c = (lane % CHUNKS) ^ (q & (CHUNKS - 1));
+      lds_direct_16_far(__builtin_amdgcn_readfirstlane(lds0 + q0 * EB), o.xq + (int64_t)items[q < n ? q : n - 1].row * o.ldx + rt * TROWS + c * 16);
     }
   };
   bool pre;
@@ -1023,7 +1023,7 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
     const int E = __builtin_amdgcn_readfirstlane(ioff[256]);
     pre = E <= room;
     if (pre && E > 0) {
-      Item* items = reinterpret_cast<Item*>(area + room * 256);
+      Item* items = reinterpret_cast<Item*>(area + room * EB);
       for (int k = 0; k < cnt; ++k) items[incl - cnt + k].row = s0 + k;
       __syncthreads();
       for (int q = t; q < E; q += NTHREADS) {
@@ -1034,15 +1034,17 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
       load_rows(items, E, area);
     }
   }
-  v16f acc[4][4];
-  mfma_mainloop<false, NoHook, BLOCKED_KSTEP, true, 2>(p.xt + ((int64_t)rt * p.kbn + p.kb0) * BLOCKED_KSTEP, BK, p.ghat_t + (int64_t)(2 * ct) * BLOCKED_KSTEP, BLOCKED_KSTEP, p.KT,
+  v16f acc[NA][4];
+  // (128 rows: half a 256-row tile of X~, whose K blocks are 256 rows of BK bytes)
+  const uint8_t* xt = p.xt + ((int64_t)(NA == 4 ? rt : rt >> 1) * p.kbn + p.kb0) * BLOCKED_KSTEP + (NA == 4 ? 0 : (rt & 1) * TROWS * BK);
+  mfma_mainloop<false, NoHook, BLOCKED_KSTEP, true, 2, false, false, NA>(xt, BK, p.ghat_t + (int64_t)(2 * ct) * BLOCKED_KSTEP, BLOCKED_KSTEP, p.KT,
                                                        smem, acc, ct & 7, 2 * (rt & 3), wave, NoHook(), 128 * BK, p.kbv * BLOCKED_KSTEP, lsc + wb * p.KT);
   const float x_s = o.dc ? o.dc->x_s : o.x_s, scale = x_s * o.xi[0];
   T* dw = reinterpret_cast<T*>(o.dw);
   const bool vec = sizeof(T) == 2 && ((reinterpret_cast<uintptr_t>(o.dw) | (uintptr_t)(o.dw_ld * (int64_t)sizeof(T))) & 15) == 0 && (o.V % 8 == 0 || ct * 256 + 256 <= o.V);
   uint8_t* stage = (pre ? smem : area) + wave * DWO_STAGE;
   const uint8_t* xrows = pre ? area : smem;
-  const Item* items = reinterpret_cast<const Item*>(pre ? area + room * 256 : smem + DWO_GROUP * 256);
+  const Item* items = reinterpret_cast<const Item*>(pre ? area + room * EB : smem + DWO_GROUP * EB);
   int bend = pre ? 4 : 0, qsub = 0;            // row blocks whose entries are in LDS; what to take off an entry's number for its place there
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
@@ -1053,7 +1055,7 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
       while (bend < 4 && upto(bend + 1) <= DWO_GROUP) ++bend;
       bend = __builtin_amdgcn_readfirstlane(bend);
       const int total = __builtin_amdgcn_readfirstlane(upto(bend)), base0 = ioff[32 * b], sub1 = ioff[128 + 32 * b] - (ioff[32 * bend] - base0);
-      Item* list = reinterpret_cast<Item*>(smem + DWO_GROUP * 256);
+      Item* list = reinterpret_cast<Item*>(smem + DWO_GROUP * EB);
       __syncthreads();                         // every wave is done with the entries that were there
       const int t = wave * 64 + lane_id(), tb = (t & 127) >> 5;
       if (tb >= b && tb < bend) {
@@ -1072,7 +1074,7 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
       qsub = __builtin_amdgcn_readfirstlane(wb ? sub1 : base0);
     }
 #pragma unroll
-    for (int ah = 0; ah < 2; ++ah) {           // rows 64 ah .. + 63 of the quadrant
+    for (int ah = 0; ah < NA / 2; ++ah) {      // rows 64 ah .. + 63 of the quadrant
       const int lane = lane_id(), h = lane >> 5, c = wb * 128 + b * 32 + (lane & 31), v = ct * 256 + c;
       float val[32];
 #pragma unroll
@@ -1082,8 +1084,8 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
         if (k < n) {
           const int q = q0 + k;
           const float hx = items[q].h * x_s;
-          const uint8_t* xr = xrows + q * 256 + 4 * h;
-          const int sw = (8 * wa + 4 * ah) ^ (q & 15);
+          const uint8_t* xr = xrows + q * EB + 4 * h;
+          const int sw = (2 * NA * wa + 4 * ah) ^ (q & (CHUNKS - 1));
 #pragma unroll
           for (int g = 0; g < 8; ++g) {        // four rows each: 32 (g / 4) + 8 (g % 4) + 4 h on
             const uint32_t w = *reinterpret_cast<const uint32_t*>(xr + ((sw ^ (g >> 1)) << 4) + 8 * (g & 1));
@@ -1097,7 +1099,7 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
       const int L = spos[c + 1] - spos[c];
       if (__builtin_amdgcn_ballot_w64(L >= LONG_SEG) != 0) {
         if (L >= LONG_SEG) {
-          const float* ls = o.longsum + (int64_t)o.longbase[v] * o.dq + rt * 256 + wa * 128 + ah * 64 + 4 * h;
+          const float* ls = o.longsum + (int64_t)o.longbase[v] * o.dq + rt * TROWS + wa * 32 * NA + ah * 64 + 4 * h;
 #pragma unroll
           for (int g = 0; g < 8; ++g) {
             const v4f s = *reinterpret_cast<const v4f*>(ls + 32 * (g >> 2) + 8 * (g & 3));
@@ -1106,7 +1108,7 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
           }
         }
       }
-      const int j0 = rt * 256 + wa * 128 + ah * 64;
+      const int j0 = rt * TROWS + wa * 32 * NA + ah * 64;
       if (vec) {
 #pragma unroll
         for (int g = 0; g < 8; ++g) {
@@ -1139,6 +1141,31 @@ __global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
       __builtin_amdgcn_sched_barrier(0);       // one half at a time: the accumulators of all of them, moved up front, do not fit the registers
     }
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  int rt, ct;
+  if (!map_tile_rr(blockIdx.x, p.RT, p.CT, rt, ct)) return;
+  dw_out_tile<T, 4>(p, o, smem, rt, ct);
+}
+
+// The tiles of a last round that would leave more than half of the CUs idle, 128 rows to a workgroup: tiles tile0 .. tile0 + ntail - 1
+// of the round-robin order, two workgroups each, neighbours on one XCD (their columns of G are the same).
+// No partial sums and no launch to add them up, but a K loop as long as a whole tile's with half its MFMAs.  Measured, tail kernel and
+// its sum against this, V = 50304: d = 768 (79 tiles in the last round) 2048 rows of fp32 43 -> 27 us, 4096 60 -> 39, bf16 8192 80 -> 60,
+// 16384 123 -> 103; d = 1600 (99 tiles) 4096 rows 63 -> 36, 8192 94 -> 57; d = 1024 (20 tiles) 300 rows 16 -> 15, 2048 25 -> 23, 4096 29 for 34,
+// 16384 55 for 94.  As lines over kp, the pairs of K blocks, and n tiles: tail 18 + n / 4 + kp (0.25 + n / 70), this 14.5 + 1.3 kp
+// (dw_tail_plan).
+template <typename T>
+__global__ __launch_bounds__(256) void bwd_dw_half_kernel(DwParams p, DwOut o, int tile0, int ntail) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  int lin, none, rt, ct;
+  if (!map_tile(blockIdx.x, 1, 2 * ntail, none, lin)) return;
+  tile_from_index(tile0 + (lin >> 1), p.RT, p.CT, rt, ct);
+  rt = __builtin_amdgcn_readfirstlane(rt); ct = __builtin_amdgcn_readfirstlane(ct);
+  dw_out_tile<T, 2>(p, o, smem, 2 * rt + (lin & 1), ct);
 }
 
 // The same from fp32 partials: what is left are the tiles of a K-split last round (tl.tile0 >= 0: grid.y = tl.ntail tiles of

@@ -89,7 +89,8 @@ __device__ __forceinline__ void lds_direct_16_far(uint32_t lds_addr, const uint8
 //              stored in 128-byte pieces: for each of the 128 K rows of a K block, 128 bytes of N in one piece
 //              and the next 128 bytes in a second piece `ldb` bytes further on.  In LDS the K block is
 //              [2 pieces][128 K rows][128 B]; fragments are formed with the transposing LDS read (see below).
-template <bool TRB = false>
+// NA = 2: a tile of 128 A rows (see mfma_mainloop): the wave's A rows are 32 in four chunks, loads 8, 10, 12 and 14 do not exist.
+template <bool TRB = false, int NA = 4>
 struct TileLoads {
   uint32_t vo[16];    // per-lane byte offset of load n; even n: A, odd n: B
   uint32_t lds[16];   // LDS address of load n in slot 0 (wave-uniform)
@@ -103,19 +104,20 @@ struct TileLoads {
     const int lr = lane >> 3, pc = lane & 7;
 #pragma unroll
     for (int n = 0; n < 8; ++n) {
-      const int ca = (n + rot_a) & 7, cb = (n + rot_b) & 7;
-      const int rowa = wave * 64 + ca * 8 + lr, rowb = wave * 64 + cb * 8 + lr;
+      const int ca = (n + rot_a) & (2 * NA - 1), cb = (n + rot_b) & 7;
+      const int rowa = wave * 16 * NA + ca * 8 + lr, rowb = wave * 64 + cb * 8 + lr;
       const int swa = (rowa & 7) ^ ((rowa >> 3) & 1), swb = (rowb & 7) ^ ((rowb >> 3) & 1);
       vo[2 * n] = (uint32_t)((a_rows ? a_rows[rowa] : rowa) * lda + ((pc ^ swa) * 16));
       if (TRB) vo[2 * n + 1] = (uint32_t)((rowb >> 7) * ldb + (rowb & 127) * BK + ((pc ^ (rowb & 7)) * 16));
       else vo[2 * n + 1] = (uint32_t)(rowb * ldb + ((pc ^ swb) * 16));
-      lds[2 * n] = lds0 + wave * 64 * BK + ca * 8 * BK;
+      lds[2 * n] = lds0 + wave * 16 * NA * BK + ca * 8 * BK;
       lds[2 * n + 1] = lds0 + TM * BK + wave * 64 * BK + cb * 8 * BK;
     }
   }
   // load n of the K block that starts at ga / gb, into LDS slot SLOT
   template <int SLOT>
   __device__ __forceinline__ void issue(int n, const uint8_t* ga, const uint8_t* gb) const {
+    if ((n & 1) == 0 && n >= 4 * NA) return;
     lds_direct_16<SLOT * SLOT_BYTES>(lds[n], vo[n], (n & 1) ? gb : ga);
   }
 };
@@ -187,23 +189,28 @@ __device__ __forceinline__ v16f mfma_bf16_pair(const v8i& a, const v8i& b, v16f 
 // issued; the other 48 are left to the caller, who finds the pair in the two LDS slots on return (lds_fragment) and
 // issues them (mfma_tail) between the vector instructions of its epilogue of the finished accumulators, where the
 // matrix pipe would otherwise stand idle.  Nothing may be loaded into the slots until that is done.
-template <bool PREFETCHED = false, class Hook = NoHook, int KSTEP = BK, bool TRB = false, int SCALE = 0, bool BF16 = false, bool DEFER = false>
+//
+// NA = 2: a tile of 128 A rows, 64 to a wave, for a last round of tiles that would leave half the chip idle.  The slots
+// are the same 32, every other one with an MFMA; the loads and reads of the missing rows drop out of the table (no load
+// before b2, whose count the wait there relies on, is among them).
+template <bool PREFETCHED = false, class Hook = NoHook, int KSTEP = BK, bool TRB = false, int SCALE = 0, bool BF16 = false, bool DEFER = false, int NA = 4>
 __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, int64_t lda,
                                               const uint8_t* __restrict__ Bg, int64_t ldb, int KD,
-                                              uint8_t* smem, v16f (&acc)[4][4], int rot_a, int rot_b, int wave, Hook&& hook = NoHook(),
+                                              uint8_t* smem, v16f (&acc)[NA][4], int rot_a, int rot_b, int wave, Hook&& hook = NoHook(),
                                               int64_t bk1_arg = 0, int64_t bk2_arg = 0, const uint32_t* lds_scale = nullptr,
                                               const int* a_rows = nullptr) {
-  static_assert(!DEFER || (!BF16 && SCALE == 0 && !TRB), "DEFER is for the plain fp8 loop");
+  static_assert(!DEFER || (!BF16 && SCALE == 0 && !TRB && NA == 4), "DEFER is for the plain fp8 loop");
+  static_assert(NA == 4 || (NA == 2 && LOADS_EM <= 8), "loads of block k + 2 that are counted: both operands' first four each");
   const int lane = lane_id();
   const int wa = wave >> 1, wb = wave & 1;
   const int64_t bk1 = TRB ? bk1_arg : (int64_t)KSTEP, bk2 = TRB ? bk2_arg : (int64_t)(2 * KSTEP);
-  const TileLoads<TRB> ld(lda, ldb, smem, rot_a, rot_b, wave, a_rows);
+  const TileLoads<TRB, NA> ld(lda, ldb, smem, rot_a, rot_b, wave, a_rows);
   // fragments: lane reads row l%32 of a 32-row block, 32 bytes of K at (l/32)*32 within the sub-step
   const int r = lane & 31, h = lane >> 5;
   const int sw = (r & 7) ^ ((r >> 3) & 1);
-  const int abase = wa * 128 * BK + r * BK, bbase = TM * BK + wb * 128 * BK + r * BK;
+  const int abase = wa * 32 * NA * BK + r * BK, bbase = TM * BK + wb * 128 * BK + r * BK;
   // half `u` (0, 1) of fragment n (0-3: A, 4-7: B) of the sub-step with K half `half` in LDS slot `slot`: registers 4 u .. 4 u + 3
-  auto runit = [&](int slot, int half, int n, int u, v8i (&fa)[4], v8i (&fb)[4]) {
+  auto runit = [&](int slot, int half, int n, int u, v8i (&fa)[NA], v8i (&fb)[4]) {
     v4i q;
     if (TRB && n >= 4) {
       // B block b = n - 4 from the [K row][N] layout.  ds_read_b64_tr_b8 works on groups of 16 lanes: lane j of a
@@ -232,9 +239,10 @@ __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, in
     f[4 * u] = q[0]; f[4 * u + 1] = q[1]; f[4 * u + 2] = q[2]; f[4 * u + 3] = q[3];
   };
   // read units [q0, q0 + cnt) of a sub-step, in the order in which its MFMAs need them
-  auto runits = [&](int slot, int half, int q0, int cnt, v8i (&fa)[4], v8i (&fb)[4]) {
+  auto runits = [&](int slot, int half, int q0, int cnt, v8i (&fa)[NA], v8i (&fb)[4]) {
 #pragma unroll
-    for (int q = q0; q < q0 + cnt; ++q) runit(slot, half, UNIT_FRAG[q >> 1], q & 1, fa, fb);
+    for (int q = q0; q < q0 + cnt; ++q)
+      if (UNIT_FRAG[q >> 1] < NA || UNIT_FRAG[q >> 1] >= 4) runit(slot, half, UNIT_FRAG[q >> 1], q & 1, fa, fb);
   };
   // prologue: K block 0 and half of block 1 in flight, block 0 visible, fragments of sub-step 0 in registers
   if (!PREFETCHED) {
@@ -246,7 +254,7 @@ __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, in
   // K block 0 has landed once at most the loads of block 1 are in flight (vector memory operations that a caller issued
   // after its prefetch -- stores of an epilogue -- are younger still: the wait then covers block 1 as well, no more)
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(AHEAD_LOADS) : "memory");
-  v8i fa[2][4], fb[2][4];
+  v8i fa[2][NA], fb[2][4];
   runits(0, 0, 0, 16, fa[0], fb[0]);
   // block scales of the current pair of K blocks and of the next one (read one pair ahead)
   const __attribute__((address_space(3))) v2i* scp = (const __attribute__((address_space(3))) v2i*)lds_scale;
@@ -302,8 +310,10 @@ __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, in
         }
       }
       const int sub = s >> 4, i = s & 15;
+      constexpr int PER = 4 / NA;                 // slots to an MFMA
       if (DEFER && !has2 && (i & 3) != 0) {}      // last pair, B blocks 1 - 3: the caller's
-      else if (first && BLK == 0 && sub == 0) mm0(i); else mm(BLK, sub, i);
+      else if (i % PER != 0) {}
+      else if (first && BLK == 0 && sub == 0) mm0(i / PER); else mm(BLK, sub, i / PER);
       hook(32 * BLK + s);
       if (!(first && BLK == 0)) runits(BLK, 0, UNITS_N0 + ksum(KS.c0, s), KS.c0[s], fa[0], fb[0]);      // (the first block's came with the prologue)
       runits(BLK, 1, ksum(KS.r1, s), KS.r1[s], fa[1], fb[1]);

@@ -1,0 +1,45 @@
+"""The last round of dW's tiles -- 128 rows of a tile to a workgroup, shared out along K, or a workgroup to each tile like the full
+rounds -- against the way over fp32 partials that a small workspace takes: the same products, so that the difference is the
+order of an fp32 sum of a few parts, 2^-20 of the largest element here, and one unit of the output type's rounding."""
+import pytest
+import torch
+
+from slowrun_amd import configs
+from .test_gpu_dw_epilogue import _targets
+
+pytestmark = pytest.mark.gpu
+
+
+def _kernels(fn):
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        out = fn()
+        torch.cuda.synchronize()
+    return out, " ".join(e.key for e in p.key_averages())
+
+
+@pytest.mark.parametrize("kind", ["spread", "crowded", "hot"])
+@pytest.mark.parametrize("w_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("way,N,d,V,K", [
+    ("half", 1, 16, 8, 1), ("half", 513, 272, 2049, 2), ("half", 300, 1040, 4096, 3), ("half", 2048, 528, 5000, 1), ("half", 700, 112, 32701, 1),
+    ("tail", 1700, 16, 250, 1), ("tail", 4100, 272, 1003, 2),
+    ("out", 300, 16, 33100, 1), ("out", 600, 16, 65536, 1)])
+def test_last_round_of_dw(kind, w_dtype, way, N, d, V, K):
+    from slowrun_amd import _lib
+    from slowrun_amd import cuda_kernels as ck
+    inp = configs.make_inputs("tiny_track", N=N, d=d, V=V)
+    y = _targets(kind, N, V, torch.Generator().manual_seed(N + K)).clamp_(max=V - 1).cuda()
+    if N == 1:
+        y[0] = V // 2
+    x, w = inp.x.cuda().bfloat16(), inp.w.cuda().to(w_dtype)
+    mw = torch.tensor([1.0, 0.5, 0.25, 0.125][:K], device="cuda") if K > 1 else None
+    go = torch.rand(N, generator=torch.Generator().manual_seed(1)).cuda() / N
+    _out, saved, *_ = ck.ce_forward(x, w, y, inp.x_s, inp.w_s, inp.cap, "none", mtp_weights=mw)
+    args = (saved, y, go, N, d, V, inp.x_s, inp.w_s, inp.cap, 1.0, "none", torch.bfloat16, w_dtype)
+    (_dx, dw), names = _kernels(lambda: ck.ce_backward(*args, mtp_weights=mw))
+    assert [k in names for k in ("bwd_dw_half", "bwd_dw_tail", "bwd_dw_out")].index(True) == ("half", "tail", "out").index(way), names
+    ref = ck.ce_backward(*args, mtp_weights=mw, panel_rows=256, workspace_bytes=_lib.sizes_for(N, d, V, K).bwd_workspace_min_bytes)[1].double()
+    unit = 2.0 ** -8 if w_dtype == torch.bfloat16 else 2.0 ** -23
+    assert bool(((dw.double() - ref).abs() <= unit * ref.abs() + 2.0 ** -20 * ref.abs().max()).all())
+    assert float(ref.abs().max()) > 0
