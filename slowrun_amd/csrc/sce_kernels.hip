@@ -816,7 +816,12 @@ extern "C" int sce_backward(const sce_args* a) {
     // a panel with fewer than half as many tiles as there are CUs shares each tile's K loop among several workgroups
     const int tiles = dp_.RT * CTd, kpairs = (int)(S.Vp / BK / 2);
     int ksplit = tiles * 2 <= 256 ? 256 / tiles : 1;
-    if (ksplit > 8) ksplit = 8;
+    // (up to DX_MAX_PARTS of them, more than DX_FEW_PARTS only as long as each has DX_PART_PAIRS pairs of K blocks: what a part saves in
+    // its main loop it costs in partial sums, 256 KB a tile, written and read.  Measured, V = 50304, parts of a tile and time of
+    // kernel and sum: 2048 rows, d = 256 8 62.5 us, 16 45, 32 51.6; 300 rows, d = 1024 62.4, 44.5, 42.5; 2048 rows, d = 768, 24 tiles,
+    // 8 82.6, 10 78.5; 1000 rows, d = 256, V = 4096, 16 pairs in all, 8 18, 16 22.6)
+    constexpr int DX_MAX_PARTS = 16, DX_FEW_PARTS = 8, DX_PART_PAIRS = 8;
+    ksplit = std::min(ksplit, std::max(DX_FEW_PARTS, std::min(DX_MAX_PARTS, kpairs / DX_PART_PAIRS)));
     if (ksplit > kpairs) ksplit = kpairs;
     dp_.ksplit = ksplit;
     KernelTimer tm(SCE_K_DX, st);

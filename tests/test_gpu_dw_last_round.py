@@ -1,10 +1,12 @@
 """The last round of dW's tiles -- 128 rows of a tile to a workgroup, shared out along K, or a workgroup to each tile like the full
 rounds -- against the way over fp32 partials that a small workspace takes: the same products, so that the difference is the
-order of an fp32 sum of a few parts, 2^-20 of the largest element here, and one unit of the output type's rounding."""
+order of an fp32 sum of a few parts, 2^-20 of the largest element here, and one unit of the output type's rounding.  And dX of
+few tiles, whose K loop is cut into up to 16 parts."""
 import pytest
 import torch
 
 from slowrun_amd import configs
+from . import parity_util as pu
 from .test_gpu_dw_epilogue import _targets
 
 pytestmark = pytest.mark.gpu
@@ -43,3 +45,10 @@ def test_last_round_of_dw(kind, w_dtype, way, N, d, V, K):
     unit = 2.0 ** -8 if w_dtype == torch.bfloat16 else 2.0 ** -23
     assert bool(((dw.double() - ref).abs() <= unit * ref.abs() + 2.0 ** -20 * ref.abs().max()).all())
     assert float(ref.abs().max()) > 0
+
+
+@pytest.mark.parametrize("N,d,V", [(100, 16, 4096), (300, 272, 33001), (257, 64, 50257)])
+def test_dx_in_many_parts(N, d, V):
+    inp = configs.make_inputs("irregular", N=N, d=d, V=V)
+    ours = pu.run_ours(inp, "mean", keep_dlogits=True)
+    pu.check_parity(ours, pu.run_oracle(inp, ours, "mean"), "mean")
