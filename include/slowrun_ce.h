@@ -186,6 +186,10 @@ int sce_transpose_bytes(const void* src, void* dst, int64_t rows, int64_t cols,
  * (fwd_workspace_bytes) and fills args->saved. */
 int sce_forward(const sce_args* args);
 
+/* sce_forward, and what sce_target_probability forms of its losses (args->losses must be given), in the same launches:
+ * probability[i] = exp(-losses[i]), or 0 where targets[i] == ignore_index. */
+int sce_forward_probability(const sce_args* args, float* probability);
+
 /* sce_forward without a workspace: the scratch that sce_forward takes from args->workspace (the partial row
  * statistics of the vocabulary splits) lives in a static device array of the library, 8 MiB on every GPU the
  * library has run on, until the process ends.  No counterpart in the reference; it is for callers that cannot

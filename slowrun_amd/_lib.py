@@ -15,7 +15,7 @@ SCE_VERSION = 4
 
 EXPORTS = ("sce_version", "sce_last_error", "sce_sizes_for", "sce_quantize_e4m3", "sce_quantize_e4m3_dev", "sce_amax_scale",
            "sce_target_probability", "sce_transpose_bytes",
-           "sce_forward", "sce_forward_noalloc", "sce_backward", "sce_timing_enable", "sce_timing_read", "sce_bench_mfma", "sce_bench_gemm", "sce_bench_floor",
+           "sce_forward", "sce_forward_probability", "sce_forward_noalloc", "sce_backward", "sce_timing_enable", "sce_timing_read", "sce_bench_mfma", "sce_bench_gemm", "sce_bench_floor",
            "sce_test_set_gather_limit")
 
 KERNEL_KINDS = ("quantize", "fwd", "fwd_reduce", "bwd_prep", "recompute", "dx", "dw", "dw_final")
@@ -77,6 +77,7 @@ def lib():
         L.sce_target_probability.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_void_p, C.c_int32, C.c_void_p]
         L.sce_transpose_bytes.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int32, C.c_void_p]
         L.sce_forward.argtypes = [C.POINTER(SceArgs)]
+        L.sce_forward_probability.argtypes = [C.POINTER(SceArgs), C.c_void_p]
         L.sce_forward_noalloc.argtypes = [C.POINTER(SceArgs)]
         L.sce_backward.argtypes = [C.POINTER(SceArgs)]
         L.sce_bench_mfma.argtypes = [C.c_void_p, C.c_size_t, C.c_int32, C.c_int32, C.c_void_p, C.c_size_t, C.c_int32, C.c_void_p,

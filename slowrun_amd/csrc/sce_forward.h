@@ -27,8 +27,27 @@ struct FwdParams {
   float c2;
   float em2cap;            // e^{-2 cap}: what a logit of -inf adds to the sum of e^{z - cap}
   const DevConsts* dc;     // non-NULL: sc and k1 come from here (a scale lives on the device)
+  uint8_t* hdr;            // header of the saved state
   int want_argmax;         // the caller asks for the rows' argmax: the column of the running maximum is tracked
 };
+
+// What a forward call was asked for, as far as the matching backward call must have been asked the same: left in the header
+// of the saved state (HDR_MODE_OFF bytes in) by fwd_combine_kernel and compared by bwd_prep_kernel.  A backward call whose
+// flags differ would read dlogits that were never written, or mask other columns: it gets NaN gradients instead.
+struct CallMode {
+  int32_t emit, vocab_limit, n_predict, cap_bits;
+};
+constexpr int HDR_MODE_OFF = 64;
+static inline CallMode call_mode(bool emit, int vocab_limit, int n_predict, float cap) {
+  CallMode m;
+  m.emit = emit ? 1 : 0; m.vocab_limit = vocab_limit; m.n_predict = n_predict;
+  memcpy(&m.cap_bits, &cap, 4);
+  return m;
+}
+
+// ... and HDR_COUNT_OFF bytes in, how many blocks of fwd_combine_kernel are done: set to zero by the forward kernel before it.
+constexpr int HDR_COUNT_OFF = 128;
+__device__ __forceinline__ uint32_t* done_count(const FwdParams& p) { return reinterpret_cast<uint32_t*>(p.hdr + HDR_COUNT_OFF); }
 
 // Per 256 x 256 tile and per row a lane owns: add up e^{z - cap} over its 64 columns and keep the
 // largest raw accumulator.  z is bounded by +-cap, so no running maximum is needed for the sum:
@@ -575,6 +594,7 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
   if (p.dc) { p.sc = p.dc->sc; p.k1 = p.dc->k1; }
   int rt, s;
   if (!map_tile(blockIdx.x, p.RT, p.S, rt, s)) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *done_count(p) = 0;
   const int ct0 = (int)((int64_t)p.CT * s / p.S), ct1 = (int)((int64_t)p.CT * (s + 1) / p.S);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wa = wave >> 1, wb = wave & 1;
   {
@@ -766,6 +786,7 @@ __global__ __launch_bounds__(FEW_THREADS) void fwd_few_rows_kernel(FwdParams p, 
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), h = lane >> 5;
   const int ct0 = (int)((int64_t)p.CT * blockIdx.x / p.S), ct1 = (int)((int64_t)p.CT * (blockIdx.x + 1) / p.S);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *done_count(p) = 0;
   int* tgt = reinterpret_cast<int*>(smem + F::TGT_OFF);           // [4 offsets][32 NB]
   for (int e = threadIdx.x; e < p.n_predict * 32 * NB; e += FEW_THREADS) {
     const int row = e % (32 * NB), i = row + e / (32 * NB);
@@ -907,19 +928,30 @@ __global__ __launch_bounds__(FEW_THREADS) void fwd_few_rows_kernel(FwdParams p, 
 }
 
 // What a block of COMBINE_ROWS rows contributes to the mean loss: left by fwd_combine_kernel in the first 16 bytes of the
-// block's own rows of the partial records (which it has consumed by then), summed by fwd_reduce_kernel.
-struct BlockLoss {
-  double sum;      // sum of lse_i - z[i, y_i] over the valid rows
-  int32_t cnt;     // valid rows
-  int32_t bad;     // targets outside [0, V) other than ignore_index
-};
-static_assert(sizeof(BlockLoss) == 16, "one float4 slot");
+// block's own rows of the partial records (which it has consumed by then), summed by its last block:
+//   8 bytes: sum of lse_i - z[i, y_i] over the valid rows (a double); 4: valid rows; 4: targets outside [0, V) other than ignore_index
+
+// p(target) = exp(-loss), 0 for the rows without a target (fwd_combine_kernel forms it for sce_forward_probability).
+__device__ __forceinline__ float row_probability(float loss, int64_t target, int64_t ignore_index) { return target == ignore_index ? 0.f : expf(-loss); }
+
+// The same of losses from any call.  Bound by its launch: in place of five elementwise operations of
+// torch's (compare, zeros, negate, exp, where) a call that scores 61 rows at d = 2560, V = 50304 takes 65.6 us for 73.6.
+__global__ __launch_bounds__(256) void target_probability_kernel(const float* __restrict__ losses, const int64_t* __restrict__ targets, int64_t n,
+                                                                int64_t ignore_index, float* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = row_probability(losses[i], targets[i], ignore_index);
+}
 
 // Folds the V-splits of a row and writes lse / loss / argmax and the saved row statistics: COMBINE_ROWS rows to a
 // workgroup, one wave to every G-th split (its 64 rows' records are 1 KB in a row), four records in flight per lane.
 // What bounds it is the chain of loads, not their volume: with one thread per row the records of a call of 61 rows and
 // 197 splits were 197 loads of one workgroup.  Rows beyond N have no records (fwd_few_rows_kernel writes none).  G = 4 for up to 16 splits, 16 beyond (rows too few to fill the chip
 // without cutting the vocabulary finer); the order of the sums depends on G alone.
+// The block that is done last adds up what all of them left: n_valid, targets out of range, the mean, in a fixed order.  The blocks'
+// sums and the count go past the L2 caches (agent scope: every XCD has its own), the sum before the count.  As a launch of one
+// workgroup (fwd_reduce_kernel, before) the same was 4.1 us of every forward call, and exp(-loss) for a caller that scores rows another 4.1: this kernel takes 2
+// to 2.6 us longer for both (7.1 for 4.5 + 4.1 at 2048 rows, 61 rows scored 56 -> 50 us in all).  A call of 64 rows at most that no backward
+// call follows is one block, which has nobody to wait for.
 constexpr int COMBINE_ROWS = 64;
 template <int G>
 __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* __restrict__ partials, int S, int N, int Np, int V,
@@ -927,11 +959,13 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
                                                          const float* __restrict__ mtp_weights, int n_predict,
                                                          float* __restrict__ s_lse, float* __restrict__ s_zy, float* __restrict__ losses,
                                                          float* __restrict__ lse_out, int32_t* __restrict__ argmax_out,
-                                                         uint8_t* __restrict__ ghat, int64_t kbv) {
+                                                         uint8_t* __restrict__ ghat, int64_t kbv, float* __restrict__ probability, uint8_t* __restrict__ hdr,
+                                                         float* __restrict__ loss_out, int32_t* __restrict__ nvalid_out, CallMode mode) {
   static_assert(G >= 4, "one wave per prediction offset");
   __shared__ float rsum[G][COMBINE_ROWS], rmax[G][COMBINE_ROWS], rl[4][COMBINE_ROWS];
   __shared__ int rarg[G][COMBINE_ROWS];
-  const int r = threadIdx.x & 63, g = threadIdx.x >> 6, i = blockIdx.x * COMBINE_ROWS + r;      // the grid covers Np rows exactly
+  __shared__ bool last;
+  const int r = threadIdx.x & 63, g = threadIdx.x >> 6, i = blockIdx.x * COMBINE_ROWS + r;      // the grid covers Np rows exactly, or N alone if no backward call can follow
   {
     float sum = 0.f, umax = -INFINITY;
     int uarg = 0x7fffffff;
@@ -992,70 +1026,47 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) { term += __shfl_xor(term, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
       if (r == 0) {
-        BlockLoss bl;
-        bl.sum = term; bl.cnt = cnt; bl.bad = bad;
-        *reinterpret_cast<BlockLoss*>(partials + (int64_t)blockIdx.x * COMBINE_ROWS) = bl;
+        uint64_t* slot = reinterpret_cast<uint64_t*>(partials + (int64_t)blockIdx.x * COMBINE_ROWS);
+        const uint64_t counts = (uint64_t)(uint32_t)cnt | ((uint64_t)(uint32_t)bad << 32);
+        __hip_atomic_store(slot, (uint64_t)__double_as_longlong(term), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(slot + 1, counts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (gridDim.x > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // both have arrived
+        last = gridDim.x == 1 || __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hdr + HDR_COUNT_OFF), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
       }
     }
   }
-  if (!losses) return;
   __syncthreads();
-  if (g == 0 && i < N) {
+  if (losses && g == 0 && i < N) {
     float l = rl[0][r];
     for (int k = 1; k < n_predict; ++k) l += rl[k][r];
     losses[i] = l;
+    if (probability) probability[i] = row_probability(l, targets[i], ignore_index);
   }
-}
-
-// p(target) = exp(-loss) of every row, 0 for the rows without a target.  Bound by its launch: in place of five elementwise operations of
-// torch's (compare, zeros, negate, exp, where) a call that scores 61 rows at d = 2560, V = 50304 takes 65.6 us for 73.6.
-__global__ __launch_bounds__(256) void target_probability_kernel(const float* __restrict__ losses, const int64_t* __restrict__ targets, int64_t n,
-                                                                int64_t ignore_index, float* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) out[i] = targets[i] == ignore_index ? 0.f : expf(-losses[i]);
-}
-
-// What a forward call was asked for, as far as the matching backward call must have been asked the same: left in the header
-// of the saved state (HDR_MODE_OFF bytes in) by fwd_reduce_kernel and compared by bwd_prep_kernel.  A backward call whose
-// flags differ would read dlogits that were never written, or mask other columns: it gets NaN gradients instead.
-struct CallMode {
-  int32_t emit, vocab_limit, n_predict, cap_bits;
-};
-constexpr int HDR_MODE_OFF = 64;
-static inline CallMode call_mode(bool emit, int vocab_limit, int n_predict, float cap) {
-  CallMode m;
-  m.emit = emit ? 1 : 0; m.vocab_limit = vocab_limit; m.n_predict = n_predict;
-  memcpy(&m.cap_bits, &cap, 4);
-  return m;
-}
-
-// single workgroup: n_valid, number of out-of-range targets, mean loss from the per-block sums (fixed order)
-__global__ __launch_bounds__(1024) void fwd_reduce_kernel(const float4* __restrict__ partials, int nblk,
-                                                         int32_t* __restrict__ hdr, float* __restrict__ loss_out,
-                                                         int32_t* __restrict__ nvalid_out, CallMode mode) {
-  __shared__ double ssum[1024];
-  __shared__ int scnt[1024], sbad[1024];
-  const int t = threadIdx.x;
-  double acc = 0.0;
+  if (!last) return;
+  double sum = 0.0;
   int cnt = 0, bad = 0;
-  for (int b = t; b < nblk; b += 1024) {
-    const BlockLoss bl = *reinterpret_cast<const BlockLoss*>(partials + (int64_t)b * COMBINE_ROWS);
-    acc += bl.sum; cnt += bl.cnt; bad += bl.bad;
+  for (int b = threadIdx.x; b < (int)gridDim.x; b += COMBINE_ROWS * G) {      // (of one block, thread 0 reads what it stored)
+    const uint64_t* slot = reinterpret_cast<const uint64_t*>(partials + (int64_t)b * COMBINE_ROWS);
+    sum += __longlong_as_double((long long)__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    const uint64_t c = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    cnt += (int)(uint32_t)c; bad += (int)(uint32_t)(c >> 32);
   }
-  ssum[t] = acc; scnt[t] = cnt; sbad[t] = bad;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) { sum += __shfl_xor(sum, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
+  __shared__ double wsum[G];
+  __shared__ int wcnt[G], wbad[G];
+  if (r == 0) { wsum[g] = sum; wcnt[g] = cnt; wbad[g] = bad; }
   __syncthreads();
-  for (int w = 512; w > 0; w >>= 1) {
-    if (t < w) { ssum[t] += ssum[t + w]; scnt[t] += scnt[t + w]; sbad[t] += sbad[t + w]; }
-    __syncthreads();
-  }
-  if (t == 0) {
-    hdr[0] = scnt[0]; hdr[1] = sbad[0];
-    const float mean = (float)(ssum[0] / (double)scnt[0]);   // 0/0 = NaN, as F.cross_entropy gives
-    reinterpret_cast<float*>(hdr)[2] = mean;
-    if (loss_out) *loss_out = mean;
-    if (nvalid_out) { nvalid_out[0] = scnt[0]; nvalid_out[1] = sbad[0]; }
-    *reinterpret_cast<CallMode*>(reinterpret_cast<uint8_t*>(hdr) + HDR_MODE_OFF) = mode;
-  }
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < G; ++w) { sum += wsum[w]; cnt += wcnt[w]; bad += wbad[w]; }
+  const float mean = (float)(sum / (double)cnt);                 // 0/0 = NaN, as F.cross_entropy gives
+  int32_t* head = reinterpret_cast<int32_t*>(hdr);
+  head[0] = cnt; head[1] = bad;
+  reinterpret_cast<float*>(hdr)[2] = mean;
+  *reinterpret_cast<CallMode*>(hdr + HDR_MODE_OFF) = mode;
+  if (loss_out) *loss_out = mean;
+  if (nvalid_out) { nvalid_out[0] = cnt; nvalid_out[1] = bad; }
 }
+
 
 }  // namespace sce

@@ -485,7 +485,8 @@ static int check_common(const sce_args* a, bool own_scratch = false) {
 }
 
 // ws: the partial records of the V-splits (the caller's workspace, or the library's static scratch)
-static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char* ws_name) {
+// probability: exp(-loss) of every row as well (sce_forward_probability), or NULL
+static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char* ws_name, float* probability = nullptr) {
   const int64_t N = a->shape.N, d = a->shape.d, V = a->shape.V;
   if (!a->x || !a->w) return fail(SCE_EINVAL, "x or w is NULL");
   if (a->x_ld < d || a->w_ld < V) return fail(SCE_EINVAL, "row strides smaller than the row length");
@@ -579,7 +580,7 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   p.dp = S.dp; p.ldx = S.ldx; p.N = (int)N; p.V = (int)Vl; p.Np = (int)S.Np; p.RT = RT; p.CT = CTw; p.S = nsplit;
   p.sc = bf16ops ? 1.0f : (float)a->x_s * (float)a->w_s; p.k1 = p.sc * 2.0f * LOG2E / a->cap; p.c2 = -2.0f * a->cap * LOG2E; p.ic2 = 1.0f / p.c2; p.em2cap = expf(-2.0f * a->cap);
   p.dc = bf16ops ? nullptr : dcp;
-  p.want_argmax = a->argmax != nullptr;
+  p.want_argmax = a->argmax != nullptr; p.hdr = sv + S.off_hdr;
   const int grid = map_tile_grid(RT, nsplit);
   // An fp8 forward pass has its target logits computed ahead of the forward kernel (from a tile of gathered rows of W_q^T,
   // together with the rows' boosts when it emits the dlogits) as long as that tile's 32-bit offsets reach every row of
@@ -619,16 +620,14 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   KernelTimer tm_red(SCE_K_FWD_REDUCE, st);
   float* s_lse = (float*)(sv + S.off_lse);
   float* s_zy = (float*)(sv + S.off_zy);
-  const int nblk = (int)(S.Np / COMBINE_ROWS);
+  const int nblk = (int)((bf16ops ? N + COMBINE_ROWS - 1 : S.Np) / COMBINE_ROWS);
   auto combine = [&](auto kernel, int g) {
     kernel<<<nblk, COMBINE_ROWS * g, 0, st>>>(p.partials, nsplit, (int)N, (int)S.Np, (int)Vl, a->targets, a->ignore_index, a->cap, a->mtp_weights,
-                                             a->shape.n_predict, s_lse, s_zy, a->losses, a->lse, a->argmax, emit && pre ? p.ghat_t : nullptr, p.kbv);
+                                             a->shape.n_predict, s_lse, s_zy, a->losses, a->lse, a->argmax, emit && pre ? p.ghat_t : nullptr, p.kbv, probability,
+                                             p.hdr, a->reduction == SCE_REDUCE_MEAN ? a->loss : nullptr, a->n_valid, call_mode(emit, (int)Vl, a->shape.n_predict, a->cap));
   };
   if (nsplit <= 16) combine(fwd_combine_kernel<4>, 4);
   else combine(fwd_combine_kernel<16>, 16);
-  fwd_reduce_kernel<<<1, 1024, 0, st>>>(p.partials, nblk, (int32_t*)(sv + S.off_hdr),
-                                        a->reduction == SCE_REDUCE_MEAN ? a->loss : nullptr, a->n_valid,
-                                        call_mode(emit, (int)Vl, a->shape.n_predict, a->cap));
   HIP_TRY(hipGetLastError());
   return SCE_OK;
 }
@@ -636,6 +635,14 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
 extern "C" int sce_forward(const sce_args* a) {
   if (int rc = check_common(a)) return rc;
   return forward_impl(a, a->workspace, a->workspace_bytes, "forward workspace");
+}
+
+// sce_forward, and exp(-loss) of every row from the kernel that forms the losses
+extern "C" int sce_forward_probability(const sce_args* a, float* probability) {
+  if (int rc = check_common(a)) return rc;
+  if (!probability) return fail(SCE_EINVAL, "probability is NULL");
+  if (!a->losses) return fail(SCE_EINVAL, "losses is NULL: the probabilities are formed from them");
+  return forward_impl(a, a->workspace, a->workspace_bytes, "forward workspace", probability);
 }
 
 // The same launches as sce_forward with the partial records in the library's static device array instead of a

@@ -163,9 +163,11 @@ class WeightCache:
 
 
 def ce_forward(x, w, targets, x_s, w_s, cap, reduction, want_argmax=False, mtp_weights=None, vocab_size=None,
-               weight_cache=None, norm_eps=None, keep_dlogits=False, no_alloc=False, operand_dtype=None):
+               weight_cache=None, norm_eps=None, keep_dlogits=False, no_alloc=False, operand_dtype=None, probability=None):
     """One call of sce_forward.  Returns (out, saved, lse, argmax, n_valid).
 
+    probability: float32 (N,) on x's device, to receive exp(-loss) of every row (0 where the target is -1)
+    from the same launches (sce_forward_probability).
     operand_dtype: None / torch.float8_e4m3fn (the fused path's e4m3 operands) or torch.bfloat16 (the arithmetic of the
     eager head under bf16 autocast: bf16 operands, logits rounded to bf16; forward only, the scales are not used).
     no_alloc: call sce_forward_noalloc instead, which keeps its scratch in a static device array of the library (this
@@ -218,7 +220,13 @@ def ce_forward(x, w, targets, x_s, w_s, cap, reduction, want_argmax=False, mtp_w
     if weight_cache is not None:
         wbuf, valid = weight_cache.prepare(w, w_s, sz.wcache_bytes)
         a.wcache, a.wcache_bytes, a.wcache_valid = wbuf.data_ptr(), wbuf.numel(), int(valid)
-    if no_alloc:
+    if probability is not None:
+        if no_alloc:
+            raise ValueError("probability and no_alloc do not go together")
+        if probability.dtype != torch.float32 or probability.shape != (N,) or probability.device != dev or not probability.is_contiguous():
+            raise ValueError("probability must be a contiguous float32 tensor of shape (N,) on x's device")
+        _lib.check(_lib.lib().sce_forward_probability(C.byref(a), probability.data_ptr()), "sce_forward_probability")
+    elif no_alloc:
         _lib.check(_lib.lib().sce_forward_noalloc(C.byref(a)), "sce_forward_noalloc")
     else:
         _lib.check(_lib.lib().sce_forward(C.byref(a)), "sce_forward")
@@ -419,16 +427,19 @@ def softcapped_cross_entropy(x, lm_head_weight, targets, x_s=None, w_s=None, cap
     that validation losses compare; the default keeps the training path's e4m3 operands with scales ``x_s``, ``w_s``.  ``x`` may have leading batch dimensions.  With ``norm_eps``
     given, ``x`` is the hidden state before the final ``F.rms_norm(x, (d,), eps=norm_eps)`` (tiny/train.py:734),
     which is then applied inside the quantiser."""
-    lead = x.shape[:-1]
+    out = _head_forward(x, lm_head_weight, targets, x_s, w_s, cap, vocab_size, reduction, norm_eps, operand_dtype)
+    return out if reduction == "mean" else out.reshape(x.shape[:-1])
+
+
+def _head_forward(x, lm_head_weight, targets, x_s, w_s, cap, vocab_size, reduction, norm_eps, operand_dtype, probability=None):
     x2 = x.reshape(-1, x.shape[-1])
     if operand_dtype == torch.bfloat16:
         x_s = w_s = 1.0
     elif x_s is None or w_s is None:
         raise ValueError("e4m3 operands need their scales x_s and w_s")
-    out, _saved, _lse, _am, _nv = ce_forward(x2.detach(), lm_head_weight.detach(), targets.reshape(-1),
-                                             _scale_value(x_s, x2), _scale_value(w_s, lm_head_weight), float(cap),
-                                             reduction, vocab_size=vocab_size, norm_eps=norm_eps, operand_dtype=operand_dtype)
-    return out if reduction == "mean" else out.reshape(lead)
+    return ce_forward(x2.detach(), lm_head_weight.detach(), targets.reshape(-1),
+                      _scale_value(x_s, x2), _scale_value(w_s, lm_head_weight), float(cap), reduction, vocab_size=vocab_size,
+                      norm_eps=norm_eps, operand_dtype=operand_dtype, probability=probability)[0]
 
 
 def target_probability(x, lm_head_weight, targets, x_s=None, w_s=None, cap=15.0, vocab_size=None, norm_eps=None,
@@ -438,10 +449,8 @@ def target_probability(x, lm_head_weight, targets, x_s=None, w_s=None, cap=15.0,
     (``_forward_pgt``, unlimited/train.py:1063-1069).  Here it is ``exp(-loss)`` of the per-row losses of
     ``softcapped_cross_entropy(..., reduction='none')``, same arguments; a row whose target is -1 has no target
     probability and gets 0."""
-    losses = softcapped_cross_entropy(x, lm_head_weight, targets, x_s, w_s, cap, vocab_size, "none", norm_eps, operand_dtype)
-    y, out = targets.reshape(-1).contiguous(), torch.empty_like(losses)
-    _lib.check(_lib.lib().sce_target_probability(losses.data_ptr(), y.data_ptr(), losses.numel(), IGNORE_INDEX, out.data_ptr(), losses.device.index,
-                                                _stream_ptr(losses.device)), "sce_target_probability")
+    out = torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
+    _head_forward(x, lm_head_weight, targets, x_s, w_s, cap, vocab_size, "none", norm_eps, operand_dtype, out.view(-1))
     return out
 
 
