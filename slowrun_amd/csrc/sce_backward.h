@@ -976,7 +976,7 @@ static_assert(DWO_GROUP * (256 + 8) <= SMEM_BYTES && DWO_GROUP >= 64 * (LONG_SEG
 constexpr int DWO_MAX_KT = 131072 / BK;
 static_assert(SMEM_MAX - SMEM_BYTES - 8 * DWO_MAX_KT - DWO_AUX >= 4 * DWO_STAGE, "no room for the staging tiles beside the K slots");
 
-// NA = 2: 128 rows of dW (rt counts those), see bwd_dw_half_kernel.
+// NA = 2: 128 rows of dW (rt counts those), the half tiles of bwd_dw_out_kernel.
 template <typename T, int NA>
 __device__ __forceinline__ void dw_out_tile(const DwParams& p, const DwOut& o, uint8_t* smem, int rt, int ct) {
   constexpr int TROWS = 64 * NA, EB = TROWS, CHUNKS = EB / 16;               // rows of dW in the tile = bytes of X_q of an entry
@@ -1143,29 +1143,29 @@ __device__ __forceinline__ void dw_out_tile(const DwParams& p, const DwOut& o, u
   }
 }
 
+// The first half_grid workgroups take the tiles tile0 .. of a last round that would leave more than half of the CUs idle, 128 rows each, two
+// neighbours on one XCD to a tile (their columns of G are the same): nhalf of them.  No partial sums and no launch to add them up,
+// but a K loop as long as a whole tile's with half its MFMAs.  They go first, so that the CUs fall out of step: when all of them
+// store their tiles at the same time, the matrix pipes stand idle, and the stores are the whole of 19 us of a tile's 43 at 2048 rows in fp32.
+// Measured, d = 768 (79 tiles in the last round), 2048 rows, fp32: full rounds, tail kernel and its sum 98 + 27 + 17 us; half tiles in a
+// launch of their own 98 + 28; like this 108.  d = 1024 (20 tiles), bf16: 2048 rows 114 + 13 + 10, 114 + 23, 115; 4096 rows 192 + 17 + 10
+// and 200; 8192 rows 302 + 24 + 12 for 345; 32768 rows 1128 + 61 + 20 for 1379.  d = 1600 (99 tiles), 4096 rows 281 + 45 + 16 and 309.
+// So it is a matter of kp, the pairs of K blocks, and of n, the tiles of the last round, which the K-split cuts into 256 / n
+// parts: as lines, tail kernel and sum 18 + n / 4 + kp (0.25 + n / 70), this 1.3 kp and next to nothing (dw_tail_plan).
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o) {
+__global__ __launch_bounds__(256) void bwd_dw_out_kernel(DwParams p, DwOut o, int tile0, int nhalf, int half_grid) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   int rt, ct;
-  if (!map_tile_rr(blockIdx.x, p.RT, p.CT, rt, ct)) return;
+  if ((int)blockIdx.x < half_grid) {
+    int lin, none;
+    if (!map_tile(blockIdx.x, 1, nhalf, none, lin)) return;
+    tile_from_index(tile0 + (lin >> 1), p.RT, p.CT, rt, ct);
+    rt = __builtin_amdgcn_readfirstlane(rt); ct = __builtin_amdgcn_readfirstlane(ct);
+    dw_out_tile<T, 2>(p, o, smem, 2 * rt + (lin & 1), ct);
+    return;
+  }
+  if (!map_tile_rr(blockIdx.x - half_grid, p.RT, p.CT, rt, ct)) return;
   dw_out_tile<T, 4>(p, o, smem, rt, ct);
-}
-
-// The tiles of a last round that would leave more than half of the CUs idle, 128 rows to a workgroup: tiles tile0 .. tile0 + ntail - 1
-// of the round-robin order, two workgroups each, neighbours on one XCD (their columns of G are the same).
-// No partial sums and no launch to add them up, but a K loop as long as a whole tile's with half its MFMAs.  Measured, tail kernel and
-// its sum against this, V = 50304: d = 768 (79 tiles in the last round) 2048 rows of fp32 43 -> 27 us, 4096 60 -> 39, bf16 8192 80 -> 60,
-// 16384 123 -> 103; d = 1600 (99 tiles) 4096 rows 63 -> 36, 8192 94 -> 57; d = 1024 (20 tiles) 300 rows 16 -> 15, 2048 25 -> 23, 4096 29 for 34,
-// 16384 55 for 94.  As lines over kp, the pairs of K blocks, and n tiles: tail 18 + n / 4 + kp (0.25 + n / 70), this 14.5 + 1.3 kp
-// (dw_tail_plan).
-template <typename T>
-__global__ __launch_bounds__(256) void bwd_dw_half_kernel(DwParams p, DwOut o, int tile0, int ntail) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  int lin, none, rt, ct;
-  if (!map_tile(blockIdx.x, 1, 2 * ntail, none, lin)) return;
-  tile_from_index(tile0 + (lin >> 1), p.RT, p.CT, rt, ct);
-  rt = __builtin_amdgcn_readfirstlane(rt); ct = __builtin_amdgcn_readfirstlane(ct);
-  dw_out_tile<T, 2>(p, o, smem, 2 * rt + (lin & 1), ct);
 }
 
 // The same from fp32 partials: what is left are the tiles of a K-split last round (tl.tile0 >= 0: grid.y = tl.ntail tiles of

@@ -987,6 +987,8 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
   }
   __syncthreads();               // also: every wave of this block has read its partial records
   float lse = 0.f;
+  double sum = 0.0;                                              // of this block and in the end of all, in thread 0
+  int cnt = 0, bad = 0;
   if (g < n_predict && i < N) {
     float sum = 0.f;
 #pragma unroll
@@ -1005,8 +1007,6 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
     s_zy[(int64_t)g * Np + i] = zy;
     rl[g][r] = l;
     if (g == 0) {
-      double term = 0.0;
-      int cnt = 0, bad = 0;
       s_lse[i] = lse;
       if (i < N) {
         if (lse_out) lse_out[i] = lse;
@@ -1020,18 +1020,21 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
         const int64_t y = targets[i];
         if (y != ignore_index) {
           if (y < 0 || y >= V) bad = 1;
-          else { term = (double)(lse - zy); cnt = 1; }
+          else { sum = (double)(lse - zy); cnt = 1; }
         }
       }
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) { term += __shfl_xor(term, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
+      for (int o = 32; o > 0; o >>= 1) { sum += __shfl_xor(sum, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
       if (r == 0) {
-        uint64_t* slot = reinterpret_cast<uint64_t*>(partials + (int64_t)blockIdx.x * COMBINE_ROWS);
-        const uint64_t counts = (uint64_t)(uint32_t)cnt | ((uint64_t)(uint32_t)bad << 32);
-        __hip_atomic_store(slot, (uint64_t)__double_as_longlong(term), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(slot + 1, counts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (gridDim.x > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // both have arrived
-        last = gridDim.x == 1 || __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hdr + HDR_COUNT_OFF), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        last = gridDim.x == 1;
+        if (!last) {
+          uint64_t* slot = reinterpret_cast<uint64_t*>(partials + (int64_t)blockIdx.x * COMBINE_ROWS);
+          const uint64_t counts = (uint64_t)(uint32_t)cnt | ((uint64_t)(uint32_t)bad << 32);
+          __hip_atomic_store(slot, (uint64_t)__double_as_longlong(sum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_store(slot + 1, counts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // both have arrived
+          last = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hdr + HDR_COUNT_OFF), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        }
       }
     }
   }
@@ -1043,22 +1046,24 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
     if (probability) probability[i] = row_probability(l, targets[i], ignore_index);
   }
   if (!last) return;
-  double sum = 0.0;
-  int cnt = 0, bad = 0;
-  for (int b = threadIdx.x; b < (int)gridDim.x; b += COMBINE_ROWS * G) {      // (of one block, thread 0 reads what it stored)
-    const uint64_t* slot = reinterpret_cast<const uint64_t*>(partials + (int64_t)b * COMBINE_ROWS);
-    sum += __longlong_as_double((long long)__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    const uint64_t c = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    cnt += (int)(uint32_t)c; bad += (int)(uint32_t)(c >> 32);
-  }
+  if (gridDim.x > 1) {
+    __shared__ double wsum[G];
+    __shared__ int wcnt[G], wbad[G];
+    sum = 0.0; cnt = 0; bad = 0;
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += COMBINE_ROWS * G) {
+      const uint64_t* slot = reinterpret_cast<const uint64_t*>(partials + (int64_t)b * COMBINE_ROWS);
+      sum += __longlong_as_double((long long)__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      const uint64_t c = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      cnt += (int)(uint32_t)c; bad += (int)(uint32_t)(c >> 32);
+    }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) { sum += __shfl_xor(sum, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
-  __shared__ double wsum[G];
-  __shared__ int wcnt[G], wbad[G];
-  if (r == 0) { wsum[g] = sum; wcnt[g] = cnt; wbad[g] = bad; }
-  __syncthreads();
+    for (int o = 32; o > 0; o >>= 1) { sum += __shfl_xor(sum, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
+    if (r == 0) { wsum[g] = sum; wcnt[g] = cnt; wbad[g] = bad; }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int w = 1; w < G; ++w) { sum += wsum[w]; cnt += wcnt[w]; bad += wbad[w]; }
+  }
   if (threadIdx.x != 0) return;
-  for (int w = 1; w < G; ++w) { sum += wsum[w]; cnt += wcnt[w]; bad += wbad[w]; }
   const float mean = (float)(sum / (double)cnt);                 // 0/0 = NaN, as F.cross_entropy gives
   int32_t* head = reinterpret_cast<int32_t*>(hdr);
   head[0] = cnt; head[1] = bad;

@@ -160,8 +160,6 @@ static int check_device(int dev) {
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_tail_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
-      HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_half_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
-      HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_half_kernel<bf16_t>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_out_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       HIP_TRY(hipFuncSetAttribute((const void*)bwd_dw_out_kernel<bf16_t>, hipFuncAttributeMaxDynamicSharedMemorySize, SMEM_MAX));
       void* sp = nullptr;
@@ -206,7 +204,7 @@ constexpr size_t DX_PART_BYTES = (size_t)256 * 256 * 256 * 4;
 constexpr int DW_TAIL_WGS = 256;
 struct DwTailPlan {
   int full, ntail, kp, share;      // tiles in full rounds, tiles of the last round, pairs of K blocks per tile and per workgroup
-  bool half;                       // 128 rows to a workgroup instead (bwd_dw_half_kernel)
+  bool half;                       // 128 rows to a workgroup instead (bwd_dw_out_kernel)
   bool use;                        // measured: worth it when the shared-out round is at most half a tile long per workgroup
   size_t bytes;                    // partial tiles: one per (workgroup, tile it touches)
 };
@@ -218,7 +216,7 @@ static DwTailPlan dw_tail_plan(int64_t dq, int64_t Vp, int64_t krows) {
   t.ntail = tiles - t.full;
   t.share = t.ntail > 0 ? (int)(((int64_t)t.ntail * t.kp + DW_TAIL_WGS - 1) / DW_TAIL_WGS) : 0;
   t.use = t.ntail > 0 && t.share >= 1 && t.share * 2 <= t.kp;
-  t.half = t.ntail > 0 && 2 * t.ntail <= DW_TAIL_WGS && t.kp * (74 - t.ntail) < 250 + 18 * t.ntail;
+  t.half = t.ntail > 0 && 2 * t.ntail <= DW_TAIL_WGS && t.kp * (74 - t.ntail) < 1300 + 18 * t.ntail;
   t.bytes = t.use ? (size_t)(DW_TAIL_WGS + t.ntail) * 256 * 256 * 4 : 0;
   return t;
 }
@@ -865,15 +863,10 @@ extern "C" int sce_backward(const sce_args* a) {
       if (B.one) {                       // (then w0 = 0, and this is the last launch as well as the first)
         const bool half = tp.half;
         const bool share = !half && tp.use && B.tail_bytes >= tp.bytes && a->workspace_bytes >= B.off_dwtail + tp.bytes;
-        const int grid = share || half ? tp.full : map_tile_rr_grid(CTd, CTv);
+        const int hgrid = half ? map_tile_grid(1, 2 * tp.ntail) : 0, grid = hgrid + (share || half ? tp.full : map_tile_rr_grid(CTd, CTv));
         if (grid > 0) {
-          if (dw_f32) bwd_dw_out_kernel<float><<<grid, NTHREADS, SMEM_MAX, st>>>(wp, wo);
-          else bwd_dw_out_kernel<bf16_t><<<grid, NTHREADS, SMEM_MAX, st>>>(wp, wo);
-        }
-        if (half) {
-          const int hgrid = map_tile_grid(1, 2 * tp.ntail);
-          if (dw_f32) bwd_dw_half_kernel<float><<<hgrid, NTHREADS, SMEM_MAX, st>>>(wp, wo, tp.full, tp.ntail);
-          else bwd_dw_half_kernel<bf16_t><<<hgrid, NTHREADS, SMEM_MAX, st>>>(wp, wo, tp.full, tp.ntail);
+          if (dw_f32) bwd_dw_out_kernel<float><<<grid, NTHREADS, SMEM_MAX, st>>>(wp, wo, tp.full, 2 * tp.ntail, hgrid);
+          else bwd_dw_out_kernel<bf16_t><<<grid, NTHREADS, SMEM_MAX, st>>>(wp, wo, tp.full, 2 * tp.ntail, hgrid);
         }
         if (share) {
           tail.buf = (float*)(ws + B.off_dwtail); tail.tile0 = tp.full; tail.ntail = tp.ntail; tail.kp = tp.kp; tail.share = tp.share;
