@@ -76,12 +76,12 @@ __device__ __forceinline__ Scaler make_scaler(float inv_host, const float* scale
   return sc;
 }
 
-// Scale-derived constants when a scale lives on the device (sce_args.x_s_dev / w_s_dev): written by dev_consts_kernel
+// Scale-derived constants when a scale lives on the device (sce_args.x_s_dev / w_s_dev): written by quantize_operands_kernel
 // into the header of the saved state, read by every kernel that needs them in place of its by-value copies.
 struct DevConsts {
   float x_s, w_s, sc, k1;      // sc = x_s w_s; k1 = sc 2 log2(e) / cap
 };
-__global__ void dev_consts_kernel(const float* xs_dev, const float* ws_dev, float xs_host, float ws_host, float cap, DevConsts* out) {
+__device__ __forceinline__ void dev_consts(const float* xs_dev, const float* ws_dev, float xs_host, float ws_host, float cap, DevConsts* out) {
   DevConsts c;
   c.x_s = xs_dev ? *xs_dev : xs_host;
   c.w_s = ws_dev ? *ws_dev : ws_host;

@@ -541,30 +541,24 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
       else if (a->w_dtype == SCE_BF16) prep_w_bf16_kernel<bf16_t><<<gw, 256, 0, st>>>((const bf16_t*)a->w, a->w_ld, d, V, (uint16_t*)wqt, S.ldx / 2);
       else return fail(SCE_EINVAL, "unsupported w dtype %d", a->w_dtype);
     }
-    if (devsc && !bf16ops) dev_consts_kernel<<<1, 1, 0, st>>>(a->x_s_dev, a->w_s_dev, (float)a->x_s, (float)a->w_s, a->cap, dcp);
-    const int grid = grid_for((size_t)S.Np * (S.dp / 16), 256);
-    float* rstd = (float*)(sv + S.off_rstd);
-    const int ngrid = (int)((S.Np + 3) / 4);
-    if (bf16ops) {
-      // operands laid out above
-    } else if (a->norm && a->x_dtype == SCE_F32)
-      rmsnorm_quantize_kernel<float><<<ngrid, 256, 0, st>>>((const float*)a->x, a->x_ld, N, d, a->norm_eps, xq, S.Np, S.dp, S.ldx, inv_xs, a->x_s_dev, rstd);
-    else if (a->norm && a->x_dtype == SCE_BF16)
-      rmsnorm_quantize_kernel<bf16_t><<<ngrid, 256, 0, st>>>((const bf16_t*)a->x, a->x_ld, N, d, a->norm_eps, xq, S.Np, S.dp, S.ldx, inv_xs, a->x_s_dev, rstd);
-    else if (a->x_dtype == SCE_F32)
-      quantize_pad_kernel<float><<<grid, 256, 0, st>>>((const float*)a->x, a->x_ld, N, d, xq, S.Np, S.dp, S.ldx, inv_xs, a->x_s_dev);
-    else if (a->x_dtype == SCE_BF16)
-      quantize_pad_kernel<bf16_t><<<grid, 256, 0, st>>>((const bf16_t*)a->x, a->x_ld, N, d, xq, S.Np, S.dp, S.ldx, inv_xs, a->x_s_dev);
-    else return fail(SCE_EINVAL, "unsupported x dtype %d", a->x_dtype);
-    dim3 gw((unsigned)(S.Vp / QW_TILE), (unsigned)(S.dq / QW_TILE));
-    if (bf16ops) {
-    } else if (a->wcache && a->wcache_valid) {
-      // the caller vouches that the cache holds e4m3(W / w_s) of this W (unchanged since an earlier call)
-    } else if (a->w_dtype == SCE_F32)
-      quantize_w_kernel<float><<<gw, 256, 0, st>>>((const float*)a->w, a->w_ld, d, V, wq, wqt, S.dp, S.ldx, S.Vp / BK, inv_ws, a->w_s_dev);
-    else if (a->w_dtype == SCE_BF16)
-      quantize_w_kernel<bf16_t><<<gw, 256, 0, st>>>((const bf16_t*)a->w, a->w_ld, d, V, wq, wqt, S.dp, S.ldx, S.Vp / BK, inv_ws, a->w_s_dev);
-    else return fail(SCE_EINVAL, "unsupported w dtype %d", a->w_dtype);
+    if (!bf16ops) {
+      const bool w_there = a->wcache && a->wcache_valid;      // the caller vouches that the cache holds e4m3(W / w_s) of this W (unchanged since an earlier call)
+      const auto bad = [](int32_t t) { return t != SCE_F32 && t != SCE_BF16; };
+      if (bad(a->x_dtype)) return fail(SCE_EINVAL, "unsupported x dtype %d", a->x_dtype);
+      if (!w_there && bad(a->w_dtype)) return fail(SCE_EINVAL, "unsupported w dtype %d", a->w_dtype);
+      QuantizeParams q;
+      q.x = a->x; q.x_ld = a->x_ld; q.N = N; q.d = d; q.Np = S.Np; q.dp = S.dp; q.ldx = S.ldx; q.xq = xq;
+      q.rstd = a->norm ? (float*)(sv + S.off_rstd) : nullptr; q.eps = a->norm_eps; q.inv_xs = inv_xs; q.inv_ws = inv_ws; q.xs_dev = a->x_s_dev; q.ws_dev = a->w_s_dev;
+      q.nx = a->norm ? (int)((S.Np + 3) / 4) : grid_for((size_t)S.Np * (S.dp / 16), 256);
+      q.w = a->w; q.w_ld = a->w_ld; q.V = V; q.kbv = S.Vp / BK; q.nv = (int)(S.Vp / QW_TILE); q.wq = wq; q.wqt = wqt;
+      q.dc = dcp; q.xs_host = (float)a->x_s; q.ws_host = (float)a->w_s; q.cap = a->cap;
+      const unsigned grid = (unsigned)q.nx + (w_there ? 0u : (unsigned)q.nv * (unsigned)(S.dq / QW_TILE));
+      const bool xf = a->x_dtype == SCE_F32, wf = !w_there && a->w_dtype == SCE_F32;
+      if (xf && wf) quantize_operands_kernel<float, float><<<grid, 256, 0, st>>>(q);
+      else if (xf) quantize_operands_kernel<float, bf16_t><<<grid, 256, 0, st>>>(q);
+      else if (wf) quantize_operands_kernel<bf16_t, float><<<grid, 256, 0, st>>>(q);
+      else quantize_operands_kernel<bf16_t, bf16_t><<<grid, 256, 0, st>>>(q);
+    }
   }
   const bool emit = a->dlogits_from_forward != 0;
   const int CTw = emit ? (int)(S.Vp / 256) : CT;       // with the dlogits every tile is visited: the masked ones must read as zero later

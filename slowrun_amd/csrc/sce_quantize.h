@@ -46,15 +46,13 @@ __device__ __forceinline__ bool rows_aligned(const T* p, int64_t ld) { return ((
 // dst [rows_p][cols_p] e4m3 = src [rows][cols] / s, zero outside; 16 outputs per thread.  In all the quantising
 // kernels inv_scale is the reciprocal 1 / s taken once on the host, or, with scale_dev, s is read from the device.
 template <typename T>
-__global__ __launch_bounds__(256) void quantize_pad_kernel(const T* __restrict__ src, int64_t ld, int64_t rows,
-                                                          int64_t cols, uint8_t* __restrict__ dst,
-                                                          int64_t rows_p, int64_t cols_p, int64_t dst_ld, float inv_scale,
-                                                          const float* __restrict__ scale_dev) {
+__device__ __forceinline__ void quantize_pad(int block, int nblocks, const T* __restrict__ src, int64_t ld, int64_t rows, int64_t cols, uint8_t* __restrict__ dst,
+                                             int64_t rows_p, int64_t cols_p, int64_t dst_ld, float inv_scale, const float* __restrict__ scale_dev) {
   const Scaler scale = make_scaler<T>(inv_scale, scale_dev);
   const int64_t chunks_per_row = cols_p / 16;
   const int64_t total = rows_p * chunks_per_row;
   auto walk = [&](auto any) {
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t q = (int64_t)block * 256 + threadIdx.x; q < total; q += (int64_t)nblocks * 256) {
       const int64_t r = q / chunks_per_row, c0 = (q - r * chunks_per_row) * 16;
       uint32_t out[4] = {0, 0, 0, 0};
       if (r < rows && c0 < cols) {
@@ -79,13 +77,12 @@ __device__ __forceinline__ float wave_sum(float v) {
 // dst row = e4m3(round_T(h * rstd) / scale) with rstd = 1 / sqrt(mean(h^2) + eps), the normalised row rounded to
 // the input's type as the unfused path has it in memory.  One wave per row; rstd is kept for backward.
 template <typename T>
-__global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const T* __restrict__ src, int64_t ld, int64_t rows,
-                                                              int64_t cols, float eps, uint8_t* __restrict__ dst,
-                                                              int64_t rows_p, int64_t cols_p, int64_t dst_ld, float inv_scale,
-                                                              const float* __restrict__ scale_dev, float* __restrict__ rstd_out) {
+__device__ __forceinline__ void rmsnorm_quantize(int block, const T* __restrict__ src, int64_t ld, int64_t rows, int64_t cols, float eps, uint8_t* __restrict__ dst,
+                                                 int64_t rows_p, int64_t cols_p, int64_t dst_ld, float inv_scale, const float* __restrict__ scale_dev,
+                                                 float* __restrict__ rstd_out) {
   const Scaler scale = make_scaler<T>(inv_scale, scale_dev), one = {1.0f, false};
   const int lane = threadIdx.x & 63;
-  const int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int64_t r = (int64_t)block * 4 + (threadIdx.x >> 6);
   if (r >= rows_p) return;
   const int64_t chunks = cols_p / 16;
   if (r >= rows) {
@@ -206,15 +203,13 @@ constexpr int BLOCKED_KSTEP = 256 * BK;     // bytes from one K block of a tile 
 // every piece of a row that a workgroup reads or writes is at least 128 bytes long (with 64 x 64 tiles and 64-byte
 // pieces the kernel reached 3.5 TB/s at V = 131072).
 constexpr int QW_TILE = 128;
+typedef uint8_t QwTile[QW_TILE][QW_TILE + 4];
 template <typename T>
-__global__ __launch_bounds__(256) void quantize_w_kernel(const T* __restrict__ w, int64_t ld, int64_t d, int64_t V,
-                                                        uint8_t* __restrict__ wq, uint8_t* __restrict__ wqt,
-                                                        int64_t dp, int64_t ldx, int64_t kbv, float inv_scale,
-                                                        const float* __restrict__ scale_dev) {
+__device__ __forceinline__ void quantize_w(QwTile& tile, int bx, int by, const T* __restrict__ w, int64_t ld, int64_t d, int64_t V, uint8_t* __restrict__ wq,
+                                           uint8_t* __restrict__ wqt, int64_t dp, int64_t ldx, int64_t kbv, float inv_scale, const float* __restrict__ scale_dev) {
   const Scaler scale = make_scaler<T>(inv_scale, scale_dev);
-  __shared__ uint8_t tile[QW_TILE][QW_TILE + 4];
   const int t = threadIdx.x;
-  const int64_t j0 = (int64_t)blockIdx.y * QW_TILE, v0 = (int64_t)blockIdx.x * QW_TILE;
+  const int64_t j0 = (int64_t)by * QW_TILE, v0 = (int64_t)bx * QW_TILE;
   if (sizeof(T) == 4 && v0 + QW_TILE <= V && ((reinterpret_cast<uintptr_t>(w) | (uintptr_t)(ld * 4)) & 15) == 0) {
     // fp32: four elements a load, so that a wave reads 512 bytes of a row in a row (with 16 a thread its loads lay 64 bytes
     // apart: 3.2 TB/s at d = 768)
@@ -265,6 +260,37 @@ __global__ __launch_bounds__(256) void quantize_w_kernel(const T* __restrict__ w
       *reinterpret_cast<v4i*>(wqt + (v0 + vr) * ldx + j0 + jc) = (v4i){(int)out[0], (int)out[1], (int)out[2], (int)out[3]};
     }
   }
+}
+
+// Both operands of the fp8 head in one launch: workgroups [0, nx) the rows of X, with the final norm or without, the rest the tiles of W
+// (there are none with a weight cache that is filled already).  The first one also leaves what follows from scales on the device in the
+// header (dc, or NULL).  Neither operand needs the other, and on few rows X is all launch and latency.  Measured, in launches of their own
+// (quantize_pad_kernel or with the norm rmsnorm_quantize_kernel, quantize_w_kernel, one of one thread for dc) and like this: 2048 rows, d = 768, fp32, V = 50304
+// 5.6 + 53 and 54 us; 4096 rows, d = 1600 with norm and device scales 4 + 13 + 65 and 74; 1000 rows, d = 256, V = 4096 5.1 + 8.3
+// and 10; 30011 rows, d = 2560 41 + 91 and 127; 2048 rows, d = 1024 with the weight's bytes from a cache 6.5 either way.
+struct QuantizeParams {
+  const void* x;
+  int64_t x_ld, N, d, Np, dp, ldx;
+  uint8_t* xq;
+  float* rstd;                 // non-NULL: the norm is part of the call
+  float eps, inv_xs, inv_ws;
+  const float *xs_dev, *ws_dev;
+  int nx;
+  const void* w;
+  int64_t w_ld, V, kbv;
+  int nv;                      // tiles of W side by side
+  uint8_t *wq, *wqt;
+  DevConsts* dc;
+  float xs_host, ws_host, cap;
+};
+template <typename TX, typename TW>
+__global__ __launch_bounds__(256) void quantize_operands_kernel(QuantizeParams p) {
+  __shared__ QwTile tile;
+  const int b = blockIdx.x;
+  if (b == 0 && threadIdx.x == 0 && p.dc) dev_consts(p.xs_dev, p.ws_dev, p.xs_host, p.ws_host, p.cap, p.dc);
+  if (b >= p.nx) quantize_w<TW>(tile, (b - p.nx) % p.nv, (b - p.nx) / p.nv, (const TW*)p.w, p.w_ld, p.d, p.V, p.wq, p.wqt, p.dp, p.ldx, p.kbv, p.inv_ws, p.ws_dev);
+  else if (p.rstd) rmsnorm_quantize<TX>(b, (const TX*)p.x, p.x_ld, p.N, p.d, p.eps, p.xq, p.Np, p.dp, p.ldx, p.inv_xs, p.xs_dev, p.rstd);
+  else quantize_pad<TX>(b, p.nx, (const TX*)p.x, p.x_ld, p.N, p.d, p.xq, p.Np, p.dp, p.ldx, p.inv_xs, p.xs_dev);
 }
 
 // bf16 operands (the eval head, tiny/train.py:741 under bf16 autocast): no quantisation, only the layout.
