@@ -608,7 +608,7 @@ struct FoldParams {
   const int32_t *longlist, *longbase, *segoff;
   float* longsum;
   int64_t dq;
-  int slots, first;            // first: the first workgroup of the grid that folds
+  int slots;
 };
 __device__ __forceinline__ void fold_chunks(const FoldParams& f, int block, int nblocks) {
   const int ny = (int)(f.dq / 256), items = f.longlist[2] * ny;
@@ -630,17 +630,121 @@ __device__ __forceinline__ void fold_chunks(const FoldParams& f, int block, int 
 }
 __global__ __launch_bounds__(256) void bwd_dw_fold_kernel(FoldParams f) { fold_chunks(f, blockIdx.x, gridDim.x); }
 
+// One-hot part of dW for the long columns: longsum[slot][:] = sum over the column's (or the chunk's) rows of h_i X_q[i, :], 256 rows
+// of dW at a time (by).  What bounds it is the latency of the gathered rows, of which 16 lanes read 256 bytes: a
+// wave has four rows' worth of lanes and eight loads in flight in each.  A chunk is a workgroup's, folded in LDS in a fixed order; a
+// column of up to LONG_WAVE rows is one wave's, without a barrier (a workgroup each, with most of its lanes idle, took the many
+// columns of 8 to 15 rows of a mid-sized vocabulary 138 us at 50000 rows of three offsets, d = 1024, V = 16384: now 53; LONG_WAVE = 64
+// is faster there and at 48 rows a column, 16 for 22 us, but a wave's second round of loads is 2 us of a small step).  The grid is a
+// fixed one that walks the lists, whose lengths the host does not know.  The result does not depend on scheduling.
+constexpr int LONG_GRID = 1024, FOLD_GRID = 512;
+struct LongParams {
+  const int32_t* longlist;
+  int slots;
+  const int32_t *segoff, *srow;
+  const float* sh;
+  const uint8_t* xq;
+  int64_t ldx, dq;
+  const int32_t* longbase;
+  float* longsum;
+  int gx;                      // workgroups that walk the lists, for each 256 rows of dW
+};
+typedef float LongShared[16][256];
+__device__ __forceinline__ void dw_long(LongShared& red, int bx, int by, const LongParams& p) {
+  const auto &longlist = p.longlist, &segoff = p.segoff, &srow = p.srow, &longbase = p.longbase;
+  const auto& sh = p.sh;
+  const int slots = p.slots;
+  const int64_t ldx = p.ldx, dq = p.dq;
+  float* longsum = p.longsum;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = t & 15, rl = t >> 4, q = lane >> 4;
+  const int64_t jb = (int64_t)by * 256;
+  const uint8_t* xcol = p.xq + jb + c * 16;
+  // a[m] = sum over entries first, first + stride, ... of the L from s0 on, in that order, of the lane's 16 rows of dW
+  auto rows = [&](int s0, int L, int first, int stride, float (&a)[16]) {
+#pragma unroll
+    for (int m = 0; m < 16; ++m) a[m] = 0.f;
+    for (int n0 = first; n0 < L; n0 += stride * 8) {
+      v4i raw[8];
+      float h[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int n = n0 + stride * u;
+        h[u] = n < L ? sh[s0 + n] : 0.f;
+        raw[u] = *reinterpret_cast<const v4i*>(xcol + (int64_t)srow[n < L ? s0 + n : s0] * ldx);
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {        // rows in ascending order within a row-lane
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const uint32_t w = (uint32_t)raw[u][m];
+          a[4 * m + 0] = fmaf(h[u], e4m3_to_float<0>(w), a[4 * m + 0]);
+          a[4 * m + 1] = fmaf(h[u], e4m3_to_float<1>(w), a[4 * m + 1]);
+          a[4 * m + 2] = fmaf(h[u], e4m3_to_float<2>(w), a[4 * m + 2]);
+          a[4 * m + 3] = fmaf(h[u], e4m3_to_float<3>(w), a[4 * m + 3]);
+        }
+      }
+    }
+  };
+  float a[16];
+  const int nwave = longlist[0], nchunk = longlist[1];
+  for (int i = bx; i < nchunk; i += p.gx) {
+    const int slot = slots - 1 - i, v = longlist[3 + slot], ch = slot - longbase[v];
+    int nch, len;
+    const int seg0 = segoff[v], seg1 = segoff[v + 1];
+    long_chunks(seg1 - seg0, nch, len);
+    const int s0 = seg0 + ch * len;
+    rows(s0, min(seg1 - s0, len), rl, 16, a);
+#pragma unroll
+    for (int m = 0; m < 16; ++m) red[rl][c * 16 + m] = a[m];
+    __syncthreads();
+    float sfold = 0.f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) sfold += red[k][t];
+    longsum[(int64_t)slot * dq + jb + t] = sfold;
+    __syncthreads();                       // `red` is written again for the next chunk
+  }
+  // (from the other end of the grid: while there are workgroups without a chunk, none has both to do one behind the other)
+  for (int slot = (p.gx - 1 - bx) * 4 + wave; slot < nwave; slot += p.gx * 4) {
+    const int v = longlist[3 + slot], s0 = segoff[v];
+    rows(s0, segoff[v + 1] - s0, q, 4, a);
+#pragma unroll
+    for (int m = 0; m < 16; ++m) {         // over the four row lanes, pairwise; all of them get it
+      a[m] += __shfl_xor(a[m], 16);
+      a[m] += __shfl_xor(a[m], 32);
+    }
+    v4f mine;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) mine[m] = q == 0 ? a[m] : q == 1 ? a[4 + m] : q == 2 ? a[8 + m] : a[12 + m];
+    *reinterpret_cast<v4f*>(longsum + (int64_t)slot * dq + jb + c * 16 + q * 4) = mine;
+  }
+}
+__global__ __launch_bounds__(256, 5) void bwd_dw_long_kernel(LongParams p) {
+  __shared__ LongShared red;
+  dw_long(red, blockIdx.x, blockIdx.y, p);
+}
+
 // Sum of the K-split partials, row scale, one-hot term, cast: a workgroup per 32 rows x 128 columns, a wave per 32 of the
 // columns.  A thread's values are four quads of one row; they go out through LDS as whole pieces of rows.
+// The first `riders` workgroups do work that only the kernels storing dW wait for, beside a kernel that is bound by the
+// bandwidth of its partial sums: the sums of the long columns themselves (lng.gx > 0: a call of few entries), or, of a larger call, the folding
+// of those of several chunks.  Two micro-batches of 2048 rows of Zipf targets, d = 1024: the sums in a launch of their own 18.8 and this kernel
+// 29.9 us, together 39.2; 4096 rows, d = 1600 10.5 + 18.1, 24.0; 1000 rows, d = 256, V = 4096 3.9 + 6.3, 6.1; 2048 rows of uniform targets, which
+// have no long columns, d = 768 4.2 + 14.1, 17.2.  (More than RANK_MAX entries make more chunks to a column than the kernels storing dW
+// should walk, one wave to a SIMD, so there the sums come first and only the folding rides.)
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_dx_finish_kernel(DxParams p_in, FoldParams f) {
-  if ((int)blockIdx.x >= f.first) return fold_chunks(f, blockIdx.x - f.first, gridDim.x - f.first);
+__global__ __launch_bounds__(256) void bwd_dx_finish_kernel(DxParams p_in, FoldParams f, LongParams lng, int riders) {
+  __shared__ __attribute__((aligned(16))) union { LongShared red; uint8_t stage[32 * (128 * sizeof(T) + 16)]; } shared;
+  if ((int)blockIdx.x < riders) {
+    if (lng.gx > 0) return dw_long(shared.red, blockIdx.x % lng.gx, blockIdx.x / lng.gx, lng);
+    return fold_chunks(f, blockIdx.x, riders);
+  }
   DxParams p = p_in;
   if (p.dc) p.w_s = p.dc->w_s;
   constexpr int RB = 128 * (int)sizeof(T), PITCH = RB + 16, CH = RB / 16;
-  __shared__ __attribute__((aligned(16))) uint8_t stage[32 * PITCH];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wa = blockIdx.x & 1, b = (blockIdx.x >> 1) & 3, wb = (blockIdx.x >> 3) & 1;
-  const int tile = blockIdx.x >> 4, rt = tile / p.CT, ct = tile - rt * p.CT, i0 = rt * 256 + wb * 128 + b * 32, j0 = ct * 256 + wa * 128;
+  uint8_t* stage = shared.stage;
+  const int bid = blockIdx.x - riders;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, wa = bid & 1, b = (bid >> 1) & 3, wb = (bid >> 3) & 1;
+  const int tile = bid >> 4, rt = tile / p.CT, ct = tile - rt * p.CT, i0 = rt * 256 + wb * 128 + b * 32, j0 = ct * 256 + wa * 128;
   if (i0 >= p.rows || j0 >= p.d) return;
   v4f sum[4];
 #pragma unroll
@@ -858,82 +962,6 @@ __global__ __launch_bounds__(256) void bwd_xt_segments_kernel(XtSegParams p) {
   else column_segments(shared.s, bid - p.nxt, gridDim.x - p.nxt, p.skeys, p.perm, p.hcoef, p.n, p.Np, p.V, p.long_seg, p.slots, p.segoff, p.longlist, p.longbase, p.srow, p.sh);
 }
 
-// One-hot part of dW for the long columns: longsum[slot][:] = sum over the column's (or the chunk's) rows of h_i X_q[i, :], 256 rows
-// of dW at a time (blockIdx.y).  What bounds it is the latency of the gathered rows, of which 16 lanes read 256 bytes: a
-// wave has four rows' worth of lanes and eight loads in flight in each.  A chunk is a workgroup's, folded in LDS in a fixed order; a
-// column of up to LONG_WAVE rows is one wave's, without a barrier (a workgroup each, with most of its lanes idle, took the many
-// columns of 8 to 15 rows of a mid-sized vocabulary 138 us at 50000 rows of three offsets, d = 1024, V = 16384: now 53; LONG_WAVE = 64
-// is faster there and at 48 rows a column, 16 for 22 us, but a wave's second round of loads is 2 us of a small step).  The grid is a
-// fixed one that walks the lists, whose lengths the host does not know.  The result does not depend on scheduling.
-constexpr int LONG_GRID = 1024, FOLD_GRID = 512;
-__global__ __launch_bounds__(256, 5) void bwd_dw_long_kernel(const int32_t* __restrict__ longlist, int slots, const int32_t* __restrict__ segoff,
-                                                         const int32_t* __restrict__ srow, const float* __restrict__ sh,
-                                                         const uint8_t* __restrict__ xq, int64_t ldx, int64_t dq,
-                                                         const int32_t* __restrict__ longbase, float* __restrict__ longsum) {
-  __shared__ float red[16][256];
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, c = t & 15, rl = t >> 4, q = lane >> 4;
-  const int64_t jb = (int64_t)blockIdx.y * 256;
-  const uint8_t* xcol = xq + jb + c * 16;
-  // a[m] = sum over entries first, first + stride, ... of the L from s0 on, in that order, of the lane's 16 rows of dW
-  auto rows = [&](int s0, int L, int first, int stride, float (&a)[16]) {
-#pragma unroll
-    for (int m = 0; m < 16; ++m) a[m] = 0.f;
-    for (int n0 = first; n0 < L; n0 += stride * 8) {
-      v4i raw[8];
-      float h[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int n = n0 + stride * u;
-        h[u] = n < L ? sh[s0 + n] : 0.f;
-        raw[u] = *reinterpret_cast<const v4i*>(xcol + (int64_t)srow[n < L ? s0 + n : s0] * ldx);
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {        // rows in ascending order within a row-lane
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          const uint32_t w = (uint32_t)raw[u][m];
-          a[4 * m + 0] = fmaf(h[u], e4m3_to_float<0>(w), a[4 * m + 0]);
-          a[4 * m + 1] = fmaf(h[u], e4m3_to_float<1>(w), a[4 * m + 1]);
-          a[4 * m + 2] = fmaf(h[u], e4m3_to_float<2>(w), a[4 * m + 2]);
-          a[4 * m + 3] = fmaf(h[u], e4m3_to_float<3>(w), a[4 * m + 3]);
-        }
-      }
-    }
-  };
-  float a[16];
-  const int nwave = longlist[0], nchunk = longlist[1];
-  for (int i = blockIdx.x; i < nchunk; i += gridDim.x) {
-    const int slot = slots - 1 - i, v = longlist[3 + slot], ch = slot - longbase[v];
-    int nch, len;
-    const int seg0 = segoff[v], seg1 = segoff[v + 1];
-    long_chunks(seg1 - seg0, nch, len);
-    const int s0 = seg0 + ch * len;
-    rows(s0, min(seg1 - s0, len), rl, 16, a);
-#pragma unroll
-    for (int m = 0; m < 16; ++m) red[rl][c * 16 + m] = a[m];
-    __syncthreads();
-    float sfold = 0.f;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) sfold += red[k][t];
-    longsum[(int64_t)slot * dq + jb + t] = sfold;
-    __syncthreads();                       // `red` is written again for the next chunk
-  }
-  // (from the other end of the grid: while there are workgroups without a chunk, none has both to do one behind the other)
-  for (int slot = (gridDim.x - 1 - blockIdx.x) * 4 + wave; slot < nwave; slot += gridDim.x * 4) {
-    const int v = longlist[3 + slot], s0 = segoff[v];
-    rows(s0, segoff[v + 1] - s0, q, 4, a);
-#pragma unroll
-    for (int m = 0; m < 16; ++m) {         // over the four row lanes, pairwise; all of them get it
-      a[m] += __shfl_xor(a[m], 16);
-      a[m] += __shfl_xor(a[m], 32);
-    }
-    v4f mine;
-#pragma unroll
-    for (int m = 0; m < 4; ++m) mine[m] = q == 0 ? a[m] : q == 1 ? a[4 + m] : q == 2 ? a[8 + m] : a[12 + m];
-    *reinterpret_cast<v4f*>(longsum + (int64_t)slot * dq + jb + c * 16 + q * 4) = mine;
-  }
-}
-
 // Where the one-hot part of dW comes from and where dW goes (bwd_dw_out_kernel, bwd_dw_final_kernel).
 struct DwOut {
   void* dw;                    // [d][dw_ld], columns [0, V)
@@ -949,7 +977,13 @@ struct DwOut {
   int64_t ldx, dq;
   float x_s;
   int d, V, long_seg;          // long_seg: LONG_SEG wherever bwd_dw_out_kernel runs
+  bool chunks;                 // the chunk sums of a long column are not folded into the first
 };
+__device__ __forceinline__ int long_parts(const DwOut& o, int L) {
+  int nch = 1, len;
+  if (o.chunks && L > LONG_WAVE) long_chunks(L, nch, len);
+  return nch;
+}
 
 // dW straight from the main loop: dW = x_s (xi (X~^T G) - sum over the column's target entries of h_i X_q[i, :]), cast and
 // stored by the workgroup that has the tile in its accumulators.  Used whenever one launch covers all rows: up to 131072 with
@@ -1100,12 +1134,13 @@ __device__ __forceinline__ void dw_out_tile(const DwParams& p, const DwOut& o, u
       if (__builtin_amdgcn_ballot_w64(L >= LONG_SEG) != 0) {
         if (L >= LONG_SEG) {
           const float* ls = o.longsum + (int64_t)o.longbase[v] * o.dq + rt * TROWS + wa * 32 * NA + ah * 64 + 4 * h;
+          for (int c2 = long_parts(o, L); c2 > 0; --c2, ls += o.dq)
 #pragma unroll
-          for (int g = 0; g < 8; ++g) {
-            const v4f s = *reinterpret_cast<const v4f*>(ls + 32 * (g >> 2) + 8 * (g & 3));
+            for (int g = 0; g < 8; ++g) {
+              const v4f s = *reinterpret_cast<const v4f*>(ls + 32 * (g >> 2) + 8 * (g & 3));
 #pragma unroll
-            for (int m = 0; m < 4; ++m) val[4 * g + m] -= s[m] * x_s;
-          }
+              for (int m = 0; m < 4; ++m) val[4 * g + m] -= s[m] * x_s;
+            }
         }
       }
       const int j0 = rt * TROWS + wa * 32 * NA + ah * 64;
@@ -1218,10 +1253,11 @@ __global__ __launch_bounds__(256) void bwd_dw_final_kernel(const float* __restri
   const int s0 = o.segoff[v], L = o.segoff[v + 1] - s0;
   if (L >= o.long_seg) {
     const float* ls = o.longsum + (int64_t)o.longbase[v] * o.dq + j0;
+    for (int c = long_parts(o, L); c > 0; --c, ls += o.dq)
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < 4; ++q)
 #pragma unroll
-      for (int m = 0; m < 4; ++m) val[q][m] -= ls[q * step + m] * x_s;
+        for (int m = 0; m < 4; ++m) val[q][m] -= ls[q * step + m] * x_s;
   } else if (L >= LONG_SEG) {
     // where dW took several launches: the entries' sum first and then x_s, in the order in which a wave of bwd_dw_long_kernel adds
     // them (four row lanes, then the lanes pairwise)

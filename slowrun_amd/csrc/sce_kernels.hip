@@ -773,11 +773,20 @@ extern "C" int sce_backward(const sce_args* a) {
     bwd_xt_segments_kernel<<<q.nxt + segment_blocks(NE, V), 256, 0, st>>>(q);
   }
   delete tm_prep;
-  {
-    KernelTimer tm(SCE_K_DW_FINAL, st);
-    bwd_dw_long_kernel<<<dim3((unsigned)std::min<int64_t>(B.long_slots, LONG_GRID), (unsigned)(S.dq / 256)), 256, 0, st>>>(
-        longlist, (int)B.long_slots, segoff, srow, sh, xq, S.ldx, S.dq, longbase, longsum);
-  }
+  LongParams lng;
+  lng.longlist = longlist; lng.slots = (int)B.long_slots; lng.segoff = segoff; lng.srow = srow; lng.sh = sh; lng.xq = xq; lng.ldx = S.ldx; lng.dq = S.dq;
+  lng.longbase = longbase; lng.longsum = longsum; lng.gx = (int)std::min<int64_t>(B.long_slots, LONG_GRID);
+  // of few entries the sums of the long columns ride with the first finishing kernel of a K-split dX panel, and what stores dW adds a column's chunks
+  const bool few_entries = ranked && B.one;
+  bool summed = false;
+  auto ensure_summed = [&]() {
+    if (!summed) {
+      KernelTimer tm(SCE_K_DW_FINAL, st);
+      bwd_dw_long_kernel<<<dim3((unsigned)lng.gx, (unsigned)(S.dq / 256)), 256, 0, st>>>(lng);
+    }
+    summed = true;
+  };
+  if (!few_entries) ensure_summed();
   const float sc = (float)a->x_s * (float)a->w_s, k1 = sc * 2.0f * LOG2E / a->cap, c2 = -2.0f * a->cap * LOG2E;
   const int CTv = (int)(S.Vp / 256), CTd = (int)(S.dq / 256);
   int launch = 0;
@@ -785,15 +794,16 @@ extern "C" int sce_backward(const sce_args* a) {
   tail.buf = nullptr; tail.tile0 = -1; tail.ntail = 0; tail.kp = 1; tail.share = 1;
   DwOut wo;
   wo.dw = a->dw; wo.dw_ld = a->dw_ld; wo.segoff = segoff; wo.srow = srow; wo.sh = sh; wo.xq = xq; wo.longsum = longsum; wo.longbase = longbase;
-  wo.xi = xi; wo.dc = dcp; wo.ldx = S.ldx; wo.dq = S.dq; wo.x_s = (float)a->x_s; wo.d = (int)d; wo.V = (int)V; wo.long_seg = (int)B.long_seg;
+  wo.xi = xi; wo.dc = dcp; wo.ldx = S.ldx; wo.dq = S.dq; wo.x_s = (float)a->x_s; wo.d = (int)d; wo.V = (int)V; wo.long_seg = (int)B.long_seg; wo.chunks = few_entries;
   const bool dw_f32 = a->dw_dtype == SCE_F32;
   bool dw_done = false;                // every tile is stored, or will be from `tail`
   const bool dx_f32 = a->dx_dtype == SCE_F32;
   FoldParams fold;
-  fold.longlist = longlist; fold.longbase = longbase; fold.segoff = segoff; fold.longsum = longsum; fold.dq = S.dq; fold.slots = (int)B.long_slots; fold.first = 0;
+  fold.longlist = longlist; fold.longbase = longbase; fold.segoff = segoff; fold.longsum = longsum; fold.dq = S.dq; fold.slots = (int)B.long_slots;
   const int fold_blocks = (int)std::min<int64_t>(NE / (LONG_CHUNK + 1) * (S.dq / 256), FOLD_GRID);      // (0: no column can have two chunks)
-  bool folded = fold_blocks == 0;      // launched, with the finishing kernel of a K-split dX panel or by itself
+  bool folded = few_entries || fold_blocks == 0;      // launched, with the finishing kernel of a K-split dX panel or by itself
   auto ensure_folded = [&]() {
+    ensure_summed();
     if (!folded) bwd_dw_fold_kernel<<<fold_blocks, 256, 0, st>>>(fold);
     folded = true;
   };
@@ -828,16 +838,17 @@ extern "C" int sce_backward(const sce_args* a) {
       if (dx_f32) bwd_dx_kernel<float, false><<<map_tile_grid(dp_.RT, CTd), NTHREADS, smem_dx, st>>>(dp_);
       else bwd_dx_kernel<bf16_t, false><<<map_tile_grid(dp_.RT, CTd), NTHREADS, smem_dx, st>>>(dp_);
     } else if (dp_.rows > 0) {
-      FoldParams f = fold;
-      f.first = tiles * 16;
-      const int fgrid = f.first + (folded ? 0 : fold_blocks);
-      folded = true;
+      LongParams l = lng;
+      int riders = folded ? 0 : fold_blocks;
+      if (summed) l.gx = 0; else riders = l.gx * (int)(S.dq / 256);
+      const int fgrid = riders + tiles * 16;
+      folded = summed = true;
       if (dx_f32) {
         bwd_dx_kernel<float, true><<<map_tile_grid(dp_.RT, CTd * ksplit), NTHREADS, smem_dx, st>>>(dp_);
-        bwd_dx_finish_kernel<float><<<fgrid, 256, 0, st>>>(dp_, f);
+        bwd_dx_finish_kernel<float><<<fgrid, 256, 0, st>>>(dp_, fold, l, riders);
       } else {
         bwd_dx_kernel<bf16_t, true><<<map_tile_grid(dp_.RT, CTd * ksplit), NTHREADS, smem_dx, st>>>(dp_);
-        bwd_dx_finish_kernel<bf16_t><<<fgrid, 256, 0, st>>>(dp_, f);
+        bwd_dx_finish_kernel<bf16_t><<<fgrid, 256, 0, st>>>(dp_, fold, l, riders);
       }
     }
   };
