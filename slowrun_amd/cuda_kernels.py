@@ -283,14 +283,33 @@ def ce_backward(saved, targets, grad_output, N, d, V, x_s, w_s, cap, grad_scale,
 # torch.library custom ops, so that a torch.compile'd model (tiny/train.py:1254) traces the loss head
 # as two opaque calls instead of breaking the graph; the reference wraps its kernel the same way
 # (tiny/cuda_kernels.py:314).  The fake implementations only describe shapes and dtypes.
+#
+# A custom op written in Python costs 17 us of host time a call on its way through the dispatcher, and a step of 1000 rows, d = 256,
+# V = 4096 has 89 us of kernels and waits for the host.  So the autograd functions below call the body itself where nothing would see the
+# op: that step 206 -> 183 us.
 # ---------------------------------------------------------------------------------------------
-@torch.library.custom_op("slowrun_amd::ce_forward", mutates_args=())
-def ce_forward_op(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor, mtp_weights: Optional[torch.Tensor],
-                  x_s: float, w_s: float, cap: float, mean: bool, keep: bool,
-                  x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+def _seen_as_op(*tensors):
+    """Whether a call must go through the dispatcher: something traces, records or transforms calls (torch.compile, jit tracing, dispatch
+    and function modes, functorch, the profiler, autograd of a backward pass), or an argument is no plain tensor (a subclass, or a type that
+    the op's schema refuses)."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled():
+        return True
+    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active():
+        return True
+    if torch._C._autograd._profiler_enabled():
+        return True
+    return any(t is not None and type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter for t in tensors)
+
+
+def _ce_forward_body(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor, mtp_weights: Optional[torch.Tensor],
+                     x_s: float, w_s: float, cap: float, mean: bool, keep: bool,
+                     x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     out, saved, _lse, _am, _nv = ce_forward(x, w, targets, x_s if x_s_t is None else x_s_t, w_s if w_s_t is None else w_s_t, cap,
                                             "mean" if mean else "none", mtp_weights=mtp_weights, keep_dlogits=keep)
     return out, saved
+
+
+ce_forward_op = torch.library.custom_op("slowrun_amd::ce_forward", _ce_forward_body, mutates_args=())
 
 
 @ce_forward_op.register_fake
@@ -303,15 +322,17 @@ def _ce_forward_fake(x, w, targets, mtp_weights, x_s, w_s, cap, mean, keep, x_s_
     return out, x.new_empty((sz.saved_bytes + (sz.dlogits_bytes if keep else 0),), dtype=torch.uint8)
 
 
-@torch.library.custom_op("slowrun_amd::ce_backward", mutates_args=())
-def ce_backward_op(saved: torch.Tensor, targets: torch.Tensor, grad_output: torch.Tensor, mtp_weights: Optional[torch.Tensor],
-                   N: int, d: int, V: int, x_s: float, w_s: float, cap: float, grad_scale: float, mean: bool,
-                   x_bf16: bool, w_bf16: bool, keep: bool,
-                   x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+def _ce_backward_body(saved: torch.Tensor, targets: torch.Tensor, grad_output: torch.Tensor, mtp_weights: Optional[torch.Tensor],
+                      N: int, d: int, V: int, x_s: float, w_s: float, cap: float, grad_scale: float, mean: bool,
+                      x_bf16: bool, w_bf16: bool, keep: bool,
+                      x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     return ce_backward(saved, targets, grad_output, N, d, V, x_s if x_s_t is None else x_s_t, w_s if w_s_t is None else w_s_t, cap,
                        grad_scale, "mean" if mean else "none",
                        torch.bfloat16 if x_bf16 else torch.float32, torch.bfloat16 if w_bf16 else torch.float32,
                        mtp_weights=mtp_weights, keep_dlogits=keep)
+
+
+ce_backward_op = torch.library.custom_op("slowrun_amd::ce_backward", _ce_backward_body, mutates_args=())
 
 
 @ce_backward_op.register_fake
@@ -321,29 +342,33 @@ def _ce_backward_fake(saved, targets, grad_output, mtp_weights, N, d, V, x_s, w_
             saved.new_empty((d, V), dtype=torch.bfloat16 if w_bf16 else torch.float32))
 
 
-@torch.library.custom_op("slowrun_amd::norm_ce_forward", mutates_args=())
-def norm_ce_forward_op(h: torch.Tensor, w: torch.Tensor, targets: torch.Tensor, mtp_weights: Optional[torch.Tensor],
-                       x_s: float, w_s: float, cap: float, mean: bool, eps: float, keep: bool,
-                       x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+def _norm_ce_forward_body(h: torch.Tensor, w: torch.Tensor, targets: torch.Tensor, mtp_weights: Optional[torch.Tensor],
+                          x_s: float, w_s: float, cap: float, mean: bool, eps: float, keep: bool,
+                          x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     out, saved, _lse, _am, _nv = ce_forward(h, w, targets, x_s if x_s_t is None else x_s_t, w_s if w_s_t is None else w_s_t, cap,
                                             "mean" if mean else "none", mtp_weights=mtp_weights, norm_eps=eps, keep_dlogits=keep)
     return out, saved
+
+
+norm_ce_forward_op = torch.library.custom_op("slowrun_amd::norm_ce_forward", _norm_ce_forward_body, mutates_args=())
 
 
 norm_ce_forward_op.register_fake(lambda h, w, targets, mtp_weights, x_s, w_s, cap, mean, eps, keep, x_s_t=None, w_s_t=None:
                                  _ce_forward_fake(h, w, targets, mtp_weights, x_s, w_s, cap, mean, keep))
 
 
-@torch.library.custom_op("slowrun_amd::norm_ce_backward", mutates_args=())
-def norm_ce_backward_op(saved: torch.Tensor, h: torch.Tensor, targets: torch.Tensor, grad_output: torch.Tensor,
-                        mtp_weights: Optional[torch.Tensor], V: int, x_s: float, w_s: float, cap: float, grad_scale: float,
-                        mean: bool, w_bf16: bool, eps: float, keep: bool,
-                        x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
+def _norm_ce_backward_body(saved: torch.Tensor, h: torch.Tensor, targets: torch.Tensor, grad_output: torch.Tensor,
+                           mtp_weights: Optional[torch.Tensor], V: int, x_s: float, w_s: float, cap: float, grad_scale: float,
+                           mean: bool, w_bf16: bool, eps: float, keep: bool,
+                           x_s_t: Optional[torch.Tensor] = None, w_s_t: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     N, d = h.shape
     return ce_backward(saved, targets, grad_output, N, d, V, x_s if x_s_t is None else x_s_t, w_s if w_s_t is None else w_s_t, cap,
                        grad_scale, "mean" if mean else "none",
                        h.dtype, torch.bfloat16 if w_bf16 else torch.float32, mtp_weights=mtp_weights, hidden=h, norm_eps=eps,
                        keep_dlogits=keep)
+
+
+norm_ce_backward_op = torch.library.custom_op("slowrun_amd::norm_ce_backward", _norm_ce_backward_body, mutates_args=())
 
 
 @norm_ce_backward_op.register_fake
@@ -365,8 +390,9 @@ class FusedSoftcappedCrossEntropy(torch.autograd.Function):
         xs, ws_ = _scale_value(x_s, x), _scale_value(w_s, lm_head_weight)
         (xs, xst), (ws_, wst) = _split_scale(xs), _split_scale(ws_)
         keep = bool(KEEP_DLOGITS if keep_dlogits is None else keep_dlogits)
-        out, saved = ce_forward_op(x.detach(), lm_head_weight.detach(), targets, mtp_weights, xs, ws_, float(cap),
-                                   reduction == "mean", keep, xst, wst)
+        xd, wd = x.detach(), lm_head_weight.detach()
+        call = ce_forward_op if _seen_as_op(xd, wd, targets, mtp_weights, xst, wst) else _ce_forward_body
+        out, saved = call(xd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", keep, xst, wst)
         ctx.scale_tensors = (xst, wst)
         ctx.save_for_backward(saved, targets, mtp_weights if mtp_weights is not None else torch.empty(0, device=x.device))
         ctx.params = (x.shape[0], x.shape[1], lm_head_weight.shape[1], xs, ws_, float(cap), float(grad_scale),
@@ -378,8 +404,9 @@ class FusedSoftcappedCrossEntropy(torch.autograd.Function):
     def backward(ctx, grad_output):
         saved, targets, mtp_w = ctx.saved_tensors
         N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, has_mtp, keep = ctx.params
-        dx, dw = ce_backward_op(saved, targets, grad_output.contiguous(), mtp_w if has_mtp else None, N, d, V, xs, ws_, cap,
-                                gscale, mean, x_bf16, w_bf16, keep, *ctx.scale_tensors)
+        go, mtp_w = grad_output.contiguous(), mtp_w if has_mtp else None
+        call = ce_backward_op if _seen_as_op(saved, targets, go, mtp_w, *ctx.scale_tensors) else _ce_backward_body
+        dx, dw = call(saved, targets, go, mtp_w, N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, keep, *ctx.scale_tensors)
         return dx, None, None, dw, None, None, None, None, None, None, None
 
 
@@ -399,10 +426,10 @@ class FusedNormSoftcappedCrossEntropy(torch.autograd.Function):
         eps = float(torch.finfo(torch.float32).eps if eps is None else eps)
         xs, ws_ = _scale_value(x_s, h), _scale_value(w_s, lm_head_weight)
         (xs, xst), (ws_, wst) = _split_scale(xs), _split_scale(ws_)
-        hd = h.detach()
+        hd, wd = h.detach(), lm_head_weight.detach()
         keep = bool(KEEP_DLOGITS if keep_dlogits is None else keep_dlogits)
-        out, saved = norm_ce_forward_op(hd, lm_head_weight.detach(), targets, mtp_weights, xs, ws_, float(cap),
-                                        reduction == "mean", eps, keep, xst, wst)
+        call = norm_ce_forward_op if _seen_as_op(hd, wd, targets, mtp_weights, xst, wst) else _norm_ce_forward_body
+        out, saved = call(hd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", eps, keep, xst, wst)
         ctx.scale_tensors = (xst, wst)
         ctx.save_for_backward(saved, hd, targets, mtp_weights if mtp_weights is not None else torch.empty(0, device=h.device))
         ctx.params = (lm_head_weight.shape[1], xs, ws_, float(cap), float(grad_scale), reduction == "mean",
@@ -413,8 +440,9 @@ class FusedNormSoftcappedCrossEntropy(torch.autograd.Function):
     def backward(ctx, grad_output):
         saved, h, targets, mtp_w = ctx.saved_tensors
         V, xs, ws_, cap, gscale, mean, w_bf16, has_mtp, eps, keep = ctx.params
-        dh, dw = norm_ce_backward_op(saved, h, targets, grad_output.contiguous(), mtp_w if has_mtp else None, V, xs, ws_, cap,
-                                     gscale, mean, w_bf16, eps, keep, *ctx.scale_tensors)
+        go, mtp_w = grad_output.contiguous(), mtp_w if has_mtp else None
+        call = norm_ce_backward_op if _seen_as_op(saved, h, targets, go, mtp_w, *ctx.scale_tensors) else _norm_ce_backward_body
+        dh, dw = call(saved, h, targets, go, mtp_w, V, xs, ws_, cap, gscale, mean, w_bf16, eps, keep, *ctx.scale_tensors)
         return dh, None, None, dw, None, None, None, None, None, None, None, None
 
 
