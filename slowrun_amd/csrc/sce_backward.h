@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256) void bwd_recompute_kernel(RecomputeParams p_in
   v16f acc[4][4];
   // (as in the forward kernel: the last pair's MFMAs of row blocks 1 - 3 ride along with the epilogues of row blocks 0 and 1)
   mfma_mainloop<false, NoHook, BK, false, 0, false, true>(p.wqt + (int64_t)ct * 256 * p.ldx, p.ldx, p.xq + (int64_t)rt * 256 * p.ldx, p.ldx, (int)(p.dp / BK), smem, acc, 2 * (rt & 3), ct & 7, wave);
-  DeferredTail deferred(smem, wa, wb);
+  DeferredTail<> deferred(smem, wa, wb);
   auto tail = [&](int b, int k) { deferred(acc, b, k); };
   const int vlim = p.V - ct * 256;           // columns >= vlim of this tile do not exist
   const bool ragged = vlim < 256;

@@ -54,43 +54,81 @@ __device__ __forceinline__ uint32_t* done_count(const FwdParams& p) { return rei
 //   t = tanh(u/cap) = 1 - 2/(E + 1), E = e^{2u/cap};   e^{z - cap} = exp2(c2 / (E + 1)).
 // The column of the maximum is looked up only on the (rare, after the first tiles) occasion that
 // a tile raises a row's running maximum.
-template <bool EDGE>
-__device__ __forceinline__ void fwd_epilogue(const v16f (&acc)[4][4], const FwdParams& p, int vbase,
-                                             float (&sum)[4], float (&amax)[4], int (&uarg)[4]) {
+//
+// Row block b of the tile.  hook(b, k), k = 0..31: called between the stages of the arithmetic, as in form_dlogits.  The order of the sum is that of
+// the columns a lane owns.
+template <int b, bool BF16, class Hook = NoHook>
+__device__ __forceinline__ void fwd_epilogue(v16f (&acc)[4][4], const FwdParams& p, int col0, float* wave_stat, Hook&& hook = NoHook()) {
+  constexpr bool HOOKED = !std::is_same<typename std::decay<Hook>::type, NoHook>::value;
+  __builtin_amdgcn_sched_barrier(0);
+  auto stage_end = [&](int k) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (HOOKED) { hook(b, k); __builtin_amdgcn_sched_barrier(0); }
+  };
+  float tmax = -INFINITY, s = 0.f;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+#pragma unroll
+    for (int g0 = 0; g0 < 16; g0 += 8) {
+      float pt[16];
+      // the GEMM of the eager head returns bf16: the logits are rounded once, in place, and everything after sees the rounded values
+      if (BF16) {
+#pragma unroll
+        for (int r = g0; r < g0 + 8; ++r) acc[a][b][r] = round_to_bf16_hw(acc[a][b][r]);
+      }
+#pragma unroll
+      for (int r = g0; r < g0 + 8; ++r) pt[r] = fast_exp2(acc[a][b][r] * p.k1);
+      stage_end(4 * (2 * a + g0 / 8));
+      // z - cap = c2 / (1 + e^{2u/cap}) in units of log2: the reciprocal of (1 + e) / c2 gives it in one step
+#pragma unroll
+      for (int r = g0; r < g0 + 8; ++r) pt[r] = fast_rcp(fmaf(pt[r], p.ic2, p.ic2));
+      stage_end(4 * (2 * a + g0 / 8) + 1);
+#pragma unroll
+      for (int r = g0; r < g0 + 8; ++r) pt[r] = fast_exp2(pt[r]);
+      stage_end(4 * (2 * a + g0 / 8) + 2);
+#pragma unroll
+      for (int r = g0; r < g0 + 8; ++r) {
+        s += pt[r];
+        tmax = fmaxf(tmax, acc[a][b][r]);
+      }
+      stage_end(4 * (2 * a + g0 / 8) + 3);
+    }
+  }
+  float* stat = wave_stat + lane_id();      // (taken anew, as the columns are below: nothing of them stays live across the arithmetic)
+  stat[(0 + b) * NTHREADS] += s;
+  const float amax = stat[(4 + b) * NTHREADS];
+  if (p.want_argmax && __builtin_amdgcn_ballot_w64(tmax > amax) != 0) {
+    if (tmax > amax) {
+      int targ = 0x7fffffff;
+#pragma unroll
+      for (int a = 3; a >= 0; --a) {
+#pragma unroll
+        for (int r = 15; r >= 0; --r) {
+          const int vo = a * 32 + 8 * (r >> 2) + (r & 3);
+          if (acc[a][b][r] == tmax) targ = vo;   // descending scan: lowest column wins
+        }
+      }
+      stat[(4 + b) * NTHREADS] = tmax;
+      stat[(8 + b) * NTHREADS] = __int_as_float(col0 + 4 * (lane_id() >> 5) + targ);
+    }
+  }
+}
+
+// The sums of the four row blocks again, on top of the ones before this tile (stat[12 ..]), over the columns that exist (the
+// others are -inf).  They are kept out by a factor of 0 or 1: 64 comparisons would be kept in scalar registers from block to block, and spilled.
+__device__ __forceinline__ void sums_of_existing_columns(const v16f (&acc)[4][4], const FwdParams& p, int col0, float* wave_stat) {
+  float* stat = wave_stat + lane_id();
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
-    float tmax = -INFINITY, s = 0.f;
+    int left = p.V - col0 - 4 * (lane_id() >> 5);
+    asm volatile("" : "+v"(left));
+    float s = 0.f;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int vo = a * 32 + 8 * (r >> 2) + (r & 3);
-        float x = acc[a][b][r];
-        // z - cap = c2 / (1 + e^{2u/cap}) in units of log2: the reciprocal of (1 + e) / c2 gives it in one step
-        float pt = fast_exp2(fast_rcp(fmaf(fast_exp2(x * p.k1), p.ic2, p.ic2)));
-        if (EDGE) {
-          if (vo >= p.V - vbase) { pt = 0.f; x = -INFINITY; }
-        }
-        s += pt;
-        tmax = fmaxf(tmax, x);
-      }
-    }
-    sum[b] += s;
-    if (p.want_argmax && __builtin_amdgcn_ballot_w64(tmax > amax[b]) != 0) {
-      if (tmax > amax[b]) {
-        int targ = 0x7fffffff;
-#pragma unroll
-        for (int a = 3; a >= 0; --a) {
-#pragma unroll
-          for (int r = 15; r >= 0; --r) {
-            const int vo = a * 32 + 8 * (r >> 2) + (r & 3);
-            if (acc[a][b][r] == tmax && (!EDGE || vo < p.V - vbase)) targ = vo;   // descending scan: lowest column wins
-          }
-        }
-        amax[b] = tmax;
-        uarg[b] = vbase + targ;
-      }
-    }
+      for (int r = 0; r < 16; ++r)
+        s = fmaf((float)min(max(left - (a * 32 + 8 * (r >> 2) + (r & 3)), 0), 1), fast_exp2(fast_rcp(fmaf(fast_exp2(acc[a][b][r] * p.k1), p.ic2, p.ic2))), s);
+    stat[(0 + b) * NTHREADS] = stat[(12 + b) * NTHREADS] + s;
   }
 }
 
@@ -622,22 +660,20 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
   // the first K blocks of the next tile travel while the epilogue of this one runs (it does not touch the K slots)
   if (ct0 < ct1) mfma_prefetch(p.wqt + (int64_t)ct0 * 256 * p.ldx, p.ldx, Bg, p.ldx, smem, rot_a, rot_b, wave);
   for (int ct = ct0; ct < ct1; ++ct) {
-    if (EMIT) mfma_mainloop<true, NoHook, BK, false, 0, false, true>(p.wqt + (int64_t)ct * 256 * p.ldx, p.ldx, Bg, p.ldx, KT, smem, acc, rot_a, rot_b, wave);
-    else mfma_mainloop<true, NoHook, BK, false, 0, BF16>(p.wqt + (int64_t)ct * 256 * p.ldx, p.ldx, Bg, p.ldx, KT, smem, acc, rot_a, rot_b, wave);
+    mfma_mainloop<true, NoHook, BK, false, 0, BF16, true>(p.wqt + (int64_t)ct * 256 * p.ldx, p.ldx, Bg, p.ldx, KT, smem, acc, rot_a, rot_b, wave);
     auto prefetch = [&]() {
       if (ct + 1 < ct1) mfma_prefetch(p.wqt + (int64_t)(ct + 1) * 256 * p.ldx, p.ldx, Bg, p.ldx, smem, rot_a, rot_b, wave);
     };
-    if (!EMIT) prefetch();
-    float* stat = reinterpret_cast<float*>(smem + FWD_STAT_OFF) + wave * 64 + lane_id();
-    const int vbase = ct * 256 + wa * 128 + 4 * (lane_id() >> 5);
     const int* tgt = reinterpret_cast<const int*>(smem + FWD_TGT_OFF) + wb * 128;
+    DeferredTail<BF16> deferred(smem, wa, wb);
+    auto tail = [&](int b, int k) { deferred(acc, b, k); };
     if (EMIT) {
       // The main loop has left 48 of the 64 MFMAs of its last pair of K blocks undone, those of row blocks 1 - 3; the pair
       // is still in LDS.  They are issued one at a time between the stages of the epilogues of row blocks 0 and 1, where
       // the matrix pipe would stand idle: during block 0's the 32 of blocks 1 and 2 (one at each of its 32 stage
       // boundaries), during block 1's the 16 of block 3.  Only then are the slots free for the next tile's first K blocks.
-      DeferredTail deferred(smem, wa, wb);
-      auto tail = [&](int b, int k) { deferred(acc, b, k); };
+      float* stat = reinterpret_cast<float*>(smem + FWD_STAT_OFF) + wave * 64 + lane_id();
+      const int vbase = ct * 256 + wa * 128 + 4 * (lane_id() >> 5);
       const int vlim = p.V - ct * 256;
       // the wave's quadrant of G: tile of rows rt, block of columns 2 ct + wa, rows 128 wb on
       uint8_t* gq = p.ghat_t + ((int64_t)rt * p.kbv + 2 * ct + wa) * BLOCKED_KSTEP + wb * 128 * BK;
@@ -686,29 +722,32 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
       }
       if (lane_id() == 0) p.gexp[(int64_t)(2 * ct + wa) * p.kbw + 2 * rt + wb] = ew;
     } else {
-      float sum[4], amax[4];
-      int uarg[4];
+      // The same, with the epilogue that forms no dlogits: 16384 rows, d = 1024, V = 50304 with bf16 operands, where the epilogue is a third of a tile's
+      // time, a pass of 1567 us takes 1518; 8192 rows, d = 2560 in e4m3, which the card's power bounds, the same either way.  Of a tile that reaches beyond the
+      // vocabulary the columns that do not exist are struck out here too, and the sums are then formed again without them: what they add, e^{-2 cap} apiece, cannot be taken off exactly
+      const bool ragged = ct * 256 + 256 > p.V;
+      const int col0 = ct * 256 + wa * 128;
+      float* wave_stat = reinterpret_cast<float*>(smem + FWD_STAT_OFF) + wave * 64;
+      if (ragged) {
+        float* stat = wave_stat + lane_id();
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        sum[b] = stat[(0 + b) * NTHREADS]; amax[b] = stat[(4 + b) * NTHREADS]; uarg[b] = __float_as_int(stat[(8 + b) * NTHREADS]);
+        for (int b = 0; b < 4; ++b) stat[(12 + b) * NTHREADS] = stat[(0 + b) * NTHREADS];
+        strike_columns_beyond<0, 1>(acc, p.V - ct * 256, wa);
       }
-      if (BF16) {
-        // the GEMM of the eager head returns bf16: the logits are rounded once, in place, and everything after sees the rounded values
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[a][b][r] = round_to_bf16_hw(acc[a][b][r]);
-      }
-      if (ct * 256 + 256 > p.V) fwd_epilogue<true>(acc, p, vbase, sum, amax, uarg);
-      else fwd_epilogue<false>(acc, p, vbase, sum, amax, uarg);
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        stat[(0 + b) * NTHREADS] = sum[b]; stat[(4 + b) * NTHREADS] = amax[b]; stat[(8 + b) * NTHREADS] = __int_as_float(uarg[b]);
-      }
+      fwd_epilogue<0, BF16>(acc, p, col0, wave_stat, tail);
+      if (!PRE) take_target_logits<true, false, false, 256, 0, 1>(acc, tgt, p.n_predict, col0, rt * 256 + wb * 128, p.sc, p.s_uy, p.Np, nullptr, 0.f, 0.f, 0.f);
+      if (ragged) strike_columns_beyond<1, 2>(acc, p.V - ct * 256, wa);
+      fwd_epilogue<1, BF16>(acc, p, col0, wave_stat, tail);
+      if (!PRE) take_target_logits<true, false, false, 256, 1, 2>(acc, tgt, p.n_predict, col0, rt * 256 + wb * 128, p.sc, p.s_uy, p.Np, nullptr, 0.f, 0.f, 0.f);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // every wave has read its last fragment
+      prefetch();
+      if (ragged) strike_columns_beyond<2, 4>(acc, p.V - ct * 256, wa);
+      fwd_epilogue<2, BF16>(acc, p, col0, wave_stat);
+      if (!PRE) take_target_logits<true, false, false, 256, 2, 3>(acc, tgt, p.n_predict, col0, rt * 256 + wb * 128, p.sc, p.s_uy, p.Np, nullptr, 0.f, 0.f, 0.f);
+      fwd_epilogue<3, BF16>(acc, p, col0, wave_stat);
+      if (!PRE) take_target_logits<true, false, false, 256, 3, 4>(acc, tgt, p.n_predict, col0, rt * 256 + wb * 128, p.sc, p.s_uy, p.Np, nullptr, 0.f, 0.f, 0.f);
+      if (ragged) sums_of_existing_columns(acc, p, col0, wave_stat);
     }
-    if (!EMIT && !PRE) take_target_logits<true, false, false, 256>(acc, tgt, p.n_predict, ct * 256 + wa * 128, rt * 256 + wb * 128, p.sc, p.s_uy, p.Np, nullptr, 0.f, 0.f, 0.f);
   }
   float sum[4], amax[4];
   int uarg[4];

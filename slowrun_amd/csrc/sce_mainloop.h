@@ -185,7 +185,7 @@ __device__ __forceinline__ v16f mfma_bf16_pair(const v8i& a, const v8i& b, v16f 
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a1), __builtin_bit_cast(v8bf, b1), c, 0, 0, 0);
 }
 
-// DEFER (plain fp8 only): of the last pair of K blocks only the MFMAs of B block 0 (accumulators acc[.][0]) are
+// DEFER (plain fp8 or bf16 only): of the last pair of K blocks only the MFMAs of B block 0 (accumulators acc[.][0]) are
 // issued; the other 48 are left to the caller, who finds the pair in the two LDS slots on return (lds_fragment) and
 // issues them (mfma_tail) between the vector instructions of its epilogue of the finished accumulators, where the
 // matrix pipe would otherwise stand idle.  Nothing may be loaded into the slots until that is done.
@@ -199,7 +199,7 @@ __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, in
                                               uint8_t* smem, v16f (&acc)[NA][4], int rot_a, int rot_b, int wave, Hook&& hook = NoHook(),
                                               int64_t bk1_arg = 0, int64_t bk2_arg = 0, const uint32_t* lds_scale = nullptr,
                                               const int* a_rows = nullptr) {
-  static_assert(!DEFER || (!BF16 && SCALE == 0 && !TRB && NA == 4), "DEFER is for the plain fp8 loop");
+  static_assert(!DEFER || (SCALE == 0 && !TRB && NA == 4), "DEFER is for the plain loop");
   static_assert(NA == 4 || (NA == 2 && LOADS_EM <= 8), "loads of block k + 2 that are counted: both operands' first four each");
   const int lane = lane_id();
   const int wa = wave >> 1, wb = wave & 1;
@@ -468,6 +468,7 @@ constexpr bool tail_schedule_ok() {
 }
 static_assert(tail_schedule_ok(), "the deferred MFMAs: some product missing, doubled, out of order, or fed from the wrong registers");
 
+template <bool BF16 = false>
 struct DeferredTail {
   TailReader frag;
   v8i fa[2], fb[2][2];
@@ -482,7 +483,8 @@ struct DeferredTail {
   __device__ __forceinline__ DeferredTail(const uint8_t* smem, int wa, int wb) : frag(smem, wa, wb) { read(tail_prologue()); }
   __device__ __forceinline__ void operator()(v16f (&acc)[4][4], int b, int k) {
     const TailOp op = tail_op(b, k);
-    if (op.mfma) acc[op.a][op.rb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[op.fa_i], fb[op.fb_i][op.fb_j], acc[op.a][op.rb], 0, 0, 0, 0, 0, 0);
+    if (op.mfma && BF16) acc[op.a][op.rb] = mfma_bf16_pair(fa[op.fa_i], fb[op.fb_i][op.fb_j], acc[op.a][op.rb]);
+    else if (op.mfma) acc[op.a][op.rb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fa[op.fa_i], fb[op.fb_i][op.fb_j], acc[op.a][op.rb], 0, 0, 0, 0, 0, 0);
     read(op);
   }
 };
