@@ -28,6 +28,7 @@ struct FwdParams {
   float em2cap;            // e^{-2 cap}: what a logit of -inf adds to the sum of e^{z - cap}
   const DevConsts* dc;     // non-NULL: sc and k1 come from here (a scale lives on the device)
   uint8_t* hdr;            // header of the saved state
+  int halves;              // EMIT and PRE: this many tiles of every row tile are shared out in halves (fwd_halves)
   int want_argmax;         // the caller asks for the rows' argmax: the column of the running maximum is tracked
 };
 
@@ -618,6 +619,19 @@ constexpr int FWD_UY_OFF = FWD_STAT_OFF - 4096;                        // PRE: t
 constexpr int SMEM_FWD = SMEM_MAX;
 static_assert(SMEM_BYTES <= FWD_UY_OFF, "K slots and row data overlap");
 
+// PRE: which of the lane's values in the row block at row0 is a target of its row (one is looked for: two targets of a row in one
+// lane's 64 columns are the same column, or rare enough that the second may set an exponent): its known value.
+__device__ __forceinline__ float target_value(const uint8_t* smem, int n_predict, int col0, int row0) {
+  const int* tgt = reinterpret_cast<const int*>(smem + FWD_TGT_OFF) + row0;
+  const float* tuy = reinterpret_cast<const float*>(smem + FWD_UY_OFF) + row0;
+  float v = __builtin_nanf("");
+  for (int k = 0; k < n_predict; ++k) {
+    const int rel = tgt[k * 256 + (lane_id() & 31)] - col0;
+    if ((unsigned)rel < 128u && ((rel >> 2) & 1) == (lane_id() >> 5)) v = tuy[k * 256 + (lane_id() & 31)];
+  }
+  return v;
+}
+
 // EMIT: the epilogue also leaves the block-scaled dlogits of the tile in G (see form_dlogits), for a backward pass
 // that does not compute the logits again.
 // BF16 (without EMIT): bf16 operands, logits rounded to bf16 as the eager head's GEMM returns them (forward only).
@@ -633,7 +647,8 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
   int rt, s;
   if (!map_tile(blockIdx.x, p.RT, p.S, rt, s)) return;
   if (blockIdx.x == 0 && threadIdx.x == 0) *done_count(p) = 0;
-  const int ct0 = (int)((int64_t)p.CT * s / p.S), ct1 = (int)((int64_t)p.CT * (s + 1) / p.S);
+  const int cth = EMIT && PRE ? p.halves : 0;      // tiles [0, cth) as halves, one to a workgroup behind its whole tiles
+  const int ct0 = cth + (int)((int64_t)(p.CT - cth) * s / p.S), ct1 = cth + (int)((int64_t)(p.CT - cth) * (s + 1) / p.S);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wa = wave >> 1, wb = wave & 1;
   {
     float* stat = reinterpret_cast<float*>(smem + FWD_STAT_OFF) + wave * 64 + lane_id();   // [12][256]: sum, amax, uarg of the 4 row blocks
@@ -662,7 +677,8 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
   for (int ct = ct0; ct < ct1; ++ct) {
     mfma_mainloop<true, NoHook, BK, false, 0, BF16, true>(p.wqt + (int64_t)ct * 256 * p.ldx, p.ldx, Bg, p.ldx, KT, smem, acc, rot_a, rot_b, wave);
     auto prefetch = [&]() {
-      if (ct + 1 < ct1) mfma_prefetch(p.wqt + (int64_t)(ct + 1) * 256 * p.ldx, p.ldx, Bg, p.ldx, smem, rot_a, rot_b, wave);
+      const int next = ct + 1 < ct1 ? ct + 1 : s < 2 * cth ? s >> 1 : -1;
+      if (next >= 0) mfma_prefetch(p.wqt + (int64_t)next * 256 * p.ldx, p.ldx, Bg, p.ldx, smem, rot_a, rot_b, wave);
     };
     const int* tgt = reinterpret_cast<const int*>(smem + FWD_TGT_OFF) + wb * 128;
     DeferredTail<BF16> deferred(smem, wa, wb);
@@ -684,23 +700,13 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
       const bool ragged = vlim < 256;
       uint32_t ew;
       if (PRE) {
-        // which of the lane's values of row block b is a target of its row (one is looked for: two targets of a row in one
-        // lane's 64 columns are the same column, or rare enough that the second may set an exponent): its known value
-        const float* tuy = reinterpret_cast<const float*>(smem + FWD_UY_OFF) + wb * 128;
-        auto target_value = [&](int b) {
-          float v = __builtin_nanf("");
-          for (int k = 0; k < p.n_predict; ++k) {
-            const int rel = tgt[k * 256 + b * 32 + (lane_id() & 31)] - col0;
-            if ((unsigned)rel < 128u && ((rel >> 2) & 1) == (lane_id() >> 5)) v = tuy[k * 256 + b * 32 + (lane_id() & 31)];
-          }
-          return v;
-        };
+        auto target = [&](int b) { return target_value(smem, p.n_predict, col0, wb * 128 + b * 32); };
         float xc[4];                                   // (looked up a row block ahead of their use: the LDS reads have time)
         if (ragged) strike_columns_beyond<0, 1>(acc, vlim, wa, stat, p.em2cap);
-        xc[0] = target_value(0); xc[1] = target_value(1);
+        xc[0] = target(0); xc[1] = target(1);
         ew = form_dlogits<true, NTHREADS, 64, 0, 1, decltype(tail)&, true>(acc, p.k1, p.c2, vbase, gq, wa, wb, stat, lam, p.want_argmax != 0, tail, xc, p.sc);
         if (ragged) strike_columns_beyond<1, 2>(acc, vlim, wa, stat, p.em2cap);
-        xc[2] = target_value(2); xc[3] = target_value(3);
+        xc[2] = target(2); xc[3] = target(3);
         ew |= form_dlogits<true, NTHREADS, 64, 1, 2, decltype(tail)&, true>(acc, p.k1, p.c2, vbase, gq, wa, wb, stat, lam, p.want_argmax != 0, tail, xc, p.sc);
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // every wave has read its last fragment
         prefetch();
@@ -747,6 +753,24 @@ __global__ __launch_bounds__(256) void fwd_kernel(FwdParams p_in) {
       fwd_epilogue<3, BF16>(acc, p, col0, wave_stat);
       if (!PRE) take_target_logits<true, false, false, 256, 3, 4>(acc, tgt, p.n_predict, col0, rt * 256 + wb * 128, p.sc, p.s_uy, p.Np, nullptr, 0.f, 0.f, 0.f);
       if (ragged) sums_of_existing_columns(acc, p, col0, wave_stat);
+    }
+  }
+  if constexpr (EMIT && PRE) {
+    if (s < 2 * cth) {
+      // half of tile s / 2: row blocks 2 hb and 2 hb + 1 of every wave, which are blocks 0 and 1 to everything here
+      const int ct = s >> 1, hb = s & 1;
+      mfma_mainloop<true, NoHook, BK, false, 0, false, false, 4, 2>(p.wqt + (int64_t)ct * 256 * p.ldx, p.ldx, Bg, p.ldx, KT, smem, acc, rot_a, rot_b, wave, NoHook(), 0, 0,
+                                                                    nullptr, nullptr, 64 * hb);
+      float* stat = reinterpret_cast<float*>(smem + FWD_STAT_OFF) + 2 * hb * NTHREADS + wave * 64 + lane_id();
+      const float* lam = reinterpret_cast<const float*>(smem + FWD_STAT_OFF) + (12 + 2 * hb) * NTHREADS + wave * 64;
+      const int col0 = ct * 256 + wa * 128, vbase = col0 + 4 * (lane_id() >> 5), r0 = wb * 128 + hb * 64;
+      uint8_t* gq = p.ghat_t + ((int64_t)rt * p.kbv + 2 * ct + wa) * BLOCKED_KSTEP + r0 * BK;
+      float xc[2];
+#pragma unroll
+      for (int b = 0; b < 2; ++b) xc[b] = target_value(smem, p.n_predict, col0, r0 + b * 32);
+      NoHook none;
+      const uint32_t ew = form_dlogits<true, NTHREADS, 64, 0, 2, NoHook&, true>(acc, p.k1, p.c2, vbase, gq, wa, wb, stat, lam, p.want_argmax != 0, none, xc, p.sc);
+      if (lane_id() == 0) reinterpret_cast<uint16_t*>(p.gexp + (int64_t)(2 * ct + wa) * p.kbw + 2 * rt + wb)[hb] = (uint16_t)ew;
     }
   }
   float sum[4], amax[4];

@@ -357,6 +357,15 @@ static int fwd_least_splits(int RT, int CT, int ncu) {
 static int fwd_splits(int RT, int CT, int ncu) {
   return RT * FWD_MAX_SPLITS < ncu ? std::min(CT, ncu / RT) : fwd_least_splits(RT, CT, ncu);
 }
+// How many of a row tile's CT tiles an emitting forward pass shares out as halves (64 of each wave's 128 rows): where one round of workgroups does it all
+// and a few of them would have a whole tile more than the rest, twice as many have half a tile more.
+// Measured, V = 50304 (197 tiles, 5 over): 2048 rows, d = 768, fp32 7 tiles -> 6.5, a step of 385.7 us 380.0; two micro-batches of 2048,
+// d = 1024 821 -> 811; 4096 rows, d = 1600 13 -> 12.5, 1070.5 -> 1066.7.  Over several rounds of workgroups the last one is never in step, and the gain
+// would be a hundredth of the kernel; a remainder above half the splits makes some workgroups take two halves, a whole tile.
+static int fwd_halves(int RT, int CT, int nsplit, int ncu) {
+  const int over = CT % nsplit;
+  return RT * nsplit <= ncu && CT >= nsplit && 2 * over <= nsplit ? over : 0;      // (CT >= nsplit: the last tile, of which some columns may not exist, is a whole one)
+}
 // partial records of a forward pass: enough for any device (fwd_splits makes no more than MAX_CUS workgroups beyond 16 splits)
 static size_t fwd_workspace(int64_t Np) {
   return (size_t)std::max<int64_t>(FWD_MAX_SPLITS * Np, (int64_t)MAX_CUS * 256) * 16 + 256;
@@ -573,11 +582,13 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   p.sc = bf16ops ? 1.0f : (float)a->x_s * (float)a->w_s; p.k1 = p.sc * 2.0f * LOG2E / a->cap; p.c2 = -2.0f * a->cap * LOG2E; p.ic2 = 1.0f / p.c2; p.em2cap = expf(-2.0f * a->cap);
   p.dc = bf16ops ? nullptr : dcp;
   p.want_argmax = a->argmax != nullptr; p.hdr = sv + S.off_hdr;
+  p.halves = 0;
   const int grid = map_tile_grid(RT, nsplit);
   // An fp8 forward pass has its target logits computed ahead of the forward kernel (from a tile of gathered rows of W_q^T,
   // together with the rows' boosts when it emits the dlogits) as long as that tile's 32-bit offsets reach every row of
   // W_q^T; beyond, the forward kernel takes them out of its own accumulators, as the bf16 forward pass does.
   const bool pre = !bf16ops && (int64_t)S.Vp * S.ldx < g_gather_limit;
+  if (pre && emit) p.halves = fwd_halves(RT, CTw, nsplit, device_cus_or_default(a->device));
   {
     // the exponent boosts of the rows, estimated from two tiles of their logits: only for a forward pass
     // that emits the dlogits (a backward pass that forms them again knows the rows' sums and takes the boosts from those)

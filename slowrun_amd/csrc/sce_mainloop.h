@@ -193,12 +193,16 @@ __device__ __forceinline__ v16f mfma_bf16_pair(const v8i& a, const v8i& b, v16f 
 // NA = 2: a tile of 128 A rows, 64 to a wave, for a last round of tiles that would leave half the chip idle.  The slots
 // are the same 32, every other one with an MFMA; the loads and reads of the missing rows drop out of the table (no load
 // before b2, whose count the wait there relies on, is among them).
-template <bool PREFETCHED = false, class Hook = NoHook, int KSTEP = BK, bool TRB = false, int SCALE = 0, bool BF16 = false, bool DEFER = false, int NA = 4>
+//
+// NB = 2: only 64 of a wave's 128 B rows, from row b_row0 (0 or 64) of them on, as acc[.][0 .. 1]; all rows are loaded.  For the last
+// round of a walk over tiles whose way out is the longer part (see fwd_halves).
+template <bool PREFETCHED = false, class Hook = NoHook, int KSTEP = BK, bool TRB = false, int SCALE = 0, bool BF16 = false, bool DEFER = false, int NA = 4, int NB = 4>
 __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, int64_t lda,
                                               const uint8_t* __restrict__ Bg, int64_t ldb, int KD,
                                               uint8_t* smem, v16f (&acc)[NA][4], int rot_a, int rot_b, int wave, Hook&& hook = NoHook(),
                                               int64_t bk1_arg = 0, int64_t bk2_arg = 0, const uint32_t* lds_scale = nullptr,
-                                              const int* a_rows = nullptr) {
+                                              const int* a_rows = nullptr, int b_row0 = 0) {
+  static_assert(NB == 4 || (NB == 2 && NA == 4 && !DEFER && !TRB && SCALE == 0), "NB = 2 is for the plain loop");
   static_assert(!DEFER || (SCALE == 0 && !TRB && NA == 4), "DEFER is for the plain loop");
   static_assert(NA == 4 || (NA == 2 && LOADS_EM <= 8), "loads of block k + 2 that are counted: both operands' first four each");
   const int lane = lane_id();
@@ -208,7 +212,7 @@ __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, in
   // fragments: lane reads row l%32 of a 32-row block, 32 bytes of K at (l/32)*32 within the sub-step
   const int r = lane & 31, h = lane >> 5;
   const int sw = (r & 7) ^ ((r >> 3) & 1);
-  const int abase = wa * 32 * NA * BK + r * BK, bbase = TM * BK + wb * 128 * BK + r * BK;
+  const int abase = wa * 32 * NA * BK + r * BK, bbase = TM * BK + (wb * 128 + (NB == 4 ? 0 : b_row0)) * BK + r * BK;
   // half `u` (0, 1) of fragment n (0-3: A, 4-7: B) of the sub-step with K half `half` in LDS slot `slot`: registers 4 u .. 4 u + 3
   auto runit = [&](int slot, int half, int n, int u, v8i (&fa)[NA], v8i (&fb)[4]) {
     v4i q;
@@ -242,7 +246,7 @@ __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, in
   auto runits = [&](int slot, int half, int q0, int cnt, v8i (&fa)[NA], v8i (&fb)[4]) {
 #pragma unroll
     for (int q = q0; q < q0 + cnt; ++q)
-      if (UNIT_FRAG[q >> 1] < NA || UNIT_FRAG[q >> 1] >= 4) runit(slot, half, UNIT_FRAG[q >> 1], q & 1, fa, fb);
+      if (UNIT_FRAG[q >> 1] < NA || (UNIT_FRAG[q >> 1] >= 4 && UNIT_FRAG[q >> 1] < 4 + NB)) runit(slot, half, UNIT_FRAG[q >> 1], q & 1, fa, fb);
   };
   // prologue: K block 0 and half of block 1 in flight, block 0 visible, fragments of sub-step 0 in registers
   if (!PREFETCHED) {
@@ -312,7 +316,7 @@ __device__ __forceinline__ void mfma_mainloop(const uint8_t* __restrict__ Ag, in
       const int sub = s >> 4, i = s & 15;
       constexpr int PER = 4 / NA;                 // slots to an MFMA
       if (DEFER && !has2 && (i & 3) != 0) {}      // last pair, B blocks 1 - 3: the caller's
-      else if (i % PER != 0) {}
+      else if (i % PER != 0 || (i & 3) >= NB) {}
       else if (first && BLK == 0 && sub == 0) mm0(i / PER); else mm(BLK, sub, i / PER);
       hook(32 * BLK + s);
       if (!(first && BLK == 0)) runits(BLK, 0, UNITS_N0 + ksum(KS.c0, s), KS.c0[s], fa[0], fb[0]);      // (the first block's came with the prologue)
