@@ -28,7 +28,7 @@ struct FwdParams {
   float em2cap;            // e^{-2 cap}: what a logit of -inf adds to the sum of e^{z - cap}
   const DevConsts* dc;     // non-NULL: sc and k1 come from here (a scale lives on the device)
   uint8_t* hdr;            // header of the saved state
-  int halves;              // EMIT and PRE: this many tiles of every row tile are shared out in halves (fwd_halves)
+  int halves;              // EMIT and PRE: this many tiles of every row tile, whole ones of the vocabulary, are shared out in halves (fwd_halves)
   int want_argmax;         // the caller asks for the rows' argmax: the column of the running maximum is tracked
 };
 

@@ -362,9 +362,11 @@ static int fwd_splits(int RT, int CT, int ncu) {
 // Measured, V = 50304 (197 tiles, 5 over): 2048 rows, d = 768, fp32 7 tiles -> 6.5, a step of 385.7 us 380.0; two micro-batches of 2048,
 // d = 1024 821 -> 811; 4096 rows, d = 1600 13 -> 12.5, 1070.5 -> 1066.7.  Over several rounds of workgroups the last one is never in step, and the gain
 // would be a hundredth of the kernel; a remainder above half the splits makes some workgroups take two halves, a whole tile.
-static int fwd_halves(int RT, int CT, int nsplit, int ncu) {
+// A half has no code that strikes out columns beyond the vocabulary, and the vocabulary (the first Vl columns) can end in any tile: there are halves
+// only where it covers all of them.
+static int fwd_halves(int RT, int CT, int nsplit, int ncu, int64_t Vl) {
   const int over = CT % nsplit;
-  return RT * nsplit <= ncu && CT >= nsplit && 2 * over <= nsplit ? over : 0;      // (CT >= nsplit: the last tile, of which some columns may not exist, is a whole one)
+  return RT * nsplit <= ncu && CT >= nsplit && 2 * over <= nsplit && (int64_t)over * 256 <= Vl ? over : 0;
 }
 // partial records of a forward pass: enough for any device (fwd_splits makes no more than MAX_CUS workgroups beyond 16 splits)
 static size_t fwd_workspace(int64_t Np) {
@@ -588,7 +590,7 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   // together with the rows' boosts when it emits the dlogits) as long as that tile's 32-bit offsets reach every row of
   // W_q^T; beyond, the forward kernel takes them out of its own accumulators, as the bf16 forward pass does.
   const bool pre = !bf16ops && (int64_t)S.Vp * S.ldx < g_gather_limit;
-  if (pre && emit) p.halves = fwd_halves(RT, CTw, nsplit, device_cus_or_default(a->device));
+  if (pre && emit) p.halves = fwd_halves(RT, CTw, nsplit, device_cus_or_default(a->device), Vl);
   {
     // the exponent boosts of the rows, estimated from two tiles of their logits: only for a forward pass
     // that emits the dlogits (a backward pass that forms them again knows the rows' sums and takes the boosts from those)
