@@ -290,15 +290,31 @@ def ce_backward(saved, targets, grad_output, N, d, V, x_s, w_s, cap, grad_scale,
 # ---------------------------------------------------------------------------------------------
 def _seen_as_op(*tensors):
     """Whether a call must go through the dispatcher: something traces, records or transforms calls (torch.compile, jit tracing, dispatch
-    and function modes, functorch, the profiler, autograd of a backward pass), or an argument is no plain tensor (a subclass, or a type that
-    the op's schema refuses)."""
+    and function modes, functorch, the profiler, autograd of a backward pass), or an argument is no plain tensor: a subclass, a type that
+    the op's schema refuses, or a tensor that the dispatcher would turn into another before the body sees it (batched gradients without
+    functorch, negation left to be done, zeros without memory)."""
     if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled():
         return True
     if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active():
         return True
     if torch._C._autograd._profiler_enabled():
         return True
-    return any(t is not None and type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter for t in tensors)
+    for t in tensors:
+        if t is not None and ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or _dispatch_keys(t).raw_repr() & _SPECIAL_KEYS):
+            return True
+    return False
+
+
+def _plain_keys():
+    plain = _dispatch_keys(torch.empty(0, device="cpu"))
+    for name in ("CUDA", "AutogradCUDA", "AutocastCUDA", "Meta", "AutogradMeta"):
+        plain = plain | torch._C.DispatchKeySet(torch._C._dispatch_key_parse(name))
+    return plain.raw_repr()
+
+
+# All dispatch keys but those that a tensor has for being dense, on its device, and open to autograd and autocast.
+_dispatch_keys = torch._C._dispatch_keys
+_SPECIAL_KEYS = ~_plain_keys()
 
 
 def _ce_forward_body(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor, mtp_weights: Optional[torch.Tensor],

@@ -40,6 +40,68 @@ def test_only_plain_calls_pass_the_operator_by():
     assert ck._seen_as_op(x)                                   # a backward pass that is itself differentiated
 
 
+FUNCTIONS = [ck.FusedSoftcappedCrossEntropy, ck.FusedNormSoftcappedCrossEntropy]
+
+
+def _apply(fn, x, w, y, reduction="mean"):
+    return fn.apply(x, y, None, w, 0.02, 0.02, 1.0, 1.0, 15.0, reduction)
+
+
+@pytest.fixture
+def cpu_kernels(monkeypatch):
+    """Stand-ins for the two library calls, linear in the upstream gradient, that read their arguments' memory as the library does."""
+    def forward(x, w, targets, x_s, w_s, cap, reduction, **_more):
+        assert all(t.data_ptr() for t in (x, w, targets))
+        rows = torch.from_numpy(x.float().numpy()).sum(1)
+        return rows.mean() if reduction == "mean" else rows, torch.zeros(8, dtype=torch.uint8), None, None, None
+
+    def backward(saved, targets, grad_output, N, d, V, x_s, w_s, cap, grad_scale, reduction, x_dtype, w_dtype, **_more):
+        assert grad_output.data_ptr() and not grad_output.is_neg()
+        g = torch.from_numpy(grad_output.numpy()).expand(N)
+        return g[:, None].expand(N, d).to(x_dtype).contiguous(), g.sum().expand(d, V).to(w_dtype).contiguous()
+
+    monkeypatch.setattr(ck, "ce_forward", forward)
+    monkeypatch.setattr(ck, "ce_backward", backward)
+
+
+def _inputs(device="cpu", N=5, d=16, V=7):
+    return torch.ones(N, d, device=device, requires_grad=True), torch.ones(d, V, device=device, requires_grad=True), torch.zeros(N, dtype=torch.int64, device=device)
+
+
+@pytest.mark.parametrize("fn", FUNCTIONS)
+def test_batched_gradients(fn, cpu_kernels):
+    """is_grads_batched and vectorised jacobians hand backward a tensor without memory, of the plain type and outside functorch's transforms."""
+    x, w, y = _inputs()
+    dx, dw = torch.autograd.grad(_apply(fn, x, w, y), (x, w), torch.tensor([1.0, 2.0]), is_grads_batched=True)
+    assert torch.equal(dx, torch.tensor([1.0, 2.0])[:, None, None].expand(2, 5, 16)) and torch.equal(dw, 5 * torch.tensor([1.0, 2.0])[:, None, None].expand(2, 16, 7))
+    jac = torch.autograd.functional.jacobian(lambda t: _apply(fn, t, w, y, "none"), x, vectorize=True)
+    assert torch.equal(jac, torch.eye(5)[:, :, None].expand(5, 5, 16))
+
+
+@pytest.mark.parametrize("fn", FUNCTIONS)
+def test_gradients_whose_memory_is_not_their_value(fn, cpu_kernels):
+    x, w, y = _inputs()
+    for go, value in ((torch._neg_view(torch.tensor(2.0)), -2.0), (torch._efficientzerotensor(()), 0.0)):
+        (dx,) = torch.autograd.grad(_apply(fn, x, w, y), x, go)
+        assert torch.equal(dx, torch.full((5, 16), value))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fn", FUNCTIONS)
+def test_batched_gradients_on_the_gpu(fn):
+    x, w = torch.randn(300, 64, device="cuda").bfloat16().requires_grad_(True), torch.randn(64, 500, device="cuda").bfloat16().requires_grad_(True)
+    y = torch.randint(0, 500, (300,), device="cuda")
+    with torch.no_grad():
+        assert not ck._seen_as_op(x.detach(), w.detach(), y, None)
+    out = _apply(fn, x, w, y, "none")
+    go = torch.randn(3, 300, device="cuda")
+    batched = torch.autograd.grad(out, (x, w), go, is_grads_batched=True, retain_graph=True)
+    for k in range(3):
+        assert all(torch.equal(b[k], one) for b, one in zip(batched, torch.autograd.grad(out, (x, w), go[k], retain_graph=True)))
+    (dx,) = torch.autograd.grad(out, x, torch._neg_view(go[0]))
+    assert torch.equal(dx, -batched[0][0])
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("fn", [ck.FusedSoftcappedCrossEntropy, ck.FusedNormSoftcappedCrossEntropy])
 def test_both_ways_give_the_same_and_modes_see_the_operator(fn):
