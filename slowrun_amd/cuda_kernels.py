@@ -292,7 +292,7 @@ def _seen_as_op(*tensors):
     """Whether a call must go through the dispatcher: something traces, records or transforms calls (torch.compile, jit tracing, dispatch
     and function modes, functorch, the profiler, autograd of a backward pass), or an argument is no plain tensor: a subclass, a type that
     the op's schema refuses, or a tensor that the dispatcher would turn into another before the body sees it (batched gradients without
-    functorch, negation left to be done, zeros without memory)."""
+    functorch, negation left to be done, zeros without memory) or answer without it (meta tensors)."""
     if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled():
         return True
     if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active():
@@ -307,12 +307,12 @@ def _seen_as_op(*tensors):
 
 def _plain_keys():
     plain = _dispatch_keys(torch.empty(0, device="cpu"))
-    for name in ("CUDA", "AutogradCUDA", "AutocastCUDA", "Meta", "AutogradMeta"):
+    for name in ("CUDA", "AutogradCUDA", "AutocastCUDA"):
         plain = plain | torch._C.DispatchKeySet(torch._C._dispatch_key_parse(name))
     return plain.raw_repr()
 
 
-# All dispatch keys but those that a tensor has for being dense, on its device, and open to autograd and autocast.
+# All dispatch keys but those that a tensor has for being dense, on the GPU (or the CPU: the body refuses it), and open to autograd and autocast.
 _dispatch_keys = torch._C._dispatch_keys
 _SPECIAL_KEYS = ~_plain_keys()
 

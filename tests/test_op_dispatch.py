@@ -86,6 +86,22 @@ def test_gradients_whose_memory_is_not_their_value(fn, cpu_kernels):
         assert torch.equal(dx, torch.full((5, 16), value))
 
 
+@pytest.mark.parametrize("offsets,keep", [(1, False), (1, True), (3, True)])
+@pytest.mark.parametrize("fn", FUNCTIONS)
+def test_meta_tensors(fn, offsets, keep):
+    """Shapes and types of a step, from the operators' fake implementations."""
+    x, w, y = _inputs("meta")
+    x, mtp = x.detach().bfloat16().requires_grad_(True), torch.ones(offsets, device="meta") if offsets > 1 else None
+    rest = (None, keep) if fn is ck.FusedNormSoftcappedCrossEntropy else (keep,)
+    loss = fn.apply(x, y, mtp, w, 0.02, 0.02, 1.0, 1.0, 15.0, "none", *rest)
+    assert loss.is_meta and loss.shape == (5,) and loss.dtype == torch.float32
+    loss.mean().backward()
+    assert x.grad.is_meta and x.grad.shape == x.shape and x.grad.dtype == torch.bfloat16
+    assert w.grad.is_meta and w.grad.shape == w.shape and w.grad.dtype == torch.float32
+    if offsets == 1:
+        assert fn.apply(x, y, None, w, 0.02, 0.02, 1.0, 1.0, 15.0, "mean", *rest).shape == ()
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("fn", FUNCTIONS)
 def test_batched_gradients_on_the_gpu(fn):
