@@ -991,8 +991,46 @@ __global__ __launch_bounds__(FEW_THREADS) void fwd_few_rows_kernel(FwdParams p, 
 }
 
 // What a block of COMBINE_ROWS rows contributes to the mean loss: left by fwd_combine_kernel in the first 16 bytes of the
-// block's own rows of the partial records (which it has consumed by then), summed by its last block:
+// block's own rows of the partial records (which it has consumed by then), summed by its last block or by fwd_reduce_kernel:
 //   8 bytes: sum of lse_i - z[i, y_i] over the valid rows (a double); 4: valid rows; 4: targets outside [0, V) other than ignore_index
+constexpr int COMBINE_ROWS = 64, MERGE_BLOCKS = 256;
+
+// n_valid, targets out of range and the mean from what the blocks left (of a single block: sum, cnt and bad as they are), in a fixed
+// order; a workgroup of COMBINE_ROWS * G threads.
+template <int G>
+__device__ __forceinline__ void finish_mean(const float4* partials, int nblk, double sum, int cnt, int bad, uint8_t* __restrict__ hdr,
+                                            float* __restrict__ loss_out, int32_t* __restrict__ nvalid_out, const CallMode& mode) {
+  if (nblk > 1) {
+    __shared__ double wsum[G];
+    __shared__ int wcnt[G], wbad[G];
+    const int r = threadIdx.x & 63, g = threadIdx.x >> 6;
+    sum = 0.0; cnt = 0; bad = 0;
+    for (int b = threadIdx.x; b < nblk; b += COMBINE_ROWS * G) {
+      const uint64_t* slot = reinterpret_cast<const uint64_t*>(partials + (int64_t)b * COMBINE_ROWS);
+      sum += __longlong_as_double((long long)__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      const uint64_t c = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      cnt += (int)(uint32_t)c; bad += (int)(uint32_t)(c >> 32);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) { sum += __shfl_xor(sum, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
+    if (r == 0) { wsum[g] = sum; wcnt[g] = cnt; wbad[g] = bad; }
+    __syncthreads();
+    if (threadIdx.x == 0)
+      for (int w = 1; w < G; ++w) { sum += wsum[w]; cnt += wcnt[w]; bad += wbad[w]; }
+  }
+  if (threadIdx.x != 0) return;
+  const float mean = (float)(sum / (double)cnt);                 // 0/0 = NaN, as F.cross_entropy gives
+  int32_t* head = reinterpret_cast<int32_t*>(hdr);
+  head[0] = cnt; head[1] = bad;
+  reinterpret_cast<float*>(hdr)[2] = mean;
+  *reinterpret_cast<CallMode*>(hdr + HDR_MODE_OFF) = mode;
+  if (loss_out) *loss_out = mean;
+  if (nvalid_out) { nvalid_out[0] = cnt; nvalid_out[1] = bad; }
+}
+__global__ __launch_bounds__(COMBINE_ROWS * 16) void fwd_reduce_kernel(const float4* __restrict__ partials, int nblk, uint8_t* __restrict__ hdr,
+                                                                      float* __restrict__ loss_out, int32_t* __restrict__ nvalid_out, CallMode mode) {
+  finish_mean<16>(partials, nblk, 0.0, 0, 0, hdr, loss_out, nvalid_out, mode);
+}
 
 // p(target) = exp(-loss), 0 for the rows without a target (fwd_combine_kernel forms it for sce_forward_probability).
 __device__ __forceinline__ float row_probability(float loss, int64_t target, int64_t ignore_index) { return target == ignore_index ? 0.f : expf(-loss); }
@@ -1010,12 +1048,14 @@ __global__ __launch_bounds__(256) void target_probability_kernel(const float* __
 // What bounds it is the chain of loads, not their volume: with one thread per row the records of a call of 61 rows and
 // 197 splits were 197 loads of one workgroup.  Rows beyond N have no records (fwd_few_rows_kernel writes none).  G = 4 for up to 16 splits, 16 beyond (rows too few to fill the chip
 // without cutting the vocabulary finer); the order of the sums depends on G alone.
-// The block that is done last adds up what all of them left: n_valid, targets out of range, the mean, in a fixed order.  The blocks'
-// sums and the count go past the L2 caches (agent scope: every XCD has its own), the sum before the count.  As a launch of one
-// workgroup (fwd_reduce_kernel, before) the same was 4.1 us of every forward call, and exp(-loss) for a caller that scores rows another 4.1: this kernel takes 2
-// to 2.6 us longer for both (7.1 for 4.5 + 4.1 at 2048 rows, 61 rows scored 56 -> 50 us in all).  A call of 64 rows at most that no backward
-// call follows is one block, which has nobody to wait for.
-constexpr int COMBINE_ROWS = 64;
+// Up to MERGE_BLOCKS blocks the one that is done last adds up what all of them left (finish_mean).  The blocks' sums and the count go past the
+// L2 caches (agent scope: every XCD has its own), the sum before the count.  One counter takes its arrivals one at a time, some 12 ns each, and a
+// block waits for its own stores before it arrives, so of more blocks the sum is a launch of one workgroup, fwd_reduce_kernel, which takes 4.7 us
+// whatever their number.  From the end of the forward kernel to the end of the mean, emitting, d = 256, V = 16384, merged and with the launch:
+// 64 blocks (4096 rows) 5.7 and 9.7 us, 192 7.9 and 9.8, 256 8.9 and 10.1, 320 10.6 and 10.9, 384 11.1 and 10.6, 512 12.9 and 11.2, 1024 21.7 and
+// 14.0; without dlogits 256 7.9 and 9.4, 384 9.6 and 9.3, 1024 18.5 and 9.7.
+// The probabilities of a caller that scores rows ride along (a launch of their own: 4 us).  A call of 64 rows at most that no
+// backward call follows is one block, which has nobody to wait for.
 template <int G>
 __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* __restrict__ partials, int S, int N, int Np, int V,
                                                          const int64_t* __restrict__ targets, int64_t ignore_index, float cap,
@@ -1095,8 +1135,10 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
           const uint64_t counts = (uint64_t)(uint32_t)cnt | ((uint64_t)(uint32_t)bad << 32);
           __hip_atomic_store(slot, (uint64_t)__double_as_longlong(sum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           __hip_atomic_store(slot + 1, counts, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // both have arrived
-          last = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hdr + HDR_COUNT_OFF), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+          if (gridDim.x <= MERGE_BLOCKS) {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // both have arrived
+            last = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(hdr + HDR_COUNT_OFF), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+          }
         }
       }
     }
@@ -1108,33 +1150,7 @@ __global__ __launch_bounds__(COMBINE_ROWS * G) void fwd_combine_kernel(float4* _
     losses[i] = l;
     if (probability) probability[i] = row_probability(l, targets[i], ignore_index);
   }
-  if (!last) return;
-  if (gridDim.x > 1) {
-    __shared__ double wsum[G];
-    __shared__ int wcnt[G], wbad[G];
-    sum = 0.0; cnt = 0; bad = 0;
-    for (int b = threadIdx.x; b < (int)gridDim.x; b += COMBINE_ROWS * G) {
-      const uint64_t* slot = reinterpret_cast<const uint64_t*>(partials + (int64_t)b * COMBINE_ROWS);
-      sum += __longlong_as_double((long long)__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-      const uint64_t c = __hip_atomic_load(slot + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      cnt += (int)(uint32_t)c; bad += (int)(uint32_t)(c >> 32);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) { sum += __shfl_xor(sum, o); cnt += __shfl_xor(cnt, o); bad += __shfl_xor(bad, o); }
-    if (r == 0) { wsum[g] = sum; wcnt[g] = cnt; wbad[g] = bad; }
-    __syncthreads();
-    if (threadIdx.x == 0)
-      for (int w = 1; w < G; ++w) { sum += wsum[w]; cnt += wcnt[w]; bad += wbad[w]; }
-  }
-  if (threadIdx.x != 0) return;
-  const float mean = (float)(sum / (double)cnt);                 // 0/0 = NaN, as F.cross_entropy gives
-  int32_t* head = reinterpret_cast<int32_t*>(hdr);
-  head[0] = cnt; head[1] = bad;
-  reinterpret_cast<float*>(hdr)[2] = mean;
-  *reinterpret_cast<CallMode*>(hdr + HDR_MODE_OFF) = mode;
-  if (loss_out) *loss_out = mean;
-  if (nvalid_out) { nvalid_out[0] = cnt; nvalid_out[1] = bad; }
+  if (last) finish_mean<G>(partials, gridDim.x, sum, cnt, bad, hdr, loss_out, nvalid_out, mode);
 }
-
 
 }  // namespace sce

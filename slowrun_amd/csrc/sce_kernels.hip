@@ -633,6 +633,9 @@ static int forward_impl(const sce_args* a, void* ws, size_t ws_bytes, const char
   };
   if (nsplit <= 16) combine(fwd_combine_kernel<4>, 4);
   else combine(fwd_combine_kernel<16>, 16);
+  if (nblk > MERGE_BLOCKS)
+    fwd_reduce_kernel<<<1, COMBINE_ROWS * 16, 0, st>>>(p.partials, nblk, p.hdr, a->reduction == SCE_REDUCE_MEAN ? a->loss : nullptr, a->n_valid,
+                                                       call_mode(emit, (int)Vl, a->shape.n_predict, a->cap));
   HIP_TRY(hipGetLastError());
   return SCE_OK;
 }
