@@ -818,9 +818,12 @@ extern "C" int sce_backward(const sce_args* a) {
   fold.longlist = longlist; fold.longbase = longbase; fold.segoff = segoff; fold.longsum = longsum; fold.dq = S.dq; fold.slots = (int)B.long_slots;
   const int fold_blocks = (int)std::min<int64_t>(NE / (LONG_CHUNK + 1) * (S.dq / 256), FOLD_GRID);      // (0: no column can have two chunks)
   bool folded = few_entries || fold_blocks == 0;      // launched, with the finishing kernel of a K-split dX panel or by itself
-  auto ensure_folded = [&]() {
+  auto ensure_folded = [&]() {         // (not within another timer: what it launches would be counted twice)
     ensure_summed();
-    if (!folded) bwd_dw_fold_kernel<<<fold_blocks, 256, 0, st>>>(fold);
+    if (!folded) {
+      KernelTimer tm(SCE_K_DW_FINAL, st);
+      bwd_dw_fold_kernel<<<fold_blocks, 256, 0, st>>>(fold);
+    }
     folded = true;
   };
   const int smem_dx = smem_scaled((int)(S.Vp / BK), SMEM_DX);
@@ -875,9 +878,9 @@ extern "C" int sce_backward(const sce_args* a) {
     wp.xt = xt; wp.ghat_t = ghat_t + ((w0 - gorg) / 256) * (S.Vp / BK) * BLOCKED_KSTEP; wp.gexp = gexp + (w0 - gorg) / BK; wp.dwacc = (float*)((uint8_t*)dwacc + (size_t)part * B.part_stride);
     wp.kbn = S.Np / BK; wp.kbw = gkb; wp.kb0 = w0 / BK; wp.Vp = S.Vp; wp.kbv = S.Vp / BK;
     wp.RT = CTd; wp.CT = CTv; wp.KT = (int)(gathered / BK);
+    if (B.one) ensure_folded();
     {
       KernelTimer tm(SCE_K_DW, st);
-      if (B.one) ensure_folded();
       // When this launch is the only one and its last round of tiles would leave many CUs idle, that round is
       // shared out along K instead (bwd_dw_tail_kernel): the full rounds run as they are.
       const DwTailPlan tp = dw_tail_plan(S.dq, S.Vp, gathered);
@@ -941,8 +944,8 @@ extern "C" int sce_backward(const sce_args* a) {
     else rmsnorm_backward_kernel<bf16_t, bf16_t><<<ngrid, 256, 0, st>>>((bf16_t*)a->dx, a->dx_ld, (const bf16_t*)a->x, a->x_ld, rstd, N, d);
   }
   if (!dw_done || tail.tile0 >= 0) {
-    KernelTimer tm_fin(SCE_K_DW_FINAL, st);
     ensure_folded();
+    KernelTimer tm_fin(SCE_K_DW_FINAL, st);
     const dim3 g = dw_done ? dim3(16, (unsigned)tail.ntail) : dim3((unsigned)((V + 63) / 64), (unsigned)((d + 63) / 64));
     const int np = launch < nparts ? launch : nparts;
     if (dw_f32) bwd_dw_final_kernel<float><<<g, 256, 0, st>>>(dwacc, np, (int64_t)(B.part_stride / 4), S.Vp, wo, tail, CTd, CTv);

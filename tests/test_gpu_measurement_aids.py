@@ -45,3 +45,29 @@ def test_shapes_the_kernels_do_not_take_are_refused():
     assert b"random_bytes" in lib.sce_last_error()
     assert lib.sce_bench_gemm(a.data_ptr(), a.data_ptr(), 4096, 4096, 1024, 1, scratch.data_ptr(), 16, scratch.device.index, None,
                               C.byref(tf), C.byref(mhz)) == 1                                                       # scratch too small
+
+
+def test_no_launch_is_counted_twice():
+    """The times by kind of a backward pass add up to no more than the pass.  Few rows with the same target and a wide hidden state: the sum of that
+    column's rows, which only dW waits for, is a good part of the whole."""
+    from slowrun_amd import cuda_kernels as ck
+    N, d, V = 4096, 65536, 256
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn(N, d, device="cuda", generator=gen, dtype=torch.bfloat16)
+    w = torch.randn(d, V, device="cuda", generator=gen, dtype=torch.bfloat16) * d ** -0.5
+    y = torch.full((N,), 7, device="cuda")
+    _loss, saved, *_ = ck.ce_forward(x, w, y, 0.02, 0.02 * d ** -0.5, 15.0, "mean", keep_dlogits=True)
+    back = lambda: ck.ce_backward(saved, y, torch.ones((), device="cuda"), N, d, V, 0.02, 0.02 * d ** -0.5, 15.0, 1.0, "mean", torch.bfloat16, torch.bfloat16,
+                                  keep_dlogits=True)
+    back()
+    begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    _lib.timing_enable(True)
+    try:
+        begin.record()
+        back()
+        end.record()
+        kinds = _lib.timing_read()
+    finally:
+        _lib.timing_enable(False)
+    assert kinds["dw_final"][1] >= 1 and kinds["dw"][1] == 1
+    assert sum(ms for ms, _launches in kinds.values()) <= begin.elapsed_time(end) + 0.002      # (the clock of the time stamps: 10 ns a tick)
