@@ -995,8 +995,8 @@ __device__ __forceinline__ int long_parts(const DwOut& o, int L) {
 // The epilogue must not wait on memory: one wave per SIMD has nothing to hide a load behind (gathering the one-hot rows
 // with dependent loads was measured at +0.5 ms of a 20 ms step).  So the rows X_q[i] of the tile's target entries -- the
 // short columns' only; columns with LONG_SEG or more entries have their sums ready -- go to LDS with direct loads:
-// before the main loop, into what the K slots and the block exponents leave free (100 to 112 entries of 256 bytes), if they
-// fit there -- all tiles' do of 16384 rows with uniform targets over 50257 columns, four fifths of the tiles' of 65536
+// before the main loop, into what the K slots and the block exponents leave free (100 to 112 entries of 256 bytes; of a half tile an entry
+// is 128 bytes, everywhere), if they fit there -- all tiles' do of 16384 rows with uniform targets over 50257 columns, four fifths of the tiles' of 65536
 // rows with Zipf targets, next to none of 26400 uniform ones -- and otherwise into the K slots after it, as many row blocks at a
 // time as fit (a row block's 64 columns have at most 64 (LONG_SEG - 1) = 448 entries).  Each lane then walks the entries of its own
 // column.  A 16-byte chunk c of an entry's 256 bytes lies at position c ^ (entry & 15): the lanes of a wave read the same
@@ -1006,7 +1006,7 @@ __device__ __forceinline__ int long_parts(const DwOut& o, int L) {
 constexpr int DWO_AUX = 2 * 260 * 4;                         // entry offsets and segment starts of the tile's 256 columns
 constexpr int DWO_STAGE_PITCH = 64 * 2 + 16, DWO_STAGE = 32 * DWO_STAGE_PITCH;      // per wave
 constexpr int DWO_GROUP = 480;                               // entries that the K slots hold (256 bytes of X_q, row and coefficient each)
-static_assert(DWO_GROUP * (256 + 8) <= SMEM_BYTES && DWO_GROUP >= 64 * (LONG_SEG - 1) && DWO_GROUP % 4 == 0, "a row block's entries must fit the K slots");
+static_assert(DWO_GROUP * (256 + 8) <= SMEM_BYTES && DWO_GROUP >= 64 * (LONG_SEG - 1), "a row block's entries must fit the K slots");
 constexpr int DWO_MAX_KT = 131072 / BK;
 static_assert(SMEM_MAX - SMEM_BYTES - 8 * DWO_MAX_KT - DWO_AUX >= 4 * DWO_STAGE, "no room for the staging tiles beside the K slots");
 
@@ -1014,6 +1014,7 @@ static_assert(SMEM_MAX - SMEM_BYTES - 8 * DWO_MAX_KT - DWO_AUX >= 4 * DWO_STAGE,
 template <typename T, int NA>
 __device__ __forceinline__ void dw_out_tile(const DwParams& p, const DwOut& o, uint8_t* smem, int rt, int ct) {
   constexpr int TROWS = 64 * NA, EB = TROWS, CHUNKS = EB / 16;               // rows of dW in the tile = bytes of X_q of an entry
+  static_assert(DWO_GROUP % (64 / CHUNKS) == 0, "load_rows fills up its last load: beyond the group lie the entries' rows and coefficients");
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wa = wave >> 1, wb = wave & 1;
   const int KT = p.KT;
   uint32_t* lsc = reinterpret_cast<uint32_t*>(smem + SMEM_BYTES);            // block exponents of the K loop: [v half][K block]
