@@ -77,6 +77,25 @@ def test_target_probability_is_the_exponential_of_the_losses(n, shape):
     assert p.shape == losses.shape and torch.allclose(p, torch.where(y == -1, torch.zeros_like(losses), torch.exp(-losses)), rtol=1e-6, atol=0)
 
 
+@pytest.mark.parametrize("operands", ["bf16", "e4m3"])
+@pytest.mark.parametrize("N", [1, 61, 300, 16640])
+def test_both_entry_points_give_the_same_probabilities(operands, N):
+    """sce_forward_probability, which target_probability calls, and sce_target_probability of the losses of a call of its own: the same bits."""
+    from slowrun_amd import _lib, cuda_kernels as ck
+    gen = torch.Generator(device="cuda").manual_seed(N)
+    x = torch.randn(N, 64, device="cuda", generator=gen).bfloat16()
+    w = (torch.randn(64, 264, device="cuda", generator=gen) / 8).bfloat16()
+    y = torch.randint(0, 264, (N,), device="cuda", generator=gen)
+    y[::7], y[N // 2] = -1, 264 if N > 1 else 5                 # (a target out of range: NaN, or whatever its loss gives)
+    ops = dict(operand_dtype=torch.bfloat16) if operands == "bf16" else dict(x_s=0.02, w_s=0.002)
+    losses = ck.softcapped_cross_entropy(x, w, y, reduction="none", **ops)
+    got = torch.full((N,), -1.0, device="cuda")
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    assert lib.sce_target_probability(losses.data_ptr(), y.data_ptr(), N, -1, got.data_ptr(), 0, stream) == 0
+    want = ck.target_probability(x, w, y, **ops)
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32)) and bool((got[y == -1] == 0).all()) and bool((got[(y >= 0) & (y < 264)] > 0).all())
+
+
 @pytest.mark.parametrize("N,d,V", [(3, 48, 264), (64, 64, 2056), (128, 96, 520), (200, 32, 33000)])
 def test_infinities_and_nan_of_few_rows_as_in_the_general_path(N, d, V):
     """Rows with an infinity, a NaN, a largest finite value, and a column of W with each: the few-rows kernel gives what the general
