@@ -35,14 +35,17 @@ namespace sce {
 //     block; ldL = the rest of the next block's loads.  The wait that publishes a block comes at b2 of the block before.
 // The four waves of a workgroup run in step and share the compute unit's one path from L2 (64 bytes a clock: 16 clocks
 // for a wave's 1 KB load), so one load per wave and 64-clock MFMA slot already fills that path while it lasts.  What
-// costs is a slot that has both a load and fragment reads: both end in LDS, and the reads of the four waves (8 KB a slot)
-// then wait for the loads' 4 KB.  So a block's slots are four groups of eight: loads, reads, loads, reads.  The loads of the
+// costs is a slot that has both a load and fragment reads.  So a block's slots are four groups of eight: loads, reads, loads, reads.  The loads of the
 // third group go into this block's own LDS slot, behind an extra barrier that waits for the second group's reads; that
 // barrier comes a slot after the last of them, when they have landed, which leaves one load for the fourth group.
 // Measured against the schedule before it (reads in the second half of each sub-step too, but eight of the loads in the
 // slots with reads, no extra barrier), two builds in turn on one card, whole steps: 2048 rows of d = 768 476 -> 466 us, two
 // micro-batches of 2048 rows of d = 1024 974 -> 952, 4096 rows of d = 1600 1194 -> 1154, 32768 rows of d = 1024 4824 -> 4673,
-// 65536 rows of d = 2560 19370 -> 19170, the bf16 eval pass the same.  Also measured: six or more loads in slots with reads
+// 65536 rows of d = 2560 19370 -> 19170, the bf16 eval pass the same.  By the counters of the last of these, forward, dX and dW: the
+// matrix units are busy 57.3 -> 61.5, 80.7 -> 84.0 and 83.6 -> 87.2 % of the clocks (the clock falls, within the card's power, which takes most of it back), and the waves
+// wait to issue an instruction for 49.5 -> 44.9, 60.7 -> 57.1 and 59.1 -> 55.1 % of theirs.  It is not LDS instructions that wait to be issued
+// (2.1 -> 2.9, 0.2 -> 0.3, 0.7 -> 1.4 %), nor is less spent at the wait instructions (10.7 -> 11.3, 13.0 -> 14.3, 12.3 -> 13.6 %): MFMAs and loads are held
+// up less.  Also measured: six or more loads in slots with reads
 // (1 % slower than this), all loads as early as their LDS slot is free (2 %), one barrier and a load and a read in every slot
 // of the second half (2 to 4 %), the extra barrier right behind the last read (0 to 0.5 %), reads three to a slot (0.5 %), two loads
 // of a wave in one slot (5 to 10 %).
