@@ -305,22 +305,6 @@ def _seen_as_op(*tensors):
     return False
 
 
-def _call_op(op, body, tensors, *args):
-    """op(*args), or body(*args) where nothing would see the difference; `tensors`: the arguments that are tensors or None.
-    What records function calls without the profiler (an execution trace observer) cannot be asked for: it is given the call under the
-    operator's name."""
-    if _seen_as_op(*tensors):
-        return op(*args)
-    record = _record_enter(op._qualname, *args)
-    try:
-        return body(*args)
-    finally:
-        _record_exit(record)
-
-
-_record_enter, _record_exit = torch.autograd._record_function_with_args_enter, torch.autograd._record_function_with_args_exit
-
-
 def _plain_keys():
     plain = _dispatch_keys(torch.empty(0, device="cpu"))
     for name in ("CUDA", "AutogradCUDA", "AutocastCUDA"):
@@ -423,8 +407,8 @@ class FusedSoftcappedCrossEntropy(torch.autograd.Function):
         (xs, xst), (ws_, wst) = _split_scale(xs), _split_scale(ws_)
         keep = bool(KEEP_DLOGITS if keep_dlogits is None else keep_dlogits)
         xd, wd = x.detach(), lm_head_weight.detach()
-        out, saved = _call_op(ce_forward_op, _ce_forward_body, (xd, wd, targets, mtp_weights, xst, wst),
-                              xd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", keep, xst, wst)
+        call = ce_forward_op if _seen_as_op(xd, wd, targets, mtp_weights, xst, wst) else _ce_forward_body
+        out, saved = call(xd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", keep, xst, wst)
         ctx.scale_tensors = (xst, wst)
         ctx.save_for_backward(saved, targets, mtp_weights if mtp_weights is not None else torch.empty(0, device=x.device))
         ctx.params = (x.shape[0], x.shape[1], lm_head_weight.shape[1], xs, ws_, float(cap), float(grad_scale),
@@ -437,8 +421,8 @@ class FusedSoftcappedCrossEntropy(torch.autograd.Function):
         saved, targets, mtp_w = ctx.saved_tensors
         N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, has_mtp, keep = ctx.params
         go, mtp_w = grad_output.contiguous(), mtp_w if has_mtp else None
-        dx, dw = _call_op(ce_backward_op, _ce_backward_body, (saved, targets, go, mtp_w, *ctx.scale_tensors),
-                          saved, targets, go, mtp_w, N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, keep, *ctx.scale_tensors)
+        call = ce_backward_op if _seen_as_op(saved, targets, go, mtp_w, *ctx.scale_tensors) else _ce_backward_body
+        dx, dw = call(saved, targets, go, mtp_w, N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, keep, *ctx.scale_tensors)
         return dx, None, None, dw, None, None, None, None, None, None, None
 
 
@@ -460,8 +444,8 @@ class FusedNormSoftcappedCrossEntropy(torch.autograd.Function):
         (xs, xst), (ws_, wst) = _split_scale(xs), _split_scale(ws_)
         hd, wd = h.detach(), lm_head_weight.detach()
         keep = bool(KEEP_DLOGITS if keep_dlogits is None else keep_dlogits)
-        out, saved = _call_op(norm_ce_forward_op, _norm_ce_forward_body, (hd, wd, targets, mtp_weights, xst, wst),
-                              hd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", eps, keep, xst, wst)
+        call = norm_ce_forward_op if _seen_as_op(hd, wd, targets, mtp_weights, xst, wst) else _norm_ce_forward_body
+        out, saved = call(hd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", eps, keep, xst, wst)
         ctx.scale_tensors = (xst, wst)
         ctx.save_for_backward(saved, hd, targets, mtp_weights if mtp_weights is not None else torch.empty(0, device=h.device))
         ctx.params = (lm_head_weight.shape[1], xs, ws_, float(cap), float(grad_scale), reduction == "mean",
@@ -473,8 +457,8 @@ class FusedNormSoftcappedCrossEntropy(torch.autograd.Function):
         saved, h, targets, mtp_w = ctx.saved_tensors
         V, xs, ws_, cap, gscale, mean, w_bf16, has_mtp, eps, keep = ctx.params
         go, mtp_w = grad_output.contiguous(), mtp_w if has_mtp else None
-        dh, dw = _call_op(norm_ce_backward_op, _norm_ce_backward_body, (saved, h, targets, go, mtp_w, *ctx.scale_tensors),
-                          saved, h, targets, go, mtp_w, V, xs, ws_, cap, gscale, mean, w_bf16, eps, keep, *ctx.scale_tensors)
+        call = norm_ce_backward_op if _seen_as_op(saved, h, targets, go, mtp_w, *ctx.scale_tensors) else _norm_ce_backward_body
+        dh, dw = call(saved, h, targets, go, mtp_w, V, xs, ws_, cap, gscale, mean, w_bf16, eps, keep, *ctx.scale_tensors)
         return dh, None, None, dw, None, None, None, None, None, None, None, None
 
 
