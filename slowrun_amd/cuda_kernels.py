@@ -284,37 +284,46 @@ def ce_backward(saved, targets, grad_output, N, d, V, x_s, w_s, cap, grad_scale,
 # as two opaque calls instead of breaking the graph; the reference wraps its kernel the same way
 # (tiny/cuda_kernels.py:314).  The fake implementations only describe shapes and dtypes.
 #
-# A custom op written in Python costs 17 us of host time a call on its way through the dispatcher, and a step of 1000 rows, d = 256,
-# V = 4096 has 89 us of kernels and waits for the host.  So the autograd functions below call the body itself where nothing would see the
-# op: that step 206 -> 183 us.
+# A custom op written in Python costs 17 us of host time a call on its way through the dispatcher, most of it in two layers of Python around its
+# body: autograd's, which without grad mode only passes the call on, and a check for outputs that alias inputs.  A step of 1000 rows, d = 256,
+# V = 4096 has 89 us of kernels and waits for the host.  So on the GPU the body itself is the op's kernel, and the autograd functions below, which run
+# without grad mode, call the op below its autograd layer: that step 203 -> 188 us (179 with the body called without the dispatcher, which
+# batched gradients, negated views, meta tensors and execution traces would have to be told from plain calls for).
 # ---------------------------------------------------------------------------------------------
+_is_compiling, _is_tracing, _is_grad_enabled = torch.compiler.is_compiling, torch._C._is_tracing, torch.is_grad_enabled
+_dispatch_modes, _function_modes, _functorch_active = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack, torch._C._are_functorch_transforms_active
+_profiler_enabled, _Tensor, _Parameter = torch._C._autograd._profiler_enabled, torch.Tensor, torch.nn.Parameter
+
+
 def _seen_as_op(*tensors):
-    """Whether a call must go through the dispatcher: something traces, records or transforms calls (torch.compile, jit tracing, dispatch
-    and function modes, functorch, the profiler, autograd of a backward pass), or an argument is no plain tensor: a subclass, a type that
-    the op's schema refuses, or a tensor that the dispatcher would turn into another before the body sees it (batched gradients without
-    functorch, negation left to be done, zeros without memory) or answer without it (meta tensors)."""
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch.is_grad_enabled():
-        return True
-    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack() or torch._C._are_functorch_transforms_active():
-        return True
-    if torch._C._autograd._profiler_enabled():
+    """Whether a call must go through the whole dispatcher: something traces, records or transforms calls (torch.compile, jit tracing, dispatch
+    and function modes, functorch, the profiler, autograd of a backward pass), or an argument is no tensor of torch's own (a subclass, or a type
+    that the op's schema refuses)."""
+    if _is_compiling() or _is_tracing() or _is_grad_enabled() or _dispatch_modes() or _function_modes() or _functorch_active() or _profiler_enabled():
         return True
     for t in tensors:
-        if t is not None and ((type(t) is not torch.Tensor and type(t) is not torch.nn.Parameter) or _dispatch_keys(t).raw_repr() & _SPECIAL_KEYS):
+        if t is not None and type(t) is not _Tensor and type(t) is not _Parameter:
             return True
     return False
 
 
-def _plain_keys():
-    plain = _dispatch_keys(torch.empty(0, device="cpu"))
-    for name in ("CUDA", "AutogradCUDA", "AutocastCUDA"):
-        plain = plain | torch._C.DispatchKeySet(torch._C._dispatch_key_parse(name))
-    return plain.raw_repr()
+def _call_op(op, tensors, *args):
+    """op(*args), below the op's autograd layer where that has nothing to do; `tensors`: the arguments that are tensors or None."""
+    if _seen_as_op(*tensors):
+        return op(*args)
+    with torch._C._AutoDispatchBelowADInplaceOrView():
+        return _OVERLOADS[op](*args)
 
 
-# All dispatch keys but those that a tensor has for being dense, on the GPU (or the CPU: the body refuses it), and open to autograd and autocast.
-_dispatch_keys = torch._C._dispatch_keys
-_SPECIAL_KEYS = ~_plain_keys()
+_OVERLOADS = {}
+_GPU_KERNELS = torch.library.Library("slowrun_amd", "IMPL")
+
+
+def _register(name, body):
+    op = torch.library.custom_op(f"slowrun_amd::{name}", body, mutates_args=())
+    _GPU_KERNELS.impl(name, body, "CUDA")
+    _OVERLOADS[op] = getattr(torch.ops.slowrun_amd, name).default
+    return op
 
 
 def _ce_forward_body(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor, mtp_weights: Optional[torch.Tensor],
@@ -325,7 +334,7 @@ def _ce_forward_body(x: torch.Tensor, w: torch.Tensor, targets: torch.Tensor, mt
     return out, saved
 
 
-ce_forward_op = torch.library.custom_op("slowrun_amd::ce_forward", _ce_forward_body, mutates_args=())
+ce_forward_op = _register("ce_forward", _ce_forward_body)
 
 
 @ce_forward_op.register_fake
@@ -348,7 +357,7 @@ def _ce_backward_body(saved: torch.Tensor, targets: torch.Tensor, grad_output: t
                        mtp_weights=mtp_weights, keep_dlogits=keep)
 
 
-ce_backward_op = torch.library.custom_op("slowrun_amd::ce_backward", _ce_backward_body, mutates_args=())
+ce_backward_op = _register("ce_backward", _ce_backward_body)
 
 
 @ce_backward_op.register_fake
@@ -366,7 +375,7 @@ def _norm_ce_forward_body(h: torch.Tensor, w: torch.Tensor, targets: torch.Tenso
     return out, saved
 
 
-norm_ce_forward_op = torch.library.custom_op("slowrun_amd::norm_ce_forward", _norm_ce_forward_body, mutates_args=())
+norm_ce_forward_op = _register("norm_ce_forward", _norm_ce_forward_body)
 
 
 norm_ce_forward_op.register_fake(lambda h, w, targets, mtp_weights, x_s, w_s, cap, mean, eps, keep, x_s_t=None, w_s_t=None:
@@ -384,7 +393,7 @@ def _norm_ce_backward_body(saved: torch.Tensor, h: torch.Tensor, targets: torch.
                        keep_dlogits=keep)
 
 
-norm_ce_backward_op = torch.library.custom_op("slowrun_amd::norm_ce_backward", _norm_ce_backward_body, mutates_args=())
+norm_ce_backward_op = _register("norm_ce_backward", _norm_ce_backward_body)
 
 
 @norm_ce_backward_op.register_fake
@@ -407,8 +416,8 @@ class FusedSoftcappedCrossEntropy(torch.autograd.Function):
         (xs, xst), (ws_, wst) = _split_scale(xs), _split_scale(ws_)
         keep = bool(KEEP_DLOGITS if keep_dlogits is None else keep_dlogits)
         xd, wd = x.detach(), lm_head_weight.detach()
-        call = ce_forward_op if _seen_as_op(xd, wd, targets, mtp_weights, xst, wst) else _ce_forward_body
-        out, saved = call(xd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", keep, xst, wst)
+        out, saved = _call_op(ce_forward_op, (xd, wd, targets, mtp_weights, xst, wst),
+                              xd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", keep, xst, wst)
         ctx.scale_tensors = (xst, wst)
         ctx.save_for_backward(saved, targets, mtp_weights if mtp_weights is not None else torch.empty(0, device=x.device))
         ctx.params = (x.shape[0], x.shape[1], lm_head_weight.shape[1], xs, ws_, float(cap), float(grad_scale),
@@ -421,8 +430,8 @@ class FusedSoftcappedCrossEntropy(torch.autograd.Function):
         saved, targets, mtp_w = ctx.saved_tensors
         N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, has_mtp, keep = ctx.params
         go, mtp_w = grad_output.contiguous(), mtp_w if has_mtp else None
-        call = ce_backward_op if _seen_as_op(saved, targets, go, mtp_w, *ctx.scale_tensors) else _ce_backward_body
-        dx, dw = call(saved, targets, go, mtp_w, N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, keep, *ctx.scale_tensors)
+        dx, dw = _call_op(ce_backward_op, (saved, targets, go, mtp_w, *ctx.scale_tensors),
+                          saved, targets, go, mtp_w, N, d, V, xs, ws_, cap, gscale, mean, x_bf16, w_bf16, keep, *ctx.scale_tensors)
         return dx, None, None, dw, None, None, None, None, None, None, None
 
 
@@ -444,8 +453,8 @@ class FusedNormSoftcappedCrossEntropy(torch.autograd.Function):
         (xs, xst), (ws_, wst) = _split_scale(xs), _split_scale(ws_)
         hd, wd = h.detach(), lm_head_weight.detach()
         keep = bool(KEEP_DLOGITS if keep_dlogits is None else keep_dlogits)
-        call = norm_ce_forward_op if _seen_as_op(hd, wd, targets, mtp_weights, xst, wst) else _norm_ce_forward_body
-        out, saved = call(hd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", eps, keep, xst, wst)
+        out, saved = _call_op(norm_ce_forward_op, (hd, wd, targets, mtp_weights, xst, wst),
+                              hd, wd, targets, mtp_weights, xs, ws_, float(cap), reduction == "mean", eps, keep, xst, wst)
         ctx.scale_tensors = (xst, wst)
         ctx.save_for_backward(saved, hd, targets, mtp_weights if mtp_weights is not None else torch.empty(0, device=h.device))
         ctx.params = (lm_head_weight.shape[1], xs, ws_, float(cap), float(grad_scale), reduction == "mean",
@@ -457,8 +466,8 @@ class FusedNormSoftcappedCrossEntropy(torch.autograd.Function):
         saved, h, targets, mtp_w = ctx.saved_tensors
         V, xs, ws_, cap, gscale, mean, w_bf16, has_mtp, eps, keep = ctx.params
         go, mtp_w = grad_output.contiguous(), mtp_w if has_mtp else None
-        call = norm_ce_backward_op if _seen_as_op(saved, h, targets, go, mtp_w, *ctx.scale_tensors) else _norm_ce_backward_body
-        dh, dw = call(saved, h, targets, go, mtp_w, V, xs, ws_, cap, gscale, mean, w_bf16, eps, keep, *ctx.scale_tensors)
+        dh, dw = _call_op(norm_ce_backward_op, (saved, h, targets, go, mtp_w, *ctx.scale_tensors),
+                          saved, h, targets, go, mtp_w, V, xs, ws_, cap, gscale, mean, w_bf16, eps, keep, *ctx.scale_tensors)
         return dh, None, None, dw, None, None, None, None, None, None, None, None
 
 

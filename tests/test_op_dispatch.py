@@ -1,5 +1,7 @@
 """When the autograd functions call the loss head as an operator and when they call its body: whatever traces, records or transforms
 operator calls still meets the operator."""
+import json
+
 import pytest
 import torch
 from torch.utils._python_dispatch import TorchDispatchMode
@@ -100,6 +102,21 @@ def test_meta_tensors(fn, offsets, keep):
     assert w.grad.is_meta and w.grad.shape == w.shape and w.grad.dtype == torch.float32
     if offsets == 1:
         assert fn.apply(x, y, None, w, 0.02, 0.02, 1.0, 1.0, 15.0, "mean", *rest).shape == ()
+
+
+@pytest.mark.parametrize("fn", FUNCTIONS)
+def test_execution_trace_without_the_profiler(fn, cpu_kernels, tmp_path):
+    path = str(tmp_path / "trace.json")
+    observer = torch.profiler.ExecutionTraceObserver().register_callback(path)
+    observer.start()
+    x, w, y = _inputs()
+    _apply(fn, x, w, y).backward()
+    observer.stop()
+    observer.unregister_callback()
+    with open(path) as f:
+        names = [node["name"] for node in json.load(f)["nodes"]]
+    prefix = "slowrun_amd::norm_ce_" if fn is ck.FusedNormSoftcappedCrossEntropy else "slowrun_amd::ce_"
+    assert names.count(prefix + "forward") == 1 and names.count(prefix + "backward") == 1
 
 
 @pytest.mark.gpu
