@@ -1049,7 +1049,7 @@ __global__ __launch_bounds__(256) void target_probability_kernel(const float* __
 // 197 splits were 197 loads of one workgroup.  Rows beyond N have no records (fwd_few_rows_kernel writes none).  G = 4 for up to 16 splits, 16 beyond (rows too few to fill the chip
 // without cutting the vocabulary finer); the order of the sums depends on G alone.
 // Up to MERGE_BLOCKS blocks the one that is done last adds up what all of them left (finish_mean).  The blocks' sums and the count go past the
-// L2 caches (agent scope: every XCD has its own), the sum before the count.  One counter takes its arrivals one at a time, some 12 ns each, and a
+// L2 caches (agent scope: every XCD has its own), the sum before the count.  One counter takes its arrivals one at a time, some 15 ns each, and a
 // block waits for its own stores before it arrives, so of more blocks the sum is a launch of one workgroup, fwd_reduce_kernel, which takes 4.7 us
 // whatever their number.  From the end of the forward kernel to the end of the mean, emitting, d = 256, V = 16384, merged and with the launch:
 // 64 blocks (4096 rows) 5.7 and 9.7 us, 192 7.9 and 9.8, 256 8.9 and 10.1, 320 10.6 and 10.9, 384 11.1 and 10.6, 512 12.9 and 11.2, 1024 21.7 and
